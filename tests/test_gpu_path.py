@@ -1,0 +1,77 @@
+"""Plain launches (vzLaunch, the persistent path kernels) at the edges of
+their tiles, units and chunks, bit for bit against the CPU oracle; a frame of
+more passes than one chunk holds against the megakernel."""
+import sys
+
+import numpy as np
+import pytest
+
+import oracle as O
+from util import GpuTarget, book_lookat, box_lookat, gpu_params, oracle_params
+from venusaur_amd import api
+
+pytestmark = pytest.mark.gpu
+
+
+def say(*a):
+    print(*a, flush=True)
+    sys.stdout.flush()
+
+
+def _scene(kind, book):
+    if kind == "book":
+        return book, book_lookat
+    if kind == "one":  # a single sphere: no tree
+        s, m = api.box_scene(1, 4)
+        return (s[1:].copy(), m[1:].copy()), box_lookat
+    n = {"lds": 500, "mem": 700}[kind]  # either side of the tree size staged in LDS
+    return api.box_scene(n, 9), box_lookat
+
+
+# smaller than a tile, exactly one, one pixel more, each tile shape, odd
+# sizes; passes below, at and above a unit's 8, and not a multiple of it
+@pytest.mark.parametrize("kind,w,h,spp,depth", [
+    ("book", 2, 2, 1, 50), ("book", 7, 3, 9, 8), ("book", 3, 41, 2, 4), ("book", 8, 8, 8, 50),
+    ("book", 9, 7, 17, 3), ("book", 65, 33, 3, 1), ("book", 131, 67, 5, 50), ("one", 16, 9, 3, 6),
+    ("lds", 33, 17, 7, 16), ("mem", 33, 17, 7, 16), ("mem", 2, 64, 12, 255)])
+@pytest.mark.parametrize("fp64", [False, True])
+def test_launch_edges(ctx, book, kind, w, h, spp, depth, fp64):
+    say(f"case: plain launch {kind} {w}x{h} spp={spp} depth={depth} fp64={fp64}")
+    (s, m), look = _scene(kind, book)
+    cam = look(w, h)
+    sc = api.Scene(ctx, s, m)
+    tgt = GpuTarget(w, h, fp64=fp64)
+    ob = O.BVH(s)
+    want = None
+    for frame in (1, 2):
+        p = gpu_params(w, h, spp, depth, cam, subframe=frame, flags=api.ACCUM_FP64 if fp64 else 0)
+        st = sc.launch(tgt.bind(p))
+        want, img, ost = O.render(s, m, oracle_params(w, h, spp, depth, cam, subframe=frame, accum_fp64=fp64), bvh=ob,
+                                  accum=want)
+        assert np.array_equal(tgt.accum_host(), want), frame
+        assert np.abs(tgt.image_host().astype(int) - img.astype(int)).max() <= 1
+        assert (st.segments, st.hits, st.paths) == (ost.segments, ost.hits, w * h * spp)
+    p.flags |= api.COUNT_VISITS
+    p.subframe_index = 1
+    st = sc.launch(p)
+    _, _, ost = O.render(s, m, oracle_params(w, h, spp, depth, cam), bvh=ob)
+    assert (st.segments, st.node_visits, st.sphere_tests) == (ost.segments, ost.node_visits, ost.sphere_tests)
+    sc.close()
+
+
+@pytest.mark.parametrize("fp64", [False, True])
+def test_launch_of_several_chunks(ctx, book, fp64):
+    """2048x2048 holds 64 passes in a chunk: 131 passes are three chunks whose
+    sums and camera seeds carry over, the last one shorter."""
+    say(f"case: plain launch of several chunks fp64={fp64}")
+    s, m = book
+    sc = api.Scene(ctx, s, m)
+    out = []
+    flags = api.ACCUM_FP64 if fp64 else 0
+    for extra in (0, api.MEGAKERNEL):
+        tgt = GpuTarget(2048, 2048, fp64=fp64)
+        st = sc.launch(tgt.bind(gpu_params(2048, 2048, 131, 2, book_lookat(2048, 2048), flags=flags | extra)))
+        out.append((st.segments, st.paths, tgt.accum_host(), tgt.image_host()))
+    assert out[0][:2] == out[1][:2]
+    assert np.array_equal(out[0][2], out[1][2]) and np.array_equal(out[0][3], out[1][3])
+    sc.close()

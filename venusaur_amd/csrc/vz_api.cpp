@@ -12,6 +12,7 @@
 
 #include "vz_engine.h"
 #include "vz_internal.h"
+#include "vz_path.h"
 
 namespace vz {
 
@@ -79,24 +80,6 @@ static void adopt_cached_tuning(vzContext ctx)
         ctx->tuning = it->second;
         ctx->tuned = true;
     }
-}
-
-static vzStatus get_engine(vzContext ctx, Engine** out)
-{
-    if (!ctx->engine) {
-        EngineConfig cfg;
-        adopt_cached_tuning(ctx);
-        if (ctx->tuned) {
-            cfg.queue_capacity = ctx->tuning.queue_capacity;
-            cfg.tile_w = ctx->tuning.tile_w;
-            cfg.tile_h = ctx->tuning.tile_h;
-            cfg.iters_per_graph = ctx->tuning.iters_per_graph;
-            cfg.refill_lanes = ctx->tuning.refill_lanes;
-        }
-        VZ_TRY(engine_create(ctx, cfg, &ctx->engine));
-    }
-    *out = ctx->engine;
-    return VZ_SUCCESS;
 }
 
 struct DevCounters {   // per-call counters for the non-engine kernels
@@ -168,6 +151,7 @@ vzStatus vzDestroy(vzContext ctx)
     (void)hipSetDevice(ctx->device);
     (void)hipDeviceSynchronize();
     if (ctx->engine) engine_destroy(ctx->engine);
+    path_free(ctx->path);
     delete ctx;
     return VZ_SUCCESS;
 }
@@ -462,27 +446,8 @@ vzStatus vzLaunch(vzScene scene, const vzLaunchParams* params, vzStream stream, 
         }
         return VZ_SUCCESS;
     }
-    Engine* e = nullptr;
-    VZ_TRY(get_engine(ctx, &e));
-    std::vector<RunItem> items(1);
-    items[0].scene = scene;
-    items[0].params = *params;
-    RunOptions opt;
-    opt.use_graph = false;
-    opt.count_visits = (params->flags & VZ_COUNT_VISITS) != 0;
-    opt.time_trace = (params->flags & VZ_TIME_STAGES) != 0;
-    // Rays in flight for one request: four image passes, at least 1M, at
-    // most the queue.  Measured on MI355X (same box, plain launches one after
-    // another): a 120-request mix of the serving distribution 2345 against
-    // 1929 Mray-segments/s with the whole 8M queue in use, the 64-scene batch
-    // mix 2106 against 1998; 1080p frames fill the 8M queue either way (book
-    // scene 11.2 Gray-segments/s).  Six passes, or two and three (which also
-    // cut 1080p below 8M), were slower; floors from 256k to 1M were equal.
-    constexpr uint64_t kPassesInFlight = 4, kMinRaysInFlight = 1u << 20;
-    opt.rays_in_flight =
-        std::max<uint64_t>(kMinRaysInFlight, kPassesInFlight * (uint64_t)params->width * params->height);
     RunResult rr;
-    VZ_TRY(engine_run(e, items, st, opt, &rr));
+    VZ_TRY(path_launch(ctx, scene, *params, st, &rr));
     if (stats) {
         std::memset(stats, 0, sizeof(*stats));
         stats->segments = rr.segments;

@@ -280,6 +280,18 @@ VZ_DEV void camera_ray(const Cam& c, uint32_t x, uint32_t y, uint32_t& seed, v3&
     dir = sub(add(add(c.W, scl(scl(c.U, u), 0.5f)), scl(scl(c.V, v), 0.5f)), off);
 }
 
+// The draws of camera_ray alone: jitter (two), then the lens sample.
+VZ_DEV void skip_camera(uint32_t& seed)
+{
+    seed = lcg_next(lcg_next(seed));
+    for (;;) {
+        const float dx = rnd_m11(seed);
+        const float dy = rnd_m11(seed);
+        if (dx * dx + dy * dy + 0.0f * 0.0f >= 1.0f) continue;
+        break;
+    }
+}
+
 // ---- make_color (RayTracer.cu:16-47) -------------------------------------
 VZ_DEV uint32_t encode8(float c)
 {

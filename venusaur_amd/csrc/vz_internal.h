@@ -65,6 +65,7 @@ struct SceneView {           // what kernels need to traverse one scene
 };
 
 struct Engine;
+struct PathWork;
 
 // A HIP event owned by the enclosing scope, so early error returns do not
 // leak it.  ok() is false when creation failed.
@@ -104,6 +105,7 @@ struct vzContext_st {
     bool tuned = false;
     vzTuning tuning{};
     std::mutex mu;
+    vz::PathWork* path = nullptr;  // workspace of plain launches, made by the first one
     vz::Engine* engine = nullptr;  // lazily created wavefront engine
     std::atomic<uint32_t> live_scenes{0}, live_servers{0};  // vzDestroy refuses while any remain
     unsigned long long* trace_scratch = nullptr;  // this device's fixed trace scratch (vzTraceClosestNoAlloc)
