@@ -62,7 +62,7 @@ typedef struct vzHit { float t; uint32_t prim; } vzHit;
 
 /* Launch flags */
 #define VZ_ACCUM_FP64 0x1u     /* accum is double4 (required above 1024 spp) */
-#define VZ_MEGAKERNEL 0x2u     /* one-thread-per-pixel megakernel instead of the wavefront */
+#define VZ_MEGAKERNEL 0x2u     /* one-thread-per-pixel megakernel instead of the path kernels */
 #define VZ_COUNT_VISITS 0x4u   /* count BVH node fetches and sphere tests into vzStats */
 #define VZ_TIME_STAGES 0x8u    /* time every trace-kernel launch with HIP events */
 
@@ -88,7 +88,7 @@ typedef struct vzStats {
     double render_ms;        /* wall time of the launch (HIP events) */
     double trace_ms;         /* sum of trace-kernel times (VZ_TIME_STAGES only) */
     uint32_t trace_launches; /* trace-kernel launches (timed with VZ_TIME_STAGES) */
-    uint32_t iterations;     /* wavefront iterations */
+    uint32_t iterations;     /* launches of the path kernels */
     uint64_t hits;           /* segments that hit a sphere (the rest missed) */
 } vzStats;
 
@@ -187,44 +187,40 @@ typedef struct vzBatchItem {
 } vzBatchItem;
 
 typedef struct vzTuning {
-    uint32_t queue_capacity;  /* rays in flight (0 = default) */
-    uint32_t tile_w, tile_h;  /* camera-ray tile: tile_w*tile_h pixels per block of items */
-    uint32_t iters_per_graph; /* wavefront iterations captured per hipGraph (even) */
-    uint32_t refill_lanes;    /* a wave fetches new rays once fewer than this many of its lanes
-                                 still trace: 1 = only when all are done, 65 = after every
+    uint32_t queue_capacity;  /* memory of the paths in flight, in units of 96 bytes (0 = default) */
+    uint32_t tile_w, tile_h;  /* camera tile: powers of two, 64 pixels (8x8 otherwise) */
+    uint32_t iters_per_graph; /* without effect: kept for callers of earlier versions */
+    uint32_t refill_lanes;    /* a wave shades and takes new paths once fewer than this many of its
+                                 lanes still trace: 1 = only when all are done, 65 = after every
                                  node step, 0 = the default for the kernel variant: 9 for
-                                 one small scene with its nodes in LDS, 41 for one scene with
-                                 its nodes in memory, 33 for several scenes in one run */
-    uint32_t slice_split;     /* queue slices per resident step workgroup: 1, 2, 4 or 8 (0 = 4 for
-                                 batches and servers).  Slices of uneven cost (many scenes
-                                 in one run) balance better when split; vzLaunch always uses 1 */
+                                 one small scene with its nodes in LDS, 41 otherwise */
+    uint32_t slice_split;     /* without effect: kept for callers of earlier versions */
 } vzTuning;
 
-/* Renders every item in one wavefront run (its iterations replayed as
- * hipGraphs); the items share the ray queue.  Synchronises the stream. */
+/* Renders every item, as many of them in one launch of the path kernels as
+ * the tuning's memory holds.  Synchronises the stream. */
 vzStatus vzBatchLaunch(vzContext ctx, const vzBatchItem* items, uint32_t n,
                        const vzTuning* tuning, vzStream stream, vzStats* stats);
-/* Renders the batch twice per candidate tuning, timing the wavefront only,
- * and returns the candidate with the fastest run.  Stage 1: queue capacity
- * 4M/8M/12M/24M/32M/48M rays x camera tiles 32x2/16x4/8x8 (default refill, queue
- * split 4); stage 2, at the best of those: refill_lanes 25/33/49/57, then
- * slice_split 1/2/8.  The choice becomes this context's default and is cached
- * for the process per kind of device (name and CU count): contexts on the
- * same kind of device that have not tuned themselves start from it.  The
- * items' accumulators are written (as by vzBatchLaunch). */
+/* Renders the batch twice per candidate tuning, timing the render only, and
+ * returns the candidate with the fastest run.  Stage 1: queue capacity
+ * 4M/8M/12M/24M/32M/48M x camera tiles 32x2/16x4/8x8 (default refill); stage
+ * 2, at the best of those: refill_lanes 25/33/49/57.  The choice becomes this
+ * context's default and is cached for the process per kind of device (name
+ * and CU count): contexts on the same kind of device that have not tuned
+ * themselves start from it.  The items' accumulators are written (as by
+ * vzBatchLaunch). */
 vzStatus vzAutotune(vzContext ctx, const vzBatchItem* items, uint32_t n, vzStream stream,
                     vzTuning* out);
 vzStatus vzDefaultTuning(vzContext ctx, vzTuning* out);
 
 /* ---- serving form --------------------------------------------------- */
 typedef struct vzServeConfig {
-    uint64_t hbm_budget_bytes;   /* admission budget: the per-request device buffers the server
-                                    allocates (vzRequestFootprint: pass ring, per-pixel sums,
-                                    camera seeds).  Scenes are the caller's and already resident;
+    uint64_t hbm_budget_bytes;   /* admission budget: requests are admitted while the sum of their
+                                    vzRequestFootprint fits (the server's own buffers are sized by
+                                    the tuning's queue_capacity).  Scenes are the caller's and already resident;
                                     they are not counted (vzAccelInfo.device_bytes gives theirs) */
-    uint32_t max_active;         /* max requests in the device table (<= 1024) */
-    vzTuning tuning;             /* 0 fields take the serving defaults: 48M-ray queue, 8x8 tiles,
-                                    queue split 4 */
+    uint32_t max_active;         /* max requests admitted at a time (<= 1024) */
+    vzTuning tuning;             /* 0 fields take the serving defaults: 48M x 96 bytes, 8x8 tiles */
 } vzServeConfig;
 
 typedef struct vzRequestResult {

@@ -10,7 +10,6 @@
 #include <random>
 #include <string>
 
-#include "vz_engine.h"
 #include "vz_internal.h"
 #include "vz_path.h"
 
@@ -69,6 +68,9 @@ void tuning_cache_store(vzContext ctx, const vzTuning& t)
     std::lock_guard<std::mutex> lk(g_tune_mu);
     g_tune_cache[device_key(ctx)] = t;
 }
+
+// What vzDefaultTuning gives a context that has not been tuned.
+static const vzTuning kDefaultTuning = {1u << 23, 32, 2, 16, 0, 4};
 
 // Adopts the device's cached tuning if this context has none (ctx->mu held).
 static void adopt_cached_tuning(vzContext ctx)
@@ -150,7 +152,6 @@ vzStatus vzDestroy(vzContext ctx)
                                                      " server(s) of this context are still alive");
     (void)hipSetDevice(ctx->device);
     (void)hipDeviceSynchronize();
-    if (ctx->engine) engine_destroy(ctx->engine);
     path_free(ctx->path);
     delete ctx;
     return VZ_SUCCESS;
@@ -447,7 +448,7 @@ vzStatus vzLaunch(vzScene scene, const vzLaunchParams* params, vzStream stream, 
         return VZ_SUCCESS;
     }
     RunResult rr;
-    VZ_TRY(path_launch(ctx, scene, *params, st, &rr));
+    VZ_TRY(path_launch(ctx, PathItem{scene, *params}, st, &rr));
     if (stats) {
         std::memset(stats, 0, sizeof(*stats));
         stats->segments = rr.segments;
@@ -471,20 +472,8 @@ vzStatus vzDefaultTuning(vzContext ctx, vzTuning* out)
         *out = ctx->tuning;
         return VZ_SUCCESS;
     }
-    EngineConfig cfg;
-    out->queue_capacity = cfg.queue_capacity;
-    out->tile_w = cfg.tile_w;
-    out->tile_h = cfg.tile_h;
-    out->iters_per_graph = cfg.iters_per_graph;
-    out->refill_lanes = cfg.refill_lanes;
-    out->slice_split = kBatchSplit;
+    *out = kDefaultTuning;
     return VZ_SUCCESS;
-}
-
-static bool same_tuning(const EngineConfig& c, const vzTuning& t)
-{
-    return c.queue_capacity == t.queue_capacity && c.tile_w == t.tile_w && c.tile_h == t.tile_h &&
-           c.iters_per_graph == t.iters_per_graph && c.refill_lanes == t.refill_lanes;
 }
 
 vzStatus vzBatchLaunch(vzContext ctx, const vzBatchItem* items, uint32_t n, const vzTuning* tuning, vzStream stream,
@@ -492,7 +481,7 @@ vzStatus vzBatchLaunch(vzContext ctx, const vzBatchItem* items, uint32_t n, cons
 {
     if (!ctx || (n && !items)) return set_error(VZ_ERROR_INVALID_VALUE, "NULL argument");
     if (n > kMaxRequests) return set_error(VZ_ERROR_CAPACITY, "at most 1024 items per batch");
-    std::vector<RunItem> run(n);
+    std::vector<PathItem> run(n);
     for (uint32_t i = 0; i < n; i++) {
         if (!items[i].scene || items[i].scene->ctx != ctx)
             return set_error(VZ_ERROR_INVALID_VALUE, "batch item " + std::to_string(i) + " has no scene of this context");
@@ -505,37 +494,11 @@ vzStatus vzBatchLaunch(vzContext ctx, const vzBatchItem* items, uint32_t n, cons
     std::lock_guard<std::mutex> lk(ctx->mu);
     vzTuning t;
     if (tuning) t = *tuning; else VZ_TRY(vzDefaultTuning(ctx, &t));
-    if (t.queue_capacity == 0) t.queue_capacity = EngineConfig().queue_capacity;
-    if (t.tile_w == 0) t.tile_w = EngineConfig().tile_w;
-    if (t.tile_h == 0) t.tile_h = EngineConfig().tile_h;
-    if (t.iters_per_graph < 2) t.iters_per_graph = EngineConfig().iters_per_graph;
-    if (t.refill_lanes > 65) t.refill_lanes = 65;
-    if (ctx->engine && !same_tuning(ctx->engine->cfg, t)) {
-        (void)hipStreamSynchronize(as_stream(stream));
-        engine_destroy(ctx->engine);
-        ctx->engine = nullptr;
-    }
-    if (!ctx->engine) {
-        EngineConfig cfg;
-        cfg.queue_capacity = t.queue_capacity;
-        cfg.tile_w = t.tile_w;
-        cfg.tile_h = t.tile_h;
-        cfg.iters_per_graph = t.iters_per_graph;
-        cfg.refill_lanes = t.refill_lanes;
-        VZ_TRY(engine_create(ctx, cfg, &ctx->engine));
-    }
-    RunOptions opt;
-    opt.use_graph = true;
-    bool count = false, timing = false;
-    for (uint32_t i = 0; i < n; i++) {
-        count |= (items[i].params.flags & VZ_COUNT_VISITS) != 0;
-        timing |= (items[i].params.flags & VZ_TIME_STAGES) != 0;
-    }
-    opt.count_visits = count;
-    opt.time_trace = timing;
-    opt.slice_split = t.slice_split ? t.slice_split : kBatchSplit;
+    if (t.queue_capacity == 0) t.queue_capacity = kDefaultTuning.queue_capacity;
+    if (t.tile_w == 0) t.tile_w = kDefaultTuning.tile_w;
+    if (t.tile_h == 0) t.tile_h = kDefaultTuning.tile_h;
     RunResult rr;
-    VZ_TRY(engine_run(ctx->engine, run, as_stream(stream), opt, &rr));
+    VZ_TRY(path_batch(ctx, run, t, as_stream(stream), &rr));
     if (stats) {
         std::memset(stats, 0, sizeof(*stats));
         stats->segments = rr.segments;

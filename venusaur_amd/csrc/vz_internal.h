@@ -62,9 +62,12 @@ struct SceneView {           // what kernels need to traverse one scene
     const float4* mats;      // leaf order {albedo rgb, fuzz | ior}
     uint32_t n;              // primitives (leaves)
     uint32_t nw;             // 4-wide nodes (0 for a single sphere)
+    __host__ __device__ uint32_t count() const { return n; }
+    __host__ __device__ const float4* sphere_array() const { return spheres; }
+    __host__ __device__ const uint32_t* info_array() const { return leaf_info; }
+    __host__ __device__ const float4* mat_array() const { return mats; }
 };
 
-struct Engine;
 struct PathWork;
 
 // A HIP event owned by the enclosing scope, so early error returns do not
@@ -105,8 +108,7 @@ struct vzContext_st {
     bool tuned = false;
     vzTuning tuning{};
     std::mutex mu;
-    vz::PathWork* path = nullptr;  // workspace of plain launches, made by the first one
-    vz::Engine* engine = nullptr;  // lazily created wavefront engine
+    vz::PathWork* path = nullptr;  // workspace of its launches, made by the first one
     std::atomic<uint32_t> live_scenes{0}, live_servers{0};  // vzDestroy refuses while any remain
     unsigned long long* trace_scratch = nullptr;  // this device's fixed trace scratch (vzTraceClosestNoAlloc)
 };
@@ -197,6 +199,9 @@ vzStatus trace_scratch_address(unsigned long long** out);
 
 // vz_api.cpp: the process-wide autotune cache, keyed by device name and CU count
 void tuning_cache_store(vzContext ctx, const vzTuning& t);
+
+// vz_path.hip: gives back what a context kept for its launches
+void path_free(PathWork* w);
 
 // vz_megakernel.hip
 vzStatus megakernel_launch(const SceneView& sc, const vzLaunchParams& p, hipStream_t st,

@@ -1,26 +1,114 @@
-// vz_path.h -- plain launches (vzLaunch) as persistent path tracing: the
-// workspace a context keeps for them and the launch itself.
+// vz_path.h -- rendering as persistent path tracing, shared by the plain
+// launch (vzLaunch), the batched form (vzBatchLaunch) and the serving loop.
+// vz_path.hip says how a launch works and why; this file is its host side.
+//
+// A slot holds the buffers of the launches that are enqueued on one stream:
+// each launch uses them after the one before it on that stream, so a slot
+// belongs to one stream at a time.
 #pragma once
-#include "vz_engine.h"
+#include <vector>
+
+#include "vz_device.h"
+#include "vz_internal.h"
 
 namespace vz {
 
-// Buffers kept by a context between launches, freed with it.  One launch
-// uses them at a time (the context's mutex is held until the launch has
-// finished on its stream).
-struct PathWork {
-    char* paths = nullptr;      // seeds and radiances of one chunk of passes
-    size_t paths_bytes = 0;
-    char* pixels = nullptr;     // sums and camera seeds carried from chunk to chunk
-    size_t pixels_bytes = 0;
-    unsigned long long* stats = nullptr;    // device: per k_path workgroup
-    unsigned long long* h_stats = nullptr;  // pinned: their totals, written by k_path_resolve
-    Event t0, t1;
-    uint32_t grid_lds = 0, grid_mem = 0;    // resident k_path workgroups by variant
+constexpr int kPathStats = 4;         // segments, hits, node visits, sphere tests
+// Device memory per path of a launch: its camera seed and its radiance.
+constexpr uint64_t kPathBytes = 16;
+// vzTuning.queue_capacity counts rays in flight at 96 bytes each; a batch or
+// a server keeps the paths of its launches in as much memory.
+constexpr uint64_t kRayBytes = 96;
+// A plain launch: 4 GiB hold 129 passes of a 1080p frame.
+constexpr uint64_t kPlainBudget = 4ull << 30;
+// The most a slot is used for, so that a path's index fits 32 bits.
+constexpr uint64_t kMaxSlotBudget = 16ull << 30;
+
+struct PathReq {               // one request of a launch, read by scalar loads
+    Cam cam;
+    uint32_t subframe, max_depth, spp, fp64;
+    uint32_t lw;               // camera tiles are 2^lw x 2^(6 - lw) pixels
+    uint32_t tiles_x, npad;    // npad: pixels of all tiles
+    uint32_t s0, ns;           // the launch's passes [s0, s0 + ns)
+    uint32_t spu, groups;      // passes per unit, units per tile
+    uint32_t unit0, pix0, slot0;  // its first unit, padded pixel and path in the launch
+    uint32_t* camseed;         // npad: camera seed of the next launch's first pass (ns < spp)
+    void* sums;                // 3 * npad float or double, carried between launches (ns < spp)
+    void* accum;
+    uint32_t* image;
+    SceneView sc;
 };
 
-void path_free(PathWork* w);
+struct PathSlot {
+    char* paths = nullptr;     // seeds and radiances
+    size_t paths_bytes = 0;
+    char* pixels = nullptr;    // camera seeds and sums carried between the launches of one request
+    size_t pixels_bytes = 0;
+    unsigned long long* stats = nullptr;     // per workgroup, the unit counter, segments per request
+    unsigned long long* h_totals = nullptr;  // pinned: kPathStats, then segments per request
+    PathReq* reqs = nullptr;   // request table (many requests in one launch)
+    PathReq* h_reqs = nullptr; // pinned staging of it
+    uint32_t used = 0;         // its entries given to launches not yet waited for
+
+    vzStatus init(bool table);
+    void free();
+};
+
+struct PathItem {
+    const vzScene_st* scene;
+    vzLaunchParams params;
+};
+
+struct PathOptions {
+    uint32_t refill = 0;       // 0: the kernel variant's default
+    uint32_t tile_w = 8, tile_h = 8;
+    bool count = false;        // count node visits and sphere tests
+    std::vector<Event>* events = nullptr;  // appended to: a pair around every k_path launch
+};
+
+struct RunResult {
+    unsigned long long segments = 0, hits = 0, node_visits = 0, sphere_tests = 0, paths = 0;
+    double render_ms = 0.0, trace_ms = 0.0;
+    uint32_t trace_launches = 0, iterations = 0;
+};
+
+struct PathWork {              // what a context keeps between launches
+    PathSlot plain, batch;
+    Event t0, t1;
+    uint32_t grid_lds = 0, grid_mem = 0;  // resident k_path workgroups by variant
+    ~PathWork()
+    {
+        plain.free();
+        batch.free();
+    }
+};
+
+vzStatus path_work(vzContext ctx, PathWork** out);
+
+Cam make_cam(const vzLaunchParams& p);
+// The device memory a served request is admitted by: a ring of its passes
+// (at most max_depth + 2), its per-pixel sums and camera seeds.
+size_t request_bytes(const vzLaunchParams& p);
+
+// Paths of a request with its tiles' padding.
+uint64_t path_count(const vzLaunchParams& p, const PathOptions& opt);
+// Makes room in the slot for launches of up to `paths` paths; nothing on its
+// stream may still run.
+vzStatus slot_reserve(PathSlot& s, uint64_t paths);
+// Enqueues one request, in as many launches as its passes need within
+// `budget` bytes.  add: its totals add to those of the slot's launch before.
+vzStatus path_enqueue_one(PathWork* w, PathSlot& s, const PathItem& item, const PathOptions& opt, uint64_t budget,
+                          bool add, hipStream_t st, uint32_t* launches);
+// Enqueues n requests as one launch (their paths fit the slot).
+vzStatus path_enqueue_many(PathWork* w, PathSlot& s, const PathItem* const* items, uint32_t n, const PathOptions& opt,
+                           bool add, hipStream_t st);
+
 // Renders one frame and waits for it.
-vzStatus path_launch(vzContext ctx, const vzScene_st* scene, const vzLaunchParams& p, hipStream_t st, RunResult* res);
+vzStatus path_launch(vzContext ctx, const PathItem& item, hipStream_t st, RunResult* res);
+// Renders every item and waits for them.
+vzStatus path_batch(vzContext ctx, const std::vector<PathItem>& items, const vzTuning& t, hipStream_t st,
+                    RunResult* res);
+// Memory of a tuning's paths.
+uint64_t tuning_budget(const vzTuning& t);
 
 }  // namespace vz

@@ -1,24 +1,26 @@
-// vz_path.hip -- plain launches (vzLaunch) as persistent path tracing.
-// Replaces the recursive optixTrace chain of the reference's OptiX programs
+// vz_path.hip -- rendering as persistent path tracing: plain launches
+// (vzLaunch), batches (vzBatchLaunch) and the launches of a server.  Replaces
+// the recursive optixTrace chain of the reference's OptiX programs
 // (Core/RayTracer.cu:163-450).
 //
-// A launch is three kernels per chunk of passes (a pass is sample s of every
-// pixel):
-//   k_path_seeds    per pixel, the camera seed of every pass of the chunk.
-//                   The seed of pass s + 1 follows from the camera draws of
-//                   pass s alone (RayTracer.cu:163-204), so with the seeds
-//                   known every path of the chunk is independent.
+// A launch renders one request, or a table of requests of any scenes and
+// sizes, in three kernels (a pass is sample s of every pixel of a request):
+//   k_path_seeds    per pixel, the camera seed of every pass.  The seed of
+//                   pass s + 1 follows from the camera draws of pass s alone
+//                   (RayTracer.cu:163-204), so with the seeds known every
+//                   path is independent.
 //   k_path          persistent waves.  A lane traces one path from its
 //                   camera ray to its end and then takes the next (path
 //                   regeneration, Novak, Havran and Dachsbacher 2010), so a
-//                   wave stays full until the chunk runs out; its radiance
-//                   goes to the path's own slot of a buffer.
-//   k_path_resolve  adds the chunk's radiances to the per-pixel sums in
-//                   sample order and, after the last chunk, writes accum and
-//                   image.  The sums are the sequential ones whatever order
-//                   the paths finished in.
+//                   wave stays full until the launch runs out of paths; its
+//                   radiance goes to the path's own slot of a buffer.
+//   k_path_resolve  adds the radiances to the per-pixel sums in sample order
+//                   and writes accum and image.  The sums are the sequential
+//                   ones whatever order the paths finished in.
+// A request with more paths than the buffer holds takes several launches, a
+// chunk of its passes each; its sums and camera seeds carry over.
 //
-// Why.  The queue-driven wavefront this replaces for plain launches spent a
+// Why.  The queue-driven wavefront this replaces spent a
 // launch per bounce: 304 rounds of three kernels for the 1080p book frame at
 // 256 samples, each as long as its slowest workgroup, its path records
 // written and read back from HBM between them, and no fewer rounds for a
@@ -27,8 +29,9 @@
 // turn: 64x36 at 2 samples 817 -> 143 us, 400x225 at 16 samples 2.80 -> 1.12
 // ms, 1200x800 at 16 samples depth 4 3.43 -> 2.04 ms, 1080p at 256 samples
 // 115.2 -> 78.6 ms, a million spheres at 1080p and 64 samples 241 -> 187 ms,
-// 512x512 at 2048 samples in double 355 -> 135 ms; images bit for bit the
-// same.  k_path is bound by VALU issue (traversal and sphere tests with part
+// 512x512 at 2048 samples in double 355 -> 135 ms, 24 box scenes in a batch
+// 165 -> 121 ms, a burst of 20 requests to a server 336 -> 195 ms; images bit
+// for bit the same.  k_path is bound by VALU issue (traversal and sphere tests with part
 // of the lanes idle); k_path_seeds and k_path_resolve are under 1% each of
 // the 1080p frame (0.27 and 0.60 ms per 128 passes, the latter reading 3.2 GB
 // at 5.3 TB/s).
@@ -51,7 +54,8 @@ constexpr int kBlk = 256;
 constexpr uint32_t kLdsNodes = 256;   // a scene of at most this many 4-wide nodes is staged in LDS (16 KB)
 constexpr uint32_t kMaxPathBlocks = 8192;
 // A wave leaves the traversal to shade and take new paths once fewer than
-// this many of its lanes still trace.
+// this many of its lanes still trace.  Many scenes in memory, 24-scene batch:
+// 141 ms at 9, 128 at 17, 121 at 25, 117 at 33, 115 at 41, 119 at 49.
 constexpr uint32_t kRefillLds = 9;
 constexpr uint32_t kRefillGlobal = 41;
 constexpr uint32_t kFlushDen = 2;     // queued sphere tests run once 1/kFlushDen of the tracing lanes hold some
@@ -60,31 +64,31 @@ constexpr uint32_t kTile = 64;        // pixels of a camera tile: one wave of ca
 // tile, fewer while the units would not go round the waves kUnitRounds times.
 constexpr uint32_t kUnitPasses = 8;
 constexpr uint32_t kUnitRounds = 8;
-// Radiance buffer of a chunk: 16 bytes a path (seed and radiance).  4 GiB
-// holds 129 passes of a 1080p frame; every chunk ends with a fraction of a
-// millisecond in which the last long paths run alone.
-constexpr uint64_t kPathBudget = 4ull << 30;
-constexpr int kPathStats = 4;         // segments, hits, node visits, sphere tests
 
-struct PathArgs {
-    Cam cam;
-    uint32_t subframe, max_depth, spp;
-    uint32_t lw;               // tiles are 2^lw x 2^(6 - lw) pixels
-    uint32_t tiles_x, npad;    // npad: pixels of all tiles
-    uint32_t s0, ns;           // the chunk's passes [s0, s0 + ns)
-    uint32_t spu, groups;      // passes per unit, units per tile
-    uint32_t units;
+
+// Where k_path's requests and scenes come from.
+enum PathSrc {
+    kOneLds,    // one request, its scene's nodes staged in LDS
+    kOneMem,    // one request, its scene's nodes in memory
+    kManyLds,   // a table of requests of one scene, staged in LDS
+    kManyMem    // a table of requests of any scenes
+};
+
+// One launch of the three kernels: a request of its own (`one`, by value) or
+// the requests of a table.
+struct PathGroup {
+    const PathReq* reqs;       // table (many)
+    uint32_t n;                // its requests
+    uint32_t units, pixels;    // of all requests
     uint32_t refill;
+    uint32_t grid;             // k_path workgroups
+    uint32_t add;              // the totals add to those of the launch before
     uint32_t* counter;         // units claimed beyond every wave's first
-    uint32_t* seeds;           // ns * npad: camera seed of the pass
-    uint32_t* camseed;         // npad: camera seed of the next chunk's first pass
-    float* rad;                // 3 * ns * npad: radiance of each path
-    unsigned long long* stats; // kPathStats per workgroup
-    void* sums;                // 3 * npad float or double, carried between chunks
-    void* accum;
-    uint32_t* image;
-    uint32_t grid;             // k_path workgroups of the chunk
-    unsigned long long* totals;  // pinned host memory, kPathStats
+    uint32_t* seeds;           // per path: camera seed
+    float* rad;                // per path: radiance
+    unsigned long long* stats; // kPathStats per k_path workgroup
+    unsigned long long* segs;  // per request of the table: segments
+    unsigned long long* totals;  // pinned host memory: kPathStats, then segs
 };
 
 __device__ __forceinline__ uint32_t mbcnt(uint64_t m)
@@ -99,7 +103,7 @@ __device__ __forceinline__ unsigned long long wave_sum(unsigned long long v)
 }
 
 // Pixel i of the padded, tile by tile numbering.
-__device__ __forceinline__ void pixel_of(const PathArgs& P, uint32_t i, uint32_t& x, uint32_t& y)
+__device__ __forceinline__ void pixel_of(const PathReq& P, uint32_t i, uint32_t& x, uint32_t& y)
 {
     const uint32_t t = i / kTile, w = i % kTile;
     const uint32_t ty = t / P.tiles_x, tx = t - ty * P.tiles_x;
@@ -107,23 +111,70 @@ __device__ __forceinline__ void pixel_of(const PathArgs& P, uint32_t i, uint32_t
     y = (ty << (6u - P.lw)) + (w >> P.lw);
 }
 
-// The camera seed of every pass of the chunk, one thread per pixel: only the
-// draws of camera_ray, so the walk is a few LCG steps a pass.
-__global__ void __launch_bounds__(kBlk) k_path_seeds(PathArgs P)
+// The last request of the table whose first unit / first pixel is at or
+// below v (wave-uniform, so the table is read by scalar loads).
+__device__ __forceinline__ uint32_t request_of_unit(const PathReq* __restrict__ reqs, uint32_t n, uint32_t v)
 {
-    const uint32_t i = blockIdx.x * kBlk + threadIdx.x;
-    if (i == 0) *P.counter = 0u;
-    if (i >= P.npad) return;
+    uint32_t lo = 0, hi = n;
+    while (hi - lo > 1u) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (reqs[mid].unit0 <= v) lo = mid; else hi = mid;
+    }
+    return lo;
+}
+__device__ __forceinline__ uint32_t request_of_pixel(const PathReq* __restrict__ reqs, uint32_t n, uint32_t v)
+{
+    uint32_t lo = 0, hi = n;
+    while (hi - lo > 1u) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (reqs[mid].pix0 <= v) lo = mid; else hi = mid;
+    }
+    return lo;
+}
+
+// The camera seed of every pass, one thread per pixel: only the draws of
+// camera_ray, so the walk is a few LCG steps a pass.
+__device__ __forceinline__ void seed_pixel(const PathReq& P, uint32_t i, uint32_t* __restrict__ seeds)
+{
     uint32_t x, y;
     pixel_of(P, i, x, y);
     if (x >= P.cam.width || y >= P.cam.height) return;
     uint32_t seed = P.s0 == 0u ? tea4(y * P.cam.width + x, P.subframe) : P.camseed[i];
     for (uint32_t s = 0; s < P.ns; s++) {
-        P.seeds[(size_t)s * P.npad + i] = seed;
+        seeds[P.slot0 + (size_t)s * P.npad + i] = seed;
         skip_camera(seed);
     }
     if (P.s0 + P.ns < P.spp) P.camseed[i] = seed;
 }
+template <bool MANY>
+__global__ void __launch_bounds__(kBlk) k_path_seeds(PathGroup G, PathReq one)
+{
+    const uint32_t j = blockIdx.x * kBlk + threadIdx.x;
+    if (j == 0) *G.counter = 0u;
+    if (MANY)
+        for (uint32_t r = j; r < G.n; r += gridDim.x * kBlk) G.segs[r] = 0ull;
+    if (j >= G.pixels) return;
+    if (MANY) {
+        // requests have whole tiles, so a wave's pixels belong to one
+        const PathReq& P = G.reqs[request_of_pixel(G.reqs, G.n, (uint32_t)__builtin_amdgcn_readfirstlane(j))];
+        seed_pixel(P, j - P.pix0, G.seeds);
+    } else {
+        seed_pixel(one, j, G.seeds);
+    }
+}
+
+// What a lane of a many-scene launch keeps of its scene: the two arrays the
+// traversal reads.  The others are looked up in the request table where a
+// hit is shaded.
+struct LaneScene {
+    const uint4* nodes;
+    const float4* spheres;
+    const PathReq* req;
+    __device__ __forceinline__ uint32_t count() const { return ldg(&req->sc.n); }
+    __device__ __forceinline__ const float4* sphere_array() const { return spheres; }
+    __device__ __forceinline__ const uint32_t* info_array() const { return req->sc.leaf_info; }
+    __device__ __forceinline__ const float4* mat_array() const { return req->sc.mats; }
+};
 
 // Every wave takes units until none is left: the first by its place (so a
 // small frame spreads over the CUs), the others from one counter (one
@@ -131,12 +182,15 @@ __global__ void __launch_bounds__(kBlk) k_path_seeds(PathArgs P)
 // serialise across the XCDs).  Lanes without a path take the next ones of the
 // wave's unit, all lanes with a ray walk the tree until fewer than `refill`
 // of them still do, and the finished ones shade: a path that goes on starts
-// its next segment in place.  LDSN: the scene's nodes are staged in LDS.
+// its next segment in place.  A wave never waits for its lanes to finish one
+// request before it starts the next: with kManyMem each lane carries its own
+// scene.
 // COUNT: node visits and sphere tests are counted, and tests run at once so
 // that the counts follow each ray alone.
-template <bool COUNT, bool LDSN>
-__global__ void __launch_bounds__(kPathBlk) __attribute__((amdgpu_waves_per_eu(6))) k_path(SceneView sc, PathArgs P)
+template <bool COUNT, PathSrc SRC>
+__global__ void __launch_bounds__(kPathBlk) __attribute__((amdgpu_waves_per_eu(6))) k_path(PathGroup G, PathReq one)
 {
+    constexpr bool LDSN = SRC == kOneLds || SRC == kManyLds, MANY = SRC == kManyLds || SRC == kManyMem;
     constexpr bool DEFER = !COUNT && !LDSN;
     __shared__ uint32_t s_node[kStackS * kPathBlk];
     __shared__ float s_t[kStackS * kPathBlk];
@@ -145,7 +199,11 @@ __global__ void __launch_bounds__(kPathBlk) __attribute__((amdgpu_waves_per_eu(6
     __shared__ unsigned long long s_red[kPathStats][kWaves];
     const uint32_t tid = threadIdx.x, lane = __lane_id();
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(tid >> 6);
-    if (LDSN) {
+    // many requests of many scenes: the lane's own, filled in with its path
+    typename std::conditional<SRC == kManyMem, LaneScene, SceneView>::type sc;
+    if constexpr (SRC == kManyMem) sc = LaneScene{nullptr, nullptr, nullptr};
+    else sc = MANY ? G.reqs[0].sc : one.sc;
+    if constexpr (LDSN) {
         const uint32_t nn = 4u * sc.nw;
         for (uint32_t i = tid; i < nn; i += kPathBlk) s_bvh[i] = ldg(sc.nodes + i);
         __syncthreads();
@@ -154,31 +212,46 @@ __global__ void __launch_bounds__(kPathBlk) __attribute__((amdgpu_waves_per_eu(6
     Overflow ov;
     uint32_t nv = 0, ns = 0;
     uint32_t n_seg = 0, n_hit = 0;    // of the wave
-    bool active = false, tdone = false, exhausted = false;
+    bool active = false, tdone = false, exhausted = false, fresh = true;
     uint32_t unit = wave * gridDim.x + blockIdx.x;
     uint32_t cur = 0, end = 0;        // the wave's unit: its next path and their number
-    uint32_t u_tile = 0, u_x = 0, u_y = 0, u_s = 0;
+    uint32_t u_req = 0, u_tile = 0, u_x = 0, u_y = 0, u_s = 0;
+    // segments of the unit's request and of the one before it, not yet added
+    // to G.segs: an atomic per change of request, since one per segment on a
+    // request's counter made a 24-scene batch 1.4 times slower
+    uint32_t r_seg = 0, o_req = 0, o_seg = 0;
     v3 thr = mk(0.0f, 0.0f, 0.0f);    // the lane's path
-    uint32_t seed = 0, slot = 0, depth = 0;
-    bool fresh = true;
+    uint32_t seed = 0, slot = 0, depth = 0, my_req = 0;
     for (;;) {
         const uint64_t m = __ballot(!active);
         if (m && !exhausted) {
             if (cur == end) {
                 if (!fresh) {
                     uint32_t u = 0;
-                    if (lane == 0) u = atomicAdd(P.counter, 1u);
+                    if (lane == 0) u = atomicAdd(G.counter, 1u);
                     unit = kWaves * gridDim.x + (uint32_t)__builtin_amdgcn_readfirstlane(u);
                 }
                 fresh = false;
                 cur = end = 0;
-                if (unit >= P.units) {
+                if (unit >= G.units) {
                     exhausted = true;
                 } else {
+                    if (MANY) {
+                        const uint32_t r = request_of_unit(G.reqs, G.n, unit);
+                        if (r != u_req) {
+                            if (o_seg && lane == 0) atomicAdd(&G.segs[o_req], (unsigned long long)o_seg);
+                            o_req = u_req;
+                            o_seg = r_seg;
+                            r_seg = 0;
+                            u_req = r;
+                        }
+                    }
+                    const PathReq& P = MANY ? G.reqs[u_req] : one;
                     // all passes of a tile follow one another: the waves
                     // work on one part of the image at a time
-                    u_tile = unit / P.groups;
-                    u_s = (unit - u_tile * P.groups) * P.spu;
+                    const uint32_t u = unit - P.unit0;
+                    u_tile = u / P.groups;
+                    u_s = (u - u_tile * P.groups) * P.spu;
                     const uint32_t ty = u_tile / P.tiles_x;
                     u_x = (u_tile - ty * P.tiles_x) << P.lw;
                     u_y = ty << (6u - P.lw);
@@ -188,15 +261,18 @@ __global__ void __launch_bounds__(kPathBlk) __attribute__((amdgpu_waves_per_eu(6
             const uint32_t take = min((uint32_t)__popcll(m), end - cur);
             const uint32_t rk = mbcnt(m);
             if (!active && rk < take) {
+                const PathReq& P = MANY ? G.reqs[u_req] : one;
                 const uint32_t p = cur + rk, w = p % kTile;
                 const uint32_t x = u_x + (w & ((1u << P.lw) - 1u)), y = u_y + (w >> P.lw);
                 if (x < P.cam.width && y < P.cam.height) {
-                    slot = (u_s + p / kTile) * P.npad + u_tile * kTile + w;
-                    seed = ldg(P.seeds + slot);
+                    slot = P.slot0 + (u_s + p / kTile) * P.npad + u_tile * kTile + w;
+                    seed = ldg(G.seeds + slot);
                     v3 o, d;
                     camera_ray(P.cam, x, y, seed, o, d);
                     thr = mk(1.0f, 1.0f, 1.0f);
                     depth = P.max_depth - 1u;
+                    if (MANY) my_req = u_req;
+                    if constexpr (SRC == kManyMem) sc = LaneScene{P.sc.nodes, P.sc.spheres, G.reqs + u_req};
                     tdone = tr.init(sc, o, d, 0.001f, 1e16f, ns);
                     active = true;
                 }
@@ -210,7 +286,7 @@ __global__ void __launch_bounds__(kPathBlk) __attribute__((amdgpu_waves_per_eu(6
         uint64_t busy = __ballot(active && !tdone);
         while (busy) {
             if (active && !tdone) {
-                if (LDSN)
+                if constexpr (LDSN)
                     tdone = tr.step(sc, LdsNodes{s_bvh}, s_node + tid, s_t + tid, kPathBlk, ov, nv, ns, s_pend + tid);
                 else
                     tdone = tr.step(sc, GlobalNodes{sc.nodes}, s_node + tid, s_t + tid, kPathBlk, ov, nv, ns,
@@ -226,7 +302,7 @@ __global__ void __launch_bounds__(kPathBlk) __attribute__((amdgpu_waves_per_eu(6
                            kFlushDen * (uint32_t)__popcll(pm) >= (uint32_t)__popcll(busy)))
                     tr.flush(sc, s_pend + tid, kPathBlk, ns);
             }
-            if ((uint32_t)__popcll(busy) < P.refill) break;
+            if ((uint32_t)__popcll(busy) < G.refill) break;
         }
         // every queued test has run before a lane's hit is shaded
         if (DEFER) tr.flush(sc, s_pend + tid, kPathBlk, ns);
@@ -235,6 +311,17 @@ __global__ void __launch_bounds__(kPathBlk) __attribute__((amdgpu_waves_per_eu(6
         if (fm == 0ull) continue;
         n_seg += (uint32_t)__popcll(fm);
         n_hit += (uint32_t)__popcll(__ballot(fin && tr.bleaf != 0xFFFFFFFFu));
+        if (MANY) {
+            // nearly always the unit's request; after a change of request
+            // some lanes still trace the one before
+            const uint64_t same = __ballot(fin && my_req == u_req);
+            r_seg += (uint32_t)__popcll(same);
+            if (fm & ~same) {
+                const uint64_t prev = __ballot(fin && my_req != u_req && my_req == o_req);
+                o_seg += (uint32_t)__popcll(prev);
+                if (fin && my_req != u_req && my_req != o_req) atomicAdd(&G.segs[my_req], 1ull);
+            }
+        }
         if (fin) {
             v3 L = mk(0.0f, 0.0f, 0.0f);
             bool ended = true;
@@ -243,9 +330,9 @@ __global__ void __launch_bounds__(kPathBlk) __attribute__((amdgpu_waves_per_eu(6
                 L = mul(thr, sky(tr.d));
             } else if (depth > 0u) {
                 // shade (RayTracer.cu:272-440)
-                const float4 s = ldg(sc.spheres + tr.bleaf);
-                const uint32_t type = ldg(sc.leaf_info + tr.bleaf) >> 30;
-                const float4 mat = ldg(sc.mats + tr.bleaf);
+                const float4 s = ldg(sc.sphere_array() + tr.bleaf);
+                const uint32_t type = ldg(sc.info_array() + tr.bleaf) >> 30;
+                const float4 mat = ldg(sc.mat_array() + tr.bleaf);
                 const v3 pos = add(tr.o, scl(tr.d, tr.best));
                 v3 n = scl(sub(pos, mk(s.x, s.y, s.z)), recip_rn(s.w));
                 const bool front = dot(tr.d, n) < 0.0f;
@@ -259,13 +346,17 @@ __global__ void __launch_bounds__(kPathBlk) __attribute__((amdgpu_waves_per_eu(6
                 }
             }
             if (ended) {
-                float* q = P.rad + 3 * (size_t)slot;
+                float* q = G.rad + 3 * (size_t)slot;
                 q[0] = L.x;
                 q[1] = L.y;
                 q[2] = L.z;
                 active = false;
             }
         }
+    }
+    if (MANY && lane == 0) {
+        if (r_seg) atomicAdd(&G.segs[u_req], (unsigned long long)r_seg);
+        if (o_seg) atomicAdd(&G.segs[o_req], (unsigned long long)o_seg);
     }
     const unsigned long long w_nv = COUNT ? wave_sum((unsigned long long)nv) : 0ull;
     const unsigned long long w_ns = COUNT ? wave_sum((unsigned long long)ns) : 0ull;
@@ -279,27 +370,17 @@ __global__ void __launch_bounds__(kPathBlk) __attribute__((amdgpu_waves_per_eu(6
     if (tid < (uint32_t)kPathStats) {
         unsigned long long a = 0;
         for (int w = 0; w < kWaves; w++) a += s_red[tid][w];
-        P.stats[(size_t)blockIdx.x * kPathStats + tid] = a;
+        G.stats[(size_t)blockIdx.x * kPathStats + tid] = a;
     }
 }
 
-// Adds the chunk's radiances to the pixels' sums in sample order; on the last
+// Adds the radiances of pixel i to its sums in sample order; on the last
 // chunk blends the average into accum and encodes the image (RayTracer.cu:
-// 16-47, 203-216).  Its first workgroup also adds the k_path workgroups'
-// counters to the totals in host memory, which saves a copy.
+// 16-47, 203-216).
 template <bool FP64>
-__global__ void __launch_bounds__(kBlk) k_path_resolve(PathArgs P)
+__device__ __forceinline__ void resolve_pixel(const PathReq& P, uint32_t i, const float* __restrict__ rad)
 {
     using T = typename std::conditional<FP64, double, float>::type;
-    if (blockIdx.x == 0 && threadIdx.x < 64u * kPathStats) {
-        const uint32_t k = threadIdx.x >> 6;
-        unsigned long long a = 0;
-        for (uint32_t b = threadIdx.x & 63u; b < P.grid; b += 64u) a += P.stats[(size_t)b * kPathStats + k];
-        a = wave_sum(a);
-        if (__lane_id() == 0) P.totals[k] = (P.s0 ? P.totals[k] : 0ull) + a;
-    }
-    const uint32_t i = blockIdx.x * kBlk + threadIdx.x;
-    if (i >= P.npad) return;
     uint32_t x, y;
     pixel_of(P, i, x, y);
     if (x >= P.cam.width || y >= P.cam.height) return;
@@ -307,7 +388,7 @@ __global__ void __launch_bounds__(kBlk) k_path_resolve(PathArgs P)
     T s[3] = {T(0), T(0), T(0)};
     if (P.s0)
         for (int k = 0; k < 3; k++) s[k] = sums[(size_t)k * P.npad + i];
-    const float* q = P.rad + 3 * (size_t)i;
+    const float* q = rad + 3 * ((size_t)P.slot0 + i);
 #pragma unroll 8
     for (uint32_t p = 0; p < P.ns; p++, q += 3 * (size_t)P.npad)
         for (int k = 0; k < 3; k++) s[k] = s[k] + (T)q[k];
@@ -345,6 +426,33 @@ __global__ void __launch_bounds__(kBlk) k_path_resolve(PathArgs P)
     if (P.image) P.image[px] = make_color(oc[0], oc[1], oc[2]);
 }
 
+// The first workgroup also adds the k_path workgroups' counters to the
+// totals in host memory, which saves a copy.
+template <bool MANY>
+__global__ void __launch_bounds__(kBlk) k_path_resolve(PathGroup G, PathReq one)
+{
+    if (blockIdx.x == 0) {
+        static_assert(kBlk == 64 * kPathStats, "a wave per counter");
+        const uint32_t k = threadIdx.x >> 6;
+        unsigned long long a = 0;
+        for (uint32_t b = threadIdx.x & 63u; b < G.grid; b += 64u) a += G.stats[(size_t)b * kPathStats + k];
+        a = wave_sum(a);
+        if (__lane_id() == 0) G.totals[k] = (G.add ? G.totals[k] : 0ull) + a;
+        if (MANY)
+            for (uint32_t r = threadIdx.x; r < G.n; r += kBlk) G.totals[kPathStats + r] = G.segs[r];
+    }
+    const uint32_t j = blockIdx.x * kBlk + threadIdx.x;
+    if (j >= G.pixels) return;
+    if (MANY) {
+        const PathReq& P = G.reqs[request_of_pixel(G.reqs, G.n, (uint32_t)__builtin_amdgcn_readfirstlane(j))];
+        if (P.fp64) resolve_pixel<true>(P, j - P.pix0, G.rad);
+        else resolve_pixel<false>(P, j - P.pix0, G.rad);
+    } else {
+        if (one.fp64) resolve_pixel<true>(one, j, G.rad);
+        else resolve_pixel<false>(one, j, G.rad);
+    }
+}
+
 inline uint64_t align256(uint64_t v) { return (v + 255) & ~255ull; }
 
 // Grows a buffer that nothing in flight uses.
@@ -370,143 +478,386 @@ uint32_t resident_blocks(const void* kernel, uint32_t cus)
     return std::min<uint32_t>(kMaxPathBlocks, cus * (uint32_t)occ);
 }
 
+bool fits_lds(const vzScene_st* s) { return s->n >= 2 && s->nw <= kLdsNodes; }
+
+// Tile shape of a request: the options' where it is 64 pixels of powers of
+// two, 8x8 otherwise; images less than 8 pixels high or wide get tiles of
+// their shape, so that padding never multiplies the pixels by more than 4.
+uint32_t tile_lw(const vzLaunchParams& p, const PathOptions& opt)
+{
+    if (p.height < 8u) return 5u;
+    if (p.width < 8u) return 1u;
+    for (uint32_t lw = 0; lw <= 6u; lw++)
+        if (opt.tile_w == (1u << lw) && opt.tile_h == (kTile >> lw)) return lw;
+    return 3u;
+}
+
+uint64_t tile_count(const vzLaunchParams& p, uint32_t lw)
+{
+    const uint64_t tw = 1u << lw, th = kTile >> lw;
+    return ((p.width + tw - 1) / tw) * ((p.height + th - 1) / th);
+}
+
+// The request's fields that do not depend on its place in the launch.
+void fill_request(PathReq& A, const PathItem& item, const PathOptions& opt)
+{
+    const vzLaunchParams& p = item.params;
+    std::memset((void*)&A, 0, sizeof(A));
+    A.cam = make_cam(p);
+    A.subframe = p.subframe_index;
+    A.max_depth = p.max_depth;
+    A.spp = p.samples_per_pixel;
+    A.fp64 = (p.flags & VZ_ACCUM_FP64) ? 1u : 0u;
+    A.lw = tile_lw(p, opt);
+    A.tiles_x = (p.width + (1u << A.lw) - 1) >> A.lw;
+    A.npad = (uint32_t)(tile_count(p, A.lw) * kTile);
+    A.accum = p.accum;
+    A.image = (uint32_t*)p.image;
+    A.sc = item.scene->view();
+}
+
+// Passes per unit, so that the units go round the resident waves.
+uint32_t unit_passes(uint64_t tile_passes, uint32_t resident)
+{
+    uint32_t spu = kUnitPasses;
+    while (spu > 1u && tile_passes / spu < (uint64_t)kUnitRounds * resident * kWaves) spu >>= 1;
+    return spu;
+}
+
+void fill_group(PathGroup& G, PathSlot& s, bool add)
+{
+    std::memset((void*)&G, 0, sizeof(G));
+    G.add = add ? 1u : 0u;
+    G.stats = s.stats;
+    G.counter = (uint32_t*)(s.stats + kMaxPathBlocks * kPathStats);
+    G.segs = s.stats + kMaxPathBlocks * kPathStats + 1;
+    G.totals = s.h_totals;
+}
+
+// The three kernels of one launch.
+template <bool MANY>
+vzStatus launch_group(const PathGroup& G, const PathReq& one, bool lds, const PathOptions& opt, hipStream_t st)
+{
+    const dim3 pix_grid((G.pixels + kBlk - 1) / kBlk), grid(G.grid), blk(kPathBlk);
+    constexpr PathSrc L = MANY ? kManyLds : kOneLds, M = MANY ? kManyMem : kOneMem;
+    hipLaunchKernelGGL(k_path_seeds<MANY>, pix_grid, dim3(kBlk), 0, st, G, one);
+    if (opt.events) {
+        for (int k = 0; k < 2; k++) {
+            opt.events->emplace_back();
+            VZ_EVENT_TRY(opt.events->back());
+        }
+        VZ_HIP_TRY(hipEventRecord((*opt.events)[opt.events->size() - 2].e, st));
+    }
+    if (opt.count) {
+        if (lds) hipLaunchKernelGGL((k_path<true, L>), grid, blk, 0, st, G, one);
+        else hipLaunchKernelGGL((k_path<true, M>), grid, blk, 0, st, G, one);
+    } else {
+        if (lds) hipLaunchKernelGGL((k_path<false, L>), grid, blk, 0, st, G, one);
+        else hipLaunchKernelGGL((k_path<false, M>), grid, blk, 0, st, G, one);
+    }
+    if (opt.events) VZ_HIP_TRY(hipEventRecord(opt.events->back().e, st));
+    hipLaunchKernelGGL(k_path_resolve<MANY>, pix_grid, dim3(kBlk), 0, st, G, one);
+    VZ_HIP_TRY(hipGetLastError());
+    return VZ_SUCCESS;
+}
+
+uint32_t refill_of(const PathOptions& opt, uint32_t dflt)
+{
+    return opt.refill ? std::min<uint32_t>(opt.refill, 65u) : dflt;
+}
+
+}  // namespace
+
+Cam make_cam(const vzLaunchParams& p)
+{
+    auto nrm = [](v3 v) {
+        float inv = 1.0f / sqrtf(v.x * v.x + v.y * v.y + v.z * v.z);
+        v3 r;
+        r.x = v.x * inv;
+        r.y = v.y * inv;
+        r.z = v.z * inv;
+        return r;
+    };
+    Cam c;
+    c.O.x = p.origin[0]; c.O.y = p.origin[1]; c.O.z = p.origin[2];
+    c.U.x = p.u[0]; c.U.y = p.u[1]; c.U.z = p.u[2];
+    c.V.x = p.v[0]; c.V.y = p.v[1]; c.V.z = p.v[2];
+    c.W.x = p.w[0]; c.W.y = p.w[1]; c.W.z = p.w[2];
+    c.un = nrm(c.U);
+    c.vn = nrm(c.V);
+    c.lr = p.lens_radius;
+    c.width = p.width;
+    c.height = p.height;
+    return c;
+}
+
+size_t request_bytes(const vzLaunchParams& p)
+{
+    const size_t npix = (size_t)p.width * p.height;
+    const size_t K = std::min<uint32_t>(std::min<uint32_t>(p.max_depth + 2u, p.samples_per_pixel), 255u);
+    const bool fp64 = (p.flags & VZ_ACCUM_FP64) != 0;
+    return align256(K * 3 * npix * 4) + align256(3 * npix * (fp64 ? 8 : 4)) + align256(npix * 4) + align256(K * 4) +
+           align256(K * 8) + 1024;
+}
+
+vzStatus PathSlot::init(bool table)
+{
+    bool ok = stats || hipMalloc((void**)&stats, (kMaxPathBlocks * kPathStats + 1 + kMaxRequests) *
+                                                     sizeof(unsigned long long)) == hipSuccess;
+    ok = ok && (h_totals || hipHostMalloc((void**)&h_totals, (kPathStats + kMaxRequests) *
+                                                                 sizeof(unsigned long long)) == hipSuccess);
+    if (table) {
+        ok = ok && (reqs || hipMalloc((void**)&reqs, kMaxRequests * sizeof(PathReq)) == hipSuccess);
+        ok = ok && (h_reqs || hipHostMalloc((void**)&h_reqs, kMaxRequests * sizeof(PathReq)) == hipSuccess);
+    }
+    if (!ok) {
+        (void)hipGetLastError();
+        free();
+        return set_error(VZ_ERROR_OUT_OF_MEMORY, "launch table allocation failed");
+    }
+    return VZ_SUCCESS;
+}
+
+void PathSlot::free()
+{
+    void* dev[] = {paths, pixels, stats, reqs};
+    for (void* p : dev)
+        if (p) (void)hipFree(p);
+    if (h_totals) (void)hipHostFree(h_totals);
+    if (h_reqs) (void)hipHostFree(h_reqs);
+    *this = PathSlot();
+}
+
 vzStatus path_work(vzContext ctx, PathWork** out)
 {
     if (!ctx->path) {
         PathWork* w = new PathWork();
-        if (!w->t0.ok() || !w->t1.ok() ||
-            hipMalloc((void**)&w->stats, (kMaxPathBlocks * kPathStats + 1) * sizeof(unsigned long long)) != hipSuccess ||
-            hipHostMalloc((void**)&w->h_stats, kPathStats * sizeof(unsigned long long)) != hipSuccess) {
-            path_free(w);
-            return set_error(VZ_ERROR_OUT_OF_MEMORY, "launch workspace allocation failed");
+        if (!w->t0.ok() || !w->t1.ok()) {
+            delete w;
+            return set_error(VZ_ERROR_HIP, "hipEventCreate failed");
         }
         const uint32_t cus = ctx->num_cus ? ctx->num_cus : 256;
-        w->grid_lds = resident_blocks(reinterpret_cast<const void*>(k_path<false, true>), cus);
-        w->grid_mem = resident_blocks(reinterpret_cast<const void*>(k_path<false, false>), cus);
+        w->grid_lds = resident_blocks(reinterpret_cast<const void*>(k_path<false, kOneLds>), cus);
+        w->grid_mem = resident_blocks(reinterpret_cast<const void*>(k_path<false, kManyMem>), cus);
         ctx->path = w;
     }
     *out = ctx->path;
     return VZ_SUCCESS;
 }
 
-}  // namespace
+void path_free(PathWork* w) { delete w; }
 
-void path_free(PathWork* w)
+uint64_t path_count(const vzLaunchParams& p, const PathOptions& opt)
 {
-    if (!w) return;
-    if (w->paths) (void)hipFree(w->paths);
-    if (w->pixels) (void)hipFree(w->pixels);
-    if (w->stats) (void)hipFree(w->stats);
-    if (w->h_stats) (void)hipHostFree(w->h_stats);
-    delete w;
+    return tile_count(p, tile_lw(p, opt)) * kTile * p.samples_per_pixel;
 }
 
-vzStatus path_launch(vzContext ctx, const vzScene_st* scene, const vzLaunchParams& p, hipStream_t st, RunResult* res)
+vzStatus slot_reserve(PathSlot& s, uint64_t paths)
+{
+    const uint64_t need = paths * kPathBytes + 256;
+    if (!grow(&s.paths, &s.paths_bytes, need))
+        return set_error(VZ_ERROR_OUT_OF_MEMORY, "launch buffers (" + std::to_string(need) + " bytes) do not fit");
+    return VZ_SUCCESS;
+}
+
+vzStatus path_enqueue_one(PathWork* w, PathSlot& s, const PathItem& item, const PathOptions& opt, uint64_t budget,
+                          bool add, hipStream_t st, uint32_t* launches)
+{
+    const uint64_t ntiles = tile_count(item.params, tile_lw(item.params, opt));
+    if (ntiles * kTile > 0xFFFFFF00ull) return set_error(VZ_ERROR_CAPACITY, "image too large");
+    PathReq A;
+    fill_request(A, item, opt);
+    // the passes in as few equal chunks as the budget allows; less memory
+    // than that makes more chunks
+    auto split = [&](uint64_t most) {
+        const uint64_t chunks = (A.spp + most - 1) / most;
+        return (uint32_t)((A.spp + chunks - 1) / chunks);
+    };
+    budget = std::min(budget, kMaxSlotBudget);
+    uint32_t chunk = split(std::max<uint64_t>(1, std::min<uint64_t>(A.spp, budget / (kPathBytes * A.npad))));
+    const uint64_t sum_bytes = align256((A.fp64 ? 24ull : 12ull) * A.npad);
+    for (;;) {
+        const uint64_t pix = chunk < A.spp ? sum_bytes + 4ull * A.npad : 0ull;
+        const vzStatus rs = slot_reserve(s, (uint64_t)A.npad * chunk);
+        if (rs == VZ_SUCCESS && grow(&s.pixels, &s.pixels_bytes, pix)) break;
+        if (chunk == 1u) return rs != VZ_SUCCESS ? rs : set_error(VZ_ERROR_OUT_OF_MEMORY, "launch buffers do not fit");
+        chunk = split((chunk + 1) / 2);
+    }
+    const bool lds = fits_lds(item.scene);
+    const uint32_t resident = lds ? w->grid_lds : w->grid_mem;
+    PathGroup G;
+    fill_group(G, s, add);
+    G.seeds = (uint32_t*)s.paths;
+    G.rad = (float*)(s.paths + align256(4ull * A.npad * chunk));
+    G.pixels = A.npad;
+    G.refill = refill_of(opt, lds ? kRefillLds : kRefillGlobal);
+    A.sums = s.pixels;
+    A.camseed = (uint32_t*)(s.pixels + sum_bytes);
+    for (A.s0 = 0; A.s0 < A.spp; A.s0 += chunk) {
+        A.ns = std::min(chunk, A.spp - A.s0);
+        A.spu = unit_passes(ntiles * A.ns, resident);
+        A.groups = (A.ns + A.spu - 1) / A.spu;
+        G.units = (uint32_t)(ntiles * A.groups);
+        G.grid = std::min(resident, G.units);
+        VZ_TRY(launch_group<false>(G, A, lds, opt, st));
+        G.add = 1u;
+        if (launches) ++*launches;
+    }
+    return VZ_SUCCESS;
+}
+
+vzStatus path_enqueue_many(PathWork* w, PathSlot& s, const PathItem* const* items, uint32_t n, const PathOptions& opt,
+                           bool add, hipStream_t st)
+{
+    if (s.used + n > kMaxRequests) return set_error(VZ_ERROR_INTERNAL, "request table overrun");
+    PathReq* const h = s.h_reqs + s.used;
+    PathReq* const d = s.reqs + s.used;
+    bool lds = fits_lds(items[0]->scene);
+    uint64_t tile_passes = 0, paths = 0;
+    for (uint32_t i = 0; i < n; i++) {
+        fill_request(h[i], *items[i], opt);
+        lds = lds && items[i]->scene == items[0]->scene;
+        tile_passes += (uint64_t)h[i].npad / kTile * h[i].spp;
+        paths += (uint64_t)h[i].npad * h[i].spp;
+    }
+    if (paths * kPathBytes + 256 > s.paths_bytes || paths * kPathBytes > kMaxSlotBudget)
+        return set_error(VZ_ERROR_INTERNAL, "launch larger than its slot");
+    const uint32_t resident = lds ? w->grid_lds : w->grid_mem;
+    const uint32_t spu = unit_passes(tile_passes, resident);
+    PathGroup G;
+    fill_group(G, s, add);
+    uint32_t slot0 = 0;
+    for (uint32_t i = 0; i < n; i++) {
+        PathReq& A = h[i];
+        A.ns = A.spp;
+        A.spu = std::min(spu, A.spp);
+        A.groups = (A.ns + A.spu - 1) / A.spu;
+        A.unit0 = G.units;
+        A.pix0 = G.pixels;
+        A.slot0 = slot0;
+        G.units += A.npad / kTile * A.groups;
+        G.pixels += A.npad;
+        slot0 += A.npad * A.spp;
+    }
+    G.reqs = d;
+    G.n = n;
+    G.seeds = (uint32_t*)s.paths;
+    G.rad = (float*)(s.paths + align256(4ull * paths));
+    G.refill = refill_of(opt, lds ? kRefillLds : kRefillGlobal);
+    G.grid = std::min(resident, G.units);
+    VZ_HIP_TRY(hipMemcpyAsync(d, h, n * sizeof(PathReq), hipMemcpyHostToDevice, st));
+    s.used += n;
+    return launch_group<true>(G, PathReq{}, lds, opt, st);
+}
+
+// Waits for the launches of a slot, whose buffers are then free for the next
+// ones on any stream, and reads their counters and times.
+static vzStatus finish(PathWork* w, PathSlot& s, vzStatus rs, const std::vector<Event>& ev, hipStream_t st, RunResult* res)
+{
+    if (hipStreamSynchronize(st) != hipSuccess && rs == VZ_SUCCESS)
+        rs = set_error(VZ_ERROR_HIP, "hipStreamSynchronize failed");
+    VZ_TRY(rs);
+    res->segments = s.h_totals[0];
+    res->hits = s.h_totals[1];
+    res->node_visits = s.h_totals[2];
+    res->sphere_tests = s.h_totals[3];
+    float ms = 0.0f;
+    VZ_HIP_TRY(hipEventElapsedTime(&ms, w->t0.e, w->t1.e));
+    res->render_ms = ms;
+    for (size_t k = 0; k + 1 < ev.size(); k += 2) {
+        VZ_HIP_TRY(hipEventElapsedTime(&ms, ev[k].e, ev[k + 1].e));
+        res->trace_ms += ms;
+    }
+    res->trace_launches = res->iterations;
+    return VZ_SUCCESS;
+}
+
+vzStatus path_launch(vzContext ctx, const PathItem& item, hipStream_t st, RunResult* res)
 {
     PathWork* w = nullptr;
     VZ_TRY(path_work(ctx, &w));
-    PathArgs A;
-    std::memset(&A, 0, sizeof(A));
-    A.cam = make_cam(p);
-    A.subframe = p.subframe_index;
-    A.max_depth = p.max_depth;
-    A.spp = p.samples_per_pixel;
-    // 8x8 tiles; images less than 8 pixels wide or high get tiles of their
-    // shape, so that padding never multiplies the pixels by more than 4
-    A.lw = p.height < 8u ? 5u : (p.width < 8u ? 1u : 3u);
-    const uint32_t tw = 1u << A.lw, th = kTile / tw;
-    A.tiles_x = (p.width + tw - 1) / tw;
-    const uint64_t ntiles = (uint64_t)A.tiles_x * ((p.height + th - 1) / th);
-    if (ntiles * kTile > 0xFFFFFF00ull) return set_error(VZ_ERROR_CAPACITY, "image too large");
-    A.npad = (uint32_t)(ntiles * kTile);
-    const bool fp64 = (p.flags & VZ_ACCUM_FP64) != 0;
-    const bool count = (p.flags & VZ_COUNT_VISITS) != 0, timed = (p.flags & VZ_TIME_STAGES) != 0;
-
-    // the passes in as few equal chunks as the budget allows; less memory
-    // than that makes more chunks
-    auto split = [&](uint64_t most) { return (uint32_t)((A.spp + (A.spp + most - 1) / most - 1) / ((A.spp + most - 1) / most)); };
-    uint32_t chunk = split(std::max<uint64_t>(1, std::min<uint64_t>(A.spp, kPathBudget / (16ull * A.npad))));
-    for (;;) {
-        const uint64_t per = align256(4ull * A.npad * chunk) + 12ull * A.npad * chunk;
-        const uint64_t pix = chunk < A.spp ? align256((fp64 ? 24ull : 12ull) * A.npad) + 4ull * A.npad : 0ull;
-        if (grow(&w->paths, &w->paths_bytes, per) && grow(&w->pixels, &w->pixels_bytes, pix)) break;
-        if (chunk == 1u)
-            return set_error(VZ_ERROR_OUT_OF_MEMORY, "launch buffers (" + std::to_string(per + pix) + " bytes) do not fit");
-        chunk = split((chunk + 1) / 2);
-    }
-    A.seeds = (uint32_t*)w->paths;
-    A.rad = (float*)(w->paths + align256(4ull * A.npad * chunk));
-    A.sums = w->pixels;
-    A.camseed = (uint32_t*)(w->pixels + align256((fp64 ? 24ull : 12ull) * A.npad));
-    A.stats = w->stats;
-    A.counter = (uint32_t*)(w->stats + kMaxPathBlocks * kPathStats);
-    A.accum = p.accum;
-    A.image = (uint32_t*)p.image;
-    A.totals = w->h_stats;
-    const bool lds = scene->n >= 2 && scene->nw <= kLdsNodes;
-    const uint32_t resident = lds ? w->grid_lds : w->grid_mem;
-    A.refill = lds ? kRefillLds : kRefillGlobal;
-    const SceneView sc = scene->view();
-    const dim3 pix_grid((A.npad + kBlk - 1) / kBlk);
+    VZ_TRY(w->plain.init(false));
     std::vector<Event> ev;
-    uint32_t launches = 0;
+    PathOptions opt;
+    opt.count = (item.params.flags & VZ_COUNT_VISITS) != 0;
+    if (item.params.flags & VZ_TIME_STAGES) opt.events = &ev;
+    *res = RunResult();
+    res->paths = (unsigned long long)item.params.width * item.params.height * item.params.samples_per_pixel;
     auto enqueue = [&]() -> vzStatus {
         VZ_HIP_TRY(hipEventRecord(w->t0.e, st));
-        for (; A.s0 < A.spp; A.s0 += chunk, launches++) {
-            A.ns = std::min(chunk, A.spp - A.s0);
-            A.spu = kUnitPasses;
-            while (A.spu > 1u && ntiles * ((A.ns + A.spu - 1) / A.spu) < (uint64_t)kUnitRounds * resident * kWaves)
-                A.spu >>= 1;
-            A.groups = (A.ns + A.spu - 1) / A.spu;
-            A.units = (uint32_t)(ntiles * A.groups);
-            A.grid = std::min(resident, A.units);
-            hipLaunchKernelGGL(k_path_seeds, pix_grid, dim3(kBlk), 0, st, A);
-            if (timed) {
-                for (int k = 0; k < 2; k++) {
-                    ev.emplace_back();
-                    VZ_EVENT_TRY(ev.back());
-                }
-                VZ_HIP_TRY(hipEventRecord(ev[ev.size() - 2].e, st));
-            }
-            const dim3 grid(A.grid), blk(kPathBlk);
-            if (count) {
-                if (lds) hipLaunchKernelGGL((k_path<true, true>), grid, blk, 0, st, sc, A);
-                else hipLaunchKernelGGL((k_path<true, false>), grid, blk, 0, st, sc, A);
-            } else {
-                if (lds) hipLaunchKernelGGL((k_path<false, true>), grid, blk, 0, st, sc, A);
-                else hipLaunchKernelGGL((k_path<false, false>), grid, blk, 0, st, sc, A);
-            }
-            if (timed) VZ_HIP_TRY(hipEventRecord(ev.back().e, st));
-            if (fp64) hipLaunchKernelGGL(k_path_resolve<true>, pix_grid, dim3(kBlk), 0, st, A);
-            else hipLaunchKernelGGL(k_path_resolve<false>, pix_grid, dim3(kBlk), 0, st, A);
-            VZ_HIP_TRY(hipGetLastError());
+        VZ_TRY(path_enqueue_one(w, w->plain, item, opt, kPlainBudget, false, st, &res->iterations));
+        VZ_HIP_TRY(hipEventRecord(w->t1.e, st));
+        return VZ_SUCCESS;
+    };
+    return finish(w, w->plain, enqueue(), ev, st, res);
+}
+
+uint64_t tuning_budget(const vzTuning& t)
+{
+    return std::min(std::max<uint64_t>((uint64_t)t.queue_capacity * kRayBytes, 256ull << 20), kMaxSlotBudget);
+}
+
+// A batch: its items in groups as large as the slot holds, each group one
+// launch; an item too large for the slot renders by itself, a chunk of passes
+// at a time.  One stream: with the groups side by side on 2, 4 and 8 streams,
+// so that a group takes over the CUs another's last paths leave, a 24-scene
+// batch took 139-143 ms instead of 121 (groups that share the GPU also share
+// its caches).
+vzStatus path_batch(vzContext ctx, const std::vector<PathItem>& items, const vzTuning& t, hipStream_t st, RunResult* res)
+{
+    *res = RunResult();
+    if (items.empty()) return VZ_SUCCESS;
+    PathWork* w = nullptr;
+    VZ_TRY(path_work(ctx, &w));
+    PathSlot& slot = w->batch;
+    std::vector<Event> ev;
+    PathOptions opt;
+    opt.refill = t.refill_lanes;
+    opt.tile_w = t.tile_w;
+    opt.tile_h = t.tile_h;
+    for (const PathItem& it : items) {
+        opt.count |= (it.params.flags & VZ_COUNT_VISITS) != 0;
+        if (it.params.flags & VZ_TIME_STAGES) opt.events = &ev;
+        res->paths += (unsigned long long)it.params.width * it.params.height * it.params.samples_per_pixel;
+    }
+    const uint64_t budget = tuning_budget(t);
+    if (slot.paths_bytes > budget + 256) slot.free();  // a smaller tuning gives memory back
+    VZ_TRY(slot.init(true));
+    slot.used = 0;
+    // small items first, so that the slot has its size before anything runs
+    std::vector<std::vector<const PathItem*>> groups(1);
+    std::vector<const PathItem*> large;
+    uint64_t open = 0, need = 0;
+    for (const PathItem& it : items) {
+        const uint64_t n = path_count(it.params, opt);
+        if (n * kPathBytes > budget) {
+            large.push_back(&it);
+            continue;
+        }
+        if ((open + n) * kPathBytes > budget) {
+            groups.emplace_back();
+            open = 0;
+        }
+        groups.back().push_back(&it);
+        open += n;
+        need = std::max(need, open);
+    }
+    if (need) VZ_TRY(slot_reserve(slot, need));
+    auto enqueue = [&]() -> vzStatus {
+        VZ_HIP_TRY(hipEventRecord(w->t0.e, st));
+        for (const auto& g : groups) {
+            if (g.empty()) continue;
+            VZ_TRY(path_enqueue_many(w, slot, g.data(), (uint32_t)g.size(), opt, res->iterations != 0, st));
+            res->iterations++;
+        }
+        for (const PathItem* it : large) {
+            VZ_HIP_TRY(hipStreamSynchronize(st));  // its buffers may have to grow
+            VZ_TRY(path_enqueue_one(w, slot, *it, opt, budget, res->iterations != 0, st, &res->iterations));
         }
         VZ_HIP_TRY(hipEventRecord(w->t1.e, st));
         return VZ_SUCCESS;
     };
-    vzStatus rs = enqueue();
-    // the workspace is free for the next launch, on any stream, once this one
-    // has finished
-    if (hipStreamSynchronize(st) != hipSuccess && rs == VZ_SUCCESS)
-        rs = set_error(VZ_ERROR_HIP, "hipStreamSynchronize failed");
-    VZ_TRY(rs);
-    float ms = 0.0f;
-    (void)hipEventElapsedTime(&ms, w->t0.e, w->t1.e);
-    *res = RunResult();
-    res->segments = w->h_stats[0];
-    res->hits = w->h_stats[1];
-    res->node_visits = w->h_stats[2];
-    res->sphere_tests = w->h_stats[3];
-    res->paths = (unsigned long long)p.width * p.height * p.samples_per_pixel;
-    res->render_ms = ms;
-    for (size_t k = 0; k + 1 < ev.size(); k += 2) {
-        float t = 0.0f;
-        VZ_HIP_TRY(hipEventElapsedTime(&t, ev[k].e, ev[k + 1].e));
-        res->trace_ms += t;
-        res->trace_launches++;
-    }
-    if (!timed) res->trace_launches = launches;
-    res->iterations = launches;
+    VZ_TRY(finish(w, slot, enqueue(), ev, st, res));
     return VZ_SUCCESS;
 }
 

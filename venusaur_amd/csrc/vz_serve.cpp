@@ -1,19 +1,21 @@
 // vz_serve.cpp -- the serving form and the autotuner.
 //
-// Serving: a host thread owns a wavefront engine and a non-blocking stream.
-// Requests are queued FIFO by vzServerSubmit and admitted into the engine's
-// request table whenever a slot is free and the request's buffers fit the
-// HBM budget; admitted requests join the running wavefront at the next
-// iteration, so new work overlaps with requests already on the GPU
-// (continuous batching).  BVHs stay resident (vzScene objects owned by the
-// caller) and request buffers are allocated stream-ordered, so admission and
-// release never synchronise the device.  The nearest reference analogue is
-// the interactive loop that keeps the GAS and accumulator resident across
-// frames (Core/Core.cpp:358-430, Core/Renderer.h:37-54).
+// Serving: a host thread owns a few streams, each with the buffers of its
+// launches (a slot).  Requests are queued FIFO by vzServerSubmit; whenever a
+// slot is idle the requests at the head of the queue that fit it and the HBM
+// budget are rendered as one launch on its stream, at once and beside the
+// launches of the other slots, which the GPU works through in the order they
+// came: new work overlaps with requests already on the GPU (continuous
+// batching) and takes over the CUs that finishing launches leave.  BVHs stay
+// resident (vzScene objects owned by the caller) and the slots' buffers are
+// kept, so admission and release never synchronise the device.  The nearest
+// reference analogue is the interactive loop that keeps the GAS and
+// accumulator resident across frames (Core/Core.cpp:358-430,
+// Core/Renderer.h:37-54).
 //
-// Autotuner: times the caller's batch over candidate queue capacities and
-// camera-ray tile shapes and keeps the fastest (segments per millisecond),
-// cached per context.
+// Autotuner: times the caller's batch over candidate buffer sizes, camera
+// tiles and refill thresholds and keeps the fastest (segments per
+// millisecond), cached per context.
 #include <algorithm>
 #include <chrono>
 #include <condition_variable>
@@ -22,8 +24,8 @@
 #include <thread>
 #include <unordered_map>
 
-#include "vz_engine.h"
 #include "vz_internal.h"
+#include "vz_path.h"
 
 using namespace vz;
 
@@ -40,25 +42,44 @@ struct Pending {
 struct Active {
     uint64_t id;
     const vzScene_st* scene;
-    uint32_t slot;
     size_t bytes;
-    uint32_t first_step;  // first engine_step whose status includes the slot
     double submit_ms, admit_ms;
 };
+
+// Requests rendered by one launch, or one request of several launches.
+struct Flight {
+    PathSlot slot;
+    hipStream_t stream = nullptr;
+    Event done{hipEventDisableTiming};
+    std::vector<Active> active;  // empty: idle
+    bool large = false;
+};
+
+// Launches side by side: the second takes over the CUs that the first one's
+// last paths leave.  A burst of 20 requests (1k to 200k spheres, 256 to 1024
+// pixels square, 4 to 64 samples, one of 1088) took 195 ms with 2, 209 with
+// 1, 202 with 3 and 203 with 4.
+constexpr uint32_t kServeStreams = 2;
+// Paths of a launch of several requests at most.  A launch's requests finish
+// together: the burst's p50 latency is 92 ms at 8M paths, 101 at 32M and 116
+// at 64M, its throughput the same within 1%.
+constexpr uint64_t kServeGroupPaths = 16u << 20;
 
 }  // namespace
 
 struct vzServer_st {
     vzContext ctx = nullptr;
     vzServeConfig cfg{};
-    Engine* engine = nullptr;
-    hipStream_t stream = nullptr;
+    PathWork* work = nullptr;
+    PathOptions opt;
+    uint64_t slot_budget = 0;
+    std::vector<Flight> flights;
     std::thread worker;
     std::mutex mu;
     std::condition_variable cv_work, cv_done;
     std::deque<Pending> pending;
     std::unordered_map<uint64_t, vzRequestResult> results;
-    std::vector<Active> active;
+    size_t n_active = 0;
     uint64_t next_id = 1;
     size_t used_bytes = 0;
     bool stop = false;
@@ -71,29 +92,17 @@ struct vzServer_st {
         return std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     }
     void loop();
+    std::vector<Pending> admit();
+    vzStatus start(Flight& f, const std::vector<Pending>& group);
+    void harvest(Flight& f);
     // A request no longer needs its scene (finished, rejected or dropped).
     static void release_scene(const vzScene_st* sc)
     {
         const_cast<vzScene_st*>(sc)->server_refs.fetch_sub(1);
     }
-};
-
-void vzServer_st::loop()
-{
-    (void)hipSetDevice(ctx->device);
-    uint32_t k = 0;          // steps enqueued
-    uint32_t harvested = 0;  // steps whose status has been read
-    hipEvent_t ev[2];
-    (void)hipEventCreateWithFlags(&ev[0], hipEventDisableTiming);
-    (void)hipEventCreateWithFlags(&ev[1], hipEventDisableTiming);
-    auto fail = [&](vzStatus s) {
-        std::lock_guard<std::mutex> lk(mu);
-        fatal = s;
-        fatal_msg = vzGetLastError();
-        stop = true;
-        cv_done.notify_all();
-    };
-    auto reject = [&](const Pending& p, uint32_t status) {
+    // A request that will never run (mu held).
+    void reject(const Pending& p, vzStatus status)
+    {
         release_scene(p.scene);
         vzRequestResult r{};
         r.request_id = p.id;
@@ -101,109 +110,168 @@ void vzServer_st::loop()
         r.admit_ms = r.finish_ms = now_ms();
         r.status = status;
         results[p.id] = r;
-    };
-    for (;;) {
-        // 1. admit queued requests while a slot is free and the HBM budget allows
-        {
-            std::unique_lock<std::mutex> lk(mu);
-            if (k == harvested && active.empty() && pending.empty()) {
-                cv_done.notify_all();
-                cv_work.wait(lk, [&] { return stop || !pending.empty(); });
-                if (stop && pending.empty()) break;
-            }
-            while (!pending.empty() && active.size() < cfg.max_active) {
-                Pending& p = pending.front();
-                if (p.bytes > cfg.hbm_budget_bytes) {  // can never fit
-                    reject(p, VZ_ERROR_CAPACITY);
-                    pending.pop_front();
-                    continue;
-                }
-                if (used_bytes + p.bytes > cfg.hbm_budget_bytes) break;  // wait for memory
-                RunItem it;
-                it.scene = p.scene;
-                it.params = p.params;
-                uint32_t slot = 0;
-                vzStatus s = engine_admit(engine, it, stream, &slot);
-                if (s == VZ_ERROR_CAPACITY || s == VZ_ERROR_OUT_OF_MEMORY) {
-                    if (active.empty() && k == harvested) {  // nothing will free up
-                        reject(p, s);
-                        pending.pop_front();
-                        continue;
-                    }
-                    break;
-                }
-                if (s != VZ_SUCCESS) {
-                    fatal = s;
-                    fatal_msg = vzGetLastError();
-                    stop = true;
-                    cv_done.notify_all();
-                    break;
-                }
-                Active a;
-                a.id = p.id;
-                a.scene = p.scene;
-                a.slot = slot;
-                a.bytes = p.bytes;
-                a.first_step = k;
-                a.submit_ms = p.submit_ms;
-                a.admit_ms = now_ms();
-                used_bytes += p.bytes;
-                active.push_back(a);
-                pending.pop_front();
-            }
-            if (fatal != VZ_SUCCESS) break;
-        }
-        // 2. keep up to two blocks of iterations in flight
-        if (!active.empty() && k - harvested < 2u) {
-            if (engine_step(engine, stream, k) != VZ_SUCCESS || hipEventRecord(ev[k & 1u], stream) != hipSuccess) {
-                fail(VZ_ERROR_HIP);
-                break;
-            }
-            k++;
-        }
-        // 3. harvest the oldest block once two are queued (or nothing is left to queue)
-        if (k > harvested && (k - harvested >= 2u || active.empty())) {
-            uint32_t h = harvested;
-            if (hipEventSynchronize(ev[h & 1u]) != hipSuccess) {
-                fail(VZ_ERROR_HIP);
-                break;
-            }
-            harvested++;
-            double t = now_ms();
-            std::vector<Active> still;
-            for (const Active& a : active) {
-                bool act = true;
-                unsigned long long seg = 0;
-                if (h >= a.first_step) engine_slot_status(engine, h, a.slot, &act, &seg);
-                if (act) {
-                    still.push_back(a);
-                    continue;
-                }
-                if (engine_release_slot(engine, a.slot, stream) != VZ_SUCCESS) {
-                    fail(VZ_ERROR_HIP);
-                    break;
-                }
-                release_scene(a.scene);
-                std::lock_guard<std::mutex> lk(mu);
-                vzRequestResult r{};
-                r.request_id = a.id;
-                r.submit_ms = a.submit_ms;
-                r.admit_ms = a.admit_ms;
-                r.finish_ms = t;
-                r.segments = seg;
-                r.status = VZ_SUCCESS;
-                results[a.id] = r;
-                used_bytes -= a.bytes;
-            }
-            std::lock_guard<std::mutex> lk(mu);
-            active.swap(still);
-            if (fatal != VZ_SUCCESS) break;
-            cv_done.notify_all();
+    }
+    ~vzServer_st()
+    {
+        for (Flight& f : flights) {
+            f.slot.free();
+            if (f.stream) (void)hipStreamDestroy(f.stream);
         }
     }
-    (void)hipStreamSynchronize(stream);
-    (void)hipEventDestroy(ev[0]);
-    (void)hipEventDestroy(ev[1]);
+};
+
+// The next launch's requests, in arrival order, while they fit the budget,
+// the table and the slot (mu held).
+std::vector<Pending> vzServer_st::admit()
+{
+    std::vector<Pending> group;
+    uint64_t paths = 0;
+    const uint64_t most = std::min<uint64_t>(slot_budget / kPathBytes, kServeGroupPaths);
+    while (!pending.empty() && n_active < cfg.max_active) {
+        const Pending& p = pending.front();
+        if (p.bytes > cfg.hbm_budget_bytes) {  // can never fit
+            reject(p, VZ_ERROR_CAPACITY);
+            pending.pop_front();
+            continue;
+        }
+        if (used_bytes + p.bytes > cfg.hbm_budget_bytes) break;  // wait for memory
+        const uint64_t n = path_count(p.params, opt);
+        if (!group.empty() && paths + n > most) break;
+        paths += n;
+        used_bytes += p.bytes;
+        n_active++;
+        group.push_back(p);
+        pending.pop_front();
+        if (paths > most) break;  // a large request renders by itself
+    }
+    return group;
+}
+
+vzStatus vzServer_st::start(Flight& f, const std::vector<Pending>& group)
+{
+    std::vector<PathItem> items;
+    std::vector<const PathItem*> ptr;
+    items.reserve(group.size());
+    for (const Pending& p : group) items.push_back(PathItem{p.scene, p.params});
+    for (const PathItem& it : items) ptr.push_back(&it);
+    uint64_t paths = 0;
+    for (const PathItem& it : items) paths += path_count(it.params, opt);
+    f.slot.used = 0;
+    f.large = group.size() == 1 && paths * kPathBytes > slot_budget;
+    if (f.large) return path_enqueue_one(work, f.slot, items[0], opt, slot_budget, false, f.stream, nullptr);
+    VZ_TRY(slot_reserve(f.slot, paths));
+    return path_enqueue_many(work, f.slot, ptr.data(), (uint32_t)ptr.size(), opt, false, f.stream);
+}
+
+// Results of a flight whose launches have finished.
+void vzServer_st::harvest(Flight& f)
+{
+    std::lock_guard<std::mutex> lk(mu);
+    const double t = now_ms();
+    for (size_t i = 0; i < f.active.size(); i++) {
+        const Active& a = f.active[i];
+        release_scene(a.scene);
+        vzRequestResult r{};
+        r.request_id = a.id;
+        r.submit_ms = a.submit_ms;
+        r.admit_ms = a.admit_ms;
+        r.finish_ms = t;
+        r.segments = f.large ? f.slot.h_totals[0] : f.slot.h_totals[kPathStats + i];
+        r.status = VZ_SUCCESS;
+        results[a.id] = r;
+        used_bytes -= a.bytes;
+        n_active--;
+    }
+    f.active.clear();
+    cv_done.notify_all();
+}
+
+void vzServer_st::loop()
+{
+    (void)hipSetDevice(ctx->device);
+    auto fail = [&](vzStatus s) {
+        std::lock_guard<std::mutex> lk(mu);
+        fatal = s;
+        fatal_msg = vzGetLastError();
+        stop = true;
+        cv_done.notify_all();
+    };
+    for (;;) {
+        bool progress = false, busy = false;
+        // 1. finished launches
+        for (Flight& f : flights) {
+            if (f.active.empty()) continue;
+            const hipError_t e = hipEventQuery(f.done.e);
+            if (e == hipSuccess) {
+                harvest(f);
+                progress = true;
+            } else if (e == hipErrorNotReady) {
+                busy = true;
+            } else {
+                set_error(VZ_ERROR_HIP, std::string("a launch failed: ") + hipGetErrorString(e));
+                fail(VZ_ERROR_HIP);
+                goto out;
+            }
+        }
+        // 2. queued requests onto idle slots
+        for (Flight& f : flights) {
+            if (!f.active.empty()) continue;
+            std::vector<Pending> group;
+            {
+                std::lock_guard<std::mutex> lk(mu);
+                if (pending.empty()) break;
+                group = admit();
+                const double t = now_ms();
+                for (const Pending& p : group)
+                    f.active.push_back(Active{p.id, p.scene, p.bytes, p.submit_ms, t});
+                if (group.empty()) {
+                    cv_done.notify_all();  // rejected ones, if any
+                    break;
+                }
+            }
+            const vzStatus s = start(f, group);
+            if (s == VZ_ERROR_CAPACITY || s == VZ_ERROR_OUT_OF_MEMORY) {
+                // nothing of the group was enqueued beyond what the stream
+                // finishes: wait for it, and for memory if others run
+                (void)hipStreamSynchronize(f.stream);
+                std::lock_guard<std::mutex> lk(mu);
+                f.active.clear();
+                for (auto p = group.rbegin(); p != group.rend(); ++p) {
+                    used_bytes -= p->bytes;
+                    n_active--;
+                    if (busy || group.size() > 1) pending.push_front(*p);
+                    else reject(*p, s);
+                }
+                if (!busy && group.size() > 1) {
+                    // even an idle device does not hold the group: fewer at a time
+                    slot_budget = std::max<uint64_t>(slot_budget / 2, kPathBytes);
+                    progress = true;
+                }
+                cv_done.notify_all();
+                break;
+            }
+            if (s != VZ_SUCCESS || hipEventRecord(f.done.e, f.stream) != hipSuccess) {
+                if (s == VZ_SUCCESS) set_error(VZ_ERROR_HIP, "hipEventRecord failed");
+                fail(VZ_ERROR_HIP);
+                goto out;
+            }
+            progress = busy = true;
+        }
+        if (progress) continue;
+        // 3. nothing to do: wait for a submission, or a moment for the GPU
+        std::unique_lock<std::mutex> lk(mu);
+        if (busy) {
+            cv_work.wait_for(lk, std::chrono::microseconds(20));
+        } else {
+            if (pending.empty()) {
+                cv_done.notify_all();
+                if (stop) break;
+                cv_work.wait(lk, [&] { return stop || !pending.empty(); });
+            }
+        }
+    }
+out:
+    for (Flight& f : flights) (void)hipStreamSynchronize(f.stream);
 }
 
 extern "C" {
@@ -218,28 +286,29 @@ vzStatus vzServerCreate(vzContext ctx, const vzServeConfig* cfg, vzServer* out)
     s->cfg = *cfg;
     if (s->cfg.max_active == 0 || s->cfg.max_active > kMaxRequests) s->cfg.max_active = kMaxRequests;
     if (s->cfg.hbm_budget_bytes == 0) s->cfg.hbm_budget_bytes = ctx->hbm_bytes / 2;
-    EngineConfig ec;
-    // Serving defaults: a 48M-ray queue (4.8 GB for its two parities), 8x8
-    // camera tiles and the queue split 4 ways per resident step workgroup
-    // (kServeSplit).  On the first 600 requests of the 2000-request stream,
-    // all in flight at once: 5648 Mray-segments/s against 5576 for 32M, 5303
-    // for 24M and 5690 for 64M, all at split 4 (16x4 tiles at 24M: 5020).
-    ec.queue_capacity = 12u << 22;
-    ec.tile_w = 8;
-    ec.tile_h = 8;
-    if (s->cfg.tuning.queue_capacity) ec.queue_capacity = s->cfg.tuning.queue_capacity;
-    if (s->cfg.tuning.tile_w) ec.tile_w = s->cfg.tuning.tile_w;
-    if (s->cfg.tuning.tile_h) ec.tile_h = s->cfg.tuning.tile_h;
-    if (s->cfg.tuning.iters_per_graph >= 2) ec.iters_per_graph = s->cfg.tuning.iters_per_graph;
-    ec.refill_lanes = std::min<uint32_t>(s->cfg.tuning.refill_lanes, 65u);  // 0: the kernel variant's default
-    vzStatus rs = engine_create(ctx, ec, &s->engine);
-    if (rs == VZ_SUCCESS && hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking) != hipSuccess)
-        rs = set_error(VZ_ERROR_HIP, "hipStreamCreateWithFlags failed");
-    const uint32_t split = s->cfg.tuning.slice_split ? s->cfg.tuning.slice_split : kServeSplit;
-    if (rs == VZ_SUCCESS) rs = engine_serve_init(s->engine, s->stream, split);
+    // Serving defaults: the memory of a 48M-ray queue (4.8 GB) over the
+    // streams, 8x8 camera tiles
+    vzTuning t = s->cfg.tuning;
+    if (t.queue_capacity == 0) t.queue_capacity = 12u << 22;
+    s->opt.tile_w = t.tile_w ? t.tile_w : 8u;
+    s->opt.tile_h = t.tile_h ? t.tile_h : 8u;
+    s->opt.refill = std::min<uint32_t>(t.refill_lanes, 65u);  // 0: the kernel variant's default
+    const uint32_t n = std::min<uint32_t>(kServeStreams, s->cfg.max_active);
+    s->slot_budget = tuning_budget(t) / kServeStreams;
+    vzStatus rs;
+    {
+        std::lock_guard<std::mutex> lk(ctx->mu);
+        rs = path_work(ctx, &s->work);
+    }
+    s->flights = std::vector<Flight>(n);
+    for (Flight& f : s->flights) {
+        if (rs == VZ_SUCCESS && !f.done.ok()) rs = set_error(VZ_ERROR_HIP, "hipEventCreate failed");
+        if (rs == VZ_SUCCESS && hipStreamCreateWithFlags(&f.stream, hipStreamNonBlocking) != hipSuccess)
+            rs = set_error(VZ_ERROR_HIP, "hipStreamCreateWithFlags failed");
+        if (rs == VZ_SUCCESS) rs = f.slot.init(true);
+        if (rs == VZ_SUCCESS) rs = slot_reserve(f.slot, s->slot_budget / kPathBytes);
+    }
     if (rs != VZ_SUCCESS) {
-        if (s->engine) engine_destroy(s->engine);
-        if (s->stream) (void)hipStreamDestroy(s->stream);
         delete s;
         return rs;
     }
@@ -290,7 +359,7 @@ vzStatus vzServerDrain(vzServer srv)
     if (!srv) return set_error(VZ_ERROR_INVALID_VALUE, "NULL argument");
     std::unique_lock<std::mutex> lk(srv->mu);
     srv->cv_done.wait(lk, [&] {
-        return srv->fatal != VZ_SUCCESS || (srv->pending.empty() && srv->active.empty());
+        return srv->fatal != VZ_SUCCESS || (srv->pending.empty() && srv->n_active == 0);
     });
     if (srv->fatal != VZ_SUCCESS) return set_error(srv->fatal, "server stopped: " + srv->fatal_msg);
     return VZ_SUCCESS;
@@ -305,14 +374,10 @@ vzStatus vzServerDestroy(vzServer srv)
         srv->cv_work.notify_all();
     }
     if (srv->worker.joinable()) srv->worker.join();
-    (void)hipStreamSynchronize(srv->stream);
     // after a fatal error requests may remain; they will never run
     for (const Pending& p : srv->pending) vzServer_st::release_scene(p.scene);
-    for (const Active& a : srv->active) vzServer_st::release_scene(a.scene);
-    srv->pending.clear();
-    srv->active.clear();
-    engine_destroy(srv->engine);
-    (void)hipStreamDestroy(srv->stream);
+    for (const Flight& f : srv->flights)
+        for (const Active& a : f.active) vzServer_st::release_scene(a.scene);
     srv->ctx->live_servers--;
     delete srv;
     return VZ_SUCCESS;
@@ -323,10 +388,8 @@ vzStatus vzAutotune(vzContext ctx, const vzBatchItem* items, uint32_t n, vzStrea
     if (!ctx || !items || n == 0 || !out) return set_error(VZ_ERROR_INVALID_VALUE, "NULL argument or empty batch");
     // Times the batch itself, twice per candidate, and keeps each
     // candidate's faster run: the candidates are often within a few percent,
-    // and a single run let the noise pick.  The engine's render time starts
-    // after the queue allocation and graph capture, so no warm-up run is
-    // needed.  Reduced-sample probes shrank each request's pass ring and
-    // favoured small queues that lost on the real batch.
+    // and a single run let the noise pick.  The render time starts after the
+    // buffers are allocated, so no warm-up run is needed.
     std::vector<vzBatchItem> probe(items, items + n);
     for (auto& it : probe) it.params.flags &= ~(uint32_t)(VZ_COUNT_VISITS | VZ_TIME_STAGES);
     vzTuning best{};
@@ -344,7 +407,7 @@ vzStatus vzAutotune(vzContext ctx, const vzBatchItem* items, uint32_t n, vzStrea
         }
         return VZ_SUCCESS;
     };
-    // stage 1: queue capacity x camera tile at the default refill and split
+    // stage 1: buffer size x camera tile at the default refill
     const uint32_t caps[] = {1u << 22, 1u << 23, 3u << 22, 6u << 22, 8u << 22, 12u << 22};
     const uint32_t tiles[][2] = {{32, 2}, {16, 4}, {8, 8}};
     for (uint32_t cap : caps)
@@ -355,20 +418,14 @@ vzStatus vzAutotune(vzContext ctx, const vzBatchItem* items, uint32_t n, vzStrea
             cand.tile_h = t[1];
             cand.iters_per_graph = 16;
             cand.refill_lanes = 0;
-            cand.slice_split = kBatchSplit;
+            cand.slice_split = 4;
             VZ_TRY(time(cand));
         }
-    // stage 2: at the best queue and tile, the refill threshold, then the split
+    // stage 2: at the best of those, the refill threshold
     const vzTuning base = best;
     for (uint32_t refill : {25u, 33u, 49u, 57u}) {
         vzTuning cand = base;
         cand.refill_lanes = refill;
-        VZ_TRY(time(cand));
-    }
-    const vzTuning base2 = best;
-    for (uint32_t split : {1u, 2u, 8u}) {
-        vzTuning cand = base2;
-        cand.slice_split = split;
         VZ_TRY(time(cand));
     }
     {

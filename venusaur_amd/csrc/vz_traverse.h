@@ -89,7 +89,8 @@ struct Traversal {
     uint32_t npend = 0;  // DEFER: queued leaf tests (0 also for a lane that never gets a ray)
 
     // Returns true when the ray is already finished (single-sphere scene).
-    VZ_DEV bool init(const SceneView& sc, v3 o_, v3 d_, float tmin_, float tmax_, uint32_t& ns)
+    template <class Scene>
+    VZ_DEV bool init(const Scene& sc, v3 o_, v3 d_, float tmin_, float tmax_, uint32_t& ns)
     {
         o = o_;
         d = d_;
@@ -110,10 +111,10 @@ struct Traversal {
             // direction, hi for a negative one
             negm |= (inv[k] < 0.0f ? 1u : 0u) << k;
         }
-        if (sc.n == 1u) {
+        if (sc.count() == 1u) {
             float t;
             if (COUNT) ns++;
-            if (hit_gated(ldg(sc.spheres), t)) {
+            if (hit_gated(ldg(sc.sphere_array()), t)) {
                 best = t;
                 bleaf = 0;
             }
@@ -157,7 +158,8 @@ struct Traversal {
 
     // Sphere test of leaf `leaf` (sphere s); keeps the lexicographic minimum
     // of (t, prim).
-    VZ_DEV void test_leaf(const SceneView& sc, uint32_t leaf, float4 s, uint32_t& ns)
+    template <class Scene>
+    VZ_DEV void test_leaf(const Scene& sc, uint32_t leaf, float4 s, uint32_t& ns)
     {
         float t;
         if (COUNT) ns++;
@@ -167,8 +169,8 @@ struct Traversal {
                 bleaf = leaf;
                 bprim = 0xFFFFFFFFu;  // looked up lazily on a tie
             } else {
-                const uint32_t pid = ldg(sc.leaf_info + leaf) & 0x3FFFFFFFu;
-                if (bprim == 0xFFFFFFFFu && bleaf != 0xFFFFFFFFu) bprim = ldg(sc.leaf_info + bleaf) & 0x3FFFFFFFu;
+                const uint32_t pid = ldg(sc.info_array() + leaf) & 0x3FFFFFFFu;
+                if (bprim == 0xFFFFFFFFu && bleaf != 0xFFFFFFFFu) bprim = ldg(sc.info_array() + bleaf) & 0x3FFFFFFFu;
                 if (pid < bprim) {
                     best = t;
                     bleaf = leaf;
@@ -203,18 +205,19 @@ struct Traversal {
     }
 
     // DEFER: tests the queued leaves (the lane's column of lds_pend).
-    VZ_DEV void flush(const SceneView& sc, const uint32_t* lds_pend, uint32_t stride, uint32_t& ns)
+    template <class Scene>
+    VZ_DEV void flush(const Scene& sc, const uint32_t* lds_pend, uint32_t stride, uint32_t& ns)
     {
         while (npend) {
             npend--;
             const uint32_t leaf = lds_pend[npend * stride];
-            test_leaf(sc, leaf, ldg(sc.spheres + leaf), ns);
+            test_leaf(sc, leaf, ldg(sc.sphere_array() + leaf), ns);
         }
     }
 
     // One wide node visit; returns true when the traversal has finished.
-    template <class NodeSrc>
-    VZ_DEV bool step(const SceneView& sc, const NodeSrc& nodes, uint32_t* lds_node, float* lds_t,
+    template <class Scene, class NodeSrc>
+    VZ_DEV bool step(const Scene& sc, const NodeSrc& nodes, uint32_t* lds_node, float* lds_t,
                      uint32_t stride, Overflow& ov, uint32_t& nv, uint32_t& ns, uint32_t* lds_pend = nullptr)
     {
         uint4 A, B, C, D;
@@ -223,7 +226,8 @@ struct Traversal {
     }
 
     // The visit of the current node, whose 64 bytes are A..D.
-    VZ_DEV bool visit(const SceneView& sc, const uint4& A, const uint4& B, const uint4& C, const uint4& D,
+    template <class Scene>
+    VZ_DEV bool visit(const Scene& sc, const uint4& A, const uint4& B, const uint4& C, const uint4& D,
                       uint32_t* lds_node, float* lds_t, uint32_t stride, Overflow& ov, uint32_t& nv, uint32_t& ns,
                       uint32_t* lds_pend)
     {
@@ -287,7 +291,7 @@ struct Traversal {
                 lds_pend[npend * stride] = leaf;
                 npend++;
             } else {
-                test_leaf(sc, leaf, ldg(sc.spheres + leaf), ns);
+                test_leaf(sc, leaf, ldg(sc.sphere_array() + leaf), ns);
             }
             lm &= lm - 1u;
         }
