@@ -42,7 +42,7 @@
 #include <vector>
 
 #include "vz_path.h"
-#include "vz_traverse.h"
+#include "vz_traverse_lds.h"
 
 namespace vz {
 namespace {
@@ -51,14 +51,18 @@ constexpr int kPathBlk = 512;         // k_path workgroup (8 waves)
 constexpr int kWaves = kPathBlk / 64;
 constexpr int kStackS = kWideStackS;  // LDS stack slots per lane
 constexpr int kBlk = 256;
-constexpr uint32_t kLdsNodes = 256;   // a scene of at most this many 4-wide nodes is staged in LDS (16 KB)
 constexpr uint32_t kMaxPathBlocks = 8192;
 // A wave leaves the traversal to shade and take new paths once fewer than
-// this many of its lanes still trace.  Many scenes in memory, 24-scene batch:
-// 141 ms at 9, 128 at 17, 121 at 25, 117 at 33, 115 at 41, 119 at 49.
+// this many of its lanes still trace.  Nodes in LDS, 1080p book frame: 66.2
+// ms at 1, 61.7 at 5, 61.3 at 9, 61.4 at 13, 62.1 at 17, 64.6 at 25.  Many
+// scenes in memory, 24-scene batch: 141 ms at 9, 128 at 17, 121 at 25, 117 at
+// 33, 115 at 41, 119 at 49.
 constexpr uint32_t kRefillLds = 9;
 constexpr uint32_t kRefillGlobal = 41;
-constexpr uint32_t kFlushDen = 2;     // queued sphere tests run once 1/kFlushDen of the tracing lanes hold some
+// Queued sphere tests run once two thirds of the tracing lanes hold some:
+// 1080p book frame 61.1 ms against 61.3 at a half, 61.7 at a third and 65.8
+// when tested at once; a million spheres 180.1 against 181.2 and 184.5.
+constexpr uint32_t kFlushNum = 2, kFlushDen = 3;
 constexpr uint32_t kTile = 64;        // pixels of a camera tile: one wave of camera rays
 // A unit is what a wave claims at a time: up to kUnitPasses passes of one
 // tile, fewer while the units would not go round the waves kUnitRounds times.
@@ -163,6 +167,18 @@ __global__ void __launch_bounds__(kBlk) k_path_seeds(PathGroup G, PathReq one)
     }
 }
 
+// LDS of a workgroup whose nodes are in memory: traversal stacks and queued
+// sphere tests.
+struct MemScene {
+    uint32_t node[kStackS * kPathBlk];
+    float t[kStackS * kPathBlk];
+    uint32_t pend[kPend * kPathBlk];
+};
+struct NoBound {
+    template <class Scene>
+    __device__ explicit NoBound(const Scene&) {}
+};
+
 // What a lane of a many-scene launch keeps of its scene: the two arrays the
 // traversal reads.  The others are looked up in the request table where a
 // hit is shaded.
@@ -185,17 +201,15 @@ struct LaneScene {
 // its next segment in place.  A wave never waits for its lanes to finish one
 // request before it starts the next: with kManyMem each lane carries its own
 // scene.
-// COUNT: node visits and sphere tests are counted, and tests run at once so
-// that the counts follow each ray alone.
+// COUNT: node visits and sphere tests are counted, with the nodes in memory,
+// and tests run at once so that the counts follow each ray alone.
 template <bool COUNT, PathSrc SRC>
 __global__ void __launch_bounds__(kPathBlk) __attribute__((amdgpu_waves_per_eu(6))) k_path(PathGroup G, PathReq one)
 {
     constexpr bool LDSN = SRC == kOneLds || SRC == kManyLds, MANY = SRC == kManyLds || SRC == kManyMem;
-    constexpr bool DEFER = !COUNT && !LDSN;
-    __shared__ uint32_t s_node[kStackS * kPathBlk];
-    __shared__ float s_t[kStackS * kPathBlk];
-    __shared__ uint4 s_bvh[LDSN ? 4 * kLdsNodes : 1];
-    __shared__ uint32_t s_pend[DEFER ? kPend * kPathBlk : 1];
+    static_assert(!(COUNT && LDSN), "node visits are counted with the nodes in memory");
+    constexpr bool DEFER = !COUNT;  // sphere tests queued and run by many lanes together
+    __shared__ typename std::conditional<LDSN, LdsScene<kPathBlk>, MemScene>::type sh;
     __shared__ unsigned long long s_red[kPathStats][kWaves];
     const uint32_t tid = threadIdx.x, lane = __lane_id();
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(tid >> 6);
@@ -203,13 +217,14 @@ __global__ void __launch_bounds__(kPathBlk) __attribute__((amdgpu_waves_per_eu(6
     typename std::conditional<SRC == kManyMem, LaneScene, SceneView>::type sc;
     if constexpr (SRC == kManyMem) sc = LaneScene{nullptr, nullptr, nullptr};
     else sc = MANY ? G.reqs[0].sc : one.sc;
+    typename std::conditional<LDSN, PlaneBound, NoBound>::type pb(sc);
     if constexpr (LDSN) {
-        const uint32_t nn = 4u * sc.nw;
-        for (uint32_t i = tid; i < nn; i += kPathBlk) s_bvh[i] = ldg(sc.nodes + i);
+        stage_nodes(sc, sh);
         __syncthreads();
     }
-    Traversal<kStackS, COUNT, DEFER> tr;
-    Overflow ov;
+    typename std::conditional<LDSN, LdsTraversal<kPathBlk>, Traversal<kStackS, COUNT, DEFER>>::type tr;
+    typename std::conditional<LDSN, LdsOverflow, Overflow>::type ov;
+    tr.npend = 0;
     uint32_t nv = 0, ns = 0;
     uint32_t n_seg = 0, n_hit = 0;    // of the wave
     bool active = false, tdone = false, exhausted = false, fresh = true;
@@ -273,7 +288,9 @@ __global__ void __launch_bounds__(kPathBlk) __attribute__((amdgpu_waves_per_eu(6
                     depth = P.max_depth - 1u;
                     if (MANY) my_req = u_req;
                     if constexpr (SRC == kManyMem) sc = LaneScene{P.sc.nodes, P.sc.spheres, G.reqs + u_req};
-                    tdone = tr.init(sc, o, d, 0.001f, 1e16f, ns);
+                    if constexpr (LDSN) tr.init(pb, o, d, 0.001f, 1e16f);
+                    else tdone = tr.init(sc, o, d, 0.001f, 1e16f, ns);
+                    if (LDSN) tdone = false;
                     active = true;
                 }
             }
@@ -287,10 +304,10 @@ __global__ void __launch_bounds__(kPathBlk) __attribute__((amdgpu_waves_per_eu(6
         while (busy) {
             if (active && !tdone) {
                 if constexpr (LDSN)
-                    tdone = tr.step(sc, LdsNodes{s_bvh}, s_node + tid, s_t + tid, kPathBlk, ov, nv, ns, s_pend + tid);
+                    tdone = tr.step(sh, ov);
                 else
-                    tdone = tr.step(sc, GlobalNodes{sc.nodes}, s_node + tid, s_t + tid, kPathBlk, ov, nv, ns,
-                                    s_pend + tid);
+                    tdone = tr.step(sc, GlobalNodes{sc.nodes}, sh.node + tid, sh.t + tid, kPathBlk, ov, nv, ns,
+                                    sh.pend + tid);
             }
             busy = __ballot(active && !tdone);
             if (DEFER) {
@@ -299,13 +316,16 @@ __global__ void __launch_bounds__(kPathBlk) __attribute__((amdgpu_waves_per_eu(6
                 // visit queues at most 4)
                 const uint64_t pm = __ballot(tr.npend != 0u);
                 if (pm && (__ballot(tr.npend + 4u > kPend) != 0ull ||
-                           kFlushDen * (uint32_t)__popcll(pm) >= (uint32_t)__popcll(busy)))
-                    tr.flush(sc, s_pend + tid, kPathBlk, ns);
+                           kFlushDen * (uint32_t)__popcll(pm) >= kFlushNum * (uint32_t)__popcll(busy))) {
+                    if constexpr (LDSN) tr.flush(sc, sh);
+                    else tr.flush(sc, sh.pend + tid, kPathBlk, ns);
+                }
             }
             if ((uint32_t)__popcll(busy) < G.refill) break;
         }
         // every queued test has run before a lane's hit is shaded
-        if (DEFER) tr.flush(sc, s_pend + tid, kPathBlk, ns);
+        if constexpr (LDSN) tr.flush(sc, sh);
+        else if (DEFER) tr.flush(sc, sh.pend + tid, kPathBlk, ns);
         const bool fin = active && tdone;
         const uint64_t fm = __ballot(fin);
         if (fm == 0ull) continue;
@@ -342,7 +362,9 @@ __global__ void __launch_bounds__(kPathBlk) __attribute__((amdgpu_waves_per_eu(6
                     thr = mul(thr, att);
                     depth--;
                     ended = false;
-                    tdone = tr.init(sc, pos, nd, 0.001f, 1e16f, ns);
+                    if constexpr (LDSN) tr.init(pb, pos, nd, 0.001f, 1e16f);
+                    else tdone = tr.init(sc, pos, nd, 0.001f, 1e16f, ns);
+                    if (LDSN) tdone = false;
                 }
             }
             if (ended) {
@@ -548,13 +570,9 @@ vzStatus launch_group(const PathGroup& G, const PathReq& one, bool lds, const Pa
         }
         VZ_HIP_TRY(hipEventRecord((*opt.events)[opt.events->size() - 2].e, st));
     }
-    if (opt.count) {
-        if (lds) hipLaunchKernelGGL((k_path<true, L>), grid, blk, 0, st, G, one);
-        else hipLaunchKernelGGL((k_path<true, M>), grid, blk, 0, st, G, one);
-    } else {
-        if (lds) hipLaunchKernelGGL((k_path<false, L>), grid, blk, 0, st, G, one);
-        else hipLaunchKernelGGL((k_path<false, M>), grid, blk, 0, st, G, one);
-    }
+    if (opt.count) hipLaunchKernelGGL((k_path<true, M>), grid, blk, 0, st, G, one);
+    else if (lds) hipLaunchKernelGGL((k_path<false, L>), grid, blk, 0, st, G, one);
+    else hipLaunchKernelGGL((k_path<false, M>), grid, blk, 0, st, G, one);
     if (opt.events) VZ_HIP_TRY(hipEventRecord(opt.events->back().e, st));
     hipLaunchKernelGGL(k_path_resolve<MANY>, pix_grid, dim3(kBlk), 0, st, G, one);
     VZ_HIP_TRY(hipGetLastError());
@@ -683,7 +701,7 @@ vzStatus path_enqueue_one(PathWork* w, PathSlot& s, const PathItem& item, const 
         if (chunk == 1u) return rs != VZ_SUCCESS ? rs : set_error(VZ_ERROR_OUT_OF_MEMORY, "launch buffers do not fit");
         chunk = split((chunk + 1) / 2);
     }
-    const bool lds = fits_lds(item.scene);
+    const bool lds = fits_lds(item.scene) && !opt.count;
     const uint32_t resident = lds ? w->grid_lds : w->grid_mem;
     PathGroup G;
     fill_group(G, s, add);
@@ -712,7 +730,7 @@ vzStatus path_enqueue_many(PathWork* w, PathSlot& s, const PathItem* const* item
     if (s.used + n > kMaxRequests) return set_error(VZ_ERROR_INTERNAL, "request table overrun");
     PathReq* const h = s.h_reqs + s.used;
     PathReq* const d = s.reqs + s.used;
-    bool lds = fits_lds(items[0]->scene);
+    bool lds = fits_lds(items[0]->scene) && !opt.count;
     uint64_t tile_passes = 0, paths = 0;
     for (uint32_t i = 0; i < n; i++) {
         fill_request(h[i], *items[i], opt);
