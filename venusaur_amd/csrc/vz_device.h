@@ -83,6 +83,28 @@ VZ_DEV float recip_rn(float x)
     }
     return 1.0f / x;
 }
+// The traversal's 1/d: a component within 1e-20 of zero counts as 1e-20 of its
+// sign, the others are recip_rn's.  One test covers the three of an ordinary
+// ray (a sum, so that a NaN fails it); most of recip_rn's cost is its range
+// test.  Returns whether the ray was one of those.
+VZ_DEV bool ray_inverse(v3 d, float (&inv)[3])
+{
+    const float dd[3] = {d.x, d.y, d.z};
+    if (fminf(fminf(fabsf(d.x), fabsf(d.y)), fabsf(d.z)) > 1e-20f && fabsf(d.x) + fabsf(d.y) + fabsf(d.z) < 0x1p40f) {
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            const float r = __builtin_amdgcn_rcpf(dd[k]);
+            inv[k] = __builtin_fmaf(__builtin_fmaf(-dd[k], r, 1.0f), r, r);
+        }
+        return true;
+    }
+    for (int k = 0; k < 3; k++) {
+        float dk = dd[k];
+        if (!(fabsf(dk) > 1e-20f)) dk = copysignf(1e-20f, dk);
+        inv[k] = recip_rn(dk);
+    }
+    return false;
+}
 VZ_DEV v3 normalize(v3 v) { float inv = recip_rn(sqrtf(dot(v, v))); return scl(v, inv); }
 VZ_DEV v3 reflect(v3 i, v3 n) { return sub(i, scl(scl(n, 2.0f), dot(n, i))); }
 VZ_DEV v3 refract(v3 uv, v3 n, float eta)

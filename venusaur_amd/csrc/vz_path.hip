@@ -47,8 +47,11 @@
 namespace vz {
 namespace {
 
-constexpr int kPathBlk = 512;         // k_path workgroup (8 waves)
-constexpr int kWaves = kPathBlk / 64;
+// k_path workgroups, 24 waves per CU either way: three of 8 waves with the
+// nodes in memory; two of 12 with the scene in LDS, so that 160 KB hold it
+// twice and not three times.
+constexpr int kMemBlk = 512;
+constexpr int kLdsBlk = 768;
 constexpr int kStackS = kWideStackS;  // LDS stack slots per lane
 constexpr int kBlk = 256;
 constexpr uint32_t kMaxPathBlocks = 8192;
@@ -77,6 +80,8 @@ enum PathSrc {
     kManyLds,   // a table of requests of one scene, staged in LDS
     kManyMem    // a table of requests of any scenes
 };
+
+constexpr int path_threads(PathSrc src) { return src == kOneLds || src == kManyLds ? kLdsBlk : kMemBlk; }
 
 // One launch of the three kernels: a request of its own (`one`, by value) or
 // the requests of a table.
@@ -170,9 +175,9 @@ __global__ void __launch_bounds__(kBlk) k_path_seeds(PathGroup G, PathReq one)
 // LDS of a workgroup whose nodes are in memory: traversal stacks and queued
 // sphere tests.
 struct MemScene {
-    uint32_t node[kStackS * kPathBlk];
-    float t[kStackS * kPathBlk];
-    uint32_t pend[kPend * kPathBlk];
+    uint32_t node[kStackS * kMemBlk];
+    float t[kStackS * kMemBlk];
+    uint32_t pend[kPend * kMemBlk];
 };
 struct NoBound {
     template <class Scene>
@@ -204,12 +209,13 @@ struct LaneScene {
 // COUNT: node visits and sphere tests are counted, with the nodes in memory,
 // and tests run at once so that the counts follow each ray alone.
 template <bool COUNT, PathSrc SRC>
-__global__ void __launch_bounds__(kPathBlk) __attribute__((amdgpu_waves_per_eu(6))) k_path(PathGroup G, PathReq one)
+__global__ void __launch_bounds__(path_threads(SRC)) __attribute__((amdgpu_waves_per_eu(6))) k_path(PathGroup G, PathReq one)
 {
     constexpr bool LDSN = SRC == kOneLds || SRC == kManyLds, MANY = SRC == kManyLds || SRC == kManyMem;
     static_assert(!(COUNT && LDSN), "node visits are counted with the nodes in memory");
+    constexpr uint32_t NT = path_threads(SRC), kWaves = NT / 64;
     constexpr bool DEFER = !COUNT;  // sphere tests queued and run by many lanes together
-    __shared__ typename std::conditional<LDSN, LdsScene<kPathBlk>, MemScene>::type sh;
+    __shared__ typename std::conditional<LDSN, LdsScene<NT>, MemScene>::type sh;
     __shared__ unsigned long long s_red[kPathStats][kWaves];
     const uint32_t tid = threadIdx.x, lane = __lane_id();
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(tid >> 6);
@@ -219,10 +225,10 @@ __global__ void __launch_bounds__(kPathBlk) __attribute__((amdgpu_waves_per_eu(6
     else sc = MANY ? G.reqs[0].sc : one.sc;
     typename std::conditional<LDSN, PlaneBound, NoBound>::type pb(sc);
     if constexpr (LDSN) {
-        stage_nodes(sc, sh);
+        stage_scene(sc, sh);
         __syncthreads();
     }
-    typename std::conditional<LDSN, LdsTraversal<kPathBlk>, Traversal<kStackS, COUNT, DEFER>>::type tr;
+    typename std::conditional<LDSN, LdsTraversal<NT>, Traversal<kStackS, COUNT, DEFER>>::type tr;
     typename std::conditional<LDSN, LdsOverflow, Overflow>::type ov;
     tr.npend = 0;
     uint32_t nv = 0, ns = 0;
@@ -237,6 +243,7 @@ __global__ void __launch_bounds__(kPathBlk) __attribute__((amdgpu_waves_per_eu(6
     uint32_t r_seg = 0, o_req = 0, o_seg = 0;
     v3 thr = mk(0.0f, 0.0f, 0.0f);    // the lane's path
     uint32_t seed = 0, slot = 0, depth = 0, my_req = 0;
+    bool start = false;               // its next segment has not been set up
     for (;;) {
         const uint64_t m = __ballot(!active);
         if (m && !exhausted) {
@@ -282,16 +289,12 @@ __global__ void __launch_bounds__(kPathBlk) __attribute__((amdgpu_waves_per_eu(6
                 if (x < P.cam.width && y < P.cam.height) {
                     slot = P.slot0 + (u_s + p / kTile) * P.npad + u_tile * kTile + w;
                     seed = ldg(G.seeds + slot);
-                    v3 o, d;
-                    camera_ray(P.cam, x, y, seed, o, d);
+                    camera_ray(P.cam, x, y, seed, tr.o, tr.d);
                     thr = mk(1.0f, 1.0f, 1.0f);
                     depth = P.max_depth - 1u;
                     if (MANY) my_req = u_req;
                     if constexpr (SRC == kManyMem) sc = LaneScene{P.sc.nodes, P.sc.spheres, G.reqs + u_req};
-                    if constexpr (LDSN) tr.init(pb, o, d, 0.001f, 1e16f);
-                    else tdone = tr.init(sc, o, d, 0.001f, 1e16f, ns);
-                    if (LDSN) tdone = false;
-                    active = true;
+                    active = start = true;
                 }
             }
             cur += take;
@@ -300,13 +303,19 @@ __global__ void __launch_bounds__(kPathBlk) __attribute__((amdgpu_waves_per_eu(6
             if (exhausted) break;
             continue;
         }
+        if (start) {  // new paths and scattered ones alike
+            if constexpr (LDSN) tr.init(pb, tr.o, tr.d, 0.001f, 1e16f);
+            else tdone = tr.init(sc, tr.o, tr.d, 0.001f, 1e16f, ns);
+            if (LDSN) tdone = false;
+            start = false;
+        }
         uint64_t busy = __ballot(active && !tdone);
         while (busy) {
             if (active && !tdone) {
                 if constexpr (LDSN)
                     tdone = tr.step(sh, ov);
                 else
-                    tdone = tr.step(sc, GlobalNodes{sc.nodes}, sh.node + tid, sh.t + tid, kPathBlk, ov, nv, ns,
+                    tdone = tr.step(sc, GlobalNodes{sc.nodes}, sh.node + tid, sh.t + tid, kMemBlk, ov, nv, ns,
                                     sh.pend + tid);
             }
             busy = __ballot(active && !tdone);
@@ -318,14 +327,14 @@ __global__ void __launch_bounds__(kPathBlk) __attribute__((amdgpu_waves_per_eu(6
                 if (pm && (__ballot(tr.npend + 4u > kPend) != 0ull ||
                            kFlushDen * (uint32_t)__popcll(pm) >= kFlushNum * (uint32_t)__popcll(busy))) {
                     if constexpr (LDSN) tr.flush(sc, sh);
-                    else tr.flush(sc, sh.pend + tid, kPathBlk, ns);
+                    else tr.flush(sc, sh.pend + tid, kMemBlk, ns);
                 }
             }
             if ((uint32_t)__popcll(busy) < G.refill) break;
         }
         // every queued test has run before a lane's hit is shaded
         if constexpr (LDSN) tr.flush(sc, sh);
-        else if (DEFER) tr.flush(sc, sh.pend + tid, kPathBlk, ns);
+        else if (DEFER) tr.flush(sc, sh.pend + tid, kMemBlk, ns);
         const bool fin = active && tdone;
         const uint64_t fm = __ballot(fin);
         if (fm == 0ull) continue;
@@ -350,7 +359,9 @@ __global__ void __launch_bounds__(kPathBlk) __attribute__((amdgpu_waves_per_eu(6
                 L = mul(thr, sky(tr.d));
             } else if (depth > 0u) {
                 // shade (RayTracer.cu:272-440)
-                const float4 s = ldg(sc.sphere_array() + tr.bleaf);
+                float4 s;
+                if constexpr (LDSN) s = sh.spheres[tr.bleaf];
+                else s = ldg(sc.sphere_array() + tr.bleaf);
                 const uint32_t type = ldg(sc.info_array() + tr.bleaf) >> 30;
                 const float4 mat = ldg(sc.mat_array() + tr.bleaf);
                 const v3 pos = add(tr.o, scl(tr.d, tr.best));
@@ -362,9 +373,9 @@ __global__ void __launch_bounds__(kPathBlk) __attribute__((amdgpu_waves_per_eu(6
                     thr = mul(thr, att);
                     depth--;
                     ended = false;
-                    if constexpr (LDSN) tr.init(pb, pos, nd, 0.001f, 1e16f);
-                    else tdone = tr.init(sc, pos, nd, 0.001f, 1e16f, ns);
-                    if (LDSN) tdone = false;
+                    tr.o = pos;
+                    tr.d = nd;
+                    start = true;
                 }
             }
             if (ended) {
@@ -391,7 +402,7 @@ __global__ void __launch_bounds__(kPathBlk) __attribute__((amdgpu_waves_per_eu(6
     __syncthreads();
     if (tid < (uint32_t)kPathStats) {
         unsigned long long a = 0;
-        for (int w = 0; w < kWaves; w++) a += s_red[tid][w];
+        for (uint32_t w = 0; w < kWaves; w++) a += s_red[tid][w];
         G.stats[(size_t)blockIdx.x * kPathStats + tid] = a;
     }
 }
@@ -493,14 +504,14 @@ bool grow(char** p, size_t* have, size_t need)
     return true;
 }
 
-uint32_t resident_blocks(const void* kernel, uint32_t cus)
+uint32_t resident_blocks(const void* kernel, int threads, uint32_t cus)
 {
     int occ = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kernel, kPathBlk, 0) != hipSuccess || occ < 1) occ = 1;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kernel, threads, 0) != hipSuccess || occ < 1) occ = 1;
     return std::min<uint32_t>(kMaxPathBlocks, cus * (uint32_t)occ);
 }
 
-bool fits_lds(const vzScene_st* s) { return s->n >= 2 && s->nw <= kLdsNodes; }
+bool fits_lds(const vzScene_st* s) { return s->n >= 2 && s->nw <= kLdsNodes && s->n <= kLdsSpheres; }
 
 // Tile shape of a request: the options' where it is 64 pixels of powers of
 // two, 8x8 otherwise; images less than 8 pixels high or wide get tiles of
@@ -539,10 +550,10 @@ void fill_request(PathReq& A, const PathItem& item, const PathOptions& opt)
 }
 
 // Passes per unit, so that the units go round the resident waves.
-uint32_t unit_passes(uint64_t tile_passes, uint32_t resident)
+uint32_t unit_passes(uint64_t tile_passes, uint32_t waves)
 {
     uint32_t spu = kUnitPasses;
-    while (spu > 1u && tile_passes / spu < (uint64_t)kUnitRounds * resident * kWaves) spu >>= 1;
+    while (spu > 1u && tile_passes / spu < (uint64_t)kUnitRounds * waves) spu >>= 1;
     return spu;
 }
 
@@ -560,7 +571,7 @@ void fill_group(PathGroup& G, PathSlot& s, bool add)
 template <bool MANY>
 vzStatus launch_group(const PathGroup& G, const PathReq& one, bool lds, const PathOptions& opt, hipStream_t st)
 {
-    const dim3 pix_grid((G.pixels + kBlk - 1) / kBlk), grid(G.grid), blk(kPathBlk);
+    const dim3 pix_grid((G.pixels + kBlk - 1) / kBlk), grid(G.grid), blk(lds ? kLdsBlk : kMemBlk);
     constexpr PathSrc L = MANY ? kManyLds : kOneLds, M = MANY ? kManyMem : kOneMem;
     hipLaunchKernelGGL(k_path_seeds<MANY>, pix_grid, dim3(kBlk), 0, st, G, one);
     if (opt.events) {
@@ -655,8 +666,8 @@ vzStatus path_work(vzContext ctx, PathWork** out)
             return set_error(VZ_ERROR_HIP, "hipEventCreate failed");
         }
         const uint32_t cus = ctx->num_cus ? ctx->num_cus : 256;
-        w->grid_lds = resident_blocks(reinterpret_cast<const void*>(k_path<false, kOneLds>), cus);
-        w->grid_mem = resident_blocks(reinterpret_cast<const void*>(k_path<false, kManyMem>), cus);
+        w->grid_lds = resident_blocks(reinterpret_cast<const void*>(k_path<false, kOneLds>), kLdsBlk, cus);
+        w->grid_mem = resident_blocks(reinterpret_cast<const void*>(k_path<false, kManyMem>), kMemBlk, cus);
         ctx->path = w;
     }
     *out = ctx->path;
@@ -713,7 +724,7 @@ vzStatus path_enqueue_one(PathWork* w, PathSlot& s, const PathItem& item, const 
     A.camseed = (uint32_t*)(s.pixels + sum_bytes);
     for (A.s0 = 0; A.s0 < A.spp; A.s0 += chunk) {
         A.ns = std::min(chunk, A.spp - A.s0);
-        A.spu = unit_passes(ntiles * A.ns, resident);
+        A.spu = unit_passes(ntiles * A.ns, resident * (lds ? kLdsBlk : kMemBlk) / 64);
         A.groups = (A.ns + A.spu - 1) / A.spu;
         G.units = (uint32_t)(ntiles * A.groups);
         G.grid = std::min(resident, G.units);
@@ -741,7 +752,7 @@ vzStatus path_enqueue_many(PathWork* w, PathSlot& s, const PathItem* const* item
     if (paths * kPathBytes + 256 > s.paths_bytes || paths * kPathBytes > kMaxSlotBudget)
         return set_error(VZ_ERROR_INTERNAL, "launch larger than its slot");
     const uint32_t resident = lds ? w->grid_lds : w->grid_mem;
-    const uint32_t spu = unit_passes(tile_passes, resident);
+    const uint32_t spu = unit_passes(tile_passes, resident * (lds ? kLdsBlk : kMemBlk) / 64);
     PathGroup G;
     fill_group(G, s, add);
     uint32_t slot0 = 0;

@@ -99,13 +99,10 @@ struct Traversal {
         bleaf = 0xFFFFFFFFu;
         bprim = 0xFFFFFFFFu;
         npend = 0;
-        const float dd[3] = {d.x, d.y, d.z};
+        ray_inverse(d, inv);
         negm = 0u;
 #pragma unroll
         for (int k = 0; k < 3; k++) {
-            float dk = dd[k];
-            if (!(fabsf(dk) > 1e-20f)) dk = copysignf(1e-20f, dk);
-            inv[k] = recip_rn(dk);
             // lo <= hi and rounding is monotone, so (lo - o) * inv <= (hi - o) * inv
             // exactly when inv > 0: the near plane is lo for a positive
             // direction, hi for a negative one

@@ -11,8 +11,9 @@
 // Measured against the packed nodes in LDS (64 bytes, decoded at every
 // visit, sphere tests at once, children ranked pair by pair): the 1080p book
 // frame at 256 samples 78.1 -> 61.1 ms, VALU instructions 3.37e10 -> 2.49e10 a
-// launch of 128 passes.  53 KB of LDS per 512 threads keep three workgroups
-// on a CU.
+// launch of 128 passes.  The spheres are staged too (60.7 -> 59.1 ms with one
+// set-up for camera and scattered rays): a queued test otherwise waits for the
+// L1.  78 KB of LDS per 768 threads keep two workgroups, 24 waves, on a CU.
 //
 // Node, 112 bytes at a byte offset that is also its number:
 //   0   float lo[4], hi[4] of the slots on x;  32 on y;  64 on z
@@ -32,6 +33,7 @@
 namespace vz {
 
 constexpr uint32_t kLdsNodes = 256;        // a scene of at most this many 4-wide nodes is staged
+constexpr uint32_t kLdsSpheres = 3 * kLdsNodes + 1;  // leaves of so many 4-wide nodes, at most
 constexpr uint32_t kLdsNodeBytes = 112;
 constexpr uint32_t kLdsPend = 8;           // queued leaf tests per lane
 constexpr uint32_t kLdsKeyMask = 0xFFFF0000u;
@@ -41,14 +43,17 @@ constexpr uint32_t kLdsStack = kWideStackS;  // stack words per lane, the oldest
 template <uint32_t NT>
 struct LdsScene {
     uint4 nodes[kLdsNodes * kLdsNodeBytes / 16];
+    float4 spheres[kLdsSpheres];
     uint32_t stack[kLdsStack * NT];
     uint16_t pend[kLdsPend * NT];
 };
 
-// Decodes the packed nodes (64 bytes, vz_api.h) into LDS, whole workgroup.
+// Copies the spheres into LDS and decodes the packed nodes (64 bytes,
+// vz_api.h), whole workgroup.
 template <uint32_t NT>
-VZ_DEV void stage_nodes(const SceneView& sc, LdsScene<NT>& sh)
+VZ_DEV void stage_scene(const SceneView& sc, LdsScene<NT>& sh)
 {
+    for (uint32_t i = threadIdx.x; i < sc.n; i += NT) sh.spheres[i] = ldg(sc.spheres + i);
     for (uint32_t i = threadIdx.x; i < sc.nw; i += NT) {
         const uint4 A = ldg(sc.nodes + 4 * i), B = ldg(sc.nodes + 4 * i + 1);
         const uint4 C = ldg(sc.nodes + 4 * i + 2), D = ldg(sc.nodes + 4 * i + 3);
@@ -81,7 +86,9 @@ VZ_DEV void stage_nodes(const SceneView& sc, LdsScene<NT>& sh)
     }
 }
 
-// The largest |plane| of a scene on each axis: every lo plane is at or above
+// 2^-20 of the largest |plane| of a scene on each axis, at least 2^-70 (|1/d|
+// of an ordinary ray is above 2^-41, so that its bound stays a normal number):
+// every lo plane is at or above
 // the root box's lo corner, every hi plane at most one step of its node's
 // grid above an exact box, and no node's grid is coarser than the root's.
 struct PlaneBound {
@@ -92,7 +99,7 @@ struct PlaneBound {
         const float no[3] = {__uint_as_float(A.x), __uint_as_float(A.y), __uint_as_float(A.z)};
         for (int k = 0; k < 3; k++) {
             const float s = scale_of(A.w, k);
-            p[k] = fmaxf(fabsf(no[k]), fabsf(__builtin_fmaf(257.0f, s, no[k])));
+            p[k] = fmaxf(0x1p-20f * fmaxf(fabsf(no[k]), fabsf(__builtin_fmaf(257.0f, s, no[k]))), 0x1p-70f);
         }
     }
 };
@@ -126,18 +133,21 @@ struct LdsTraversal {
         best = tmax_;
         bleaf = 0xFFFFFFFFu;
         node = sp = bottom = npend = 0u;
-        const float dd[3] = {d.x, d.y, d.z}, oo[3] = {o.x, o.y, o.z};
+        const bool ordinary = ray_inverse(d, inv);
+        const float oo[3] = {o.x, o.y, o.z};
 #pragma unroll
         for (int k = 0; k < 3; k++) {
-            float dk = dd[k];
-            if (!(fabsf(dk) > 1e-20f)) dk = copysignf(1e-20f, dk);
-            inv[k] = recip_rn(dk);
             off[k] = inv[k] < 0.0f ? 16u : 0u;
             const float m = oo[k] * inv[k];
-            const float e = fmaxf((pb.p[k] + fabsf(oo[k])) * fabsf(inv[k]) * 0x1p-20f, 0x1p-126f);
+            const float e = __builtin_fmaf(fabsf(oo[k]), 0x1p-20f, pb.p[k]) * fabsf(inv[k]);
             bn[k] = -m - e;
             bf[k] = __builtin_fmaf(2.0f, e, -m);
         }
+        if (!ordinary)  // a bound that may underflow
+            for (int k = 0; k < 3; k++) {
+                bn[k] -= 0x1p-126f;
+                bf[k] += 0x1p-125f;
+            }
     }
 
     // As Traversal::hit_gated.
@@ -163,7 +173,7 @@ struct LdsTraversal {
             npend--;
             const uint32_t leaf = sh.pend[npend * NT + threadIdx.x];
             float t;
-            if (hit_gated(ldg(sc.spheres + leaf), t)) {
+            if (hit_gated(sh.spheres[leaf], t)) {
                 if (t < best) {
                     best = t;
                     bleaf = leaf;
