@@ -9,6 +9,7 @@ import pytest
 import oracle as O
 from util import GpuTarget, book_lookat, box_lookat, gpu_params, oracle_params
 from venusaur_amd import api
+from venusaur_amd.hipmem import DeviceBuffer
 
 pytestmark = pytest.mark.gpu
 
@@ -74,4 +75,41 @@ def test_launch_of_several_chunks(ctx, book, fp64):
         out.append((st.segments, st.paths, tgt.accum_host(), tgt.image_host()))
     assert out[0][:2] == out[1][:2]
     assert np.array_equal(out[0][2], out[1][2]) and np.array_equal(out[0][3], out[1][3])
+    sc.close()
+
+
+# without stats the rays go through persistent waves (a small scene in LDS):
+# sizes around a wave, a workgroup and all resident waves, and ray intervals
+# that start behind the origin, end before it, or are empty
+@pytest.mark.parametrize("kind", ["book", "one", "lds", "mem"])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 769, 49153, 500001])
+def test_trace_without_stats(ctx, book, kind, n):
+    say(f"case: hits without stats {kind} n={n}")
+    (s, m), look = _scene(kind, book)
+    rng = np.random.default_rng([n, 3])
+    rays = np.zeros(n, api.RAY_DT)
+    pick = s[rng.integers(0, len(s), n)]
+    for f, c in (("ox", "cx"), ("oy", "cy"), ("oz", "cz")):
+        rays[f] = rng.uniform(-30, 30, n)
+        rays["d" + f[1]] = pick[c] - rays[f] + rng.normal(0, 0.3, n)
+    rays["dx"][::17] = 0.0
+    rays["dy"][::23] = 0.0
+    rays["tmin"], rays["tmax"] = 0.001, 1e16
+    k = rng.integers(0, 6, n)
+    rays["tmin"][k == 1], rays["tmax"][k == 1] = -50.0, 50.0
+    rays["tmin"][k == 2], rays["tmax"][k == 2] = -1e16, 1e16
+    rays["tmin"][k == 3], rays["tmax"][k == 3] = 0.0, 0.5
+    rays["tmin"][k == 4], rays["tmax"][k == 4] = 0.9, 0.2
+    sc = api.Scene(ctx, s, m)
+    rb = DeviceBuffer.from_array(rays)
+    hits = []
+    for call in (sc.trace, sc.trace_noalloc):
+        h = DeviceBuffer(n * 8)
+        call(rb.value, n, h.value)
+        hits.append(h.download(api.HIT_DT))
+    want = O.trace_brute(s, rays[:20000])
+    assert hits[0][:20000].tobytes() == want.tobytes()
+    h = DeviceBuffer(n * 8)
+    sc.trace(rb.value, n, h.value, stats=True)
+    assert hits[0].tobytes() == hits[1].tobytes() == h.download(api.HIT_DT).tobytes()
     sc.close()

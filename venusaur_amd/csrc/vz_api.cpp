@@ -342,6 +342,12 @@ vzStatus vzTraceClosest(vzScene scene, const vzRay* rays, uint32_t n, vzHit* hit
 {
     if (!scene || (n && (!rays || !hits))) return set_error(VZ_ERROR_INVALID_VALUE, "NULL argument");
     hipStream_t st = as_stream(stream);
+    if (!stats) {
+        vzStatus rs = trace_hits(scene->ctx, scene->view(), rays, n, hits, st);
+        if (hipStreamSynchronize(st) != hipSuccess && rs == VZ_SUCCESS)
+            rs = set_error(VZ_ERROR_HIP, "hipStreamSynchronize failed");
+        return rs;
+    }
     // per-workgroup partial counters, then the 4 summed counters
     const size_t nparts = (size_t)trace_blocks(n) * kTraceParts;
     DevCounters c;
@@ -350,28 +356,26 @@ vzStatus vzTraceClosest(vzScene scene, const vzRay* rays, uint32_t n, vzHit* hit
     VZ_EVENT_TRY(e0);
     VZ_EVENT_TRY(e1);
     VZ_HIP_TRY(hipEventRecord(e0.e, st));
-    vzStatus rs = trace_rays(scene->view(), rays, n, hits, st, stats != nullptr, c.d, c.d + nparts);
+    vzStatus rs = trace_rays(scene->view(), rays, n, hits, st, c.d, c.d + nparts);
     unsigned long long h[8] = {};
     if (rs == VZ_SUCCESS && hipEventRecord(e1.e, st) != hipSuccess)
         rs = set_error(VZ_ERROR_HIP, "hipEventRecord failed");
-    if (rs == VZ_SUCCESS && stats &&
+    if (rs == VZ_SUCCESS &&
         hipMemcpyAsync(h, c.d + nparts, 4 * sizeof(unsigned long long), hipMemcpyDeviceToHost, st) != hipSuccess)
         rs = set_error(VZ_ERROR_HIP, "hipMemcpyAsync of the trace counters failed");
     // c.d is freed on return: the kernel must be done with it, on every path
     if (hipStreamSynchronize(st) != hipSuccess && rs == VZ_SUCCESS)
         rs = set_error(VZ_ERROR_HIP, "hipStreamSynchronize failed");
     VZ_TRY(rs);
-    if (stats) {
-        float ms = 0.0f;
-        (void)hipEventElapsedTime(&ms, e0.e, e1.e);
-        std::memset(stats, 0, sizeof(*stats));
-        stats->segments = h[0];
-        stats->node_visits = h[2];
-        stats->sphere_tests = h[3];
-        stats->render_ms = ms;
-        stats->trace_ms = ms;
-        stats->trace_launches = 1;
-    }
+    float ms = 0.0f;
+    (void)hipEventElapsedTime(&ms, e0.e, e1.e);
+    std::memset(stats, 0, sizeof(*stats));
+    stats->segments = h[0];
+    stats->node_visits = h[2];
+    stats->sphere_tests = h[3];
+    stats->render_ms = ms;
+    stats->trace_ms = ms;
+    stats->trace_launches = 1;
     return VZ_SUCCESS;
 }
 
@@ -391,19 +395,18 @@ vzStatus vzTraceClosestNoAlloc(vzScene scene, const vzRay* rays, uint32_t n, vzH
         return set_error(VZ_ERROR_INVALID_VALUE, "the current device is not the scene's device");
     if (!ctx->trace_scratch) return set_error(VZ_ERROR_INTERNAL, "trace scratch address not set");
     hipStream_t st = as_stream(stream);
+    if (!stats) return trace_hits(ctx, scene->view(), rays, n, hits, st);
     unsigned long long* parts = ctx->trace_scratch;
     unsigned long long* counters = parts + (size_t)kTraceScratchBlocks * kTraceParts;
-    VZ_TRY(trace_rays(scene->view(), rays, n, hits, st, stats != nullptr, parts, counters));
-    if (stats) {
-        unsigned long long h[4] = {};
-        VZ_HIP_TRY(hipMemcpyAsync(h, counters, sizeof(h), hipMemcpyDeviceToHost, st));
-        VZ_HIP_TRY(hipStreamSynchronize(st));
-        std::memset(stats, 0, sizeof(*stats));
-        stats->segments = h[0];
-        stats->node_visits = h[2];
-        stats->sphere_tests = h[3];
-        stats->trace_launches = 1;
-    }
+    VZ_TRY(trace_rays(scene->view(), rays, n, hits, st, parts, counters));
+    unsigned long long h[4] = {};
+    VZ_HIP_TRY(hipMemcpyAsync(h, counters, sizeof(h), hipMemcpyDeviceToHost, st));
+    VZ_HIP_TRY(hipStreamSynchronize(st));
+    std::memset(stats, 0, sizeof(*stats));
+    stats->segments = h[0];
+    stats->node_visits = h[2];
+    stats->sphere_tests = h[3];
+    stats->trace_launches = 1;
     return VZ_SUCCESS;
 }
 

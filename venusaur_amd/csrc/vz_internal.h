@@ -188,11 +188,13 @@ void lbvh_free(vzScene s);
 // vz_trace.hip
 // Workgroups of a trace of n rays (each writes kTraceParts partial counters).
 uint32_t trace_blocks(uint32_t n);
-// Closest hits of n rays; parts holds trace_blocks(n) * kTraceParts words,
+// Closest hits of n rays, enqueued.
+vzStatus trace_hits(vzContext ctx, const SceneView& sc, const vzRay* rays, uint32_t n, vzHit* hits, hipStream_t st);
+// The same, counted; parts holds trace_blocks(n) * kTraceParts words,
 // counters 4 words (segments, 0, node visits, sphere tests), both device
 // memory written (not accumulated) by the call.
 vzStatus trace_rays(const SceneView& sc, const vzRay* rays, uint32_t n, vzHit* hits,
-                    hipStream_t st, bool count, unsigned long long* parts, unsigned long long* counters);
+                    hipStream_t st, unsigned long long* parts, unsigned long long* counters);
 // Device address of the current device's fixed trace scratch:
 // kTraceScratchBlocks * kTraceParts partial words, then 8 counter words.
 vzStatus trace_scratch_address(unsigned long long** out);

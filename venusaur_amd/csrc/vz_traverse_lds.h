@@ -109,7 +109,10 @@ struct LdsOverflow {
     uint32_t w[kWideOverflow];
 };
 
-template <uint32_t NT>
+// ANYT: tmin may be negative or NaN.  Entries then hold distances from zero
+// up and none is dropped for its distance while the best hit lies behind the
+// origin.
+template <uint32_t NT, bool ANYT = false>
 struct LdsTraversal {
     v3 o, d;
     float inv[3], bn[3], bf[3];
@@ -177,7 +180,8 @@ struct LdsTraversal {
                 if (t < best) {
                     best = t;
                     bleaf = leaf;
-                } else {  // t == best
+                } else {  // a tie
+                    best = t;
                     const uint32_t pid = ldg(sc.leaf_info + leaf) & 0x3FFFFFFFu;
                     const uint32_t bpid =
                         bleaf == 0xFFFFFFFFu ? 0xFFFFFFFFu : ldg(sc.leaf_info + bleaf) & 0x3FFFFFFFu;
@@ -227,7 +231,7 @@ struct LdsTraversal {
             const float lo_t = fmaxf(fmaxf(fmaxf(tmin, n3[0]), n3[1]), n3[2]);
             const float hi_t = fminf(fminf(fminf(lim, f3[0]), f3[1]), f3[2]);
             hit[c] = lo_t <= hi_t;
-            const uint32_t e = ((__float_as_uint(lo_t) & kLdsKeyMask) | (node + 96u + 4u * c)) | (w[c] & kLdsKeyMask);
+            const uint32_t e = ((__float_as_uint(ANYT ? fmaxf(lo_t, 0.0f) : lo_t) & kLdsKeyMask) | (node + 96u + 4u * c)) | (w[c] & kLdsKeyMask);
             key[c] = hit[c] ? e : 0xFFFFFFFFu;
         }
 #pragma unroll
@@ -267,7 +271,7 @@ struct LdsTraversal {
                 } else {
                     e = sh.stack[(sp % kLdsStack) * NT + threadIdx.x];
                 }
-                if (__uint_as_float(e & kLdsKeyMask) <= lim) break;
+                if (__uint_as_float(e & kLdsKeyMask) <= (ANYT ? fmaxf(lim, 0.0f) : lim)) break;
             }
         }
         node = *reinterpret_cast<const uint32_t*>(base + (e & 0xFFFFu));
