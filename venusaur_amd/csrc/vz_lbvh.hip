@@ -385,12 +385,20 @@ __global__ void __launch_bounds__(kBlk) k_karras(const uint32_t* __restrict__ K,
 // tree stays within the traversal's kMaxWideDepth.
 // Nodes use the Karras layout (children g and g + 1 for a split after leaf
 // position g, the root is node 0), so refit, collapse and traversal are the
-// LBVH's.  One workgroup, level by level: each wave takes one range of the
-// level per round.  Bin boxes are kept as order-preserving integer keys and
-// merged with LDS integer min/max, counts with adds, so the bins do not
-// depend on the order lanes ran in; the sweep and the partition are
-// sequential in bin and leaf order.  The result equals the oracle's
-// sah_range bit for bit.
+// LBVH's.  One workgroup; a wave splits a range by itself.  Bin boxes are
+// kept as order-preserving integer keys and merged with LDS integer min/max,
+// counts with adds, so the bins do not depend on the order lanes ran in; the
+// sweep's unions are exact in any order and the partition is stable.  The
+// result equals the oracle's sah_range bit for bit.
+//
+// What a split costs is the latency of its cross-lane steps, some 500 of
+// them when every step of every scan was a shuffle through the LDS crossbar,
+// and the barriers of a workgroup that took one range per wave and round:
+// 409 us for the book scene's 486 spheres, 3.15 ms for the 1536 treelets of a
+// million.  Scans and reductions now run in DPP (four-cycle VALU moves
+// inside and between rows of 16 lanes), the prefix and the suffix of an axis
+// side by side in the two halves of the wave, and waves take ranges from a
+// queue without barriers: 173 us and 1.21 ms.
 constexpr uint32_t kSahMaxPrims = 1024;
 constexpr int kSahBins = 32;
 constexpr uint32_t kSahDepthCap = 24;
@@ -402,11 +410,20 @@ constexpr uint32_t kSahDepthCap = 24;
 // spheres up they visit 4-6% fewer.
 constexpr uint32_t kTreeletMinPrims = 131072;
 constexpr uint32_t kTreeletBlocks = 2048;  // grid of k_sah_treelets (grid-stride over the treelets)
-constexpr int kSahWaves = 8;
-constexpr int kSahThreads = 64 * kSahWaves;
+constexpr int kSahWaves = 8;       // of a treelet's workgroup
+constexpr int kSahSoloWaves = 16;  // of the one workgroup that builds a small scene
 constexpr int kSahBinWords = 3 * kSahBins * 7;  // per wave: [axis][bin] lo xyz, hi xyz keys, count
 static_assert(kSahMaxPrims <= kRefitLeaves, "every SAH range lies in one refit workgroup");
 static_assert(kSahWaves * kSahBinWords >= (int)kSahMaxPrims, "the bins hold a treelet's keys at the end");
+// A wave goes on with the larger part of a split; the smaller one goes to the
+// queue from kSahShare spheres up (at most kSahMaxPrims / kSahShare of them),
+// and is finished first otherwise.
+constexpr uint32_t kSahShare = 24;
+constexpr uint32_t kSahTasks = 64;
+static_assert(kSahMaxPrims / kSahShare + 1 + kSahSoloWaves <= kSahTasks, "a ticket per task and waiting wave");
+constexpr uint32_t kSahLocal = 8;  // ranges a wave has put aside: each at most half of the one before
+static_assert((kSahShare >> kSahLocal) == 0, "the smaller parts halve");
+constexpr uint32_t kSahNone = 0xFFFFFFFFu;
 static_assert(kSahDepthCap + 10 + 1 <= kMaxWideDepth, "SAH tree depth within the traversal stack");
 
 __device__ __forceinline__ uint32_t ord_key(float f)
@@ -429,31 +446,68 @@ __device__ __forceinline__ float box_area6(const float* b)
     const float dx = b[3] - b[0], dy = b[4] - b[1], dz = b[5] - b[2];
     return dx * dy + dy * dz + dz * dx;
 }
-__device__ __forceinline__ float wave_min(float v)
+// v of another lane by DPP; lanes without a source keep their own.
+template <int CTRL, int ROWS = 0xF>
+__device__ __forceinline__ float dpp_f(float v)
 {
-    for (int o = 32; o >= 1; o >>= 1) v = fminf(v, __shfl_xor(v, o));
-    return v;
+    const int x = __float_as_int(v);
+    return __int_as_float(__builtin_amdgcn_update_dpp(x, x, CTRL, ROWS, 0xF, false));
 }
-__device__ __forceinline__ float wave_max(float v)
+template <int CTRL, int ROWS = 0xF>
+__device__ __forceinline__ uint32_t dpp_add(uint32_t v)  // v + v of another lane, + 0 where there is none
 {
-    for (int o = 32; o >= 1; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
-    return v;
+    return v + (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xF, false);
 }
-__device__ __forceinline__ uint32_t wave_sum(uint32_t v)
+constexpr int kRowShr = 0x110, kRowBcast15 = 0x142, kRowBcast31 = 0x143;
+// Inclusive prefix in each half of the wave (lanes 0-31, 32-63).
+template <bool MIN>
+__device__ __forceinline__ float half_scan(float v)
 {
-    for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
-    return v;
+    auto op = [](float a, float b) { return MIN ? fminf(a, b) : fmaxf(a, b); };
+    v = op(v, dpp_f<kRowShr + 1>(v));
+    v = op(v, dpp_f<kRowShr + 2>(v));
+    v = op(v, dpp_f<kRowShr + 4>(v));
+    v = op(v, dpp_f<kRowShr + 8>(v));
+    return op(v, dpp_f<kRowBcast15, 0xA>(v));
+}
+__device__ __forceinline__ uint32_t half_scan_add(uint32_t v)
+{
+    v = dpp_add<kRowShr + 1>(v);
+    v = dpp_add<kRowShr + 2>(v);
+    v = dpp_add<kRowShr + 4>(v);
+    v = dpp_add<kRowShr + 8>(v);
+    return dpp_add<kRowBcast15, 0xA>(v);
+}
+// Over the whole wave, the same value in every lane.
+template <bool MIN>
+__device__ __forceinline__ float wave_reduce(float v)
+{
+    v = half_scan<MIN>(v);
+    const float o = dpp_f<kRowBcast31, 0xC>(v);
+    v = MIN ? fminf(v, o) : fmaxf(v, o);
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+// Orders LDS accesses of the wave's lanes (which the hardware runs in order)
+// for the compiler, and brings its lanes together after a branch that only
+// some took.
+__device__ __forceinline__ void wave_order()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 
-// LDS of one treelet build: the range's spheres by local index (gathered
-// once: every phase of every round reads them), the local permutation, two
-// level lists of ranges, and per wave the bins.
+// LDS of one treelet build by NW waves: the range's spheres by local index
+// (gathered once), the local permutation, the queue of ranges, and per wave
+// the ranges put aside and the bins.  A range is (a | b << 10 | depth << 20
+// local, node index).
+template <int NW>
 struct SahShared {
     float4 sph[kSahMaxPrims];
     uint32_t perm[kSahMaxPrims], tmp[kSahMaxPrims];
-    uint2 task[2][kSahMaxPrims / 2];  // (a | b << 10 local, node index)
-    uint32_t ntask[2];
-    uint32_t bin[kSahWaves][kSahBinWords];
+    uint2 task[kSahTasks];            // .x kSahNone: not written yet
+    uint32_t head, tail, open;        // tickets taken, tasks written, tasks not finished
+    uint2 local[NW][kSahLocal];
+    uint32_t bin[NW][kSahBinWords];
 };
 
 // The SAH split of a range of two spheres [x, x + 1] (node `self`: the
@@ -465,18 +519,18 @@ struct SahShared {
 // what the binned sweep gives for two spheres (they fall in bins 0 and 31).
 __device__ __forceinline__ void sah_pair(uint32_t x, uint32_t f, uint32_t self, uint32_t d,
                                          uint32_t* __restrict__ child, uint32_t* __restrict__ parent_leaf,
-                                         SahShared& sh)
+                                         const float4* sph, uint32_t* perm)
 {
     const uint32_t X = f + x;  // split after leaf X: both children leaves
-    const float4 s0 = sh.sph[sh.perm[x]], s1 = sh.sph[sh.perm[x + 1u]];
+    const float4 s0 = sph[perm[x]], s1 = sph[perm[x + 1u]];
     if (d < kSahDepthCap) {
         for (int k = 0; k < 3; k++) {
             const float c0 = sah_cen(s0, k), c1 = sah_cen(s1, k);
             if (c0 != c1) {
                 if (c0 > c1) {
-                    const uint32_t t = sh.perm[x];
-                    sh.perm[x] = sh.perm[x + 1u];
-                    sh.perm[x + 1u] = t;
+                    const uint32_t t = perm[x];
+                    perm[x] = perm[x + 1u];
+                    perm[x + 1u] = t;
                 }
                 break;
             }
@@ -488,192 +542,229 @@ __device__ __forceinline__ void sah_pair(uint32_t x, uint32_t f, uint32_t self, 
     child[self] = X | (3u << 30);
 }
 
+// Splits the range [a, b] (at least 3 spheres) at depth d, by one wave: its
+// permutation is partitioned; returns the last index of the left part.
+__device__ __forceinline__ uint32_t sah_split(const float4* sph, uint32_t* perm, uint32_t* tmp, uint32_t* bins, uint32_t a,
+                                              uint32_t b, uint32_t d)
+{
+    const uint32_t lane = __lane_id(), m = b - a + 1u;
+    // centre bounds; a range of at most a wave stays in registers
+    float lo[3] = {3.4e38f, 3.4e38f, 3.4e38f}, hi[3] = {-3.4e38f, -3.4e38f, -3.4e38f};
+    uint32_t p = 0;
+    float4 sp = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (uint32_t i = a + lane; i <= b; i += 64u) {
+        p = perm[i];
+        sp = sph[p];
+        for (int k = 0; k < 3; k++) {
+            lo[k] = fminf(lo[k], sah_cen(sp, k));
+            hi[k] = fmaxf(hi[k], sah_cen(sp, k));
+        }
+    }
+    float ext[3];
+    bool any = false;
+    for (int k = 0; k < 3; k++) {
+        lo[k] = wave_reduce<true>(lo[k]);
+        hi[k] = wave_reduce<false>(hi[k]);
+        ext[k] = hi[k] - lo[k];
+        any = any || ext[k] > 0.0f;
+    }
+    if (!any || d >= kSahDepthCap) return a + m / 2u - 1u;
+    for (int x = (int)lane; x < kSahBinWords; x += 64) bins[x] = x % 7 < 3 ? 0xFFFFFFFFu : 0u;
+    wave_order();
+    int mine[3] = {0, 0, 0};
+    for (uint32_t i = a + lane; i <= b; i += 64u) {
+        if (m > 64u) sp = sph[perm[i]];
+        const float rr = fabsf(sp.w);
+        const uint32_t klo[3] = {ord_key(sp.x - rr), ord_key(sp.y - rr), ord_key(sp.z - rr)};
+        const uint32_t khi[3] = {ord_key(sp.x + rr), ord_key(sp.y + rr), ord_key(sp.z + rr)};
+        for (int k = 0; k < 3; k++) {
+            if (!(ext[k] > 0.0f)) continue;
+            mine[k] = sah_bin(sah_cen(sp, k), lo[k], ext[k]);
+            uint32_t* bn = &bins[(k * kSahBins + mine[k]) * 7];
+            for (int q = 0; q < 3; q++) {
+                atomicMin(&bn[q], klo[q]);
+                atomicMax(&bn[3 + q], khi[q]);
+            }
+            atomicAdd(&bn[6], 1u);
+        }
+    }
+    wave_order();
+    // The cheapest split of each axis: lane j < 32 holds the union of bins
+    // 0..j (min and max, exact in any order), lane 32 + j that of bins 31-j..31;
+    // the split after bin j adds lane j's and lane 62 - j's products.
+    int bk = -1, bj = 0;
+    uint32_t nl = 0;
+    float bc = 0.0f;
+    for (int k = 0; k < 3; k++) {
+        if (!(ext[k] > 0.0f)) continue;
+        const int j = (int)(lane < 32u ? lane : 63u - lane);
+        const uint32_t* bn = &bins[(k * kSahBins + j) * 7];
+        uint32_t cnt = bn[6];
+        float box[6];
+        for (int q = 0; q < 3; q++) {
+            box[q] = half_scan<true>(cnt ? ord_val(bn[q]) : 3.4e38f);
+            box[3 + q] = half_scan<false>(cnt ? ord_val(bn[3 + q]) : -3.4e38f);
+        }
+        cnt = half_scan_add(cnt);
+        const float part = box_area6(box) * (float)cnt;
+        const uint32_t rn = __shfl(cnt, (int)(62u - lane) & 63);
+        const float right = __shfl(part, (int)(62u - lane) & 63);
+        const bool ok = lane < (uint32_t)kSahBins - 1u && cnt > 0u && rn > 0u;
+        const float cost = part + right;
+        const uint64_t okm = __ballot(ok);
+        if (okm == 0ull) continue;
+        // the first minimum (the first split at all if no cost is a number)
+        const float best = wave_reduce<true>(ok ? cost : __builtin_huge_valf());
+        const uint64_t bm = __ballot(ok && cost == best);
+        const int cj = __ffsll((unsigned long long)(bm ? bm : okm)) - 1;
+        const float c = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cost), cj));
+        if (bk < 0 || c < bc) {
+            bk = k;
+            bj = cj;
+            bc = c;
+            nl = (uint32_t)__builtin_amdgcn_readlane((int)cnt, cj);
+        }
+    }
+    if (bk < 0) return a + m / 2u - 1u;
+    // stable partition
+    if (m <= 64u) {
+        const bool valid = lane < m;
+        const int bin = bk == 0 ? mine[0] : (bk == 1 ? mine[1] : mine[2]);
+        const bool left = valid && bin <= bj;
+        const uint64_t ml = __ballot(left), mr = __ballot(valid && !left);
+        if (valid) perm[left ? a + mbcnt(ml) : a + nl + mbcnt(mr)] = p;
+        wave_order();
+        return a + nl - 1u;
+    }
+    uint32_t offl = a, offr = a + nl;
+    const float blo = bk == 0 ? lo[0] : (bk == 1 ? lo[1] : lo[2]), bext = bk == 0 ? ext[0] : (bk == 1 ? ext[1] : ext[2]);
+    for (uint32_t i0 = a; i0 <= b; i0 += 64u) {
+        const uint32_t i = i0 + lane;
+        const bool valid = i <= b;
+        const uint32_t pi = valid ? perm[i] : 0u;
+        const bool left = valid && sah_bin(sah_cen(sph[pi], bk), blo, bext) <= bj;
+        const uint64_t ml = __ballot(left), mr = __ballot(valid && !left);
+        if (valid) tmp[left ? offl + mbcnt(ml) : offr + mbcnt(mr)] = pi;
+        offl += (uint32_t)__popcll(ml);
+        offr += (uint32_t)__popcll(mr);
+    }
+    wave_order();
+    for (uint32_t i = a + lane; i <= b; i += 64u) perm[i] = tmp[i];
+    wave_order();
+    return a + nl - 1u;
+}
+
 // Rebuilds the subtree over leaves [f, f + m) (2 <= m <= kSahMaxPrims), root
 // node r at depth d0, in place: leaf_prim and keys are permuted within the
 // range, and the child words and parent links of the subtree's nodes are
 // rewritten.  In the Karras layout a subtree's node indices are fixed by its
 // leaf range and root index, so the nodes above it are untouched.  Called
-// by a whole workgroup.
+// by a whole workgroup of NW waves.
+template <int NW>
 __device__ __forceinline__ void sah_treelet(const float4* __restrict__ sph, uint32_t f, uint32_t m, uint32_t r,
                                             uint32_t d0, uint32_t* __restrict__ leaf_prim,
                                             uint32_t* __restrict__ keys, uint32_t* __restrict__ child,
                                             uint32_t* __restrict__ parent_int, uint32_t* __restrict__ parent_leaf,
-                                            SahShared& sh)
+                                            SahShared<NW>& sh)
 {
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
-    for (uint32_t i = tid; i < m; i += kSahThreads) {
+    constexpr uint32_t NT = 64 * NW;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(tid >> 6);
+    for (uint32_t i = tid; i < m; i += NT) {
         sh.sph[i] = sph[leaf_prim[f + i]];
         sh.perm[i] = i;
     }
+    if (tid < kSahTasks) sh.task[tid] = tid == 0u ? make_uint2((m - 1u) << 10 | d0 << 20, r) : make_uint2(kSahNone, 0u);
     if (tid == 0) {
-        sh.task[0][0] = make_uint2((m - 1u) << 10, r);
-        sh.ntask[0] = 1u;
-        sh.ntask[1] = 0u;
+        sh.head = 0u;
+        sh.tail = 1u;
+        sh.open = 1u;
     }
-    uint32_t cur = 0;
-    for (uint32_t level = 0; level < 64u; level++) {
-        __syncthreads();
-        const uint32_t nt = sh.ntask[cur];
-        if (nt == 0u) break;
-        for (uint32_t round = 0; round < nt; round += kSahWaves) {
-            const uint32_t t = round + w;
-            const bool has = t < nt;
-            const uint2 tw = has ? sh.task[cur][t] : make_uint2(0u, 0u);
-            const uint32_t a = tw.x & 0x3FFu, b = (tw.x >> 10) & 0x3FFu, self = tw.y;
-            // centre bounds of the range
-            float lo[3] = {3.4e38f, 3.4e38f, 3.4e38f}, hi[3] = {-3.4e38f, -3.4e38f, -3.4e38f};
-            if (has)
-                for (uint32_t i = a + lane; i <= b; i += 64u) {
-                    const float4 sp = sh.sph[sh.perm[i]];
-                    for (int k = 0; k < 3; k++) {
-                        lo[k] = fminf(lo[k], sah_cen(sp, k));
-                        hi[k] = fmaxf(hi[k], sah_cen(sp, k));
-                    }
-                }
-            float ext[3];
-            bool any = false;
-            for (int k = 0; k < 3; k++) {
-                lo[k] = wave_min(lo[k]);
-                hi[k] = wave_max(hi[k]);
-                ext[k] = hi[k] - lo[k];
-                any = any || ext[k] > 0.0f;
-            }
-            const bool sah = has && d0 + level < kSahDepthCap && any;
-            if (sah)
-                for (int x = (int)lane; x < kSahBinWords; x += 64) sh.bin[w][x] = x % 7 < 3 ? 0xFFFFFFFFu : 0u;
-            __syncthreads();
-            if (sah)
-                for (uint32_t i = a + lane; i <= b; i += 64u) {
-                    const float4 sp = sh.sph[sh.perm[i]];
-                    const float rr = fabsf(sp.w);
-                    const float lb[6] = {sp.x - rr, sp.y - rr, sp.z - rr, sp.x + rr, sp.y + rr, sp.z + rr};
-                    for (int k = 0; k < 3; k++) {
-                        if (!(ext[k] > 0.0f)) continue;
-                        uint32_t* bn = &sh.bin[w][(k * kSahBins + sah_bin(sah_cen(sp, k), lo[k], ext[k])) * 7];
-                        for (int q = 0; q < 3; q++) {
-                            atomicMin(&bn[q], ord_key(lb[q]));
-                            atomicMax(&bn[3 + q], ord_key(lb[3 + q]));
-                        }
-                        atomicAdd(&bn[6], 1u);
-                    }
-                }
-            __syncthreads();
-            // the cheapest split, per axis with one lane per bin: inclusive
-            // prefix and suffix unions (min/max, exact in any order) and
-            // counts over the 32 bins, the cost of the split after each bin,
-            // then the first minimum.  The unions start from the box
-            // (3.4e38, -3.4e38) as the sequential sweep of the oracle does.
-            int bk = -1, bj = -1;
-            if (sah) {
-                float bc = 0.0f;
-                const int j = (int)(lane & 31u);
-                for (int k = 0; k < 3; k++) {
-                    if (!(ext[k] > 0.0f)) continue;
-                    const uint32_t* bn = &sh.bin[w][(k * kSahBins + j) * 7];
-                    const uint32_t c = bn[6];
-                    float P[6], S[6];
-                    for (int q = 0; q < 3; q++) {
-                        P[q] = S[q] = c ? ord_val(bn[q]) : 3.4e38f;
-                        P[3 + q] = S[3 + q] = c ? ord_val(bn[3 + q]) : -3.4e38f;
-                    }
-                    uint32_t pc = c, sc = c;
-                    for (int d = 1; d < kSahBins; d <<= 1) {
-                        for (int q = 0; q < 6; q++) {
-                            const float up = __shfl_up(P[q], d, kSahBins), dn = __shfl_down(S[q], d, kSahBins);
-                            if (j >= d) P[q] = q < 3 ? fminf(P[q], up) : fmaxf(P[q], up);
-                            if (j + d < kSahBins) S[q] = q < 3 ? fminf(S[q], dn) : fmaxf(S[q], dn);
-                        }
-                        const uint32_t upc = __shfl_up(pc, d, kSahBins), dnc = __shfl_down(sc, d, kSahBins);
-                        if (j >= d) pc += upc;
-                        if (j + d < kSahBins) sc += dnc;
-                    }
-                    float L[6], R[6];
-                    for (int q = 0; q < 6; q++) {
-                        const float r1 = __shfl_down(S[q], 1, kSahBins);  // bins j+1 .. 31
-                        L[q] = q < 3 ? fminf(3.4e38f, P[q]) : fmaxf(-3.4e38f, P[q]);
-                        R[q] = q < 3 ? fminf(3.4e38f, r1) : fmaxf(-3.4e38f, r1);
-                    }
-                    const uint32_t rn = __shfl_down(sc, 1, kSahBins);
-                    bool ok = j < kSahBins - 1 && pc > 0u && rn > 0u;
-                    float cost = ok ? box_area6(L) * (float)pc + box_area6(R) * (float)rn : 0.0f;
-                    int cj = j;
-                    for (int o = kSahBins / 2; o >= 1; o >>= 1) {
-                        const bool ook = __shfl_xor(ok ? 1 : 0, o, kSahBins) != 0;
-                        const float oc = __shfl_xor(cost, o, kSahBins);
-                        const int oj = __shfl_xor(cj, o, kSahBins);
-                        if ((ook && !ok) || (ook == ok && (oc < cost || (oc == cost && oj < cj)))) {
-                            ok = ook;
-                            cost = oc;
-                            cj = oj;
-                        }
-                    }
-                    if (ok && (bk < 0 || cost < bc)) {
-                        bk = k;
-                        bj = cj;
-                        bc = cost;
-                    }
-                }
-            }
-            uint32_t g = a + (b - a + 1u) / 2u - 1u;
-            if (bk >= 0) {
-                uint32_t cl = 0;
-                for (uint32_t i = a + lane; i <= b; i += 64u)
-                    cl += sah_bin(sah_cen(sh.sph[sh.perm[i]], bk), lo[bk], ext[bk]) <= bj ? 1u : 0u;
-                const uint32_t nl = wave_sum(cl);
-                uint32_t offl = a, offr = a + nl;
-                for (uint32_t i0 = a; i0 <= b; i0 += 64u) {
-                    const uint32_t i = i0 + lane;
-                    const bool valid = i <= b;
-                    const uint32_t p = valid ? sh.perm[i] : 0u;
-                    const bool left = valid && sah_bin(sah_cen(sh.sph[p], bk), lo[bk], ext[bk]) <= bj;
-                    const uint64_t ml = __ballot(left), mr = __ballot(valid && !left);
-                    if (left) sh.tmp[offl + mbcnt(ml)] = p;
-                    else if (valid) sh.tmp[offr + mbcnt(mr)] = p;
-                    offl += (uint32_t)__popcll(ml);
-                    offr += (uint32_t)__popcll(mr);
-                }
-                g = a + nl - 1u;
-            }
-            __syncthreads();
-            if (bk >= 0)
-                for (uint32_t i = a + lane; i <= b; i += 64u) sh.perm[i] = sh.tmp[i];
-            if (has && lane == 0u) {
-                const uint32_t G = f + g;  // split after leaf G: children G and G + 1
-                const uint32_t up = self | (((f + a) / kRefitLeaves == (f + b) / kRefitLeaves) ? kLocalBit : 0u);
-                uint32_t fl = 0;
-                if (g == a) { fl |= 1u; parent_leaf[G] = up; } else { parent_int[G] = up; }
-                if (g + 1u == b) { fl |= 2u; parent_leaf[G + 1u] = up; } else { parent_int[G + 1u] = up; }
-                child[self] = G | (fl << 30);
-                // children of two spheres are finished here; larger ones are
-                // the next level's ranges
-                const uint32_t ca[2] = {a, g + 1u}, cb[2] = {g, b};
-                for (int c = 0; c < 2; c++) {
-                    if (cb[c] == ca[c]) continue;
-                    const uint32_t node = f + (c == 0 ? g : g + 1u);  // Karras layout index
-                    if (cb[c] == ca[c] + 1u)
-                        sah_pair(ca[c], f, node, d0 + level + 1u, child, parent_leaf, sh);
-                    else
-                        sh.task[cur ^ 1u][atomicAdd(&sh.ntask[cur ^ 1u], 1u)] =
-                            make_uint2(ca[c] | (cb[c] << 10), node);
-                }
-            }
+    __syncthreads();
+    for (;;) {
+        // A ticket names a task, perhaps one that has not been written yet.
+        // Every open task is being worked on by some wave (or is this wave's
+        // to take), which writes no task after it has closed its own; so the
+        // wait ends with this ticket's task or with none open.
+        uint32_t ticket = 0, tx = kSahNone;
+        if (lane == 0) ticket = atomicAdd(&sh.head, 1u);
+        wave_order();
+        ticket = (uint32_t)__builtin_amdgcn_readfirstlane(ticket);
+        for (;;) {
+            const uint32_t open = __hip_atomic_load(&sh.open, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
+            tx = __hip_atomic_load(&sh.task[ticket].x, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
+            if (tx != kSahNone || open == 0u) break;
+            __builtin_amdgcn_s_sleep(1);
         }
-        __syncthreads();
-        if (tid == 0) sh.ntask[cur] = 0u;
-        cur ^= 1u;
+        tx = (uint32_t)__builtin_amdgcn_readfirstlane(tx);
+        if (tx == kSahNone) break;
+        uint32_t self = (uint32_t)__builtin_amdgcn_readfirstlane(sh.task[ticket].y), aside = 0;
+        for (;;) {
+            const uint32_t a = tx & 0x3FFu, b = (tx >> 10) & 0x3FFu, d = tx >> 20;
+            if (b == a + 1u) {  // a root of two spheres
+                if (lane == 0) sah_pair(a, f, self, d, child, parent_leaf, sh.sph, sh.perm);
+            } else {
+                const uint32_t g = sah_split(sh.sph, sh.perm, sh.tmp, sh.bin[w], a, b, d);
+                const uint32_t G = f + g;  // split after leaf G: children G and G + 1
+                const uint32_t ml = g - a + 1u, mr = b - g;
+                if (lane == 0) {
+                    const uint32_t up = self | (((f + a) / kRefitLeaves == (f + b) / kRefitLeaves) ? kLocalBit : 0u);
+                    if (ml == 1u) parent_leaf[G] = up; else parent_int[G] = up;
+                    if (mr == 1u) parent_leaf[G + 1u] = up; else parent_int[G + 1u] = up;
+                    child[self] = G | (ml == 1u ? 1u << 30 : 0u) | (mr == 1u ? 2u << 30 : 0u);
+                    if (ml == 2u) sah_pair(a, f, G, d + 1u, child, parent_leaf, sh.sph, sh.perm);
+                    if (mr == 2u) sah_pair(g + 1u, f, G + 1u, d + 1u, child, parent_leaf, sh.sph, sh.perm);
+                }
+                wave_order();
+                const uint2 tl = make_uint2(a | g << 10 | (d + 1u) << 20, G);
+                const uint2 tr = make_uint2((g + 1u) | b << 10 | (d + 1u) << 20, G + 1u);
+                const uint2 big = ml >= mr ? tl : tr, small = ml >= mr ? tr : tl;
+                const uint32_t ms = min(ml, mr);
+                if (ms >= kSahShare) {
+                    if (lane == 0) {
+                        atomicAdd(&sh.open, 1u);
+                        const uint32_t at = atomicAdd(&sh.tail, 1u);
+                        sh.task[at].y = small.y;
+                        __hip_atomic_store(&sh.task[at].x, small.x, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    }
+                    wave_order();
+                } else if (ms >= 3u) {
+                    if (lane == 0) sh.local[w][aside] = big;
+                    wave_order();
+                    aside++;
+                    tx = small.x;
+                    self = small.y;
+                    continue;
+                }
+                if (max(ml, mr) >= 3u) {
+                    tx = big.x;
+                    self = big.y;
+                    continue;
+                }
+            }
+            if (aside == 0u) break;
+            aside--;
+            tx = (uint32_t)__builtin_amdgcn_readfirstlane(sh.local[w][aside].x);
+            self = (uint32_t)__builtin_amdgcn_readfirstlane(sh.local[w][aside].y);
+        }
+        if (lane == 0) __hip_atomic_fetch_sub(&sh.open, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+        // keeps the wave's lanes together: without it the compiler sent all
+        // lanes but the first straight past the next `if (lane == 0)`, and
+        // they took ticket 0 again, by themselves, for ever
+        wave_order();
     }
     __syncthreads();
     // permute the range's primitive ids and keys in place, staged through
     // LDS (the bins are free now) so every global read has landed before the
     // barrier that precedes the writes
     uint32_t* kbuf = &sh.bin[0][0];
-    for (uint32_t i = tid; i < m; i += kSahThreads) {
+    for (uint32_t i = tid; i < m; i += NT) {
         const uint32_t p = sh.perm[i];
         sh.tmp[i] = leaf_prim[f + p];
         kbuf[i] = keys[f + p];
     }
     __syncthreads();
-    for (uint32_t i = tid; i < m; i += kSahThreads) {
+    for (uint32_t i = tid; i < m; i += NT) {
         leaf_prim[f + i] = sh.tmp[i];
         keys[f + i] = kbuf[i];
     }
@@ -682,16 +773,16 @@ __device__ __forceinline__ void sah_treelet(const float4* __restrict__ sph, uint
 
 // A small scene: the whole tree is one SAH build (keys and identity
 // permutation in sphere order in, leaf order out).
-__global__ void __launch_bounds__(kSahThreads) k_sah_build(const float4* __restrict__ sph, uint32_t n,
+__global__ void __launch_bounds__(64 * kSahSoloWaves) k_sah_build(const float4* __restrict__ sph, uint32_t n,
                                                            uint32_t* __restrict__ leaf_prim,
                                                            uint32_t* __restrict__ keys,
                                                            uint32_t* __restrict__ child,
                                                            uint32_t* __restrict__ parent_int,
                                                            uint32_t* __restrict__ parent_leaf)
 {
-    __shared__ SahShared sh;
+    __shared__ SahShared<kSahSoloWaves> sh;
     if (threadIdx.x == 0) parent_int[0] = 0xFFFFFFFFu;
-    sah_treelet(sph, 0u, n, 0u, 0u, leaf_prim, keys, child, parent_int, parent_leaf, sh);
+    sah_treelet<kSahSoloWaves>(sph, 0u, n, 0u, 0u, leaf_prim, keys, child, parent_int, parent_leaf, sh);
 }
 
 // A large LBVH: the roots of its treelets, the maximal subtrees of at most
@@ -719,7 +810,7 @@ __global__ void __launch_bounds__(kBlk) k_treelet_roots(const uint2* __restrict_
     list[atomicAdd(count, 1u)] = make_uint4(ri.x, m, i, d);
 }
 
-__global__ void __launch_bounds__(kSahThreads) k_sah_treelets(const float4* __restrict__ sph,
+__global__ void __launch_bounds__(64 * kSahWaves) k_sah_treelets(const float4* __restrict__ sph,
                                                               const uint4* __restrict__ list,
                                                               const uint32_t* __restrict__ count,
                                                               uint32_t* __restrict__ leaf_prim,
@@ -728,11 +819,11 @@ __global__ void __launch_bounds__(kSahThreads) k_sah_treelets(const float4* __re
                                                               uint32_t* __restrict__ parent_int,
                                                               uint32_t* __restrict__ parent_leaf)
 {
-    __shared__ SahShared sh;
+    __shared__ SahShared<kSahWaves> sh;
     const uint32_t cnt = *count;
     for (uint32_t t = blockIdx.x; t < cnt; t += gridDim.x) {
         const uint4 e = list[t];
-        sah_treelet(sph, e.x, e.y, e.z, e.w, leaf_prim, keys, child, parent_int, parent_leaf, sh);
+        sah_treelet<kSahWaves>(sph, e.x, e.y, e.z, e.w, leaf_prim, keys, child, parent_int, parent_leaf, sh);
     }
 }
 
@@ -1333,7 +1424,7 @@ vzStatus lbvh_build(vzScene s, hipStream_t st)
     s->d_morton = s->d_keys[0];
     s->d_leaf_prim = s->d_vals[0];
     if (s->builder == VZ_BUILD_SAH) {
-        hipLaunchKernelGGL(k_sah_build, dim3(1), dim3(kSahThreads), 0, st, s->d_sph_in, n, s->d_leaf_prim,
+        hipLaunchKernelGGL(k_sah_build, dim3(1), dim3(64 * kSahSoloWaves), 0, st, s->d_sph_in, n, s->d_leaf_prim,
                            s->d_morton, s->d_child, s->d_parent_int, s->d_parent_leaf);
     } else {
         uint32_t tiles = s->hist_blocks;
@@ -1358,7 +1449,7 @@ vzStatus lbvh_build(vzScene s, hipStream_t st)
                 hipLaunchKernelGGL(k_zero, dim3(1), dim3(kBlk), 0, st, count, 1u);
                 hipLaunchKernelGGL(k_treelet_roots, dim3(blocks_for(n - 1, kBlk)), dim3(kBlk), 0, st, range,
                                    s->d_parent_int, n - 1, list, count);
-                hipLaunchKernelGGL(k_sah_treelets, dim3(kTreeletBlocks), dim3(kSahThreads), 0, st, s->d_sph_in,
+                hipLaunchKernelGGL(k_sah_treelets, dim3(kTreeletBlocks), dim3(64 * kSahWaves), 0, st, s->d_sph_in,
                                    list, count, s->d_leaf_prim, s->d_morton, s->d_child, s->d_parent_int,
                                    s->d_parent_leaf);
             }
