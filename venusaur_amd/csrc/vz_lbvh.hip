@@ -867,16 +867,31 @@ __device__ __forceinline__ void leaf_box(const float4 sp, float* b)
     b[3] = sp.x + r; b[4] = sp.y + r; b[5] = sp.z + r;
 }
 
-// Union of the two child boxes into nb, and the 32-byte packed node p.
-__device__ __forceinline__ void pack_node(uint32_t p, const float (&cb)[2][6], uint32_t g, uint32_t flags,
-                                          float (&nb)[6], uint4* __restrict__ nodes)
+// Union of the two child boxes.
+__device__ __forceinline__ void join_boxes(const float (&cb)[2][6], float (&nb)[6])
 {
     for (int k = 0; k < 3; k++) {
         nb[k] = fminf(cb[0][k], cb[1][k]);
         nb[3 + k] = fmaxf(cb[0][3 + k], cb[1][3 + k]);
     }
+}
+
+// The 32-byte packed node p, once every box is known: one thread per node.
+// The refit's climbs used to pack each node on their way, which put some 20
+// divisions on every level of their serial chains (local part of a million
+// spheres 315 us, of the book scene 65 us).
+__device__ __forceinline__ void pack_node(uint32_t p, const float4* __restrict__ sph, const uint32_t* __restrict__ child,
+                                          const float* __restrict__ boxes, uint4* __restrict__ nodes)
+{
+    const uint32_t cw = child[p], g = cw & 0x3FFFFFFFu, flags = cw >> 30;
+    float cb[2][6], nb[6];
+    for (uint32_t c = 0; c < 2; c++) {
+        if ((flags >> c) & 1u) leaf_box(sph[g + c], cb[c]);
+        else
+            for (int k = 0; k < 6; k++) cb[c][k] = boxes[(size_t)(g + c) * 6 + k];
+    }
+    join_boxes(cb, nb);
     uint32_t meta = 0, q[3];
-    float o[3];
     for (int k = 0; k < 3; k++) {
         const float lo = nb[k], hi = nb[3 + k];
         const uint32_t e = pick_exp(lo, hi);
@@ -884,12 +899,18 @@ __device__ __forceinline__ void pack_node(uint32_t p, const float (&cb)[2][6], u
         meta |= e << (8 * k);
         const uint32_t l0 = quant_lo(cb[0][k], lo, sc), h0 = quant_hi(cb[0][3 + k], lo, sc);
         const uint32_t l1 = quant_lo(cb[1][k], lo, sc), h1 = quant_hi(cb[1][3 + k], lo, sc);
-        o[k] = lo;
         q[k] = l0 | (h0 << 8) | (l1 << 16) | (h1 << 24);
     }
     meta |= flags << 24;
-    nodes[2 * p] = make_uint4(__float_as_uint(o[0]), __float_as_uint(o[1]), __float_as_uint(o[2]), meta);
-    nodes[2 * p + 1] = make_uint4(q[0], q[1], q[2], g);
+    nodes[2 * (size_t)p] = make_uint4(__float_as_uint(nb[0]), __float_as_uint(nb[1]), __float_as_uint(nb[2]), meta);
+    nodes[2 * (size_t)p + 1] = make_uint4(q[0], q[1], q[2], g);
+}
+__global__ void __launch_bounds__(kBlk) k_pack_nodes(const float4* __restrict__ sph, const uint32_t* __restrict__ child,
+                                                     const float* __restrict__ boxes, uint32_t ni,
+                                                     uint4* __restrict__ nodes)
+{
+    const uint32_t p = blockIdx.x * kBlk + threadIdx.x;
+    if (p < ni) pack_node(p, sph, child, boxes, nodes);
 }
 
 // Bottom-up refit (Karras 2012, section 4): one thread per leaf climbs, and
@@ -921,7 +942,6 @@ __global__ void __launch_bounds__(kRefitThreads) k_refit_local(const float4* __r
                                                                const uint32_t* __restrict__ parent_leaf,
                                                                float* __restrict__ boxes,
                                                                uint32_t* __restrict__ height,
-                                                               uint4* __restrict__ nodes,
                                                                uint32_t* __restrict__ frontier,
                                                                uint32_t* __restrict__ fcount)
 {
@@ -966,11 +986,11 @@ __global__ void __launch_bounds__(kRefitThreads) k_refit_local(const float4* __r
                     h = max(h, __hip_atomic_load(&s_h[cs], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
                 }
             }
-            pack_node(p, cb, g, flags, nb, nodes);
+            join_boxes(cb, nb);
             nh = h + 1u;
             for (int k = 0; k < 6; k++) {
                 __hip_atomic_store(&s_box[k][slot], nb[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                boxes[(size_t)p * 6 + k] = nb[k];  // every node's exact box: the 4-wide collapse reads them
+                boxes[(size_t)p * 6 + k] = nb[k];  // every node's exact box: packing and the 4-wide collapse read them
             }
             __hip_atomic_store(&s_h[slot], nh, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             done = p;
@@ -997,7 +1017,7 @@ __global__ void __launch_bounds__(kRefitThreads) k_refit_top(const float4* __res
                                                     const uint32_t* __restrict__ parent_leaf,
                                                     const uint32_t* __restrict__ frontier,
                                                     const uint32_t* __restrict__ fcount, uint32_t* visit,
-                                                    float* boxes, uint32_t* height, uint4* __restrict__ nodes)
+                                                    float* boxes, uint32_t* height)
 {
     const uint32_t count = *fcount;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < count; i += gridDim.x * blockDim.x) {
@@ -1020,7 +1040,7 @@ __global__ void __launch_bounds__(kRefitThreads) k_refit_top(const float4* __res
                 }
             }
             float nb[6];
-            pack_node(p, cb, g, flags, nb, nodes);
+            join_boxes(cb, nb);
             for (int k = 0; k < 6; k++) __hip_atomic_store(&boxes[p * 6 + k], nb[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __hip_atomic_store(&height[p], h + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (p == 0u) break;
@@ -1069,48 +1089,95 @@ __global__ void __launch_bounds__(kBlk) k_wide_init(uint32_t* __restrict__ wflag
     }
 }
 
+// The children of wide root r: starts as its binary node's two, and opens the
+// internal one of largest box area while there are fewer than 4.  Areas are
+// kept, so every box is read once.
+__device__ __forceinline__ uint32_t wide_children(uint32_t r, const uint32_t* __restrict__ child,
+                                                  const float* __restrict__ boxes, uint32_t (&ks)[4])
+{
+    const uint32_t cw = child[r];
+    float area[4] = {-1.0f, -1.0f, -1.0f, -1.0f};  // of leaves and absent slots: never opened
+    ks[0] = child_ref(cw, 0);
+    ks[1] = child_ref(cw, 1);
+    ks[2] = ks[3] = 0u;
+    bool internal[4] = {!(ks[0] & kLeafRef), !(ks[1] & kLeafRef), false, false};
+    for (int k = 0; k < 2; k++)
+        if (internal[k]) area[k] = box_area(boxes + (size_t)ks[k] * 6);
+    uint32_t n_k = 2;
+#pragma unroll
+    for (int round = 0; round < 2; round++) {
+        int best = -1;
+        float ba = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            if (internal[k] && (best < 0 || area[k] > ba)) {
+                best = k;
+                ba = area[k];
+            }
+        if (best < 0) break;
+        const uint32_t opened = best == 0 ? ks[0] : (best == 1 ? ks[1] : (best == 2 ? ks[2] : ks[3]));
+        const uint32_t ow = child[opened];
+        const uint32_t c0 = child_ref(ow, 0), c1 = child_ref(ow, 1);
+        const bool i0 = !(c0 & kLeafRef), i1 = !(c1 & kLeafRef);
+        const float a0 = i0 ? box_area(boxes + (size_t)c0 * 6) : -1.0f;
+        const float a1 = i1 ? box_area(boxes + (size_t)c1 * 6) : -1.0f;
+        // c0 takes the opened slot, c1 the next; the slots after move up
+#pragma unroll
+        for (int k = 3; k >= 0; k--) {
+            if (k > best + 1) {
+                ks[k] = ks[k > 0 ? k - 1 : 0];
+                area[k] = area[k > 0 ? k - 1 : 0];
+                internal[k] = internal[k > 0 ? k - 1 : 0];
+            } else if (k == best + 1) {
+                ks[k] = c1;
+                area[k] = a1;
+                internal[k] = i1;
+            } else if (k == best) {
+                ks[k] = c0;
+                area[k] = a0;
+                internal[k] = i0;
+            }
+        }
+        n_k++;
+    }
+    return n_k;
+}
+
 // One level: every wide root of the frontier picks its children; internal
-// children are the next level's frontier.  cnt[level + 1] starts at zero.
+// children are the next level's frontier.  cnt[level + 1] starts at zero and
+// is added to once per wave (once per child, and a maximum per root for the
+// depth, kept one address busy: 414 us for the levels of a million spheres).
 __global__ void __launch_bounds__(kBlk) k_wide_level(const uint32_t* __restrict__ child,
                                                      const float* __restrict__ boxes,
                                                      const uint32_t* __restrict__ front_in,
                                                      uint32_t* __restrict__ front_out, uint32_t* __restrict__ cnt,
                                                      uint32_t level, uint32_t* __restrict__ wkids,
-                                                     uint32_t* __restrict__ wflag, uint32_t* __restrict__ wdepth)
+                                                     uint32_t* __restrict__ wflag)
 {
-    const uint32_t count = cnt[level];
-    for (uint32_t i = blockIdx.x * kBlk + threadIdx.x; i < count; i += gridDim.x * kBlk) {
-        const uint32_t r = front_in[i];
-        const uint32_t cw = child[r];
-        uint32_t ks[4] = {child_ref(cw, 0), child_ref(cw, 1), 0u, 0u};
-        uint32_t n_k = 2;
-        while (n_k < 4u) {
-            int best = -1;
-            float ba = 0.0f;
-            for (uint32_t k = 0; k < n_k; k++) {
-                if (ks[k] & kLeafRef) continue;
-                const float a = box_area(boxes + (size_t)ks[k] * 6);
-                if (best < 0 || a > ba) {
-                    best = (int)k;
-                    ba = a;
-                }
-            }
-            if (best < 0) break;
-            const uint32_t ow = child[ks[best]];
-            for (int k = (int)n_k - 1; k > best; k--) ks[k + 1] = ks[k];
-            ks[best] = child_ref(ow, 0);
-            ks[best + 1] = child_ref(ow, 1);
-            n_k++;
+    const uint32_t count = cnt[level], lane = lane_id();
+    for (uint32_t i0 = (blockIdx.x * kBlk + threadIdx.x) & ~63u; i0 < count; i0 += gridDim.x * kBlk) {
+        const uint32_t i = i0 + lane;
+        uint32_t ks[4] = {0u, 0u, 0u, 0u}, n_k = 0, n_in = 0;
+        if (i < count) {
+            const uint32_t r = front_in[i];
+            n_k = wide_children(r, child, boxes, ks);
+            reinterpret_cast<uint4*>(wkids)[r] = make_uint4(ks[0], ks[1], ks[2], ks[3]);
+            wflag[r] = kWideRoot | n_k;
+            for (uint32_t k = 0; k < 4u; k++) n_in += k < n_k && !(ks[k] & kLeafRef) ? 1u : 0u;
         }
-        reinterpret_cast<uint4*>(wkids)[r] = make_uint4(ks[0], ks[1], ks[2], ks[3]);
-        wflag[r] = kWideRoot | n_k;
-        for (uint32_t k = 0; k < n_k; k++) {
-            const uint32_t c = ks[k];
-            if (c & kLeafRef) continue;
-            wflag[c] = kWideRoot;
-            front_out[atomicAdd(&cnt[level + 1], 1u)] = c;
+        uint32_t incl = n_in;
+        for (uint32_t off = 1; off < 64u; off <<= 1) {
+            const uint32_t x = __shfl_up(incl, off);
+            if (lane >= off) incl += x;
         }
-        atomicMax(wdepth, level + 2u);  // wide levels 1..level+1, plus the leaf level
+        uint32_t base = 0;
+        if (lane == 63u && incl) base = atomicAdd(&cnt[level + 1], incl);
+        uint32_t at = __shfl(base, 63) + incl - n_in;
+        for (uint32_t k = 0; k < 4u; k++) {
+            if (k >= n_k || (ks[k] & kLeafRef)) continue;
+            wflag[ks[k]] = kWideRoot;
+            front_out[at++] = ks[k];
+        }
     }
 }
 
@@ -1340,7 +1407,7 @@ __global__ void __launch_bounds__(kBlk) k_wide_verify(const uint32_t* __restrict
 static vzStatus collapse_wide(vzScene s, hipStream_t st)
 {
     const uint32_t n = s->n, ni = n - 1;
-    uint32_t* cnt = s->d_wcnt;  // [0, kMaxDepth]: per level; then nw, the wide depth
+    uint32_t* cnt = s->d_wcnt;  // [0, kMaxDepth]: roots per level; then nw, a spare word, the check's result
     uint32_t* tsum = s->d_widx + ni;
     const uint32_t ntile = blocks_for(ni, kScanTile);
     hipLaunchKernelGGL(k_zero, dim3(blocks_for(ni, kBlk)), dim3(kBlk), 0, st, s->d_wflag, ni);
@@ -1348,8 +1415,7 @@ static vzStatus collapse_wide(vzScene s, hipStream_t st)
     const uint32_t grid = std::min<uint32_t>(1024u, blocks_for(ni, kBlk));
     for (uint32_t L = 0; L + 1 < s->depth && L < kMaxDepth; L++)
         hipLaunchKernelGGL(k_wide_level, dim3(grid), dim3(kBlk), 0, st, s->d_child, s->d_boxes,
-                           s->d_wfront[L & 1u], s->d_wfront[(L + 1) & 1u], cnt, L, s->d_wkids, s->d_wflag,
-                           cnt + kMaxDepth + 2);
+                           s->d_wfront[L & 1u], s->d_wfront[(L + 1) & 1u], cnt, L, s->d_wkids, s->d_wflag);
     hipLaunchKernelGGL(k_wscan_tiles, dim3(ntile), dim3(kBlk), 0, st, s->d_wflag, ni, tsum);
     hipLaunchKernelGGL(k_wscan_top, dim3(1), dim3(kBlk), 0, st, tsum, ntile, cnt + kMaxDepth + 1);
     hipLaunchKernelGGL(k_wscan_apply, dim3(ntile), dim3(kBlk), 0, st, s->d_wflag, ni, tsum, s->d_widx);
@@ -1366,12 +1432,14 @@ static vzStatus collapse_wide(vzScene s, hipStream_t st)
     hipLaunchKernelGGL(k_wide_verify, dim3(grid), dim3(kBlk), 0, st, cnt + kMaxDepth + 1, n, wref, lref,
                        cnt + kMaxDepth + 3);
     VZ_HIP_TRY(hipGetLastError());
-    uint32_t h[3] = {0u, 0u, 0u};
-    VZ_HIP_TRY(hipMemcpyAsync(h, cnt + kMaxDepth + 1, sizeof(h), hipMemcpyDeviceToHost, st));
+    uint32_t h[kMaxDepth + 8] = {};
+    VZ_HIP_TRY(hipMemcpyAsync(h, cnt, sizeof(h), hipMemcpyDeviceToHost, st));
     VZ_HIP_TRY(hipStreamSynchronize(st));
-    s->nw = h[0];
-    s->wdepth = h[1];
-    if (h[2] != 0u) return set_error(VZ_ERROR_INTERNAL, "4-wide BVH failed its structural check");
+    s->nw = h[kMaxDepth + 1];
+    s->wdepth = 1;  // the leaf level below the deepest roots'
+    for (uint32_t L = 0; L <= kMaxDepth; L++)
+        if (h[L]) s->wdepth = L + 2;
+    if (h[kMaxDepth + 3] != 0u) return set_error(VZ_ERROR_INTERNAL, "4-wide BVH failed its structural check");
     if (s->wdepth > kMaxWideDepth)
         return set_error(VZ_ERROR_CAPACITY, "4-wide BVH depth " + std::to_string(s->wdepth) +
                                                 " exceeds the traversal stack (" + std::to_string(kMaxWideDepth) + ")");
@@ -1385,11 +1453,14 @@ static vzStatus refit_core(vzScene s, hipStream_t st)
     hipLaunchKernelGGL(k_zero, dim3(blocks_for(n - 1, kBlk)), dim3(kBlk), 0, st, s->d_visit, n - 1);
     hipLaunchKernelGGL(k_zero, dim3(1), dim3(kBlk), 0, st, s->d_fcount, 1u);
     hipLaunchKernelGGL(k_refit_local, dim3(blocks_for(n, kRefitLeaves)), dim3(kRefitThreads), 0, st, s->d_sph,
-                       n, s->d_child, s->d_parent_int, s->d_parent_leaf, s->d_boxes, s->d_height, s->d_nodes,
+                       n, s->d_child, s->d_parent_int, s->d_parent_leaf, s->d_boxes, s->d_height,
                        s->d_frontier, s->d_fcount);
-    hipLaunchKernelGGL(k_refit_top, dim3(kTopBlocks), dim3(kRefitThreads), 0, st, s->d_sph, s->d_child,
-                       s->d_parent_int, s->d_parent_leaf, s->d_frontier, s->d_fcount, s->d_visit, s->d_boxes,
-                       s->d_height, s->d_nodes);
+    if (n > kRefitLeaves)  // nodes that cross the workgroups' ranges
+        hipLaunchKernelGGL(k_refit_top, dim3(kTopBlocks), dim3(kRefitThreads), 0, st, s->d_sph, s->d_child,
+                           s->d_parent_int, s->d_parent_leaf, s->d_frontier, s->d_fcount, s->d_visit, s->d_boxes,
+                           s->d_height);
+    hipLaunchKernelGGL(k_pack_nodes, dim3(blocks_for(n - 1, kBlk)), dim3(kBlk), 0, st, s->d_sph, s->d_child,
+                       s->d_boxes, n - 1, s->d_nodes);
     VZ_HIP_TRY(hipGetLastError());
     uint32_t h = 0;
     VZ_HIP_TRY(hipMemcpyAsync(&h, s->d_height, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
