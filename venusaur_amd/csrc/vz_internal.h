@@ -100,6 +100,32 @@ struct Event {
 
 }  // namespace vz
 
+namespace vz {
+// Blocks of destroyed scenes, kept for the next ones: mapping and unmapping
+// the 300 MB of a million-sphere scene takes longer than building it.  At
+// most kKeepBytes are kept, given back when an allocation of the context
+// fails and with the context.  A scene is destroyed after the device has
+// gone idle, so a kept block is free for any stream.
+class SceneBlocks {
+public:
+    static constexpr size_t kKeepBytes = 1ull << 30;
+    // A block of at least `bytes`; *got is its size.  NULL when out of memory.
+    void* take(size_t bytes, size_t* got);
+    void give(void* p, size_t bytes);
+    void trim();
+    ~SceneBlocks() { trim(); }
+
+private:
+    struct Block {
+        void* p;
+        size_t bytes;
+    };
+    std::mutex mu_;
+    std::vector<Block> kept_;
+    size_t kept_bytes_ = 0;
+};
+}  // namespace vz
+
 struct vzContext_st {
     int device = 0;
     uint32_t num_cus = 0;
@@ -109,6 +135,7 @@ struct vzContext_st {
     vzTuning tuning{};
     std::mutex mu;
     vz::PathWork* path = nullptr;  // workspace of its launches, made by the first one
+    vz::SceneBlocks scene_blocks;
     std::atomic<uint32_t> live_scenes{0}, live_servers{0};  // vzDestroy refuses while any remain
     unsigned long long* trace_scratch = nullptr;  // this device's fixed trace scratch (vzTraceClosestNoAlloc)
 };
@@ -123,6 +150,9 @@ struct vzScene_st {
     // Server requests (queued or running) that name this scene; while any
     // remain, vzSceneDestroy refuses.
     std::atomic<uint32_t> server_refs{0};
+    // one block of device memory holds all of the arrays below
+    void* arena = nullptr;
+    size_t arena_bytes = 0;
     // inputs (original order)
     float4* d_sph_in = nullptr;
     vzMaterial* d_mat_in = nullptr;

@@ -1310,57 +1310,111 @@ inline uint32_t blocks_for(uint32_t n, uint32_t per) { return (n + per - 1) / pe
 
 }  // namespace
 
+void* SceneBlocks::take(size_t bytes, size_t* got)
+{
+    {
+        std::lock_guard<std::mutex> lk(mu_);
+        size_t best = kept_.size();
+        for (size_t i = 0; i < kept_.size(); i++)  // the smallest that fits, not above twice the size
+            if (kept_[i].bytes >= bytes && kept_[i].bytes <= 2 * bytes &&
+                (best == kept_.size() || kept_[i].bytes < kept_[best].bytes))
+                best = i;
+        if (best < kept_.size()) {
+            void* p = kept_[best].p;
+            *got = kept_[best].bytes;
+            kept_bytes_ -= *got;
+            kept_.erase(kept_.begin() + best);
+            return p;
+        }
+    }
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        trim();
+        if (hipMalloc(&p, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+    }
+    *got = bytes;
+    return p;
+}
+
+void SceneBlocks::give(void* p, size_t bytes)
+{
+    {
+        std::lock_guard<std::mutex> lk(mu_);
+        if (kept_.size() < 256 && kept_bytes_ + bytes <= kKeepBytes) {
+            kept_.push_back({p, bytes});
+            kept_bytes_ += bytes;
+            return;
+        }
+    }
+    (void)hipFree(p);
+}
+
+void SceneBlocks::trim()
+{
+    std::lock_guard<std::mutex> lk(mu_);
+    for (const Block& b : kept_) (void)hipFree(b.p);
+    kept_.clear();
+    kept_bytes_ = 0;
+}
+
 vzStatus lbvh_alloc(vzScene s)
 {
-    uint32_t n = s->n, ni = n > 1 ? n - 1 : 1;
+    const uint32_t n = s->n, ni = n > 1 ? n - 1 : 1;
     s->hist_blocks = blocks_for(n, kTile);
-    uint64_t bytes = 0;
-    auto al = [&](void** p, size_t b) -> vzStatus {
-        hipError_t e = hipMalloc(p, b);
-        if (e != hipSuccess) return set_error(VZ_ERROR_OUT_OF_MEMORY, "hipMalloc of scene buffers failed");
-        bytes += b;
-        return VZ_SUCCESS;
+    uint64_t bytes = 0;   // the arrays' own sizes (vzAccelInfo.device_bytes)
+    size_t at = 0;        // their places in the block, 256-byte aligned
+    struct Part {
+        void** p;
+        size_t at;
     };
-    VZ_TRY(al((void**)&s->d_sph_in, sizeof(float4) * n));
-    VZ_TRY(al((void**)&s->d_mat_in, sizeof(vzMaterial) * n));
+    std::vector<Part> parts;
+    auto part = [&](auto** p, size_t b) {
+        parts.push_back({(void**)p, at});
+        at += (b + 255) & ~(size_t)255;
+        bytes += b;
+    };
+    part(&s->d_sph_in, sizeof(float4) * n);
+    part(&s->d_mat_in, sizeof(vzMaterial) * n);
     for (int i = 0; i < 2; i++) {
-        VZ_TRY(al((void**)&s->d_keys[i], sizeof(uint32_t) * n));
-        VZ_TRY(al((void**)&s->d_vals[i], sizeof(uint32_t) * n));
+        part(&s->d_keys[i], sizeof(uint32_t) * n);
+        part(&s->d_vals[i], sizeof(uint32_t) * n);
     }
-    VZ_TRY(al((void**)&s->d_hist, sizeof(uint32_t) * 256 * (s->hist_blocks + 1)));
-    VZ_TRY(al((void**)&s->d_bounds, sizeof(float) * (6 * 1024 + 32)));  // partials, grid A, grid B
-    VZ_TRY(al((void**)&s->d_sph, sizeof(float4) * n));
-    VZ_TRY(al((void**)&s->d_leaf_info, sizeof(uint32_t) * n));
-    VZ_TRY(al((void**)&s->d_mat, sizeof(float4) * n));
-    VZ_TRY(al((void**)&s->d_nodes, sizeof(uint4) * 2 * ni));
-    VZ_TRY(al((void**)&s->d_boxes, sizeof(float) * 6 * ni));
-    VZ_TRY(al((void**)&s->d_child, sizeof(uint32_t) * ni));
-    VZ_TRY(al((void**)&s->d_parent_int, sizeof(uint32_t) * ni));
-    VZ_TRY(al((void**)&s->d_parent_leaf, sizeof(uint32_t) * n));
-    VZ_TRY(al((void**)&s->d_visit, sizeof(uint32_t) * ni));
-    VZ_TRY(al((void**)&s->d_height, sizeof(uint32_t) * ni));
-    VZ_TRY(al((void**)&s->d_frontier, sizeof(uint32_t) * n));
-    VZ_TRY(al((void**)&s->d_fcount, 256));
-    VZ_TRY(al((void**)&s->d_wnodes, sizeof(uint4) * 4 * ni));
-    VZ_TRY(al((void**)&s->d_wkids, sizeof(uint32_t) * 4 * ni));
-    VZ_TRY(al((void**)&s->d_wflag, sizeof(uint32_t) * ni));
-    VZ_TRY(al((void**)&s->d_widx, sizeof(uint32_t) * (ni + blocks_for(ni, kScanTile) + 1)));  // + tile sums
-    VZ_TRY(al((void**)&s->d_wfront[0], sizeof(uint32_t) * ni));
-    VZ_TRY(al((void**)&s->d_wfront[1], sizeof(uint32_t) * ni));
-    VZ_TRY(al((void**)&s->d_wcnt, sizeof(uint32_t) * (kMaxDepth + 8)));
+    part(&s->d_hist, sizeof(uint32_t) * 256 * (s->hist_blocks + 1));
+    part(&s->d_bounds, sizeof(float) * (6 * 1024 + 32));  // partials, grid A, grid B
+    part(&s->d_sph, sizeof(float4) * n);
+    part(&s->d_leaf_info, sizeof(uint32_t) * n);
+    part(&s->d_mat, sizeof(float4) * n);
+    part(&s->d_nodes, sizeof(uint4) * 2 * ni);
+    part(&s->d_boxes, sizeof(float) * 6 * ni);
+    part(&s->d_child, sizeof(uint32_t) * ni);
+    part(&s->d_parent_int, sizeof(uint32_t) * ni);
+    part(&s->d_parent_leaf, sizeof(uint32_t) * n);
+    part(&s->d_visit, sizeof(uint32_t) * ni);
+    part(&s->d_height, sizeof(uint32_t) * ni);
+    part(&s->d_frontier, sizeof(uint32_t) * n);
+    part(&s->d_fcount, 256);
+    part(&s->d_wnodes, sizeof(uint4) * 4 * ni);
+    part(&s->d_wkids, sizeof(uint32_t) * 4 * ni);
+    part(&s->d_wflag, sizeof(uint32_t) * ni);
+    part(&s->d_widx, sizeof(uint32_t) * (ni + blocks_for(ni, kScanTile) + 1));  // + tile sums
+    part(&s->d_wfront[0], sizeof(uint32_t) * ni);
+    part(&s->d_wfront[1], sizeof(uint32_t) * ni);
+    part(&s->d_wcnt, sizeof(uint32_t) * (kMaxDepth + 8));
+    s->arena = s->ctx->scene_blocks.take(at, &s->arena_bytes);
+    if (!s->arena) return set_error(VZ_ERROR_OUT_OF_MEMORY, "hipMalloc of scene buffers failed");
+    for (const Part& q : parts) *q.p = (char*)s->arena + q.at;
     s->device_bytes = bytes;
     return VZ_SUCCESS;
 }
 
 void lbvh_free(vzScene s)
 {
-    void* ptrs[] = {s->d_sph_in, s->d_mat_in, s->d_keys[0], s->d_keys[1], s->d_vals[0], s->d_vals[1],
-                    s->d_hist, s->d_bounds, s->d_sph, s->d_leaf_info, s->d_mat, s->d_nodes,
-                    s->d_boxes, s->d_child, s->d_parent_int, s->d_parent_leaf, s->d_visit,
-                    s->d_height, s->d_frontier, s->d_fcount, s->d_wnodes, s->d_wkids, s->d_wflag,
-                    s->d_widx, s->d_wfront[0], s->d_wfront[1], s->d_wcnt};
-    for (void* p : ptrs)
-        if (p) (void)hipFree(p);
+    if (s->arena) s->ctx->scene_blocks.give(s->arena, s->arena_bytes);
+    s->arena = nullptr;
 }
 
 // Structural check of the packed 4-wide tree, so that traversal needs no

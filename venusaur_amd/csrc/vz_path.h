@@ -40,6 +40,7 @@ struct PathReq {               // one request of a launch, read by scalar loads
 };
 
 struct PathSlot {
+    vzContext ctx = nullptr;
     char* paths = nullptr;     // seeds and radiances
     size_t paths_bytes = 0;
     char* pixels = nullptr;    // camera seeds and sums carried between the launches of one request
@@ -50,7 +51,7 @@ struct PathSlot {
     PathReq* h_reqs = nullptr; // pinned staging of it
     uint32_t used = 0;         // its entries given to launches not yet waited for
 
-    vzStatus init(bool table);
+    vzStatus init(vzContext c, bool table);
     void free();
 };
 

@@ -489,7 +489,7 @@ __global__ void __launch_bounds__(kBlk) k_path_resolve(PathGroup G, PathReq one)
 inline uint64_t align256(uint64_t v) { return (v + 255) & ~255ull; }
 
 // Grows a buffer that nothing in flight uses.
-bool grow(char** p, size_t* have, size_t need)
+bool grow(vzContext ctx, char** p, size_t* have, size_t need)
 {
     if (*have >= need) return true;
     if (*p) (void)hipFree(*p);
@@ -497,8 +497,12 @@ bool grow(char** p, size_t* have, size_t need)
     *have = 0;
     if (hipMalloc((void**)p, need) != hipSuccess) {
         (void)hipGetLastError();
-        *p = nullptr;
-        return false;
+        ctx->scene_blocks.trim();
+        if (hipMalloc((void**)p, need) != hipSuccess) {
+            (void)hipGetLastError();
+            *p = nullptr;
+            return false;
+        }
     }
     *have = need;
     return true;
@@ -629,8 +633,9 @@ size_t request_bytes(const vzLaunchParams& p)
            align256(K * 8) + 1024;
 }
 
-vzStatus PathSlot::init(bool table)
+vzStatus PathSlot::init(vzContext c, bool table)
 {
+    ctx = c;
     bool ok = stats || hipMalloc((void**)&stats, (kMaxPathBlocks * kPathStats + 1 + kMaxRequests) *
                                                      sizeof(unsigned long long)) == hipSuccess;
     ok = ok && (h_totals || hipHostMalloc((void**)&h_totals, (kPathStats + kMaxRequests) *
@@ -684,7 +689,7 @@ uint64_t path_count(const vzLaunchParams& p, const PathOptions& opt)
 vzStatus slot_reserve(PathSlot& s, uint64_t paths)
 {
     const uint64_t need = paths * kPathBytes + 256;
-    if (!grow(&s.paths, &s.paths_bytes, need))
+    if (!grow(s.ctx, &s.paths, &s.paths_bytes, need))
         return set_error(VZ_ERROR_OUT_OF_MEMORY, "launch buffers (" + std::to_string(need) + " bytes) do not fit");
     return VZ_SUCCESS;
 }
@@ -708,7 +713,7 @@ vzStatus path_enqueue_one(PathWork* w, PathSlot& s, const PathItem& item, const 
     for (;;) {
         const uint64_t pix = chunk < A.spp ? sum_bytes + 4ull * A.npad : 0ull;
         const vzStatus rs = slot_reserve(s, (uint64_t)A.npad * chunk);
-        if (rs == VZ_SUCCESS && grow(&s.pixels, &s.pixels_bytes, pix)) break;
+        if (rs == VZ_SUCCESS && grow(s.ctx, &s.pixels, &s.pixels_bytes, pix)) break;
         if (chunk == 1u) return rs != VZ_SUCCESS ? rs : set_error(VZ_ERROR_OUT_OF_MEMORY, "launch buffers do not fit");
         chunk = split((chunk + 1) / 2);
     }
@@ -805,7 +810,7 @@ vzStatus path_launch(vzContext ctx, const PathItem& item, hipStream_t st, RunRes
 {
     PathWork* w = nullptr;
     VZ_TRY(path_work(ctx, &w));
-    VZ_TRY(w->plain.init(false));
+    VZ_TRY(w->plain.init(ctx, false));
     std::vector<Event> ev;
     PathOptions opt;
     opt.count = (item.params.flags & VZ_COUNT_VISITS) != 0;
@@ -851,7 +856,7 @@ vzStatus path_batch(vzContext ctx, const std::vector<PathItem>& items, const vzT
     }
     const uint64_t budget = tuning_budget(t);
     if (slot.paths_bytes > budget + 256) slot.free();  // a smaller tuning gives memory back
-    VZ_TRY(slot.init(true));
+    VZ_TRY(slot.init(ctx, true));
     slot.used = 0;
     // small items first, so that the slot has its size before anything runs
     std::vector<std::vector<const PathItem*>> groups(1);

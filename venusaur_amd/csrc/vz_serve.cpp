@@ -305,7 +305,7 @@ vzStatus vzServerCreate(vzContext ctx, const vzServeConfig* cfg, vzServer* out)
         if (rs == VZ_SUCCESS && !f.done.ok()) rs = set_error(VZ_ERROR_HIP, "hipEventCreate failed");
         if (rs == VZ_SUCCESS && hipStreamCreateWithFlags(&f.stream, hipStreamNonBlocking) != hipSuccess)
             rs = set_error(VZ_ERROR_HIP, "hipStreamCreateWithFlags failed");
-        if (rs == VZ_SUCCESS) rs = f.slot.init(true);
+        if (rs == VZ_SUCCESS) rs = f.slot.init(ctx, true);
         if (rs == VZ_SUCCESS) rs = slot_reserve(f.slot, s->slot_budget / kPathBytes);
     }
     if (rs != VZ_SUCCESS) {
