@@ -330,7 +330,10 @@ __global__ void __launch_bounds__(path_threads(SRC)) __attribute__((amdgpu_waves
                     else tr.flush(sc, sh.pend + tid, kMemBlk, ns);
                 }
             }
-            if ((uint32_t)__popcll(busy) < G.refill) break;
+            // with no paths left to take, the wave finishes its rays first:
+            // leaving at every step made the last paths of a launch slower
+            // (400x225 at 16 samples 1005 us against 812)
+            if (!exhausted && (uint32_t)__popcll(busy) < G.refill) break;
         }
         // every queued test has run before a lane's hit is shaded
         if constexpr (LDSN) tr.flush(sc, sh);
