@@ -62,10 +62,12 @@ struct SceneView {           // what kernels need to traverse one scene
     const float4* mats;      // leaf order {albedo rgb, fuzz | ior}
     uint32_t n;              // primitives (leaves)
     uint32_t nw;             // 4-wide nodes (0 for a single sphere)
-    __host__ __device__ uint32_t count() const { return n; }
-    __host__ __device__ const float4* sphere_array() const { return spheres; }
-    __host__ __device__ const uint32_t* info_array() const { return leaf_info; }
-    __host__ __device__ const float4* mat_array() const { return mats; }
+    // the same for the traversals that do not count: 48-byte nodes, leaves in
+    // their order (a single sphere: the arrays above)
+    const uint4* tnodes;
+    const float4* tspheres;
+    const uint32_t* tinfo;
+    const float4* tmats;
 };
 
 struct PathWork;
@@ -179,6 +181,12 @@ struct vzScene_st {
     uint32_t* d_fcount = nullptr;
     // the 4-wide tree collapsed from the binary one (traversed by every kernel)
     uint4* d_wnodes = nullptr;        // 4 uint4 per wide node, at most n-1 of them
+    // the same tree and its leaves as the traversals that do not count read
+    // them (vz_traverse_mem.h)
+    uint4* d_tnodes = nullptr;        // 3 uint4 per wide node, level order
+    float4* d_tsph = nullptr;         // the leaves' spheres, info and materials, 3 spare spheres at the end
+    uint32_t* d_tinfo = nullptr;
+    float4* d_tmat = nullptr;
     uint32_t* d_wkids = nullptr;      // 4 binary child references per wide root
     uint32_t* d_wflag = nullptr;      // per binary node: wide-root bit and child count
     uint32_t* d_widx = nullptr;       // per binary node: its wide node index (roots only)
@@ -193,12 +201,16 @@ struct vzScene_st {
     vz::SceneView view() const
     {
         vz::SceneView v;
-        v.nodes = d_wnodes;
+        v.nodes = nw ? d_wnodes : nullptr;
         v.spheres = d_sph;
         v.leaf_info = d_leaf_info;
         v.mats = d_mat;
         v.n = n;
         v.nw = nw;
+        v.tnodes = nw ? d_tnodes : nullptr;
+        v.tspheres = nw ? d_tsph : d_sph;
+        v.tinfo = nw ? d_tinfo : d_leaf_info;
+        v.tmats = nw ? d_tmat : d_mat;
         return v;
     }
 };

@@ -1063,6 +1063,7 @@ __global__ void __launch_bounds__(kRefitThreads) k_refit_top(const float4* __res
 // 24-27) and valid flags (28-31).
 constexpr uint32_t kWideRoot = 0x80000000u;  // wide-root flag of a binary node
 constexpr uint32_t kLeafRef = 0x80000000u;   // a wide child that is a leaf
+constexpr uint32_t kLeafCount = kMaxDepth + 2;  // word of the level counts: leaves given a place so far
 constexpr uint32_t kScanItems = 4;            // root flags per thread in the index scan
 constexpr uint32_t kScanTile = kBlk * kScanItems;
 
@@ -1152,27 +1153,44 @@ __global__ void __launch_bounds__(kBlk) k_wide_level(const uint32_t* __restrict_
                                                      const uint32_t* __restrict__ front_in,
                                                      uint32_t* __restrict__ front_out, uint32_t* __restrict__ cnt,
                                                      uint32_t level, uint32_t* __restrict__ wkids,
-                                                     uint32_t* __restrict__ wflag)
+                                                     uint32_t* __restrict__ wflag, uint32_t* __restrict__ tidx,
+                                                     uint32_t* __restrict__ tchild, uint32_t* __restrict__ tleaf)
 {
     const uint32_t count = cnt[level], lane = lane_id();
+    // roots of the levels above: the first of this level in level order
+    uint32_t before = lane < level ? cnt[lane] : 0u;
+    for (int o = 32; o >= 1; o >>= 1) before += __shfl_xor(before, o);
     for (uint32_t i0 = (blockIdx.x * kBlk + threadIdx.x) & ~63u; i0 < count; i0 += gridDim.x * kBlk) {
         const uint32_t i = i0 + lane;
-        uint32_t ks[4] = {0u, 0u, 0u, 0u}, n_k = 0, n_in = 0;
+        uint32_t ks[4] = {0u, 0u, 0u, 0u}, n_k = 0, n_in = 0, r = 0;
         if (i < count) {
-            const uint32_t r = front_in[i];
+            r = front_in[i];
             n_k = wide_children(r, child, boxes, ks);
             reinterpret_cast<uint4*>(wkids)[r] = make_uint4(ks[0], ks[1], ks[2], ks[3]);
             wflag[r] = kWideRoot | n_k;
             for (uint32_t k = 0; k < 4u; k++) n_in += k < n_k && !(ks[k] & kLeafRef) ? 1u : 0u;
         }
-        uint32_t incl = n_in;
+        const uint32_t n_leaf = n_k - n_in;
+        uint32_t incl = n_in, lincl = n_leaf;
         for (uint32_t off = 1; off < 64u; off <<= 1) {
-            const uint32_t x = __shfl_up(incl, off);
-            if (lane >= off) incl += x;
+            const uint32_t x = __shfl_up(incl, off), y = __shfl_up(lincl, off);
+            if (lane >= off) {
+                incl += x;
+                lincl += y;
+            }
         }
-        uint32_t base = 0;
-        if (lane == 63u && incl) base = atomicAdd(&cnt[level + 1], incl);
+        uint32_t base = 0, lbase = 0;
+        if (lane == 63u) {
+            if (incl) base = atomicAdd(&cnt[level + 1], incl);
+            if (lincl) lbase = atomicAdd(&cnt[kLeafCount], lincl);
+        }
         uint32_t at = __shfl(base, 63) + incl - n_in;
+        const uint32_t lat = __shfl(lbase, 63) + lincl - n_leaf;
+        if (i < count) {  // the root's place in level order, its children's, its leaves'
+            tidx[r] = before + i;
+            tchild[r] = before + count + at;
+            tleaf[r] = lat;
+        }
         for (uint32_t k = 0; k < 4u; k++) {
             if (k >= n_k || (ks[k] & kLeafRef)) continue;
             wflag[ks[k]] = kWideRoot;
@@ -1235,11 +1253,35 @@ __global__ void __launch_bounds__(kBlk) k_wscan_apply(const uint32_t* __restrict
     }
 }
 
+// What k_wide_pack writes for the traversals that do not count: the same tree
+// as 48-byte nodes, three 16-byte loads a visit instead of four, and the
+// leaves in the order of the nodes that name them.  A node's internal
+// children come first in its slots and lie next to each other in level
+// order, its leaves after them likewise, so one index each stands for all of
+// them (a traversal of many rays is bound by the L1's accesses as much as by
+// the VALU).  Words: the node box's lo corner (3 floats); scale exponents
+// (bytes 0-2) and the number of internal children (byte 3); the quantised lo
+// planes of the 4 slots for x, y, z, then the hi planes (byte c = slot c; an
+// empty slot's lie the wrong way round); the first internal child (in units
+// of 16 bytes), the first leaf.  An empty slot that an extreme ray passes all
+// the same names a leaf of some other node, or one of the spare ones at the
+// end: testing it is harmless.
+struct TravOut {
+    const uint32_t *tidx, *tchild, *tleaf;
+    const uint32_t* info;   // leaf order
+    const float4* mat;
+    uint32_t n;             // leaves
+    uint4* nodes;           // 3 per node
+    float4* sph;            // traversal order, 3 spare at the end
+    uint32_t* tinfo;
+    float4* tmat;
+};
+
 __global__ void __launch_bounds__(kBlk) k_wide_pack(const float4* __restrict__ sph, const uint32_t* __restrict__ wkids,
                                                     const uint32_t* __restrict__ wflag,
                                                     const uint32_t* __restrict__ widx,
                                                     const float* __restrict__ boxes, uint32_t ni,
-                                                    uint4* __restrict__ wnodes)
+                                                    uint4* __restrict__ wnodes, TravOut T)
 {
     const uint32_t r = blockIdx.x * kBlk + threadIdx.x;
     if (r >= ni) return;
@@ -1248,28 +1290,45 @@ __global__ void __launch_bounds__(kBlk) k_wide_pack(const float4* __restrict__ s
     const uint32_t cnt = fl & 7u;
     const float* nb = boxes + (size_t)r * 6;
     uint32_t meta = 0, qlo[3] = {0u, 0u, 0u}, qhi[3] = {0u, 0u, 0u}, ch[4] = {0u, 0u, 0u, 0u};
+    uint32_t tlo[3] = {0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu}, thi[3] = {0u, 0u, 0u};
     float sc[3];
     for (int k = 0; k < 3; k++) {
         const uint32_t e = pick_exp(nb[k], nb[3 + k]);
         sc[k] = __uint_as_float(e << 23);
         meta |= e << (8 * k);
     }
+    const uint4 refs = reinterpret_cast<const uint4*>(wkids)[r];
+    const uint32_t ref[4] = {refs.x, refs.y, refs.z, refs.w};
+    uint32_t n_in = 0;
+    for (uint32_t c = 0; c < cnt; c++) n_in += (ref[c] & kLeafRef) ? 0u : 1u;
+    const uint32_t scales = meta, leaf0 = T.tleaf[r];
+    uint32_t slot_in = 0, slot_leaf = n_in;
     for (uint32_t c = 0; c < cnt; c++) {
-        const uint32_t ref = wkids[(size_t)r * 4 + c];
         float cb[6];
-        if (ref & kLeafRef) {
-            const uint32_t leaf = ref & ~kLeafRef;
-            leaf_box(sph[leaf], cb);
+        uint32_t t;  // the child's slot in the 48-byte node
+        if (ref[c] & kLeafRef) {
+            const uint32_t leaf = ref[c] & ~kLeafRef;
+            const float4 s = sph[leaf];
+            leaf_box(s, cb);
             ch[c] = leaf;
             meta |= 1u << (24 + c);
+            t = slot_leaf++;
+            const uint32_t at = leaf0 + t - n_in;
+            T.sph[at] = s;
+            T.tinfo[at] = T.info[leaf];
+            T.tmat[at] = T.mat[leaf];
         } else {
-            for (int k = 0; k < 6; k++) cb[k] = boxes[(size_t)ref * 6 + k];
-            ch[c] = widx[ref];
+            for (int k = 0; k < 6; k++) cb[k] = boxes[(size_t)ref[c] * 6 + k];
+            ch[c] = widx[ref[c]];
+            t = slot_in++;
         }
         meta |= 1u << (28 + c);
         for (int k = 0; k < 3; k++) {
-            qlo[k] |= quant_lo(cb[k], nb[k], sc[k]) << (8 * c);
-            qhi[k] |= quant_hi(cb[3 + k], nb[k], sc[k]) << (8 * c);
+            const uint32_t lo = quant_lo(cb[k], nb[k], sc[k]), hi = quant_hi(cb[3 + k], nb[k], sc[k]);
+            qlo[k] |= lo << (8 * c);
+            qhi[k] |= hi << (8 * c);
+            tlo[k] = (tlo[k] & ~(0xFFu << (8 * t))) | lo << (8 * t);
+            thi[k] |= hi << (8 * t);
         }
     }
     uint4* w = wnodes + (size_t)widx[r] * 4;
@@ -1277,6 +1336,16 @@ __global__ void __launch_bounds__(kBlk) k_wide_pack(const float4* __restrict__ s
     w[1] = make_uint4(qlo[0], qlo[1], qlo[2], qhi[0]);
     w[2] = make_uint4(qhi[1], qhi[2], ch[0], ch[1]);
     w[3] = make_uint4(ch[2], ch[3], 0u, 0u);
+    uint4* v = T.nodes + (size_t)T.tidx[r] * 3;
+    v[0] = make_uint4(__float_as_uint(nb[0]), __float_as_uint(nb[1]), __float_as_uint(nb[2]), scales | n_in << 24);
+    v[1] = make_uint4(tlo[0], tlo[1], tlo[2], thi[0]);
+    v[2] = make_uint4(thi[1], thi[2], 3u * T.tchild[r], leaf0);
+    if (r == 0u)  // the spare leaves are one of the scene's once more
+        for (uint32_t k = 0; k < 3; k++) {
+            T.sph[T.n + k] = sph[0];
+            T.tinfo[T.n + k] = T.info[0];
+            T.tmat[T.n + k] = T.mat[0];
+        }
 }
 
 __global__ void k_zero(uint32_t* a, uint32_t n)
@@ -1398,6 +1467,10 @@ vzStatus lbvh_alloc(vzScene s)
     part(&s->d_frontier, sizeof(uint32_t) * n);
     part(&s->d_fcount, 256);
     part(&s->d_wnodes, sizeof(uint4) * 4 * ni);
+    part(&s->d_tnodes, sizeof(uint4) * 3 * ni);
+    part(&s->d_tsph, sizeof(float4) * (n + 3));
+    part(&s->d_tinfo, sizeof(uint32_t) * (n + 3));
+    part(&s->d_tmat, sizeof(float4) * (n + 3));
     part(&s->d_wkids, sizeof(uint32_t) * 4 * ni);
     part(&s->d_wflag, sizeof(uint32_t) * ni);
     part(&s->d_widx, sizeof(uint32_t) * (ni + blocks_for(ni, kScanTile) + 1));  // + tile sums
@@ -1417,13 +1490,18 @@ void lbvh_free(vzScene s)
     s->arena = nullptr;
 }
 
-// Structural check of the packed 4-wide tree, so that traversal needs no
-// per-visit guards: every child index in range, every leaf referenced by
-// exactly one slot, every wide node but the root by exactly one slot and the
-// root by none.  Then a walk from the root reaches each node at most once
-// and ends.  Any violation sets *err.
-__global__ void __launch_bounds__(kBlk) k_wide_refs(const uint4* __restrict__ wnodes, const uint32_t* __restrict__ nwp,
-                                                    uint32_t n, uint32_t* __restrict__ wref,
+// Structural check of both packed forms of the 4-wide tree, so that traversal
+// needs no per-visit guards: every child index in range, every leaf
+// referenced by exactly one slot, every wide node but the root by exactly one
+// slot and the root by none.  Then a walk from the root reaches each node at
+// most once and ends.  References count 1 from a 64-byte node and kTravRef
+// from a 48-byte one.  Any violation sets *err.
+constexpr uint32_t kTravRef = 0x10000u;
+__global__ void __launch_bounds__(kBlk) k_wide_refs(const uint4* __restrict__ wnodes, const uint4* __restrict__ tnodes,
+                                                    const uint32_t* __restrict__ wflag,
+                                                    const uint32_t* __restrict__ tidx, uint32_t ni,
+                                                    const uint32_t* __restrict__ nwp, uint32_t n,
+                                                    uint32_t* __restrict__ wref, uint32_t* __restrict__ tref,
                                                     uint32_t* __restrict__ lref, uint32_t* __restrict__ err)
 {
     const uint32_t nw = *nwp;
@@ -1442,16 +1520,36 @@ __global__ void __launch_bounds__(kBlk) k_wide_refs(const uint4* __restrict__ wn
             }
         }
     }
+    for (uint32_t r = blockIdx.x * kBlk + threadIdx.x; r < ni; r += gridDim.x * kBlk) {
+        const uint32_t fl = wflag[r];
+        if (!(fl & kWideRoot)) continue;
+        const uint32_t t = tidx[r];
+        if (t >= nw) {
+            *err = 1u;
+            continue;
+        }
+        const uint32_t meta = tnodes[3 * (size_t)t].w, first3 = tnodes[3 * (size_t)t + 2].z, first = first3 / 3u;
+        const uint32_t leaf = tnodes[3 * (size_t)t + 2].w, n_in = meta >> 24, n_leaf = (fl & 7u) - n_in;
+        if (n_in > 4u || n_leaf > 4u || leaf > n || n_leaf > n - leaf || (n_in && first == 0u) ||
+            (n_in && first3 != 3u * first) || (n_in && first > nw) ||
+            (n_in && n_in > nw - first)) {
+            *err = 1u;
+            continue;
+        }
+        for (uint32_t k = 0; k < n_in; k++) atomicAdd(&tref[first + k], 1u);
+        for (uint32_t k = 0; k < n_leaf; k++) atomicAdd(&lref[leaf + k], kTravRef);
+    }
 }
 
 __global__ void __launch_bounds__(kBlk) k_wide_verify(const uint32_t* __restrict__ nwp, uint32_t n,
                                                       const uint32_t* __restrict__ wref,
+                                                      const uint32_t* __restrict__ tref,
                                                       const uint32_t* __restrict__ lref, uint32_t* __restrict__ err)
 {
     const uint32_t nw = *nwp;
     for (uint32_t i = blockIdx.x * kBlk + threadIdx.x; i < n; i += gridDim.x * kBlk) {
-        if (lref[i] != 1u) *err = 1u;
-        if (i < nw && wref[i] != (i == 0u ? 0u : 1u)) *err = 1u;
+        if (lref[i] != 1u + kTravRef) *err = 1u;
+        if (i < nw && (wref[i] != (i == 0u ? 0u : 1u) || tref[i] != wref[i])) *err = 1u;
     }
 }
 
@@ -1461,7 +1559,10 @@ __global__ void __launch_bounds__(kBlk) k_wide_verify(const uint32_t* __restrict
 static vzStatus collapse_wide(vzScene s, hipStream_t st)
 {
     const uint32_t n = s->n, ni = n - 1;
-    uint32_t* cnt = s->d_wcnt;  // [0, kMaxDepth]: roots per level; then nw, a spare word, the check's result
+    uint32_t* cnt = s->d_wcnt;  // [0, kMaxDepth]: roots per level; then nw, leaves placed, the check's result
+    // places in level order, in buffers free at this point: the refit's
+    // counters and the sort's second buffers
+    uint32_t *tidx = s->d_visit, *tchild = s->d_keys[1], *tleaf = s->d_vals[1];
     uint32_t* tsum = s->d_widx + ni;
     const uint32_t ntile = blocks_for(ni, kScanTile);
     hipLaunchKernelGGL(k_zero, dim3(blocks_for(ni, kBlk)), dim3(kBlk), 0, st, s->d_wflag, ni);
@@ -1469,21 +1570,25 @@ static vzStatus collapse_wide(vzScene s, hipStream_t st)
     const uint32_t grid = std::min<uint32_t>(1024u, blocks_for(ni, kBlk));
     for (uint32_t L = 0; L + 1 < s->depth && L < kMaxDepth; L++)
         hipLaunchKernelGGL(k_wide_level, dim3(grid), dim3(kBlk), 0, st, s->d_child, s->d_boxes,
-                           s->d_wfront[L & 1u], s->d_wfront[(L + 1) & 1u], cnt, L, s->d_wkids, s->d_wflag);
+                           s->d_wfront[L & 1u], s->d_wfront[(L + 1) & 1u], cnt, L, s->d_wkids, s->d_wflag, tidx,
+                           tchild, tleaf);
     hipLaunchKernelGGL(k_wscan_tiles, dim3(ntile), dim3(kBlk), 0, st, s->d_wflag, ni, tsum);
     hipLaunchKernelGGL(k_wscan_top, dim3(1), dim3(kBlk), 0, st, tsum, ntile, cnt + kMaxDepth + 1);
     hipLaunchKernelGGL(k_wscan_apply, dim3(ntile), dim3(kBlk), 0, st, s->d_wflag, ni, tsum, s->d_widx);
     hipLaunchKernelGGL(k_wide_pack, dim3(blocks_for(ni, kBlk)), dim3(kBlk), 0, st, s->d_sph, s->d_wkids,
-                       s->d_wflag, s->d_widx, s->d_boxes, ni, s->d_wnodes);
+                       s->d_wflag, s->d_widx, s->d_boxes, ni, s->d_wnodes,
+                       TravOut{tidx, tchild, tleaf, s->d_leaf_info, s->d_mat, n, s->d_tnodes, s->d_tsph, s->d_tinfo,
+                               s->d_tmat});
     // reference counts in buffers free at this point: the level fronts and
     // the refit frontier (both rebuilt by every refit)
-    uint32_t* wref = s->d_wfront[0];
+    uint32_t *wref = s->d_wfront[0], *tref = s->d_wfront[1];
     uint32_t* lref = s->d_frontier;
     hipLaunchKernelGGL(k_zero, dim3(blocks_for(ni, kBlk)), dim3(kBlk), 0, st, wref, ni);
+    hipLaunchKernelGGL(k_zero, dim3(blocks_for(ni, kBlk)), dim3(kBlk), 0, st, tref, ni);
     hipLaunchKernelGGL(k_zero, dim3(blocks_for(n, kBlk)), dim3(kBlk), 0, st, lref, n);
-    hipLaunchKernelGGL(k_wide_refs, dim3(grid), dim3(kBlk), 0, st, s->d_wnodes, cnt + kMaxDepth + 1, n, wref, lref,
-                       cnt + kMaxDepth + 3);
-    hipLaunchKernelGGL(k_wide_verify, dim3(grid), dim3(kBlk), 0, st, cnt + kMaxDepth + 1, n, wref, lref,
+    hipLaunchKernelGGL(k_wide_refs, dim3(grid), dim3(kBlk), 0, st, s->d_wnodes, s->d_tnodes, s->d_wflag, tidx, ni,
+                       cnt + kMaxDepth + 1, n, wref, tref, lref, cnt + kMaxDepth + 3);
+    hipLaunchKernelGGL(k_wide_verify, dim3(grid), dim3(kBlk), 0, st, cnt + kMaxDepth + 1, n, wref, tref, lref,
                        cnt + kMaxDepth + 3);
     VZ_HIP_TRY(hipGetLastError());
     uint32_t h[kMaxDepth + 8] = {};

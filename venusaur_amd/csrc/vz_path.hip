@@ -43,6 +43,7 @@
 
 #include "vz_path.h"
 #include "vz_traverse_lds.h"
+#include "vz_traverse_mem.h"
 
 namespace vz {
 namespace {
@@ -172,29 +173,27 @@ __global__ void __launch_bounds__(kBlk) k_path_seeds(PathGroup G, PathReq one)
     }
 }
 
-// LDS of a workgroup whose nodes are in memory: traversal stacks and queued
-// sphere tests.
-struct MemScene {
+// LDS of a workgroup whose nodes are in memory, where visits are counted.
+struct CountScene {
     uint32_t node[kStackS * kMemBlk];
     float t[kStackS * kMemBlk];
-    uint32_t pend[kPend * kMemBlk];
 };
 struct NoBound {
-    template <class Scene>
-    __device__ explicit NoBound(const Scene&) {}
+    __device__ explicit NoBound(const SceneView&) {}
 };
 
 // What a lane of a many-scene launch keeps of its scene: the two arrays the
-// traversal reads.  The others are looked up in the request table where a
-// hit is shaded.
+// traversal reads (as SceneArrays).  The others are looked up in the request
+// table where a hit is shaded.
+template <bool COUNT>
 struct LaneScene {
     const uint4* nodes;
     const float4* spheres;
     const PathReq* req;
-    __device__ __forceinline__ uint32_t count() const { return ldg(&req->sc.n); }
+    __device__ __forceinline__ const uint4* node_array() const { return nodes; }
     __device__ __forceinline__ const float4* sphere_array() const { return spheres; }
-    __device__ __forceinline__ const uint32_t* info_array() const { return req->sc.leaf_info; }
-    __device__ __forceinline__ const float4* mat_array() const { return req->sc.mats; }
+    __device__ __forceinline__ const uint32_t* info_array() const { return COUNT ? req->sc.leaf_info : req->sc.tinfo; }
+    __device__ __forceinline__ const float4* mat_array() const { return COUNT ? req->sc.mats : req->sc.tmats; }
 };
 
 // Every wave takes units until none is left: the first by its place (so a
@@ -214,23 +213,28 @@ __global__ void __launch_bounds__(path_threads(SRC)) __attribute__((amdgpu_waves
     constexpr bool LDSN = SRC == kOneLds || SRC == kManyLds, MANY = SRC == kManyLds || SRC == kManyMem;
     static_assert(!(COUNT && LDSN), "node visits are counted with the nodes in memory");
     constexpr uint32_t NT = path_threads(SRC), kWaves = NT / 64;
-    constexpr bool DEFER = !COUNT;  // sphere tests queued and run by many lanes together
-    __shared__ typename std::conditional<LDSN, LdsScene<NT>, MemScene>::type sh;
+    __shared__ typename std::conditional<LDSN, LdsScene<NT>,
+                                         typename std::conditional<COUNT, CountScene, MemScene<NT>>::type>::type sh;
     __shared__ unsigned long long s_red[kPathStats][kWaves];
     const uint32_t tid = threadIdx.x, lane = __lane_id();
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(tid >> 6);
     // many requests of many scenes: the lane's own, filled in with its path
-    typename std::conditional<SRC == kManyMem, LaneScene, SceneView>::type sc;
-    if constexpr (SRC == kManyMem) sc = LaneScene{nullptr, nullptr, nullptr};
-    else sc = MANY ? G.reqs[0].sc : one.sc;
-    typename std::conditional<LDSN, PlaneBound, NoBound>::type pb(sc);
+    typename std::conditional<LDSN, SceneView,
+                              typename std::conditional<MANY, LaneScene<COUNT>, SceneArrays>::type>::type sc;
+    const SceneView& view = MANY ? G.reqs[0].sc : one.sc;
+    if constexpr (SRC == kManyMem) sc = LaneScene<COUNT>{nullptr, nullptr, nullptr};
+    else if constexpr (LDSN) sc = view;
+    else sc = scene_arrays<COUNT>(view);
+    typename std::conditional<LDSN, PlaneBound, NoBound>::type pb(view);
     if constexpr (LDSN) {
         stage_scene(sc, sh);
         __syncthreads();
     }
-    typename std::conditional<LDSN, LdsTraversal<NT>, Traversal<kStackS, COUNT, DEFER>>::type tr;
-    typename std::conditional<LDSN, LdsOverflow, Overflow>::type ov;
-    tr.npend = 0;
+    typename std::conditional<LDSN, LdsTraversal<NT>,
+                              typename std::conditional<COUNT, Traversal<kStackS, true>, MemTraversal<NT>>::type>::type tr;
+    typename std::conditional<LDSN, LdsOverflow,
+                              typename std::conditional<COUNT, Overflow, MemOverflow>::type>::type ov;
+    if constexpr (!COUNT) tr.npend = 0;
     uint32_t nv = 0, ns = 0;
     uint32_t n_seg = 0, n_hit = 0;    // of the wave
     bool active = false, tdone = false, exhausted = false, fresh = true;
@@ -293,7 +297,10 @@ __global__ void __launch_bounds__(path_threads(SRC)) __attribute__((amdgpu_waves
                     thr = mk(1.0f, 1.0f, 1.0f);
                     depth = P.max_depth - 1u;
                     if (MANY) my_req = u_req;
-                    if constexpr (SRC == kManyMem) sc = LaneScene{P.sc.nodes, P.sc.spheres, G.reqs + u_req};
+                    if constexpr (SRC == kManyMem) {
+                        const SceneArrays v = scene_arrays<COUNT>(P.sc);
+                        sc = LaneScene<COUNT>{v.nodes, v.spheres, G.reqs + u_req};
+                    }
                     active = start = true;
                 }
             }
@@ -305,7 +312,8 @@ __global__ void __launch_bounds__(path_threads(SRC)) __attribute__((amdgpu_waves
         }
         if (start) {  // new paths and scattered ones alike
             if constexpr (LDSN) tr.init(pb, tr.o, tr.d, 0.001f, 1e16f);
-            else tdone = tr.init(sc, tr.o, tr.d, 0.001f, 1e16f, ns);
+            else if constexpr (COUNT) tdone = tr.init(sc, tr.o, tr.d, 0.001f, 1e16f, ns);
+            else tdone = tr.init(sc, sh, tr.o, tr.d, 0.001f, 1e16f);
             if (LDSN) tdone = false;
             start = false;
         }
@@ -314,20 +322,20 @@ __global__ void __launch_bounds__(path_threads(SRC)) __attribute__((amdgpu_waves
             if (active && !tdone) {
                 if constexpr (LDSN)
                     tdone = tr.step(sh, ov);
+                else if constexpr (COUNT)
+                    tdone = tr.step(sc, sh.node + tid, sh.t + tid, NT, ov, nv, ns);
                 else
-                    tdone = tr.step(sc, GlobalNodes{sc.nodes}, sh.node + tid, sh.t + tid, kMemBlk, ov, nv, ns,
-                                    sh.pend + tid);
+                    tdone = tr.step(sc, sh, ov);
             }
             busy = __ballot(active && !tdone);
-            if (DEFER) {
+            if constexpr (!COUNT) {
                 // flush once enough lanes hold queued tests, relative to the
                 // lanes still tracing, or before a queue could overflow (a
                 // visit queues at most 4)
                 const uint64_t pm = __ballot(tr.npend != 0u);
                 if (pm && (__ballot(tr.npend + 4u > kPend) != 0ull ||
                            kFlushDen * (uint32_t)__popcll(pm) >= kFlushNum * (uint32_t)__popcll(busy))) {
-                    if constexpr (LDSN) tr.flush(sc, sh);
-                    else tr.flush(sc, sh.pend + tid, kMemBlk, ns);
+                    tr.flush(sc, sh);
                 }
             }
             // with no paths left to take, the wave finishes its rays first:
@@ -336,8 +344,7 @@ __global__ void __launch_bounds__(path_threads(SRC)) __attribute__((amdgpu_waves
             if (!exhausted && (uint32_t)__popcll(busy) < G.refill) break;
         }
         // every queued test has run before a lane's hit is shaded
-        if constexpr (LDSN) tr.flush(sc, sh);
-        else if (DEFER) tr.flush(sc, sh.pend + tid, kMemBlk, ns);
+        if constexpr (!COUNT) tr.flush(sc, sh);
         const bool fin = active && tdone;
         const uint64_t fm = __ballot(fin);
         if (fm == 0ull) continue;
@@ -362,11 +369,17 @@ __global__ void __launch_bounds__(path_threads(SRC)) __attribute__((amdgpu_waves
                 L = mul(thr, sky(tr.d));
             } else if (depth > 0u) {
                 // shade (RayTracer.cu:272-440)
-                float4 s;
-                if constexpr (LDSN) s = sh.spheres[tr.bleaf];
-                else s = ldg(sc.sphere_array() + tr.bleaf);
-                const uint32_t type = ldg(sc.info_array() + tr.bleaf) >> 30;
-                const float4 mat = ldg(sc.mat_array() + tr.bleaf);
+                float4 s, mat;
+                uint32_t type;
+                if constexpr (LDSN) {
+                    s = sh.spheres[tr.bleaf];
+                    type = ldg(sc.leaf_info + tr.bleaf) >> 30;
+                    mat = ldg(sc.mats + tr.bleaf);
+                } else {
+                    s = ldg(sc.sphere_array() + tr.bleaf);
+                    type = ldg(sc.info_array() + tr.bleaf) >> 30;
+                    mat = ldg(sc.mat_array() + tr.bleaf);
+                }
                 const v3 pos = add(tr.o, scl(tr.d, tr.best));
                 v3 n = scl(sub(pos, mk(s.x, s.y, s.z)), recip_rn(s.w));
                 const bool front = dot(tr.d, n) < 0.0f;

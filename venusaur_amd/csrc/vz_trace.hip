@@ -15,6 +15,7 @@
 #include <type_traits>
 
 #include "vz_traverse_lds.h"
+#include "vz_traverse_mem.h"
 
 namespace vz {
 
@@ -48,7 +49,7 @@ __global__ void __launch_bounds__(kTraceBlk) k_trace(SceneView sc, const vzRay* 
     if (i < n) {
         const float4* rp = reinterpret_cast<const float4*>(rays + i);
         float4 a = rp[0], b = rp[1];
-        TraceResult r = closest_hit<S, COUNT>(sc, GlobalNodes{sc.nodes}, mk(a.x, a.y, a.z), mk(b.x, b.y, b.z), a.w, b.w,
+        TraceResult r = closest_hit<S, COUNT>(sc, mk(a.x, a.y, a.z), mk(b.x, b.y, b.z), a.w, b.w,
                                               s_node + threadIdx.x, s_t + threadIdx.x, kTraceBlk, nv, ns);
         uint32_t prim = r.leaf == 0xFFFFFFFFu ? VZ_MISS : (sc.leaf_info[r.leaf] & 0x3FFFFFFFu);
         reinterpret_cast<uint2*>(hits)[i] = make_uint2(__float_as_uint(r.t), prim);
@@ -112,31 +113,29 @@ constexpr uint32_t kTraceMemBlk = 512;
 constexpr uint32_t kTraceRefill = 32;
 constexpr uint32_t kFlushNum = 2, kFlushDen = 3;  // as in vz_path.hip
 
-struct TraceMem {
-    uint32_t node[kWideStackS * kTraceMemBlk];
-    float t[kWideStackS * kTraceMemBlk];
-    uint32_t pend[kPend * kTraceMemBlk];
-};
 struct TraceNoBound {
     VZ_DEV explicit TraceNoBound(const SceneView&) {}
 };
 
 template <bool LDSN>
 __global__ void __launch_bounds__(LDSN ? kTraceLdsBlk : kTraceMemBlk) __attribute__((amdgpu_waves_per_eu(6)))
-k_trace_hits(SceneView sc, const vzRay* __restrict__ rays, uint32_t n, vzHit* __restrict__ hits)
+k_trace_hits(SceneView view, const vzRay* __restrict__ rays, uint32_t n, vzHit* __restrict__ hits)
 {
     constexpr uint32_t NT = LDSN ? kTraceLdsBlk : kTraceMemBlk;
-    __shared__ typename std::conditional<LDSN, LdsScene<NT>, TraceMem>::type sh;
+    __shared__ typename std::conditional<LDSN, LdsScene<NT>, MemScene<NT>>::type sh;
     const uint32_t tid = threadIdx.x, wave = (uint32_t)__builtin_amdgcn_readfirstlane(tid >> 6);
-    const typename std::conditional<LDSN, PlaneBound, TraceNoBound>::type pb(sc);
+    const typename std::conditional<LDSN, PlaneBound, TraceNoBound>::type pb(view);
+    typename std::conditional<LDSN, SceneView, SceneArrays>::type sc;
+    if constexpr (LDSN) sc = view;
+    else sc = scene_arrays<false>(view);
     if constexpr (LDSN) {
         stage_scene(sc, sh);
         __syncthreads();
     }
-    typename std::conditional<LDSN, LdsTraversal<NT, true>, Traversal<kWideStackS, false, true>>::type tr;
-    typename std::conditional<LDSN, LdsOverflow, Overflow>::type ov;
+    typename std::conditional<LDSN, LdsTraversal<NT, true>, MemTraversal<NT, true>>::type tr;
+    typename std::conditional<LDSN, LdsOverflow, MemOverflow>::type ov;
     tr.npend = 0;
-    uint32_t nv = 0, ns = 0, mine = 0;
+    uint32_t mine = 0;
     bool active = false, tdone = false;
     // the wave's next ray, the end of its packet and the packets' stride
     const uint32_t stride = gridDim.x * NT;
@@ -150,7 +149,7 @@ k_trace_hits(SceneView sc, const vzRay* __restrict__ rays, uint32_t n, vzHit* __
                 const float4* rp = reinterpret_cast<const float4*>(rays + mine);
                 const float4 a = ldg(rp), b = ldg(rp + 1);
                 if constexpr (LDSN) tr.init(pb, mk(a.x, a.y, a.z), mk(b.x, b.y, b.z), a.w, b.w);
-                else tdone = tr.init(sc, mk(a.x, a.y, a.z), mk(b.x, b.y, b.z), a.w, b.w, ns);
+                else tdone = tr.init(sc, sh, mk(a.x, a.y, a.z), mk(b.x, b.y, b.z), a.w, b.w);
                 if (LDSN) tdone = false;
                 active = true;
             }
@@ -168,22 +167,19 @@ k_trace_hits(SceneView sc, const vzRay* __restrict__ rays, uint32_t n, vzHit* __
                 if constexpr (LDSN)
                     tdone = tr.step(sh, ov);
                 else
-                    tdone = tr.step(sc, GlobalNodes{sc.nodes}, sh.node + tid, sh.t + tid, kTraceMemBlk, ov, nv, ns,
-                                    sh.pend + tid);
+                    tdone = tr.step(sc, sh, ov);
             }
             busy = __ballot(active && !tdone);
             const uint64_t pm = __ballot(tr.npend != 0u);
             if (pm && (__ballot(tr.npend + 4u > kPend) != 0ull ||
                        kFlushDen * (uint32_t)__popcll(pm) >= kFlushNum * (uint32_t)__popcll(busy))) {
-                if constexpr (LDSN) tr.flush(sc, sh);
-                else tr.flush(sc, sh.pend + tid, kTraceMemBlk, ns);
+                tr.flush(sc, sh);
             }
             if (more && (uint32_t)__popcll(busy) < kTraceRefill) break;
         }
-        if constexpr (LDSN) tr.flush(sc, sh);
-        else tr.flush(sc, sh.pend + tid, kTraceMemBlk, ns);
+        tr.flush(sc, sh);
         if (active && tdone) {
-            const uint32_t prim = tr.bleaf == 0xFFFFFFFFu ? VZ_MISS : (ldg(sc.leaf_info + tr.bleaf) & 0x3FFFFFFFu);
+            const uint32_t prim = tr.bleaf == 0xFFFFFFFFu ? VZ_MISS : (ldg((LDSN ? view.leaf_info : view.tinfo) + tr.bleaf) & 0x3FFFFFFFu);
             reinterpret_cast<uint2*>(hits)[mine] = make_uint2(__float_as_uint(tr.best), prim);
             active = false;
         }

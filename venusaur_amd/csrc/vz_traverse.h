@@ -26,34 +26,78 @@ namespace vz {
 
 constexpr float kRobust = 1.0f + 0x1p-20f;  // >= 1 + 2*gamma_3 (Ize 2013)
 
+constexpr uint32_t kPend = 8;  // queued leaf tests per lane (traversals that do not count)
+
 struct TraceResult {
     float t;
     uint32_t leaf;  // leaf (Morton-order) index, 0xFFFFFFFF on a miss
 };
 
-// Where the 64-byte nodes come from: the scene's array in HBM, or a copy a
-// workgroup staged in LDS (a small scene rendered alone).
-struct LdsNodes {
-    const uint4* p;  // points into __shared__ memory
-    VZ_DEV void fetch(uint32_t i, uint4& a, uint4& b, uint4& c, uint4& d) const
-    {
-        a = p[4 * i];
-        b = p[4 * i + 1];
-        c = p[4 * i + 2];
-        d = p[4 * i + 3];
+// The sphere test (root in [tmin, best]) gated by the sphere's own box: the
+// root counts only if the ray enters [c - |r|, c + |r|] by t, by the same
+// robust slab test as the nodes.  OptiX runs an intersection program only for
+// primitives whose box the ray enters; the gate also drops the spurious
+// grazing roots that float rounding of |oc|^2 - r^2 gives tiny distant
+// spheres, and it makes the closest hit independent of the tree: every node
+// box contains its leaves' boxes, so it passes whenever the gate does, and any
+// BVH reaches every gated root.
+VZ_DEV bool hit_gated(v3 o, v3 d, const float (&inv)[3], float tmin, float best, float4 s, float& t)
+{
+    if (!hit_sphere(o, d, tmin, best, s, t)) return false;
+    const float r = fabsf(s.w);
+    const float c[3] = {s.x, s.y, s.z}, org[3] = {o.x, o.y, o.z};
+    float lo_t = tmin, hi_t = t;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        // the near plane is c - r for a positive inv, c + r for a negative
+        // one: with sr = copysign(r, inv), c - sr and c + sr are exactly
+        // those planes (x - (-y) rounds as x + y), and rounding is monotone,
+        // so these are min(t0, t1) and max(t0, t1) of the two plane distances
+        // bit for bit
+        const float sr = copysignf(r, inv[k]);
+        lo_t = fmaxf(lo_t, ((c[k] - sr) - org[k]) * inv[k]);
+        hi_t = fminf(hi_t, ((c[k] + sr) - org[k]) * inv[k]);
     }
-};
-struct GlobalNodes {
-    const uint4* p;
-    VZ_DEV void fetch(uint32_t i, uint4& a, uint4& b, uint4& c, uint4& d) const
-    {
-        const uint4* q = p + 4 * (size_t)i;
-        a = ldg(q);
-        b = ldg(q + 1);
-        c = ldg(q + 2);
-        d = ldg(q + 3);
+    return lo_t <= hi_t * kRobust;
+}
+
+// A gated root t <= best of leaf `leaf`: keeps the lexicographic minimum of
+// (t, prim).
+VZ_DEV void keep_nearer(float t, uint32_t leaf, const uint32_t* info, float& best, uint32_t& bleaf)
+{
+    if (t < best) {
+        best = t;
+        bleaf = leaf;
+        return;
     }
+    const uint32_t pid = ldg(info + leaf) & 0x3FFFFFFFu;
+    const uint32_t bpid = bleaf == 0xFFFFFFFFu ? 0xFFFFFFFFu : ldg(info + bleaf) & 0x3FFFFFFFu;
+    if (pid < bpid) {
+        best = t;
+        bleaf = leaf;
+    }
+}
+
+// The arrays of a scene in memory that a traversal reads, with its nodes null
+// for a single sphere: the 64-byte nodes and the leaves in their order for
+// the traversal that counts, the 48-byte ones and theirs for the others.
+struct SceneArrays {
+    const uint4* nodes;
+    const float4* spheres;
+    const uint32_t* info;
+    const float4* mats;
+    VZ_DEV const uint4* node_array() const { return nodes; }
+    VZ_DEV const float4* sphere_array() const { return spheres; }
+    VZ_DEV const uint32_t* info_array() const { return info; }
+    VZ_DEV const float4* mat_array() const { return mats; }
 };
+template <bool COUNT>
+VZ_DEV SceneArrays scene_arrays(const SceneView& sc)
+{
+    return COUNT ? SceneArrays{sc.nodes, sc.spheres, sc.leaf_info, sc.mats}
+                 : SceneArrays{sc.tnodes, sc.tspheres, sc.tinfo, sc.tmats};
+}
+
 
 // The oldest stack entries of a lane once its LDS ring is full.  Kept apart
 // from Traversal so the traversal's scalars stay in registers: the compiler
@@ -69,24 +113,13 @@ struct Overflow {
 // as its traversal ends instead of waiting for the slowest lane.
 // S: LDS slots per lane (power of two); lds_node/lds_t point at this lane's
 // column, consecutive slots `stride` words apart.
-// DEFER: leaf slots that a visit hits are queued (the lane's column of
-// lds_pend, at most kPend entries) instead of tested at once, and flush()
-// tests them; the caller flushes when many lanes of the wave hold some, so a
-// wave's sphere tests run with more lanes at a time.  Culling meanwhile uses
-// the best hit found so far, which is no smaller than it would otherwise be:
-// no node that holds the closest hit is culled, and the closest hit (the
-// least (t, prim) over the spheres tested) does not depend on the order of
-// the tests.  Node-visit and sphere-test counts do depend on when the wave
-// flushes, so the counting kernels test at once.
-constexpr uint32_t kPend = 8;
-template <int S, bool COUNT, bool DEFER = false>
+template <int S, bool COUNT>
 struct Traversal {
     v3 o, d;
     float inv[3];
     float tmin, best;
     uint32_t negm;  // bit k: the ray runs towards -k, so a slot's near plane on axis k is its hi plane
-    uint32_t bleaf, bprim, node, sp, bottom;
-    uint32_t npend = 0;  // DEFER: queued leaf tests (0 also for a lane that never gets a ray)
+    uint32_t bleaf, node, sp, bottom;
 
     // Returns true when the ray is already finished (single-sphere scene).
     template <class Scene>
@@ -97,8 +130,6 @@ struct Traversal {
         tmin = tmin_;
         best = tmax_;
         bleaf = 0xFFFFFFFFu;
-        bprim = 0xFFFFFFFFu;
-        npend = 0;
         ray_inverse(d, inv);
         negm = 0u;
 #pragma unroll
@@ -108,73 +139,24 @@ struct Traversal {
             // direction, hi for a negative one
             negm |= (inv[k] < 0.0f ? 1u : 0u) << k;
         }
-        if (sc.count() == 1u) {
-            float t;
-            if (COUNT) ns++;
-            if (hit_gated(ldg(sc.sphere_array()), t)) {
-                best = t;
-                bleaf = 0;
-            }
-            return true;
-        }
         sp = 0;
         bottom = 0;
         node = 0;
         // the build checks every child index and that each node has one
         // parent, so a walk from the root ends: no guards per visit
-        return false;
+        if (sc.node_array() != nullptr) return false;
+        test_leaf(sc, 0u, ns);
+        return true;
     }
 
-    // The sphere test (root in [tmin, best]) gated by the sphere's own box:
-    // the root counts only if the ray enters [c - |r|, c + |r|] by t, by the
-    // same robust slab test as the nodes.  OptiX runs an intersection program
-    // only for primitives whose box the ray enters; the gate also drops the
-    // spurious grazing roots that float rounding of |oc|^2 - r^2 gives tiny
-    // distant spheres, and it makes the closest hit independent of the tree:
-    // every node box contains its leaves' boxes, so it passes whenever the
-    // gate does, and any BVH reaches every gated root.
-    VZ_DEV bool hit_gated(float4 s, float& t) const
-    {
-        if (!hit_sphere(o, d, tmin, best, s, t)) return false;
-        const float r = fabsf(s.w);
-        const float c[3] = {s.x, s.y, s.z}, org[3] = {o.x, o.y, o.z};
-        float lo_t = tmin, hi_t = t;
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-            // the near plane is c - r for a positive inv, c + r for a negative
-            // one: with sr = copysign(r, inv), c - sr and c + sr are exactly
-            // those planes (x - (-y) rounds as x + y), and rounding is
-            // monotone, so these are min(t0, t1) and max(t0, t1) of the two
-            // plane distances bit for bit
-            const float sr = copysignf(r, inv[k]);
-            lo_t = fmaxf(lo_t, ((c[k] - sr) - org[k]) * inv[k]);
-            hi_t = fminf(hi_t, ((c[k] + sr) - org[k]) * inv[k]);
-        }
-        return lo_t <= hi_t * kRobust;
-    }
-
-    // Sphere test of leaf `leaf` (sphere s); keeps the lexicographic minimum
-    // of (t, prim).
+    // Sphere test of leaf `leaf`; keeps the lexicographic minimum of (t, prim).
     template <class Scene>
-    VZ_DEV void test_leaf(const Scene& sc, uint32_t leaf, float4 s, uint32_t& ns)
+    VZ_DEV void test_leaf(const Scene& sc, uint32_t leaf, uint32_t& ns)
     {
         float t;
         if (COUNT) ns++;
-        if (hit_gated(s, t)) {
-            if (t < best) {
-                best = t;
-                bleaf = leaf;
-                bprim = 0xFFFFFFFFu;  // looked up lazily on a tie
-            } else {
-                const uint32_t pid = ldg(sc.info_array() + leaf) & 0x3FFFFFFFu;
-                if (bprim == 0xFFFFFFFFu && bleaf != 0xFFFFFFFFu) bprim = ldg(sc.info_array() + bleaf) & 0x3FFFFFFFu;
-                if (pid < bprim) {
-                    best = t;
-                    bleaf = leaf;
-                    bprim = pid;
-                }
-            }
-        }
+        if (hit_gated(o, d, inv, tmin, best, ldg(sc.sphere_array() + leaf), t))
+            keep_nearer(t, leaf, sc.info_array(), best, bleaf);
     }
 
     // Pops the nearest stacked node that can still hold a closer hit.
@@ -201,33 +183,13 @@ struct Traversal {
         return true;
     }
 
-    // DEFER: tests the queued leaves (the lane's column of lds_pend).
-    template <class Scene>
-    VZ_DEV void flush(const Scene& sc, const uint32_t* lds_pend, uint32_t stride, uint32_t& ns)
-    {
-        while (npend) {
-            npend--;
-            const uint32_t leaf = lds_pend[npend * stride];
-            test_leaf(sc, leaf, ldg(sc.sphere_array() + leaf), ns);
-        }
-    }
-
     // One wide node visit; returns true when the traversal has finished.
-    template <class Scene, class NodeSrc>
-    VZ_DEV bool step(const Scene& sc, const NodeSrc& nodes, uint32_t* lds_node, float* lds_t,
-                     uint32_t stride, Overflow& ov, uint32_t& nv, uint32_t& ns, uint32_t* lds_pend = nullptr)
-    {
-        uint4 A, B, C, D;
-        nodes.fetch(node, A, B, C, D);
-        return visit(sc, A, B, C, D, lds_node, lds_t, stride, ov, nv, ns, lds_pend);
-    }
-
-    // The visit of the current node, whose 64 bytes are A..D.
     template <class Scene>
-    VZ_DEV bool visit(const Scene& sc, const uint4& A, const uint4& B, const uint4& C, const uint4& D,
-                      uint32_t* lds_node, float* lds_t, uint32_t stride, Overflow& ov, uint32_t& nv, uint32_t& ns,
-                      uint32_t* lds_pend)
+    VZ_DEV bool step(const Scene& sc, uint32_t* lds_node, float* lds_t, uint32_t stride, Overflow& ov, uint32_t& nv,
+                     uint32_t& ns)
     {
+        const uint4* q = sc.node_array() + 4 * (size_t)node;
+        const uint4 A = ldg(q), B = ldg(q + 1), C = ldg(q + 2), D = ldg(q + 3);
         if (COUNT) nv++;
         const float no[3] = {__uint_as_float(A.x), __uint_as_float(A.y), __uint_as_float(A.z)};
         const float org[3] = {o.x, o.y, o.z};
@@ -284,12 +246,7 @@ struct Traversal {
             const uint32_t c = (uint32_t)__builtin_ctz(lm);
             const uint32_t lo = (c & 1u) ? ch[1] : ch[0], hi = (c & 1u) ? ch[3] : ch[2];
             const uint32_t leaf = (c & 2u) ? hi : lo;  // selects, not branches
-            if (DEFER) {
-                lds_pend[npend * stride] = leaf;
-                npend++;
-            } else {
-                test_leaf(sc, leaf, ldg(sc.sphere_array() + leaf), ns);
-            }
+            test_leaf(sc, leaf, ns);
             lm &= lm - 1u;
         }
         // internal slots that were hit and can still hold a closer hit
@@ -345,15 +302,15 @@ struct Traversal {
 };
 
 // Whole-ray traversal: init, then step until done.
-template <int S, bool COUNT, class NodeSrc>
-VZ_DEV TraceResult closest_hit(const SceneView& sc, const NodeSrc& nodes, v3 o, v3 d, float tmin,
-                               float tmax, uint32_t* lds_node, float* lds_t, uint32_t stride,
-                               uint32_t& nv, uint32_t& ns)
+template <int S, bool COUNT>
+VZ_DEV TraceResult closest_hit(const SceneView& view, v3 o, v3 d, float tmin, float tmax, uint32_t* lds_node,
+                               float* lds_t, uint32_t stride, uint32_t& nv, uint32_t& ns)
 {
+    const SceneArrays sc = scene_arrays<true>(view);
     Traversal<S, COUNT> tr;
     Overflow ov;
     if (!tr.init(sc, o, d, tmin, tmax, ns))
-        while (!tr.step(sc, nodes, lds_node, lds_t, stride, ov, nv, ns)) {
+        while (!tr.step(sc, lds_node, lds_t, stride, ov, nv, ns)) {
         }
     return TraceResult{tr.best, tr.bleaf};
 }

@@ -35,7 +35,6 @@ namespace vz {
 constexpr uint32_t kLdsNodes = 256;        // a scene of at most this many 4-wide nodes is staged
 constexpr uint32_t kLdsSpheres = 3 * kLdsNodes + 1;  // leaves of so many 4-wide nodes, at most
 constexpr uint32_t kLdsNodeBytes = 112;
-constexpr uint32_t kLdsPend = 8;           // queued leaf tests per lane
 constexpr uint32_t kLdsKeyMask = 0xFFFF0000u;
 constexpr uint32_t kLdsStack = kWideStackS;  // stack words per lane, the oldest beyond them in private memory
 
@@ -45,7 +44,7 @@ struct LdsScene {
     uint4 nodes[kLdsNodes * kLdsNodeBytes / 16];
     float4 spheres[kLdsSpheres];
     uint32_t stack[kLdsStack * NT];
-    uint16_t pend[kLdsPend * NT];
+    uint16_t pend[kPend * NT];
 };
 
 // Copies the spheres into LDS and decodes the packed nodes (64 bytes,
@@ -153,22 +152,6 @@ struct LdsTraversal {
             }
     }
 
-    // As Traversal::hit_gated.
-    VZ_DEV bool hit_gated(float4 s, float& t) const
-    {
-        if (!hit_sphere(o, d, tmin, best, s, t)) return false;
-        const float r = fabsf(s.w);
-        const float c[3] = {s.x, s.y, s.z}, org[3] = {o.x, o.y, o.z};
-        float lo_t = tmin, hi_t = t;
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-            const float sr = copysignf(r, inv[k]);
-            lo_t = fmaxf(lo_t, ((c[k] - sr) - org[k]) * inv[k]);
-            hi_t = fminf(hi_t, ((c[k] + sr) - org[k]) * inv[k]);
-        }
-        return lo_t <= hi_t * kRobust;
-    }
-
     // Tests the queued leaves; keeps the lexicographic minimum of (t, prim).
     VZ_DEV void flush(const SceneView& sc, const LdsScene<NT>& sh)
     {
@@ -176,18 +159,8 @@ struct LdsTraversal {
             npend--;
             const uint32_t leaf = sh.pend[npend * NT + threadIdx.x];
             float t;
-            if (hit_gated(sh.spheres[leaf], t)) {
-                if (t < best) {
-                    best = t;
-                    bleaf = leaf;
-                } else {  // a tie
-                    best = t;
-                    const uint32_t pid = ldg(sc.leaf_info + leaf) & 0x3FFFFFFFu;
-                    const uint32_t bpid =
-                        bleaf == 0xFFFFFFFFu ? 0xFFFFFFFFu : ldg(sc.leaf_info + bleaf) & 0x3FFFFFFFu;
-                    if (pid < bpid) bleaf = leaf;
-                }
-            }
+            if (hit_gated(o, d, inv, tmin, best, sh.spheres[leaf], t))
+                keep_nearer(t, leaf, sc.leaf_info, best, bleaf);
         }
     }
 
