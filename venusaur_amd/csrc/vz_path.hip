@@ -48,10 +48,10 @@
 namespace vz {
 namespace {
 
-// k_path workgroups, 24 waves per CU either way: three of 8 waves with the
-// nodes in memory; two of 12 with the scene in LDS, so that 160 KB hold it
-// twice and not three times.
-constexpr int kMemBlk = 512;
+// k_path workgroups: with the scene in LDS two of 12 waves per CU, so that
+// 160 KB hold it twice and not three times; with the nodes in memory seven of 4
+// waves (vz_traverse_mem.h).
+constexpr int kMemBlk = kMemThreads;
 constexpr int kLdsBlk = 768;
 constexpr int kStackS = kWideStackS;  // LDS stack slots per lane
 constexpr int kBlk = 256;
@@ -60,12 +60,14 @@ constexpr uint32_t kMaxPathBlocks = 8192;
 // this many of its lanes still trace.  Nodes in LDS, 1080p book frame: 66.2
 // ms at 1, 61.7 at 5, 61.3 at 9, 61.4 at 13, 62.1 at 17, 64.6 at 25.  Many
 // scenes in memory, 24-scene batch: 141 ms at 9, 128 at 17, 121 at 25, 117 at
-// 33, 115 at 41, 119 at 49.
+// 33, 115 at 41, 119 at 49 (64-byte nodes, 24 waves); 93.3 at 33, 93.4 at 41,
+// 93.5 at 49 now, where a million spheres take 143.9, 142.9 and 146.6.
 constexpr uint32_t kRefillLds = 9;
 constexpr uint32_t kRefillGlobal = 41;
 // Queued sphere tests run once two thirds of the tracing lanes hold some:
 // 1080p book frame 61.1 ms against 61.3 at a half, 61.7 at a third and 65.8
-// when tested at once; a million spheres 180.1 against 181.2 and 184.5.
+// when tested at once; a million spheres 142.9 against 144.2 at a half and
+// 143.2 when all of them do.
 constexpr uint32_t kFlushNum = 2, kFlushDen = 3;
 constexpr uint32_t kTile = 64;        // pixels of a camera tile: one wave of camera rays
 // A unit is what a wave claims at a time: up to kUnitPasses passes of one
@@ -208,7 +210,7 @@ struct LaneScene {
 // COUNT: node visits and sphere tests are counted, with the nodes in memory,
 // and tests run at once so that the counts follow each ray alone.
 template <bool COUNT, PathSrc SRC>
-__global__ void __launch_bounds__(path_threads(SRC)) __attribute__((amdgpu_waves_per_eu(6))) k_path(PathGroup G, PathReq one)
+__global__ void __launch_bounds__(path_threads(SRC)) __attribute__((amdgpu_waves_per_eu(SRC == kOneLds || SRC == kManyLds || COUNT ? 6 : kMemWaves))) k_path(PathGroup G, PathReq one)
 {
     constexpr bool LDSN = SRC == kOneLds || SRC == kManyLds, MANY = SRC == kManyLds || SRC == kManyMem;
     static_assert(!(COUNT && LDSN), "node visits are counted with the nodes in memory");
@@ -333,7 +335,7 @@ __global__ void __launch_bounds__(path_threads(SRC)) __attribute__((amdgpu_waves
                 // lanes still tracing, or before a queue could overflow (a
                 // visit queues at most 4)
                 const uint64_t pm = __ballot(tr.npend != 0u);
-                if (pm && (__ballot(tr.npend + 4u > kPend) != 0ull ||
+                if (pm && (__ballot(LDSN ? tr.npend + 4u > kPend : tr.npend == kMemPend) != 0ull ||
                            kFlushDen * (uint32_t)__popcll(pm) >= kFlushNum * (uint32_t)__popcll(busy))) {
                     tr.flush(sc, sh);
                 }

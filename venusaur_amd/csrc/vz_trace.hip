@@ -109,7 +109,7 @@ __global__ void __launch_bounds__(kTraceBlk) k_trace_reduce(const unsigned long 
 // neighbouring rays together: 81 us with packets of 16, 73 us with an equal
 // share of consecutive rays per wave.
 constexpr uint32_t kTraceLdsBlk = 768;
-constexpr uint32_t kTraceMemBlk = 512;
+constexpr uint32_t kTraceMemBlk = kMemThreads;
 constexpr uint32_t kTraceRefill = 32;
 constexpr uint32_t kFlushNum = 2, kFlushDen = 3;  // as in vz_path.hip
 
@@ -118,7 +118,7 @@ struct TraceNoBound {
 };
 
 template <bool LDSN>
-__global__ void __launch_bounds__(LDSN ? kTraceLdsBlk : kTraceMemBlk) __attribute__((amdgpu_waves_per_eu(6)))
+__global__ void __launch_bounds__(LDSN ? kTraceLdsBlk : kTraceMemBlk) __attribute__((amdgpu_waves_per_eu(LDSN ? 6 : kMemWaves)))
 k_trace_hits(SceneView view, const vzRay* __restrict__ rays, uint32_t n, vzHit* __restrict__ hits)
 {
     constexpr uint32_t NT = LDSN ? kTraceLdsBlk : kTraceMemBlk;
@@ -171,7 +171,7 @@ k_trace_hits(SceneView view, const vzRay* __restrict__ rays, uint32_t n, vzHit* 
             }
             busy = __ballot(active && !tdone);
             const uint64_t pm = __ballot(tr.npend != 0u);
-            if (pm && (__ballot(tr.npend + 4u > kPend) != 0ull ||
+            if (pm && (__ballot(LDSN ? tr.npend + 4u > kPend : tr.npend == kMemPend) != 0ull ||
                        kFlushDen * (uint32_t)__popcll(pm) >= kFlushNum * (uint32_t)__popcll(busy))) {
                 tr.flush(sc, sh);
             }
@@ -205,13 +205,13 @@ vzStatus trace_hits(vzContext ctx, const SceneView& sc, const vzRay* rays, uint3
     if (n == 0) return VZ_SUCCESS;
     const bool lds = sc.n >= 2 && sc.nw <= kLdsNodes && sc.n <= kLdsSpheres;
     const uint32_t packets = n / 64u + (n % 64u ? 1u : 0u), cus = ctx->num_cus ? ctx->num_cus : 256;
-    // as many workgroups as are resident at 24 waves a CU; few rays spread
+    // as many workgroups as are resident (24 and 28 waves a CU); few rays spread
     // over the CUs, a packet to a workgroup
     if (lds)
         hipLaunchKernelGGL(k_trace_hits<true>, dim3(std::min(packets, 2u * cus)), dim3(kTraceLdsBlk), 0, st, sc, rays, n,
                            hits);
     else
-        hipLaunchKernelGGL(k_trace_hits<false>, dim3(std::min(packets, 3u * cus)), dim3(kTraceMemBlk), 0, st, sc, rays, n,
+        hipLaunchKernelGGL(k_trace_hits<false>, dim3(std::min(packets, kMemWaves * cus)), dim3(kTraceMemBlk), 0, st, sc, rays, n,
                            hits);
     VZ_HIP_TRY(hipGetLastError());
     return VZ_SUCCESS;

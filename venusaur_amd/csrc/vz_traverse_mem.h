@@ -4,28 +4,43 @@
 //
 // It reads the scene's 48-byte nodes (k_wide_pack, vz_lbvh.hip): three
 // 16-byte loads a visit, one index for all internal children and one for all
-// leaves of a node.  A wave's 64 rays read mostly different nodes, and the L1
-// takes about one line per cycle, so the loads bound a visit as much as the
-// VALU does: with the 64-byte nodes the L1 was busy 77% of the cycles in a
-// frame of a million spheres.  Children hit are put in order by five min/max
-// pairs on their entry distances, whose four lowest bits hold the child's
-// place (cut, so never beyond the distance), with leaf and missed slots above
-// any distance.  A stack entry is (node, distance) in LDS, [slot][lane], the
-// oldest beyond kWideStackS of them in private memory.  Sphere tests are
-// queued and run when many lanes of the wave hold some.
+// leaves of a node.  A wave's 64 rays read mostly different nodes, nearly
+// every visit misses the 32 KB L1, and the L1 takes about one line per cycle:
+// with the 64-byte nodes it was busy 77% of the cycles in a frame of a million
+// spheres, the VALU (two thirds of a visit are conversions, min, max and
+// selects, 4 cycles each) most of the rest.  Children hit are put in order by
+// five min/max pairs on their entry distances, whose four lowest bits hold the
+// child's place (cut, so never beyond the distance), with leaf and missed
+// slots above any distance.  Million spheres at 1080p and 64 samples 181 ->
+// 162 ms.
+//
+// LDS decides the waves that hide the loads' latency: a stack entry is a node
+// and the upper 16 bits of its distance, a queued visit's leaves are one index
+// and a mask of four.  12 entries and 3 visits are 87 bytes a lane, 28 waves
+// on a CU, and hardly an entry goes to private memory: the same frame 162 ms
+// with 8 entries of 8 bytes and 24 waves, 193 with 4, 148 with 14 of 6 bytes
+// and 24 waves, 143 as it is, 146 with 10 and 32 waves (64 registers).
 #pragma once
 #include "vz_traverse.h"
 
 namespace vz {
 
-// LDS of a workgroup of NT threads.
+constexpr uint32_t kMemWaves = 7;       // waves per SIMD
+constexpr uint32_t kMemThreads = 256;   // a wave per SIMD and workgroup, so that any number of them fits evenly
+constexpr uint32_t kMemStack = 12;      // stack entries per lane in LDS, later ones in private memory
+constexpr uint32_t kMemPend = 3;        // queued visits per lane
+
+// LDS of a workgroup of NT threads, [wave][slot][lane].
 template <uint32_t NT>
 struct MemScene {
-    uint2 stack[kWideStackS * NT];
-    uint32_t pend[kPend * NT];
+    uint32_t node[NT / 64][kMemStack][64];
+    uint32_t leaf[NT / 64][kMemPend][64];
+    uint16_t dist[NT / 64][kMemStack][64];
+    uint8_t mask[NT / 64][kMemPend][64];
 };
 
-// Nodes are numbered in units of 16 bytes: 3 times their index.
+// Stack entries beyond those in LDS.  Nodes are numbered in units of 16
+// bytes: 3 times their index.
 struct MemOverflow {
     uint2 e[kWideOverflow];
 };
@@ -40,7 +55,7 @@ struct MemTraversal {
     v3 o, d;
     float inv[3];
     float tmin, best;
-    uint32_t bleaf, node, sp, bottom, npend;
+    uint32_t bleaf, node, sp, npend;
 
     // Returns true when there is nothing to walk: a single sphere, queued.
     template <class Scene>
@@ -51,11 +66,10 @@ struct MemTraversal {
         tmin = tmin_;
         best = tmax_;
         bleaf = kMiss;
-        node = sp = bottom = npend = 0u;
+        node = sp = npend = 0u;
         ray_inverse(d, inv);
         if (sc.node_array() != nullptr) return false;
-        sh.pend[threadIdx.x] = 0u;
-        npend = 1u;
+        queue(sh, 0u, 1u);
         return true;
     }
 
@@ -63,9 +77,16 @@ struct MemTraversal {
     template <class Scene>
     VZ_DEV void flush(const Scene& sc, const MemScene<NT>& sh)
     {
-        while (npend) {
-            npend--;
-            const uint32_t leaf = sh.pend[npend * NT + threadIdx.x];
+        const uint32_t w = threadIdx.x / 64, l = threadIdx.x % 64;
+        uint32_t m = 0u, leaf0 = 0u;
+        while (m | npend) {
+            if (m == 0u) {
+                npend--;
+                m = sh.mask[w][npend][l];
+                leaf0 = sh.leaf[w][npend][l];
+            }
+            const uint32_t leaf = leaf0 + (uint32_t)__builtin_ctz(m);
+            m &= m - 1u;
             float t;
             if (hit_gated(o, d, inv, tmin, best, ldg(sc.sphere_array() + leaf), t))
                 keep_nearer(t, leaf, sc.info_array(), best, bleaf);
@@ -73,8 +94,8 @@ struct MemTraversal {
     }
 
     // One node visit; returns true when the traversal has finished.  Leaf
-    // slots that are hit are queued (at most 4; the caller flushes before
-    // the queue could overflow, and before it reads the hit).
+    // slots that are hit are queued, an entry a visit (the caller flushes
+    // before the queue could overflow, and before it reads the hit).
     template <class Scene>
     VZ_DEV bool step(const Scene& sc, MemScene<NT>& sh, MemOverflow& ov)
     {
@@ -110,7 +131,7 @@ struct MemTraversal {
         }
         const float lim = best * kRobust;
         uint32_t key[4];
-        bool leaf[4];
+        bool hit[4];
 #pragma unroll
         for (uint32_t c = 0; c < 4; c++) {
             float n3[3], f3[3];
@@ -121,17 +142,16 @@ struct MemTraversal {
             }
             const float lo_t = fmaxf(fmaxf(fmaxf(tmin, n3[0]), n3[1]), n3[2]);
             const float hi_t = fminf(fminf(fminf(lim, f3[0]), f3[1]), f3[2]);
-            const bool hit = lo_t <= hi_t, in = c < n_in;
-            leaf[c] = hit && !in;
-            key[c] = hit && in ? (__float_as_uint(ANYT ? fmaxf(lo_t, 0.0f) : lo_t) & ~15u) | 3u * c : kMiss;
+            hit[c] = lo_t <= hi_t;
+            const uint32_t e = (__float_as_uint(ANYT ? fmaxf(lo_t, 0.0f) : lo_t) & ~15u) | 3u * c;
+            key[c] = hit[c] && c < n_in ? e : kMiss;
         }
-        const uint32_t leaf0 = C.w - n_in;
-#pragma unroll
-        for (uint32_t c = 0; c < 4; c++)
-            if (leaf[c]) {
-                sh.pend[npend * NT + threadIdx.x] = leaf0 + c;
-                npend++;
-            }
+        uint32_t leaves = hit[3] ? 1u : 0u;
+        leaves = leaves + leaves + (hit[2] ? 1u : 0u);  // an add with carry each
+        leaves = leaves + leaves + (hit[1] ? 1u : 0u);
+        leaves = leaves + leaves + (hit[0] ? 1u : 0u);
+        leaves >>= n_in;  // internal children come first
+        if (leaves) queue(sh, C.w, leaves);
         // ascending by five compare-exchanges
         auto order = [](uint32_t& x, uint32_t& y) {
             const uint32_t lo = min(x, y), hi = max(x, y);
@@ -145,17 +165,25 @@ struct MemTraversal {
         order(key[1], key[2]);
         if (key[0] != kMiss) {
             if (key[1] != kMiss) {
-                // room in LDS for three: the oldest go to the overflow (never
-                // more than it holds: kMaxWideDepth)
-                while (sp + 3u - bottom > kWideStackS) {
-                    if (bottom < kWideOverflow) ov.e[bottom] = sh.stack[(bottom % kWideStackS) * NT + threadIdx.x];
-                    bottom++;
+                if (sp <= (kMemStack - 3u) * kRow) {  // room in LDS for three
+                    if (key[2] != kMiss) {
+                        if (key[3] != kMiss) push(sh, C.z, key[3]);
+                        push(sh, C.z, key[2]);
+                    }
+                    push(sh, C.z, key[1]);
+                } else {
+                    for (int c = 3; c >= 1; c--)
+                        if (key[c] != kMiss) {
+                            if (sp < kMemStack * kRow) {
+                                push(sh, C.z, key[c]);
+                            } else {
+                                // never more than it holds (kMaxWideDepth)
+                                const uint32_t i = sp / kRow - kMemStack;
+                                if (i < kWideOverflow) ov.e[i] = make_uint2(C.z + (key[c] & 15u), key[c] & ~15u);
+                                sp += kRow;
+                            }
+                        }
                 }
-                if (key[2] != kMiss) {
-                    if (key[3] != kMiss) push(sh, C.z, key[3]);
-                    push(sh, C.z, key[2]);
-                }
-                push(sh, C.z, key[1]);
             }
             node = C.z + (key[0] & 15u);
             return false;
@@ -163,24 +191,44 @@ struct MemTraversal {
         // the nearest stacked child that can still hold a closer hit
         for (;;) {
             if (sp == 0u) return true;
-            sp--;
-            uint2 e;
-            if (sp < bottom) {
-                e = ov.e[sp < kWideOverflow ? sp : kWideOverflow - 1u];
-                bottom = sp;
+            sp -= kRow;
+            float t;
+            if (sp < kMemStack * kRow) {
+                node = *node_at(sh, sp);
+                t = __uint_as_float((uint32_t)*dist_at(sh, sp) << 16);
             } else {
-                e = sh.stack[(sp % kWideStackS) * NT + threadIdx.x];
+                const uint32_t i = min(sp / kRow - kMemStack, kWideOverflow - 1u);
+                node = ov.e[i].x;
+                t = __uint_as_float(ov.e[i].y);
             }
-            node = e.x;
-            if (__uint_as_float(e.y) <= (ANYT ? fmaxf(lim, 0.0f) : lim)) return false;
+            if (t <= (ANYT ? fmaxf(lim, 0.0f) : lim)) return false;
         }
     }
 
 private:
+    // sp counts bytes of a row of distances (a wave's, 2 bytes a lane)
+    static constexpr uint32_t kRow = 128;
+    static VZ_DEV uint32_t* node_at(MemScene<NT>& sh, uint32_t at)
+    {
+        return reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(&sh.node[threadIdx.x / 64][0][threadIdx.x % 64]) +
+                                           2u * at);
+    }
+    static VZ_DEV uint16_t* dist_at(MemScene<NT>& sh, uint32_t at)
+    {
+        return reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(&sh.dist[threadIdx.x / 64][0][threadIdx.x % 64]) +
+                                           at);
+    }
     VZ_DEV void push(MemScene<NT>& sh, uint32_t base, uint32_t key)
     {
-        sh.stack[(sp % kWideStackS) * NT + threadIdx.x] = make_uint2(base + (key & 15u), key & ~15u);
-        sp++;
+        *node_at(sh, sp) = base + (key & 15u);
+        *dist_at(sh, sp) = (uint16_t)(key >> 16);
+        sp += kRow;
+    }
+    VZ_DEV void queue(MemScene<NT>& sh, uint32_t leaf0, uint32_t m)
+    {
+        sh.leaf[threadIdx.x / 64][npend][threadIdx.x % 64] = leaf0;
+        sh.mask[threadIdx.x / 64][npend][threadIdx.x % 64] = (uint8_t)m;
+        npend++;
     }
 };
 
