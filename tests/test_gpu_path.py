@@ -113,3 +113,37 @@ def test_trace_without_stats(ctx, book, kind, n):
     sc.trace(rb.value, n, h.value, stats=True)
     assert hits[0].tobytes() == hits[1].tobytes() == h.download(api.HIT_DT).tobytes()
     sc.close()
+
+
+# scenes in memory whose rays enter nearly every box: more stacked children
+# than the LDS entries of a lane, full leaf queues, ties between copies of a
+# sphere; then refitted to other places
+@pytest.mark.parametrize("n", [770, 1000, 3001, 20000])
+@pytest.mark.parametrize("copies", [1, 3])
+def test_trace_overlapping_boxes(ctx, n, copies):
+    say(f"case: hits among overlapping boxes n={n} copies={copies}")
+    rng = np.random.default_rng([n, copies])
+    s, m = api.box_scene(n - 1, 5)
+    s, m = s.copy(), m.copy()
+    for f in ("cx", "cy", "cz"):
+        s[f] = np.tile(rng.normal(0, 0.5, n // copies + 1), copies)[:n].astype(np.float32)
+    s["r"] = np.tile(rng.uniform(1.0, 4.0, n // copies + 1), copies)[:n].astype(np.float32)
+    rays = np.zeros(4000, api.RAY_DT)
+    for f in ("ox", "oy", "oz"):
+        rays[f] = rng.uniform(-6, 6, len(rays))
+        rays["d" + f[1]] = rng.normal(0, 1, len(rays))
+    rays["tmin"], rays["tmax"] = 0.001, 1e16
+    rays["tmin"][::7] = -20.0
+    sc = api.Scene(ctx, s, m)
+    rb = DeviceBuffer.from_array(rays)
+    for moved in (False, True):
+        if moved:
+            s["cx"] += rng.normal(0, 2.0, n).astype(np.float32)
+            sc.update_spheres(s)
+        out = []
+        for stats in (False, True):
+            h = DeviceBuffer(len(rays) * 8)
+            sc.trace(rb.value, len(rays), h.value, stats=stats)
+            out.append(h.download(api.HIT_DT))
+        assert out[0].tobytes() == out[1].tobytes() == O.trace_brute(s, rays).tobytes(), moved
+    sc.close()
