@@ -147,3 +147,48 @@ def test_trace_overlapping_boxes(ctx, n, copies):
             out.append(h.download(api.HIT_DT))
         assert out[0].tobytes() == out[1].tobytes() == O.trace_brute(s, rays).tobytes(), moved
     sc.close()
+
+
+# a tree whose wide levels go on far below its wide ones: beside a box of
+# spheres, ever smaller cells of the Morton grid with one sphere each and a
+# crowd in the last one
+@pytest.mark.parametrize("n", [6000, 30000, 140000])
+def test_uneven_tree(ctx, n):
+    say(f"case: uneven tree n={n}")
+    s, m = api.box_scene(n, 3)
+    s, m = s[1:].copy(), m[1:].copy()
+    lo = np.array([s[f].min() for f in ("cx", "cy", "cz")])
+    ext = float(max(s[f].max() - s[f].min() for f in ("cx", "cy", "cz")))
+    chain = [lo + ext * 2.0 ** -k * np.eye(3)[a] for k in range(1, 11) for a in range(3)]
+    crowd = lo + np.random.default_rng(n).uniform(0, ext / 2048, (min(n // 3, 4000), 3))
+    extra = np.concatenate([chain, crowd])
+    keep = np.ones(len(s), bool)  # the box leaves the chain's octant: nothing else there
+    for a, f in enumerate(("cx", "cy", "cz")):
+        keep &= s[f] < lo[a] + ext * 0.45
+    s, m = s[~keep], m[~keep]
+    t = np.zeros(len(extra), s.dtype)
+    for a, f in enumerate(("cx", "cy", "cz")):
+        t[f] = extra[:, a]
+    t["r"] = ext * 1e-5
+    s = np.concatenate([s, t])
+    m = np.concatenate([m, np.resize(m, len(t))])
+    sc = api.Scene(ctx, s, m)
+    ob = O.BVH(s)
+    assert sc.info().num_prims > 2048 and sc.info().wide_depth == ob.wide_depth()
+    say(f"wide depth {ob.wide_depth()}")
+    assert sc.download_wide().tobytes() == ob.wide_nodes().tobytes()
+    rng = np.random.default_rng([n, 1])
+    rays = np.zeros(3000, api.RAY_DT)
+    pick = s[rng.integers(0, len(s), len(rays))]
+    for f, c in (("ox", "cx"), ("oy", "cy"), ("oz", "cz")):
+        rays[f] = rng.uniform(lo.min() - ext, lo.min() + 2 * ext, len(rays))
+        rays["d" + f[1]] = pick[c] - rays[f]
+    rays["tmin"], rays["tmax"] = 0.001, 1e16
+    rb = DeviceBuffer.from_array(rays)
+    out = []
+    for stats in (False, True):
+        h = DeviceBuffer(len(rays) * 8)
+        sc.trace(rb.value, len(rays), h.value, stats=stats)
+        out.append(h.download(api.HIT_DT))
+    assert out[0].tobytes() == out[1].tobytes() == O.trace_brute(s, rays).tobytes()
+    sc.close()

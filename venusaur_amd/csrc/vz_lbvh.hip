@@ -72,10 +72,26 @@ __global__ void __launch_bounds__(kBlk) k_bounds_partial(const float4* __restric
     if (threadIdx.x < 6) partial[blockIdx.x * 6 + threadIdx.x] = s[threadIdx.x][0];
 }
 
-// out: lo[3], hi[3], scale[3] with scale = ext > 0 ? 1024/ext : 0 (iso: one
+// A grid: lo[3], hi[3], scale[3] with scale = ext > 0 ? 1024/ext : 0 (iso: one
 // scale 1024/max ext for every axis), and the large-sphere threshold
-// out[9] = max extent / 4; an axis that no sphere reached gets lo = hi = 0.  min and max are exact, so the reduction order
-// does not change the result.
+// out[9] = max extent / 4; an axis that no sphere reached gets lo = hi = 0.
+// min and max are exact, so the reduction order does not change the result.
+__device__ __forceinline__ void write_grid(const float (&lo)[3], const float (&hi)[3], uint32_t iso, float* out)
+{
+    float extmax = 0.0f;
+    for (int k = 0; k < 3; k++) {
+        float l = lo[k], h = hi[k];
+        if (l > h) l = h = 0.0f;
+        const float ext = h - l;
+        out[k] = l;
+        out[3 + k] = h;
+        out[6 + k] = ext > 0.0f ? 1024.0f / ext : 0.0f;
+        extmax = fmaxf(extmax, ext);
+    }
+    if (iso)  // one scale for every axis: cubic Morton cells
+        for (int k = 0; k < 3; k++) out[6 + k] = extmax > 0.0f ? 1024.0f / extmax : 0.0f;
+    out[9] = 0.25f * extmax;
+}
 __global__ void __launch_bounds__(kBlk) k_bounds_final(const float* __restrict__ partial, uint32_t nb,
                                                        uint32_t iso, float* __restrict__ out)
 {
@@ -97,19 +113,8 @@ __global__ void __launch_bounds__(kBlk) k_bounds_final(const float* __restrict__
         __syncthreads();
     }
     if (threadIdx.x == 0) {
-        float extmax = 0.0f;
-        for (int k = 0; k < 3; k++) {
-            float l = s[k][0], h = s[3 + k][0];
-            if (l > h) l = h = 0.0f;
-            const float ext = h - l;
-            out[k] = l;
-            out[3 + k] = h;
-            out[6 + k] = ext > 0.0f ? 1024.0f / ext : 0.0f;
-            extmax = fmaxf(extmax, ext);
-        }
-        if (iso)  // one scale for every axis: cubic Morton cells
-            for (int k = 0; k < 3; k++) out[6 + k] = extmax > 0.0f ? 1024.0f / extmax : 0.0f;
-        out[9] = 0.25f * extmax;
+        for (int k = 0; k < 3; k++) { lo[k] = s[k][0]; hi[k] = s[3 + k][0]; }
+        write_grid(lo, hi, iso, out);
     }
 }
 
@@ -131,14 +136,8 @@ __device__ __forceinline__ uint32_t expand10(uint32_t v)
 // Morton code on grid B: the centroids of the small spheres only, with cubic
 // cells, so a thin slab of spheres is not split along its thin axis as often
 // as along the others.
-__global__ void __launch_bounds__(kBlk) k_morton(const float4* __restrict__ sph, uint32_t n,
-                                                 const float* __restrict__ grid_a,
-                                                 const float* __restrict__ grid_b,
-                                                 uint32_t* __restrict__ keys, uint32_t* __restrict__ vals)
+__device__ __forceinline__ uint32_t morton_key(const float4 c, const float* grid_a, const float* grid_b)
 {
-    uint32_t i = blockIdx.x * kBlk + threadIdx.x;
-    if (i >= n) return;
-    float4 c = sph[i];
     const bool large = 2.0f * fabsf(c.w) > grid_a[9];
     const float* bnd = large ? grid_a : grid_b;
     float cc[3] = {c.x, c.y, c.z};
@@ -149,7 +148,16 @@ __global__ void __launch_bounds__(kBlk) k_morton(const float4* __restrict__ sph,
         qi = qi < 0 ? 0 : (qi > 1023 ? 1023 : qi);
         q[k] = (uint32_t)qi;
     }
-    keys[i] = (expand10(q[0]) << 2) | (expand10(q[1]) << 1) | expand10(q[2]) | (large ? kLargeKey : 0u);
+    return (expand10(q[0]) << 2) | (expand10(q[1]) << 1) | expand10(q[2]) | (large ? kLargeKey : 0u);
+}
+__global__ void __launch_bounds__(kBlk) k_morton(const float4* __restrict__ sph, uint32_t n,
+                                                 const float* __restrict__ grid_a,
+                                                 const float* __restrict__ grid_b,
+                                                 uint32_t* __restrict__ keys, uint32_t* __restrict__ vals)
+{
+    uint32_t i = blockIdx.x * kBlk + threadIdx.x;
+    if (i >= n) return;
+    keys[i] = morton_key(sph[i], grid_a, grid_b);
     vals[i] = i;
 }
 
@@ -494,6 +502,48 @@ __device__ __forceinline__ void wave_order()
 {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
+}
+
+// Stages 1 and 2 of a small scene, one workgroup, a thread per sphere: five
+// launches in one.
+constexpr uint32_t kSmallThreads = 1024;
+static_assert(kSahMaxPrims <= kSmallThreads, "a thread per sphere");
+__global__ void __launch_bounds__(kSmallThreads) k_small_keys(const float4* __restrict__ sph, uint32_t n,
+                                                              uint32_t* __restrict__ keys, uint32_t* __restrict__ vals)
+{
+    __shared__ float part[6][kSmallThreads / 64];
+    __shared__ float grid[2][10];
+    const uint32_t t = threadIdx.x, w = t / 64;
+    const float4 c = t < n ? sph[t] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (uint32_t g = 0; g < 2u; g++) {  // grid A: every centroid; grid B: those of the small spheres
+        const bool in = t < n && (g == 0u || !(2.0f * fabsf(c.w) > grid[0][9]));
+        const float cc[3] = {c.x, c.y, c.z};
+        for (int k = 0; k < 3; k++) {
+            const float lo = wave_reduce<true>(in ? cc[k] : 3.4e38f), hi = wave_reduce<false>(in ? cc[k] : -3.4e38f);
+            if (t % 64 == 0u) {
+                part[k][w] = lo;
+                part[3 + k][w] = hi;
+            }
+        }
+        __syncthreads();
+        if (t == 0u) {
+            float lo[3], hi[3];
+            for (int k = 0; k < 3; k++) {
+                lo[k] = part[k][0];
+                hi[k] = part[3 + k][0];
+                for (uint32_t i = 1; i < kSmallThreads / 64; i++) {
+                    lo[k] = fminf(lo[k], part[k][i]);
+                    hi[k] = fmaxf(hi[k], part[3 + k][i]);
+                }
+            }
+            write_grid(lo, hi, g, grid[g]);
+        }
+        __syncthreads();
+    }
+    if (t < n) {
+        keys[t] = morton_key(c, grid[0], grid[1]);
+        vals[t] = t;
+    }
 }
 
 // LDS of one treelet build by NW waves: the range's spheres by local index
@@ -1063,7 +1113,13 @@ __global__ void __launch_bounds__(kRefitThreads) k_refit_top(const float4* __res
 // 24-27) and valid flags (28-31).
 constexpr uint32_t kWideRoot = 0x80000000u;  // wide-root flag of a binary node
 constexpr uint32_t kLeafRef = 0x80000000u;   // a wide child that is a leaf
-constexpr uint32_t kLeafCount = kMaxDepth + 2;  // word of the level counts: leaves given a place so far
+// Words behind the roots per level [0, kMaxDepth].
+constexpr uint32_t kWideCount = kMaxDepth + 1;   // wide nodes
+constexpr uint32_t kLeafCount = kMaxDepth + 2;   // leaves given a place so far
+constexpr uint32_t kWideError = kMaxDepth + 3;   // the structural check's result
+constexpr uint32_t kTreeHeight = kMaxDepth + 4;  // of the binary tree
+constexpr uint32_t kFirstLevel = kMaxDepth + 5;  // first level that k_wide_few left
+constexpr uint32_t kWideWords = kMaxDepth + 6;
 constexpr uint32_t kScanItems = 4;            // root flags per thread in the index scan
 constexpr uint32_t kScanTile = kBlk * kScanItems;
 
@@ -1077,17 +1133,6 @@ __device__ __forceinline__ uint32_t child_ref(uint32_t cw, int c)
 {
     const uint32_t g = (cw & 0x3FFFFFFFu) + (uint32_t)c;
     return ((cw >> (30 + c)) & 1u) ? (g | kLeafRef) : g;
-}
-
-__global__ void __launch_bounds__(kBlk) k_wide_init(uint32_t* __restrict__ wflag, uint32_t* __restrict__ front,
-                                                    uint32_t* __restrict__ cnt, uint32_t ncnt)
-{
-    const uint32_t t = threadIdx.x;
-    for (uint32_t i = t; i < ncnt; i += kBlk) cnt[i] = i == 0u ? 1u : 0u;
-    if (t == 0) {
-        wflag[0] = kWideRoot;
-        front[0] = 0u;
-    }
 }
 
 // The children of wide root r: starts as its binary node's two, and opens the
@@ -1144,30 +1189,34 @@ __device__ __forceinline__ uint32_t wide_children(uint32_t r, const uint32_t* __
     return n_k;
 }
 
+struct LevelArrays {
+    const uint32_t* child;
+    const float* boxes;
+    uint32_t* front[2];   // roots of the even levels, of the odd ones
+    uint32_t *wkids, *wflag;
+    uint32_t *tidx, *tchild, *tleaf;  // of a root: its place in level order, its first child's, its first leaf's
+};
+
 // One level: every wide root of the frontier picks its children; internal
-// children are the next level's frontier.  cnt[level + 1] starts at zero and
-// is added to once per wave (once per child, and a maximum per root for the
-// depth, kept one address busy: 414 us for the levels of a million spheres).
-__global__ void __launch_bounds__(kBlk) k_wide_level(const uint32_t* __restrict__ child,
-                                                     const float* __restrict__ boxes,
-                                                     const uint32_t* __restrict__ front_in,
-                                                     uint32_t* __restrict__ front_out, uint32_t* __restrict__ cnt,
-                                                     uint32_t level, uint32_t* __restrict__ wkids,
-                                                     uint32_t* __restrict__ wflag, uint32_t* __restrict__ tidx,
-                                                     uint32_t* __restrict__ tchild, uint32_t* __restrict__ tleaf)
+// children are the next level's frontier.  alloc(in, leaves, at, leaf_at),
+// called by the last lane of a wave, gives the wave's children and leaves
+// their places (once per child, and a maximum per root for the depth, kept one
+// address busy: 414 us for the levels of a million spheres).
+template <class Alloc>
+__device__ __forceinline__ void wide_roots(const LevelArrays& A, uint32_t level, uint32_t count, uint32_t before,
+                                           uint32_t first, uint32_t stride, Alloc alloc)
 {
-    const uint32_t count = cnt[level], lane = lane_id();
-    // roots of the levels above: the first of this level in level order
-    uint32_t before = lane < level ? cnt[lane] : 0u;
-    for (int o = 32; o >= 1; o >>= 1) before += __shfl_xor(before, o);
-    for (uint32_t i0 = (blockIdx.x * kBlk + threadIdx.x) & ~63u; i0 < count; i0 += gridDim.x * kBlk) {
+    const uint32_t lane = lane_id();
+    const uint32_t* front_in = A.front[level & 1u];
+    uint32_t* front_out = A.front[(level & 1u) ^ 1u];
+    for (uint32_t i0 = first & ~63u; i0 < count; i0 += stride) {
         const uint32_t i = i0 + lane;
         uint32_t ks[4] = {0u, 0u, 0u, 0u}, n_k = 0, n_in = 0, r = 0;
         if (i < count) {
             r = front_in[i];
-            n_k = wide_children(r, child, boxes, ks);
-            reinterpret_cast<uint4*>(wkids)[r] = make_uint4(ks[0], ks[1], ks[2], ks[3]);
-            wflag[r] = kWideRoot | n_k;
+            n_k = wide_children(r, A.child, A.boxes, ks);
+            reinterpret_cast<uint4*>(A.wkids)[r] = make_uint4(ks[0], ks[1], ks[2], ks[3]);
+            A.wflag[r] = kWideRoot | n_k;
             for (uint32_t k = 0; k < 4u; k++) n_in += k < n_k && !(ks[k] & kLeafRef) ? 1u : 0u;
         }
         const uint32_t n_leaf = n_k - n_in;
@@ -1180,23 +1229,111 @@ __global__ void __launch_bounds__(kBlk) k_wide_level(const uint32_t* __restrict_
             }
         }
         uint32_t base = 0, lbase = 0;
-        if (lane == 63u) {
-            if (incl) base = atomicAdd(&cnt[level + 1], incl);
-            if (lincl) lbase = atomicAdd(&cnt[kLeafCount], lincl);
-        }
+        if (lane == 63u) alloc(incl, lincl, base, lbase);
         uint32_t at = __shfl(base, 63) + incl - n_in;
         const uint32_t lat = __shfl(lbase, 63) + lincl - n_leaf;
-        if (i < count) {  // the root's place in level order, its children's, its leaves'
-            tidx[r] = before + i;
-            tchild[r] = before + count + at;
-            tleaf[r] = lat;
+        if (i < count) {
+            A.tidx[r] = before + i;
+            A.tchild[r] = before + count + at;
+            A.tleaf[r] = lat;
         }
         for (uint32_t k = 0; k < 4u; k++) {
             if (k >= n_k || (ks[k] & kLeafRef)) continue;
-            wflag[ks[k]] = kWideRoot;
+            A.wflag[ks[k]] = kWideRoot;
             front_out[at++] = ks[k];
         }
     }
+}
+
+// Levels by one workgroup, while they have at most `limit` roots.
+constexpr uint32_t kFewThreads = 1024;
+struct FewShared {
+    uint32_t next[3];  // roots of the next level; three by turns, so that one barrier a level is enough
+    uint32_t leaves;
+};
+__device__ __forceinline__ void few_levels(const LevelArrays& A, uint32_t* cnt, uint32_t& level, uint32_t& count,
+                                           uint32_t before, uint32_t limit, FewShared& sh)
+{
+    uint32_t turn = 0;
+    while (count != 0u && count <= limit && level < kMaxDepth) {
+        uint32_t* next = &sh.next[turn];
+        turn = turn == 2u ? 0u : turn + 1u;
+        if (threadIdx.x == 0u) sh.next[turn] = 0u;
+        wide_roots(A, level, count, before, threadIdx.x, kFewThreads,
+                   [&](uint32_t in, uint32_t leaves, uint32_t& at, uint32_t& leaf_at) {
+                       if (in) at = atomicAdd(next, in);
+                       if (leaves) leaf_at = atomicAdd(&sh.leaves, leaves);
+                   });
+        __syncthreads();
+        before += count;
+        count = *next;
+        level++;
+        if (threadIdx.x == 0u) cnt[level] = count;
+    }
+}
+
+// Clears the level words and sets up level 0: the root, unless the tree is
+// deeper than the host will take.
+__device__ __forceinline__ uint32_t first_level(const LevelArrays& A, uint32_t* cnt, const uint32_t* height,
+                                                FewShared& sh)
+{
+    const uint32_t t = threadIdx.x, h = height[0], count = h + 1u <= kMaxDepth ? 1u : 0u;
+    if (t < kWideWords) cnt[t] = t == 0u ? count : (t == kTreeHeight ? h : 0u);
+    if (t == 0u) {
+        A.wflag[0] = kWideRoot;
+        A.front[0][0] = 0u;
+        sh.next[0] = 0u;
+        sh.leaves = 0u;
+    }
+    __syncthreads();
+    return count;
+}
+
+// The levels of a larger scene.  One workgroup takes those at the top, which
+// have few roots; the next `mids` levels have a launch each; whatever is left
+// below, one workgroup again.  A launch for every level that the binary depth
+// allows for, most of them empty, cost 4 us each: 22 of them at 200k spheres,
+// 25 at a million.  With kFewRoots at a workgroup's size the top levels
+// take some 4 us each, no longer than a launch.
+constexpr uint32_t kFewRoots = 2048;
+__global__ void __launch_bounds__(kFewThreads) k_wide_few(LevelArrays A, uint32_t* cnt, const uint32_t* height,
+                                                          uint32_t resume, uint32_t mids)
+{
+    __shared__ FewShared sh;
+    uint32_t level = 0, count, before = 0;
+    if (!resume) {
+        count = first_level(A, cnt, height, sh);
+        few_levels(A, cnt, level, count, 0u, kFewRoots, sh);
+        if (threadIdx.x == 0u) {
+            cnt[kFirstLevel] = level;
+            cnt[kLeafCount] = sh.leaves;
+        }
+        return;
+    }
+    level = cnt[kFirstLevel] + mids;
+    if (level >= kMaxDepth) return;
+    count = cnt[level];
+    for (uint32_t l = 0; l < level; l++) before += cnt[l];
+    if (threadIdx.x == 0u) {
+        sh.next[0] = 0u;
+        sh.leaves = cnt[kLeafCount];
+    }
+    __syncthreads();
+    few_levels(A, cnt, level, count, before, 0xFFFFFFFFu, sh);
+}
+__global__ void __launch_bounds__(kBlk) k_wide_level(LevelArrays A, uint32_t* __restrict__ cnt, uint32_t mid)
+{
+    const uint32_t level = cnt[kFirstLevel] + mid, lane = lane_id();
+    if (level >= kMaxDepth) return;
+    const uint32_t count = cnt[level];
+    // roots of the levels above: the first of this level in level order
+    uint32_t before = lane < level ? cnt[lane] : 0u;
+    for (int o = 32; o >= 1; o >>= 1) before += __shfl_xor(before, o);
+    wide_roots(A, level, count, before, blockIdx.x * kBlk + threadIdx.x, gridDim.x * kBlk,
+               [&](uint32_t in, uint32_t leaves, uint32_t& at, uint32_t& leaf_at) {
+                   if (in) at = atomicAdd(&cnt[level + 1], in);
+                   if (leaves) leaf_at = atomicAdd(&cnt[kLeafCount], leaves);
+               });
 }
 
 // Wide indices: an exclusive scan of the root flags over the binary nodes,
@@ -1277,14 +1414,9 @@ struct TravOut {
     float4* tmat;
 };
 
-__global__ void __launch_bounds__(kBlk) k_wide_pack(const float4* __restrict__ sph, const uint32_t* __restrict__ wkids,
-                                                    const uint32_t* __restrict__ wflag,
-                                                    const uint32_t* __restrict__ widx,
-                                                    const float* __restrict__ boxes, uint32_t ni,
-                                                    uint4* __restrict__ wnodes, TravOut T)
+__device__ __forceinline__ void wide_pack(uint32_t r, const float4* sph, const uint32_t* wkids, const uint32_t* wflag,
+                                          const uint32_t* widx, const float* boxes, uint4* wnodes, const TravOut& T)
 {
-    const uint32_t r = blockIdx.x * kBlk + threadIdx.x;
-    if (r >= ni) return;
     const uint32_t fl = wflag[r];
     if (!(fl & kWideRoot)) return;
     const uint32_t cnt = fl & 7u;
@@ -1347,11 +1479,27 @@ __global__ void __launch_bounds__(kBlk) k_wide_pack(const float4* __restrict__ s
             T.tmat[T.n + k] = T.mat[0];
         }
 }
+__global__ void __launch_bounds__(kBlk) k_wide_pack(const float4* __restrict__ sph, const uint32_t* __restrict__ wkids,
+                                                    const uint32_t* __restrict__ wflag,
+                                                    const uint32_t* __restrict__ widx,
+                                                    const float* __restrict__ boxes, uint32_t ni,
+                                                    uint4* __restrict__ wnodes, TravOut T)
+{
+    const uint32_t r = blockIdx.x * kBlk + threadIdx.x;
+    if (r < ni) wide_pack(r, sph, wkids, wflag, widx, boxes, wnodes, T);
+}
 
 __global__ void k_zero(uint32_t* a, uint32_t n)
 {
     uint32_t i = blockIdx.x * kBlk + threadIdx.x;
     if (i < n) a[i] = 0u;
+}
+__global__ void k_zero3(uint32_t* a, uint32_t na, uint32_t* b, uint32_t nb, uint32_t* c, uint32_t nc)
+{
+    uint32_t i = blockIdx.x * kBlk + threadIdx.x;
+    if (i < na) a[i] = 0u;
+    if (i < nb) b[i] = 0u;
+    if (i < nc) c[i] = 0u;
 }
 
 __global__ void k_fill(uint32_t* a, uint32_t n, uint32_t v)
@@ -1476,7 +1624,7 @@ vzStatus lbvh_alloc(vzScene s)
     part(&s->d_widx, sizeof(uint32_t) * (ni + blocks_for(ni, kScanTile) + 1));  // + tile sums
     part(&s->d_wfront[0], sizeof(uint32_t) * ni);
     part(&s->d_wfront[1], sizeof(uint32_t) * ni);
-    part(&s->d_wcnt, sizeof(uint32_t) * (kMaxDepth + 8));
+    part(&s->d_wcnt, sizeof(uint32_t) * kWideWords);
     s->arena = s->ctx->scene_blocks.take(at, &s->arena_bytes);
     if (!s->arena) return set_error(VZ_ERROR_OUT_OF_MEMORY, "hipMalloc of scene buffers failed");
     for (const Part& q : parts) *q.p = (char*)s->arena + q.at;
@@ -1497,6 +1645,48 @@ void lbvh_free(vzScene s)
 // most once and ends.  References count 1 from a 64-byte node and kTravRef
 // from a 48-byte one.  Any violation sets *err.
 constexpr uint32_t kTravRef = 0x10000u;
+__device__ __forceinline__ void wide_refs(uint32_t i, const uint4* wnodes, uint32_t nw, uint32_t n, uint32_t* wref,
+                                          uint32_t* lref, uint32_t* err)
+{
+    const uint4 a = wnodes[4 * (size_t)i], c = wnodes[4 * (size_t)i + 2], d = wnodes[4 * (size_t)i + 3];
+    const uint32_t valid = a.w >> 28, leafm = (a.w >> 24) & 0xFu;
+    const uint32_t ch[4] = {c.z, c.w, d.x, d.y};
+    for (int k = 0; k < 4; k++) {
+        if (!((valid >> k) & 1u)) continue;
+        if ((leafm >> k) & 1u) {
+            if (ch[k] < n) atomicAdd(&lref[ch[k]], 1u);
+            else *err = 1u;
+        } else {
+            if (ch[k] != 0u && ch[k] < nw) atomicAdd(&wref[ch[k]], 1u);
+            else *err = 1u;
+        }
+    }
+}
+// r: a binary node, fl its wide-root flag word.
+__device__ __forceinline__ void trav_refs(uint32_t r, uint32_t fl, const uint4* tnodes, const uint32_t* tidx,
+                                          uint32_t nw, uint32_t n, uint32_t* tref, uint32_t* lref, uint32_t* err)
+{
+    if (!(fl & kWideRoot)) return;
+    const uint32_t t = tidx[r];
+    if (t >= nw) {
+        *err = 1u;
+        return;
+    }
+    const uint32_t meta = tnodes[3 * (size_t)t].w, first3 = tnodes[3 * (size_t)t + 2].z, first = first3 / 3u;
+    const uint32_t leaf = tnodes[3 * (size_t)t + 2].w, n_in = meta >> 24, n_leaf = (fl & 7u) - n_in;
+    if (n_in > 4u || n_leaf > 4u || leaf > n || n_leaf > n - leaf || (n_in && first == 0u) ||
+        (n_in && first3 != 3u * first) || (n_in && first > nw) || (n_in && n_in > nw - first)) {
+        *err = 1u;
+        return;
+    }
+    for (uint32_t k = 0; k < n_in; k++) atomicAdd(&tref[first + k], 1u);
+    for (uint32_t k = 0; k < n_leaf; k++) atomicAdd(&lref[leaf + k], kTravRef);
+}
+__device__ __forceinline__ bool refs_wrong(uint32_t i, uint32_t nw, const uint32_t* wref, const uint32_t* tref,
+                                           const uint32_t* lref)
+{
+    return lref[i] != 1u + kTravRef || (i < nw && (wref[i] != (i == 0u ? 0u : 1u) || tref[i] != wref[i]));
+}
 __global__ void __launch_bounds__(kBlk) k_wide_refs(const uint4* __restrict__ wnodes, const uint4* __restrict__ tnodes,
                                                     const uint32_t* __restrict__ wflag,
                                                     const uint32_t* __restrict__ tidx, uint32_t ni,
@@ -1505,100 +1695,119 @@ __global__ void __launch_bounds__(kBlk) k_wide_refs(const uint4* __restrict__ wn
                                                     uint32_t* __restrict__ lref, uint32_t* __restrict__ err)
 {
     const uint32_t nw = *nwp;
-    for (uint32_t i = blockIdx.x * kBlk + threadIdx.x; i < nw; i += gridDim.x * kBlk) {
-        const uint4 a = wnodes[4 * (size_t)i], c = wnodes[4 * (size_t)i + 2], d = wnodes[4 * (size_t)i + 3];
-        const uint32_t valid = a.w >> 28, leafm = (a.w >> 24) & 0xFu;
-        const uint32_t ch[4] = {c.z, c.w, d.x, d.y};
-        for (int k = 0; k < 4; k++) {
-            if (!((valid >> k) & 1u)) continue;
-            if ((leafm >> k) & 1u) {
-                if (ch[k] < n) atomicAdd(&lref[ch[k]], 1u);
-                else *err = 1u;
-            } else {
-                if (ch[k] != 0u && ch[k] < nw) atomicAdd(&wref[ch[k]], 1u);
-                else *err = 1u;
-            }
-        }
-    }
-    for (uint32_t r = blockIdx.x * kBlk + threadIdx.x; r < ni; r += gridDim.x * kBlk) {
-        const uint32_t fl = wflag[r];
-        if (!(fl & kWideRoot)) continue;
-        const uint32_t t = tidx[r];
-        if (t >= nw) {
-            *err = 1u;
-            continue;
-        }
-        const uint32_t meta = tnodes[3 * (size_t)t].w, first3 = tnodes[3 * (size_t)t + 2].z, first = first3 / 3u;
-        const uint32_t leaf = tnodes[3 * (size_t)t + 2].w, n_in = meta >> 24, n_leaf = (fl & 7u) - n_in;
-        if (n_in > 4u || n_leaf > 4u || leaf > n || n_leaf > n - leaf || (n_in && first == 0u) ||
-            (n_in && first3 != 3u * first) || (n_in && first > nw) ||
-            (n_in && n_in > nw - first)) {
-            *err = 1u;
-            continue;
-        }
-        for (uint32_t k = 0; k < n_in; k++) atomicAdd(&tref[first + k], 1u);
-        for (uint32_t k = 0; k < n_leaf; k++) atomicAdd(&lref[leaf + k], kTravRef);
+    for (uint32_t i = blockIdx.x * kBlk + threadIdx.x; i < ni; i += gridDim.x * kBlk) {
+        if (i < nw) wide_refs(i, wnodes, nw, n, wref, lref, err);
+        trav_refs(i, wflag[i], tnodes, tidx, nw, n, tref, lref, err);
     }
 }
-
 __global__ void __launch_bounds__(kBlk) k_wide_verify(const uint32_t* __restrict__ nwp, uint32_t n,
                                                       const uint32_t* __restrict__ wref,
                                                       const uint32_t* __restrict__ tref,
                                                       const uint32_t* __restrict__ lref, uint32_t* __restrict__ err)
 {
     const uint32_t nw = *nwp;
-    for (uint32_t i = blockIdx.x * kBlk + threadIdx.x; i < n; i += gridDim.x * kBlk) {
-        if (lref[i] != 1u + kTravRef) *err = 1u;
-        if (i < nw && (wref[i] != (i == 0u ? 0u : 1u) || tref[i] != wref[i])) *err = 1u;
-    }
+    for (uint32_t i = blockIdx.x * kBlk + threadIdx.x; i < n; i += gridDim.x * kBlk)
+        if (refs_wrong(i, nw, wref, tref, lref)) *err = 1u;
 }
 
-// The 4-wide tree of the current binary tree (after every build and refit).
-// One launch per wide level: the binary depth bounds the wide depth, and
-// levels past the deepest find an empty frontier.
+// Everything that follows the refit of a small scene (at most kSahMaxPrims
+// spheres, a thread each), one workgroup: the binary nodes, the levels, the
+// wide indices, both packed forms and their check.  As launches of their own
+// these were 22, each shorter than the gap to the next, and the host waited
+// once between them: loading and tracing the book scene 440 -> 324 us with
+// k_small_keys.
+__global__ void __launch_bounds__(kSmallThreads) k_wide_small(LevelArrays A, const float4* sph, uint32_t n,
+                                                              uint4* nodes, const uint32_t* height, uint32_t* cnt,
+                                                              uint32_t* widx, uint4* wnodes, TravOut T)
+{
+    __shared__ FewShared sh;
+    __shared__ uint32_t wref[kSmallThreads], tref[kSmallThreads], lref[kSmallThreads], wsum[kSmallThreads / 64];
+    const uint32_t t = threadIdx.x, ni = n - 1u;
+    wref[t] = tref[t] = lref[t] = 0u;
+    if (t > 0u && t < ni) A.wflag[t] = 0u;
+    if (t < ni) pack_node(t, sph, A.child, A.boxes, nodes);
+    uint32_t level = 0, count = first_level(A, cnt, height, sh);
+    if (count == 0u) return;
+    few_levels(A, cnt, level, count, 0u, 0xFFFFFFFFu, sh);
+    const uint32_t fl = t < ni ? A.wflag[t] : 0u;
+    const uint64_t m = __ballot((fl & kWideRoot) != 0u);
+    if (t % 64 == 0u) wsum[t / 64] = (uint32_t)__popcll(m);
+    __syncthreads();
+    uint32_t nw = 0, idx = mbcnt(m);
+    for (uint32_t w = 0; w < kSmallThreads / 64; w++) {
+        if (w < t / 64) idx += wsum[w];
+        nw += wsum[w];
+    }
+    if (fl & kWideRoot) widx[t] = idx;
+    if (t == 0u) cnt[kWideCount] = nw;
+    __syncthreads();
+    if (t < ni) wide_pack(t, sph, A.wkids, A.wflag, widx, A.boxes, wnodes, T);
+    __syncthreads();
+    if (t < nw) wide_refs(t, wnodes, nw, n, wref, lref, cnt + kWideError);
+    trav_refs(t, fl, T.nodes, A.tidx, nw, n, tref, lref, cnt + kWideError);
+    __syncthreads();
+    if (t < n && refs_wrong(t, nw, wref, tref, lref)) cnt[kWideError] = 1u;
+}
+
+// The packed nodes and the 4-wide tree of the current binary tree (after
+// every build and refit).
 static vzStatus collapse_wide(vzScene s, hipStream_t st)
 {
     const uint32_t n = s->n, ni = n - 1;
-    uint32_t* cnt = s->d_wcnt;  // [0, kMaxDepth]: roots per level; then nw, leaves placed, the check's result
+    uint32_t* cnt = s->d_wcnt;
     // places in level order, in buffers free at this point: the refit's
     // counters and the sort's second buffers
-    uint32_t *tidx = s->d_visit, *tchild = s->d_keys[1], *tleaf = s->d_vals[1];
-    uint32_t* tsum = s->d_widx + ni;
-    const uint32_t ntile = blocks_for(ni, kScanTile);
-    hipLaunchKernelGGL(k_zero, dim3(blocks_for(ni, kBlk)), dim3(kBlk), 0, st, s->d_wflag, ni);
-    hipLaunchKernelGGL(k_wide_init, dim3(1), dim3(kBlk), 0, st, s->d_wflag, s->d_wfront[0], cnt, kMaxDepth + 8);
-    const uint32_t grid = std::min<uint32_t>(1024u, blocks_for(ni, kBlk));
-    for (uint32_t L = 0; L + 1 < s->depth && L < kMaxDepth; L++)
-        hipLaunchKernelGGL(k_wide_level, dim3(grid), dim3(kBlk), 0, st, s->d_child, s->d_boxes,
-                           s->d_wfront[L & 1u], s->d_wfront[(L + 1) & 1u], cnt, L, s->d_wkids, s->d_wflag, tidx,
-                           tchild, tleaf);
-    hipLaunchKernelGGL(k_wscan_tiles, dim3(ntile), dim3(kBlk), 0, st, s->d_wflag, ni, tsum);
-    hipLaunchKernelGGL(k_wscan_top, dim3(1), dim3(kBlk), 0, st, tsum, ntile, cnt + kMaxDepth + 1);
-    hipLaunchKernelGGL(k_wscan_apply, dim3(ntile), dim3(kBlk), 0, st, s->d_wflag, ni, tsum, s->d_widx);
-    hipLaunchKernelGGL(k_wide_pack, dim3(blocks_for(ni, kBlk)), dim3(kBlk), 0, st, s->d_sph, s->d_wkids,
-                       s->d_wflag, s->d_widx, s->d_boxes, ni, s->d_wnodes,
-                       TravOut{tidx, tchild, tleaf, s->d_leaf_info, s->d_mat, n, s->d_tnodes, s->d_tsph, s->d_tinfo,
-                               s->d_tmat});
-    // reference counts in buffers free at this point: the level fronts and
-    // the refit frontier (both rebuilt by every refit)
-    uint32_t *wref = s->d_wfront[0], *tref = s->d_wfront[1];
-    uint32_t* lref = s->d_frontier;
-    hipLaunchKernelGGL(k_zero, dim3(blocks_for(ni, kBlk)), dim3(kBlk), 0, st, wref, ni);
-    hipLaunchKernelGGL(k_zero, dim3(blocks_for(ni, kBlk)), dim3(kBlk), 0, st, tref, ni);
-    hipLaunchKernelGGL(k_zero, dim3(blocks_for(n, kBlk)), dim3(kBlk), 0, st, lref, n);
-    hipLaunchKernelGGL(k_wide_refs, dim3(grid), dim3(kBlk), 0, st, s->d_wnodes, s->d_tnodes, s->d_wflag, tidx, ni,
-                       cnt + kMaxDepth + 1, n, wref, tref, lref, cnt + kMaxDepth + 3);
-    hipLaunchKernelGGL(k_wide_verify, dim3(grid), dim3(kBlk), 0, st, cnt + kMaxDepth + 1, n, wref, tref, lref,
-                       cnt + kMaxDepth + 3);
+    const LevelArrays A{s->d_child, s->d_boxes, {s->d_wfront[0], s->d_wfront[1]}, s->d_wkids, s->d_wflag,
+                        s->d_visit, s->d_keys[1], s->d_vals[1]};
+    const TravOut T{A.tidx, A.tchild, A.tleaf, s->d_leaf_info, s->d_mat, n, s->d_tnodes, s->d_tsph, s->d_tinfo,
+                    s->d_tmat};
+    if (n <= kSahMaxPrims) {
+        hipLaunchKernelGGL(k_wide_small, dim3(1), dim3(kSmallThreads), 0, st, A, s->d_sph, n, s->d_nodes, s->d_height,
+                           cnt, s->d_widx, s->d_wnodes, T);
+    } else {
+        const dim3 all(blocks_for(n, kBlk));
+        hipLaunchKernelGGL(k_pack_nodes, all, dim3(kBlk), 0, st, s->d_sph, s->d_child, s->d_boxes, ni, s->d_nodes);
+        // the levels of more than kFewRoots roots: some log4(n) - 6 of them
+        // below the top, more where the tree is uneven (empty ones cost a
+        // launch, ones left over one workgroup's time)
+        uint32_t mids = 0;
+        if (ni > kFewRoots)
+            for (uint32_t v = ni; v > 4u; v /= 4u) mids++;
+        const uint32_t grid = std::min<uint32_t>(1024u, blocks_for(ni, kBlk));
+        hipLaunchKernelGGL(k_wide_few, dim3(1), dim3(kFewThreads), 0, st, A, cnt, s->d_height, 0u, 0u);
+        for (uint32_t m = 0; m < mids; m++)
+            hipLaunchKernelGGL(k_wide_level, dim3(grid), dim3(kBlk), 0, st, A, cnt, m);
+        if (mids) hipLaunchKernelGGL(k_wide_few, dim3(1), dim3(kFewThreads), 0, st, A, cnt, s->d_height, 1u, mids);
+        uint32_t* tsum = s->d_widx + ni;
+        const uint32_t ntile = blocks_for(ni, kScanTile);
+        hipLaunchKernelGGL(k_wscan_tiles, dim3(ntile), dim3(kBlk), 0, st, s->d_wflag, ni, tsum);
+        hipLaunchKernelGGL(k_wscan_top, dim3(1), dim3(kBlk), 0, st, tsum, ntile, cnt + kWideCount);
+        hipLaunchKernelGGL(k_wscan_apply, dim3(ntile), dim3(kBlk), 0, st, s->d_wflag, ni, tsum, s->d_widx);
+        hipLaunchKernelGGL(k_wide_pack, all, dim3(kBlk), 0, st, s->d_sph, s->d_wkids, s->d_wflag, s->d_widx,
+                           s->d_boxes, ni, s->d_wnodes, T);
+        // reference counts in buffers free at this point: the level fronts and
+        // the refit frontier (both rebuilt by every refit)
+        uint32_t *wref = s->d_wfront[0], *tref = s->d_wfront[1], *lref = s->d_frontier;
+        hipLaunchKernelGGL(k_zero3, all, dim3(kBlk), 0, st, wref, ni, tref, ni, lref, n);
+        hipLaunchKernelGGL(k_wide_refs, dim3(grid), dim3(kBlk), 0, st, s->d_wnodes, s->d_tnodes, s->d_wflag, A.tidx,
+                           ni, cnt + kWideCount, n, wref, tref, lref, cnt + kWideError);
+        hipLaunchKernelGGL(k_wide_verify, dim3(grid), dim3(kBlk), 0, st, cnt + kWideCount, n, wref, tref, lref,
+                           cnt + kWideError);
+    }
     VZ_HIP_TRY(hipGetLastError());
-    uint32_t h[kMaxDepth + 8] = {};
+    uint32_t h[kWideWords] = {};
     VZ_HIP_TRY(hipMemcpyAsync(h, cnt, sizeof(h), hipMemcpyDeviceToHost, st));
     VZ_HIP_TRY(hipStreamSynchronize(st));
-    s->nw = h[kMaxDepth + 1];
+    s->depth = h[kTreeHeight] + 1;
+    if (s->depth > kMaxDepth)
+        return set_error(VZ_ERROR_CAPACITY, "BVH depth " + std::to_string(s->depth) +
+                                                " exceeds the traversal stack (" +
+                                                std::to_string(kMaxDepth) + ")");
+    s->nw = h[kWideCount];
     s->wdepth = 1;  // the leaf level below the deepest roots'
     for (uint32_t L = 0; L <= kMaxDepth; L++)
         if (h[L]) s->wdepth = L + 2;
-    if (h[kMaxDepth + 3] != 0u) return set_error(VZ_ERROR_INTERNAL, "4-wide BVH failed its structural check");
+    if (h[kWideError] != 0u) return set_error(VZ_ERROR_INTERNAL, "4-wide BVH failed its structural check");
     if (s->wdepth > kMaxWideDepth)
         return set_error(VZ_ERROR_CAPACITY, "4-wide BVH depth " + std::to_string(s->wdepth) +
                                                 " exceeds the traversal stack (" + std::to_string(kMaxWideDepth) + ")");
@@ -1609,8 +1818,9 @@ static vzStatus refit_core(vzScene s, hipStream_t st)
 {
     uint32_t n = s->n;
     if (n < 2) return VZ_SUCCESS;
-    hipLaunchKernelGGL(k_zero, dim3(blocks_for(n - 1, kBlk)), dim3(kBlk), 0, st, s->d_visit, n - 1);
-    hipLaunchKernelGGL(k_zero, dim3(1), dim3(kBlk), 0, st, s->d_fcount, 1u);
+    if (n > kSahMaxPrims)
+        hipLaunchKernelGGL(k_zero3, dim3(blocks_for(n - 1, kBlk)), dim3(kBlk), 0, st, s->d_visit, n - 1, s->d_fcount, 1u,
+                           s->d_wflag, n - 1);
     hipLaunchKernelGGL(k_refit_local, dim3(blocks_for(n, kRefitLeaves)), dim3(kRefitThreads), 0, st, s->d_sph,
                        n, s->d_child, s->d_parent_int, s->d_parent_leaf, s->d_boxes, s->d_height,
                        s->d_frontier, s->d_fcount);
@@ -1618,17 +1828,6 @@ static vzStatus refit_core(vzScene s, hipStream_t st)
         hipLaunchKernelGGL(k_refit_top, dim3(kTopBlocks), dim3(kRefitThreads), 0, st, s->d_sph, s->d_child,
                            s->d_parent_int, s->d_parent_leaf, s->d_frontier, s->d_fcount, s->d_visit, s->d_boxes,
                            s->d_height);
-    hipLaunchKernelGGL(k_pack_nodes, dim3(blocks_for(n - 1, kBlk)), dim3(kBlk), 0, st, s->d_sph, s->d_child,
-                       s->d_boxes, n - 1, s->d_nodes);
-    VZ_HIP_TRY(hipGetLastError());
-    uint32_t h = 0;
-    VZ_HIP_TRY(hipMemcpyAsync(&h, s->d_height, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-    VZ_HIP_TRY(hipStreamSynchronize(st));
-    s->depth = h + 1;
-    if (s->depth > kMaxDepth)
-        return set_error(VZ_ERROR_CAPACITY, "BVH depth " + std::to_string(s->depth) +
-                                                " exceeds the traversal stack (" +
-                                                std::to_string(kMaxDepth) + ")");
     return collapse_wide(s, st);
 }
 
@@ -1643,12 +1842,17 @@ vzStatus lbvh_build(vzScene s, hipStream_t st)
     float* partial = s->d_bounds;
     float* fin = s->d_bounds + 6 * 1024;
     float* grid_b = fin + 16;
-    hipLaunchKernelGGL(k_bounds_partial, dim3(nb), dim3(kBlk), 0, st, s->d_sph_in, n, nullptr, partial);
-    hipLaunchKernelGGL(k_bounds_final, dim3(1), dim3(kBlk), 0, st, partial, nb, 0u, fin);
-    hipLaunchKernelGGL(k_bounds_partial, dim3(nb), dim3(kBlk), 0, st, s->d_sph_in, n, fin, partial);
-    hipLaunchKernelGGL(k_bounds_final, dim3(1), dim3(kBlk), 0, st, partial, nb, 1u, grid_b);
-    hipLaunchKernelGGL(k_morton, dim3(blocks_for(n, kBlk)), dim3(kBlk), 0, st, s->d_sph_in, n, fin, grid_b,
-                       s->d_keys[0], s->d_vals[0]);
+    if (n <= kSahMaxPrims) {
+        hipLaunchKernelGGL(k_small_keys, dim3(1), dim3(kSmallThreads), 0, st, s->d_sph_in, n, s->d_keys[0],
+                           s->d_vals[0]);
+    } else {
+        hipLaunchKernelGGL(k_bounds_partial, dim3(nb), dim3(kBlk), 0, st, s->d_sph_in, n, nullptr, partial);
+        hipLaunchKernelGGL(k_bounds_final, dim3(1), dim3(kBlk), 0, st, partial, nb, 0u, fin);
+        hipLaunchKernelGGL(k_bounds_partial, dim3(nb), dim3(kBlk), 0, st, s->d_sph_in, n, fin, partial);
+        hipLaunchKernelGGL(k_bounds_final, dim3(1), dim3(kBlk), 0, st, partial, nb, 1u, grid_b);
+        hipLaunchKernelGGL(k_morton, dim3(blocks_for(n, kBlk)), dim3(kBlk), 0, st, s->d_sph_in, n, fin, grid_b,
+                           s->d_keys[0], s->d_vals[0]);
+    }
     s->builder = (n >= 2 && n <= kSahMaxPrims) ? VZ_BUILD_SAH : VZ_BUILD_LBVH;
     // keys and leaf order end in buffers 0 either way
     s->d_morton = s->d_keys[0];
