@@ -592,6 +592,57 @@ __device__ __forceinline__ void sah_pair(uint32_t x, uint32_t f, uint32_t self, 
     child[self] = X | (3u << 30);
 }
 
+// The cheapest split of a range of m <= kSahFew spheres without bins: lane (k,
+// i) weighs the split of axis k after sphere i's bin, against each sphere in
+// turn.  Every split of the binned sweep that differs from the one before it
+// is one of these, and the sums are the same, so the result is: the least
+// cost, of equal ones the first axis and the lowest bin.  Most ranges
+// are this small, and clearing, filling and scanning 96 bins took each of them
+// as long as a large one.  p and sp: sphere i in lane i.  Returns false where
+// a cost is not a number (the sweep decides) or no axis splits.
+constexpr uint32_t kSahFew = 21;  // 3 axes in a wave
+__device__ __forceinline__ bool sah_few(const float4* sph, uint32_t m, uint32_t p, const float4 sp, const float (&lo)[3],
+                                        const float (&ext)[3], int& axis, int& split, uint32_t& n_left, int& lane_bin)
+{
+    const uint32_t lane = __lane_id(), k = lane / kSahFew, i = lane - k * kSahFew;
+    const float lo_k = k == 0u ? lo[0] : (k == 1u ? lo[1] : lo[2]), ext_k = k == 0u ? ext[0] : (k == 1u ? ext[1] : ext[2]);
+    const uint32_t pi = __shfl(p, (int)i);
+    const bool on = k < 3u && i < m && ext_k > 0.0f;
+    int bin = 0;
+    if (on) bin = sah_bin(sah_cen(sph[pi], (int)k), lo_k, ext_k);
+    float l[6], r[6];
+    for (int q = 0; q < 3; q++) {
+        l[q] = r[q] = 3.4e38f;
+        l[3 + q] = r[3 + q] = -3.4e38f;
+    }
+    uint32_t nl = 0;
+    for (uint32_t j = 0; j < m; j++) {
+        auto of = [&](float v) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), (int)j)); };
+        const float c[3] = {of(sp.x), of(sp.y), of(sp.z)}, rr = fabsf(of(sp.w));
+        const bool left = __shfl(bin, (int)(k * kSahFew + j)) <= bin;
+        nl += left ? 1u : 0u;
+        for (int q = 0; q < 3; q++) {
+            const float b0 = c[q] - rr, b1 = c[q] + rr;
+            l[q] = fminf(l[q], left ? b0 : 3.4e38f);
+            l[3 + q] = fmaxf(l[3 + q], left ? b1 : -3.4e38f);
+            r[q] = fminf(r[q], left ? 3.4e38f : b0);
+            r[3 + q] = fmaxf(r[3 + q], left ? -3.4e38f : b1);
+        }
+    }
+    const float cost = box_area6(l) * (float)nl + box_area6(r) * (float)(m - nl);
+    const bool ok = on && nl < m;
+    if (__ballot(ok && !(cost == cost)) != 0ull || __ballot(ok) == 0ull) return false;
+    const float best = wave_reduce<true>(ok ? cost : __builtin_huge_valf());
+    const float key = (float)(k * (uint32_t)kSahBins) + (float)bin;  // axis, then bin
+    const float first = wave_reduce<true>(ok && cost == best ? key : 1e6f);
+    const int at = __ffsll((unsigned long long)__ballot(ok && cost == best && key == first)) - 1;
+    axis = at / (int)kSahFew;
+    split = __builtin_amdgcn_readlane(bin, at);
+    n_left = (uint32_t)__builtin_amdgcn_readlane((int)nl, at);
+    lane_bin = __shfl(bin, axis * (int)kSahFew + (int)min(lane, kSahFew - 1u));
+    return true;
+}
+
 // Splits the range [a, b] (at least 3 spheres) at depth d, by one wave: its
 // permutation is partitioned; returns the last index of the left part.
 __device__ __forceinline__ uint32_t sah_split(const float4* sph, uint32_t* perm, uint32_t* tmp, uint32_t* bins, uint32_t a,
@@ -619,6 +670,19 @@ __device__ __forceinline__ uint32_t sah_split(const float4* sph, uint32_t* perm,
         any = any || ext[k] > 0.0f;
     }
     if (!any || d >= kSahDepthCap) return a + m / 2u - 1u;
+    // stable partition of a range in registers: spheres of bins up to bj to the left
+    auto part_wave = [&](int bin, int bj, uint32_t nl) {
+        const bool valid = lane < m, left = valid && bin <= bj;
+        const uint64_t ml = __ballot(left), mr = __ballot(valid && !left);
+        if (valid) perm[left ? a + mbcnt(ml) : a + nl + mbcnt(mr)] = p;
+        wave_order();
+        return a + nl - 1u;
+    };
+    if (m <= kSahFew) {
+        int k, split, bin;
+        uint32_t n_left;
+        if (sah_few(sph, m, p, sp, lo, ext, k, split, n_left, bin)) return part_wave(bin, split, n_left);
+    }
     for (int x = (int)lane; x < kSahBinWords; x += 64) bins[x] = x % 7 < 3 ? 0xFFFFFFFFu : 0u;
     wave_order();
     int mine[3] = {0, 0, 0};
@@ -676,16 +740,7 @@ __device__ __forceinline__ uint32_t sah_split(const float4* sph, uint32_t* perm,
         }
     }
     if (bk < 0) return a + m / 2u - 1u;
-    // stable partition
-    if (m <= 64u) {
-        const bool valid = lane < m;
-        const int bin = bk == 0 ? mine[0] : (bk == 1 ? mine[1] : mine[2]);
-        const bool left = valid && bin <= bj;
-        const uint64_t ml = __ballot(left), mr = __ballot(valid && !left);
-        if (valid) perm[left ? a + mbcnt(ml) : a + nl + mbcnt(mr)] = p;
-        wave_order();
-        return a + nl - 1u;
-    }
+    if (m <= 64u) return part_wave(bk == 0 ? mine[0] : (bk == 1 ? mine[1] : mine[2]), bj, nl);
     uint32_t offl = a, offr = a + nl;
     const float blo = bk == 0 ? lo[0] : (bk == 1 ? lo[1] : lo[2]), bext = bk == 0 ? ext[0] : (bk == 1 ? ext[1] : ext[2]);
     for (uint32_t i0 = a; i0 <= b; i0 += 64u) {
