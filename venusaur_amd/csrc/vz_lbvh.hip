@@ -425,12 +425,16 @@ static_assert(kSahMaxPrims <= kRefitLeaves, "every SAH range lies in one refit w
 static_assert(kSahWaves * kSahBinWords >= (int)kSahMaxPrims, "the bins hold a treelet's keys at the end");
 // A wave goes on with the larger part of a split; the smaller one goes to the
 // queue from kSahShare spheres up (at most kSahMaxPrims / kSahShare of them),
-// and is finished first otherwise.
-constexpr uint32_t kSahShare = 24;
-constexpr uint32_t kSahTasks = 64;
+// and is finished first otherwise.  Ranges of up to kSahFew spheres are built
+// to the end by sah_few.
+#ifndef SSH
+#define SSH 8
+#endif
+constexpr uint32_t kSahFew = 21;  // times 3 axes in a wave
+constexpr uint32_t kSahShare = SSH;
+constexpr uint32_t kSahTasks = 192;
 static_assert(kSahMaxPrims / kSahShare + 1 + kSahSoloWaves <= kSahTasks, "a ticket per task and waiting wave");
-constexpr uint32_t kSahLocal = 8;  // ranges a wave has put aside: each at most half of the one before
-static_assert((kSahShare >> kSahLocal) == 0, "the smaller parts halve");
+static_assert(kSahShare <= kSahFew, "what a wave finishes first is built by sah_few");
 constexpr uint32_t kSahNone = 0xFFFFFFFFu;
 static_assert(kSahDepthCap + 10 + 1 <= kMaxWideDepth, "SAH tree depth within the traversal stack");
 
@@ -547,8 +551,8 @@ __global__ void __launch_bounds__(kSmallThreads) k_small_keys(const float4* __re
 }
 
 // LDS of one treelet build by NW waves: the range's spheres by local index
-// (gathered once), the local permutation, the queue of ranges, and per wave
-// the ranges put aside and the bins.  A range is (a | b << 10 | depth << 20
+// (gathered once), the local permutation, the queue of ranges, and the bins of
+// each wave.  A range is (a | b << 10 | depth << 20
 // local, node index).
 template <int NW>
 struct SahShared {
@@ -556,94 +560,114 @@ struct SahShared {
     uint32_t perm[kSahMaxPrims], tmp[kSahMaxPrims];
     uint2 task[kSahTasks];            // .x kSahNone: not written yet
     uint32_t head, tail, open;        // tickets taken, tasks written, tasks not finished
-    uint2 local[NW][kSahLocal];
     uint32_t bin[NW][kSahBinWords];
 };
 
-// The SAH split of a range of two spheres [x, x + 1] (node `self`: the
-// range's right end for a left child, its left end for a right child) at
-// depth d, in closed form: the two leaf boxes are the two sides whatever the axis,
-// so every axis of positive centre extent costs area(A) + area(B) alike and
-// the first one wins; the sphere with the smaller centre on it goes left.
-// With no such axis, or from the depth cap on, the order stays.  This is
-// what the binned sweep gives for two spheres (they fall in bins 0 and 31).
-__device__ __forceinline__ void sah_pair(uint32_t x, uint32_t f, uint32_t self, uint32_t d,
-                                         uint32_t* __restrict__ child, uint32_t* __restrict__ parent_leaf,
-                                         const float4* sph, uint32_t* perm)
+// The whole subtree over the range [a, a + m), 2 <= m <= kSahFew, node `self`
+// at depth d, by one wave: lane (k, i) holds the sphere at place i and weighs
+// axis k, for all ranges of a level at a time.  A split of the binned sweep
+// that differs from the one before it comes after some sphere's bin; the lane
+// of that sphere sums both sides over its range's spheres in turn, and the
+// least cost is taken, of equal ones the first axis and the lowest bin: the
+// sweep's choice, without clearing, filling and scanning 96 bins.  Range by
+// range a split of few spheres took 1.8 us, bound by the latency of one
+// wave's instructions, and they are most of a build: XXXX.
+__device__ __forceinline__ void sah_few(const float4* sph, uint32_t* perm, uint32_t a, uint32_t m, uint32_t d,
+                                        uint32_t f, uint32_t self, uint32_t* __restrict__ child,
+                                        uint32_t* __restrict__ parent_int, uint32_t* __restrict__ parent_leaf)
 {
-    const uint32_t X = f + x;  // split after leaf X: both children leaves
-    const float4 s0 = sph[perm[x]], s1 = sph[perm[x + 1u]];
-    if (d < kSahDepthCap) {
-        for (int k = 0; k < 3; k++) {
-            const float c0 = sah_cen(s0, k), c1 = sah_cen(s1, k);
-            if (c0 != c1) {
-                if (c0 > c1) {
-                    const uint32_t t = perm[x];
-                    perm[x] = perm[x + 1u];
-                    perm[x + 1u] = t;
-                }
-                break;
+    const uint32_t lane = __lane_id(), k = lane / kSahFew, i = lane - k * kSahFew, row = k * kSahFew;
+    const bool in = k < 3u && i < m;
+    uint32_t s = in ? 0u : 1u, e = in ? m - 1u : 0u;  // the range of place i
+    const uint64_t below = (1ull << i) - 1ull;        // places before it
+    for (;;) {
+        const bool on = s < e;
+        if (__ballot(on) == 0ull) return;
+        const uint32_t p = in ? perm[a + i] : 0u;
+        const float4 sp = sph[p];
+        const float c = sah_cen(sp, (int)min(k, 2u));
+        float lo = 3.4e38f, hi = -3.4e38f;
+        for (uint32_t j = s; __ballot(on && j <= e) != 0ull; j++) {
+            const float o = __shfl(c, (int)(row + j) & 63);
+            lo = fminf(lo, j <= e ? o : 3.4e38f);
+            hi = fmaxf(hi, j <= e ? o : -3.4e38f);
+        }
+        const float ext = hi - lo;
+        const bool axis_on = on && ext > 0.0f && d < kSahDepthCap;
+        int bin = 0;
+        if (axis_on) bin = sah_bin(c, lo, ext);
+        float l[6], r[6];
+        for (int q = 0; q < 3; q++) {
+            l[q] = r[q] = 3.4e38f;
+            l[3 + q] = r[3 + q] = -3.4e38f;
+        }
+        uint32_t nl = 0;
+        for (uint32_t j = s; __ballot(on && j <= e) != 0ull; j++) {
+            const float4 o = sph[perm[a + min(j, m - 1u)]];
+            const float cc[3] = {o.x, o.y, o.z}, rr = fabsf(o.w);
+            const bool left = __shfl(bin, (int)(row + j) & 63) <= bin, use = j <= e;
+            nl += use && left ? 1u : 0u;
+            for (int q = 0; q < 3; q++) {
+                const float b0 = cc[q] - rr, b1 = cc[q] + rr;
+                l[q] = fminf(l[q], use && left ? b0 : 3.4e38f);
+                l[3 + q] = fmaxf(l[3 + q], use && left ? b1 : -3.4e38f);
+                r[q] = fminf(r[q], use && !left ? b0 : 3.4e38f);
+                r[3 + q] = fmaxf(r[3 + q], use && !left ? b1 : -3.4e38f);
             }
         }
-    }
-    const uint32_t up = self | (((X / kRefitLeaves) == ((X + 1u) / kRefitLeaves)) ? kLocalBit : 0u);
-    parent_leaf[X] = up;
-    parent_leaf[X + 1u] = up;
-    child[self] = X | (3u << 30);
-}
-
-// The cheapest split of a range of m <= kSahFew spheres without bins: lane (k,
-// i) weighs the split of axis k after sphere i's bin, against each sphere in
-// turn.  Every split of the binned sweep that differs from the one before it
-// is one of these, and the sums are the same, so the result is: the least
-// cost, of equal ones the first axis and the lowest bin.  Most ranges
-// are this small, and clearing, filling and scanning 96 bins took each of them
-// as long as a large one.  p and sp: sphere i in lane i.  Returns false where
-// a cost is not a number (the sweep decides) or no axis splits.
-constexpr uint32_t kSahFew = 21;  // 3 axes in a wave
-__device__ __forceinline__ bool sah_few(const float4* sph, uint32_t m, uint32_t p, const float4 sp, const float (&lo)[3],
-                                        const float (&ext)[3], int& axis, int& split, uint32_t& n_left, int& lane_bin)
-{
-    const uint32_t lane = __lane_id(), k = lane / kSahFew, i = lane - k * kSahFew;
-    const float lo_k = k == 0u ? lo[0] : (k == 1u ? lo[1] : lo[2]), ext_k = k == 0u ? ext[0] : (k == 1u ? ext[1] : ext[2]);
-    const uint32_t pi = __shfl(p, (int)i);
-    const bool on = k < 3u && i < m && ext_k > 0.0f;
-    int bin = 0;
-    if (on) bin = sah_bin(sah_cen(sph[pi], (int)k), lo_k, ext_k);
-    float l[6], r[6];
-    for (int q = 0; q < 3; q++) {
-        l[q] = r[q] = 3.4e38f;
-        l[3 + q] = r[3 + q] = -3.4e38f;
-    }
-    uint32_t nl = 0;
-    for (uint32_t j = 0; j < m; j++) {
-        auto of = [&](float v) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), (int)j)); };
-        const float c[3] = {of(sp.x), of(sp.y), of(sp.z)}, rr = fabsf(of(sp.w));
-        const bool left = __shfl(bin, (int)(k * kSahFew + j)) <= bin;
-        nl += left ? 1u : 0u;
-        for (int q = 0; q < 3; q++) {
-            const float b0 = c[q] - rr, b1 = c[q] + rr;
-            l[q] = fminf(l[q], left ? b0 : 3.4e38f);
-            l[3 + q] = fmaxf(l[3 + q], left ? b1 : -3.4e38f);
-            r[q] = fminf(r[q], left ? 3.4e38f : b0);
-            r[3 + q] = fmaxf(r[3 + q], left ? -3.4e38f : b1);
+        const uint32_t len = e - s + 1u;
+        const float cost = box_area6(l) * (float)nl + box_area6(r) * (float)(len - nl);
+        // costs are not negative: they compare as their bits, NaN last
+        uint32_t key = 0xFFFFFFFFu;  // no split here
+        if (axis_on && nl < len) key = cost == cost ? __float_as_uint(cost + 0.0f) : 0x7FFFFFFFu;
+        // the axis's choice over the range
+        uint32_t bkey = 0xFFFFFFFFu, bsplit = 0;  // bin | left spheres << 8
+        const uint32_t mine = (uint32_t)bin | nl << 8;
+        for (uint32_t j = s; __ballot(on && j <= e) != 0ull; j++) {
+            const uint32_t ok = __shfl(key, (int)(row + j) & 63), os = __shfl(mine, (int)(row + j) & 63);
+            if (j <= e && (ok < bkey || (ok == bkey && (os & 0xFFu) < (bsplit & 0xFFu)))) {
+                bkey = ok;
+                bsplit = os;
+            }
+        }
+        // the range's choice over the axes
+        uint32_t best = 0xFFFFFFFFu, split = 0, axis = 3u;
+        for (uint32_t q = 0; q < 3u; q++) {
+            const uint32_t ok = __shfl(bkey, (int)(q * kSahFew + i) & 63), os = __shfl(bsplit, (int)(q * kSahFew + i) & 63);
+            // as floats: a cost that is not a number neither beats nor is beaten
+            if (ok != 0xFFFFFFFFu && (axis == 3u || (ok < best && best != 0x7FFFFFFFu))) {
+                best = ok;
+                split = os;
+                axis = q;
+            }
+        }
+        const int my_bin = __shfl(bin, (int)(min(axis, 2u) * kSahFew + i) & 63);
+        const uint32_t left_n = axis == 3u ? len / 2u : split >> 8;
+        const bool left = axis == 3u ? i - s < left_n : my_bin <= (int)(split & 0xFFu);
+        // stable partition of every range
+        const uint64_t ml = __ballot(left && k == 0u);
+        const uint64_t seg = (2ull << e) - (1ull << s);  // places of the range
+        const uint32_t before = (uint32_t)__popcll(ml & seg & below);
+        if (on && k == 0u) perm[a + (left ? s + before : s + left_n + (i - s - before))] = p;
+        const uint32_t g = s + left_n - 1u;  // last place of the left part
+        if (on && k == 0u && i == s) {
+            const uint32_t G = f + a + g, mr = len - left_n;  // children G and G + 1
+            const uint32_t up = self | (((f + a + s) / kRefitLeaves == (f + a + e) / kRefitLeaves) ? kLocalBit : 0u);
+            if (left_n == 1u) parent_leaf[G] = up; else parent_int[G] = up;
+            if (mr == 1u) parent_leaf[G + 1u] = up; else parent_int[G + 1u] = up;
+            child[self] = G | (left_n == 1u ? 1u << 30 : 0u) | (mr == 1u ? 2u << 30 : 0u);
+        }
+        wave_order();
+        if (on) {
+            self = f + a + g + (i <= g ? 0u : 1u);
+            d++;
+            if (i <= g) e = g;
+            else s = g + 1u;
         }
     }
-    const float cost = box_area6(l) * (float)nl + box_area6(r) * (float)(m - nl);
-    const bool ok = on && nl < m;
-    if (__ballot(ok && !(cost == cost)) != 0ull || __ballot(ok) == 0ull) return false;
-    const float best = wave_reduce<true>(ok ? cost : __builtin_huge_valf());
-    const float key = (float)(k * (uint32_t)kSahBins) + (float)bin;  // axis, then bin
-    const float first = wave_reduce<true>(ok && cost == best ? key : 1e6f);
-    const int at = __ffsll((unsigned long long)__ballot(ok && cost == best && key == first)) - 1;
-    axis = at / (int)kSahFew;
-    split = __builtin_amdgcn_readlane(bin, at);
-    n_left = (uint32_t)__builtin_amdgcn_readlane((int)nl, at);
-    lane_bin = __shfl(bin, axis * (int)kSahFew + (int)min(lane, kSahFew - 1u));
-    return true;
 }
 
-// Splits the range [a, b] (at least 3 spheres) at depth d, by one wave: its
+// Splits the range [a, b] (more than kSahFew spheres) at depth d, by one wave: its
 // permutation is partitioned; returns the last index of the left part.
 __device__ __forceinline__ uint32_t sah_split(const float4* sph, uint32_t* perm, uint32_t* tmp, uint32_t* bins, uint32_t a,
                                               uint32_t b, uint32_t d)
@@ -678,11 +702,6 @@ __device__ __forceinline__ uint32_t sah_split(const float4* sph, uint32_t* perm,
         wave_order();
         return a + nl - 1u;
     };
-    if (m <= kSahFew) {
-        int k, split, bin;
-        uint32_t n_left;
-        if (sah_few(sph, m, p, sp, lo, ext, k, split, n_left, bin)) return part_wave(bin, split, n_left);
-    }
     for (int x = (int)lane; x < kSahBinWords; x += 64) bins[x] = x % 7 < 3 ? 0xFFFFFFFFu : 0u;
     wave_order();
     int mine[3] = {0, 0, 0};
@@ -803,54 +822,40 @@ __device__ __forceinline__ void sah_treelet(const float4* __restrict__ sph, uint
         }
         tx = (uint32_t)__builtin_amdgcn_readfirstlane(tx);
         if (tx == kSahNone) break;
-        uint32_t self = (uint32_t)__builtin_amdgcn_readfirstlane(sh.task[ticket].y), aside = 0;
+        uint32_t self = (uint32_t)__builtin_amdgcn_readfirstlane(sh.task[ticket].y);
         for (;;) {
             const uint32_t a = tx & 0x3FFu, b = (tx >> 10) & 0x3FFu, d = tx >> 20;
-            if (b == a + 1u) {  // a root of two spheres
-                if (lane == 0) sah_pair(a, f, self, d, child, parent_leaf, sh.sph, sh.perm);
-            } else {
-                const uint32_t g = sah_split(sh.sph, sh.perm, sh.tmp, sh.bin[w], a, b, d);
-                const uint32_t G = f + g;  // split after leaf G: children G and G + 1
-                const uint32_t ml = g - a + 1u, mr = b - g;
+            if (b - a < kSahFew) {
+                sah_few(sh.sph, sh.perm, a, b - a + 1u, d, f, self, child, parent_int, parent_leaf);
+                break;
+            }
+            const uint32_t g = sah_split(sh.sph, sh.perm, sh.tmp, sh.bin[w], a, b, d);
+            const uint32_t G = f + g;  // split after leaf G: children G and G + 1
+            const uint32_t ml = g - a + 1u, mr = b - g;
+            if (lane == 0) {
+                const uint32_t up = self | (((f + a) / kRefitLeaves == (f + b) / kRefitLeaves) ? kLocalBit : 0u);
+                if (ml == 1u) parent_leaf[G] = up; else parent_int[G] = up;
+                if (mr == 1u) parent_leaf[G + 1u] = up; else parent_int[G + 1u] = up;
+                child[self] = G | (ml == 1u ? 1u << 30 : 0u) | (mr == 1u ? 2u << 30 : 0u);
+            }
+            wave_order();
+            const uint2 tl = make_uint2(a | g << 10 | (d + 1u) << 20, G);
+            const uint2 tr = make_uint2((g + 1u) | b << 10 | (d + 1u) << 20, G + 1u);
+            const uint2 big = ml >= mr ? tl : tr, small = ml >= mr ? tr : tl;
+            const uint32_t ms = min(ml, mr);
+            if (ms >= kSahShare) {
                 if (lane == 0) {
-                    const uint32_t up = self | (((f + a) / kRefitLeaves == (f + b) / kRefitLeaves) ? kLocalBit : 0u);
-                    if (ml == 1u) parent_leaf[G] = up; else parent_int[G] = up;
-                    if (mr == 1u) parent_leaf[G + 1u] = up; else parent_int[G + 1u] = up;
-                    child[self] = G | (ml == 1u ? 1u << 30 : 0u) | (mr == 1u ? 2u << 30 : 0u);
-                    if (ml == 2u) sah_pair(a, f, G, d + 1u, child, parent_leaf, sh.sph, sh.perm);
-                    if (mr == 2u) sah_pair(g + 1u, f, G + 1u, d + 1u, child, parent_leaf, sh.sph, sh.perm);
+                    atomicAdd(&sh.open, 1u);
+                    const uint32_t at = atomicAdd(&sh.tail, 1u);
+                    sh.task[at].y = small.y;
+                    __hip_atomic_store(&sh.task[at].x, small.x, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
                 }
                 wave_order();
-                const uint2 tl = make_uint2(a | g << 10 | (d + 1u) << 20, G);
-                const uint2 tr = make_uint2((g + 1u) | b << 10 | (d + 1u) << 20, G + 1u);
-                const uint2 big = ml >= mr ? tl : tr, small = ml >= mr ? tr : tl;
-                const uint32_t ms = min(ml, mr);
-                if (ms >= kSahShare) {
-                    if (lane == 0) {
-                        atomicAdd(&sh.open, 1u);
-                        const uint32_t at = atomicAdd(&sh.tail, 1u);
-                        sh.task[at].y = small.y;
-                        __hip_atomic_store(&sh.task[at].x, small.x, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-                    }
-                    wave_order();
-                } else if (ms >= 3u) {
-                    if (lane == 0) sh.local[w][aside] = big;
-                    wave_order();
-                    aside++;
-                    tx = small.x;
-                    self = small.y;
-                    continue;
-                }
-                if (max(ml, mr) >= 3u) {
-                    tx = big.x;
-                    self = big.y;
-                    continue;
-                }
+            } else if (ms >= 2u) {
+                sah_few(sh.sph, sh.perm, small.x & 0x3FFu, ms, d + 1u, f, small.y, child, parent_int, parent_leaf);
             }
-            if (aside == 0u) break;
-            aside--;
-            tx = (uint32_t)__builtin_amdgcn_readfirstlane(sh.local[w][aside].x);
-            self = (uint32_t)__builtin_amdgcn_readfirstlane(sh.local[w][aside].y);
+            tx = big.x;
+            self = big.y;
         }
         if (lane == 0) __hip_atomic_fetch_sub(&sh.open, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
         // keeps the wave's lanes together: without it the compiler sent all
