@@ -571,7 +571,8 @@ struct SahShared {
 // least cost is taken, of equal ones the first axis and the lowest bin: the
 // sweep's choice, without clearing, filling and scanning 96 bins.  Range by
 // range a split of few spheres took 1.8 us, bound by the latency of one
-// wave's instructions, and they are most of a build: XXXX.
+// wave's instructions, and they are most of a build: k_sah_build of the book
+// scene 155 -> 101 us, k_sah_treelets of a million spheres 836 -> 673 us.
 __device__ __forceinline__ void sah_few(const float4* sph, uint32_t* perm, uint32_t a, uint32_t m, uint32_t d,
                                         uint32_t f, uint32_t self, uint32_t* __restrict__ child,
                                         uint32_t* __restrict__ parent_int, uint32_t* __restrict__ parent_leaf)
@@ -1035,13 +1036,15 @@ __global__ void __launch_bounds__(kBlk) k_pack_nodes(const float4* __restrict__ 
 //                  the frontier list.
 //   k_refit_top    climbs from every frontier entry through the crossing
 //                  nodes (about n / kRefitLeaves * log2 kRefitLeaves of them)
-//                  in global memory at agent scope.  Starting from a clean L2
-//                  (the kernel boundary wrote the local results back), each
-//                  release only writes back the few lines this kernel
-//                  dirtied: 0.8 ms for the whole 1M-sphere build against
-//                  1.2 ms with the top done by one workgroup at workgroup
-//                  scope, and 10 ms with every node at agent scope in one
-//                  kernel.
+//                  in global memory: up to kTopOneLeaves leaves by one
+//                  workgroup at workgroup scope, above by kTopBlocks of them
+//                  at agent scope, where each step writes back what its L2
+//                  holds dirty (little: the kernel boundary wrote the local
+//                  results back) and so takes some 4 us, but many run at a
+//                  time.  200k spheres: 37 us by one workgroup, 76 by many; a
+//                  million: 190 and 122; the lines cross near 490k.  With
+//                  every node at agent scope in one kernel the build of a
+//                  million spheres took 10 ms.
 constexpr uint32_t kLeafItem = 0x80000000u;  // frontier entry is a leaf index
 constexpr uint32_t kRefitThreads = 1024;
 constexpr uint32_t kLeavesPerThread = kRefitLeaves / kRefitThreads;
@@ -1120,7 +1123,9 @@ __global__ void __launch_bounds__(kRefitThreads) k_refit_local(const float4* __r
 }
 
 constexpr uint32_t kTopBlocks = 64;
+constexpr uint32_t kTopOneLeaves = 192 * kRefitLeaves;
 
+template <int SCOPE>  // of the climbs' counters, boxes and heights
 __global__ void __launch_bounds__(kRefitThreads) k_refit_top(const float4* __restrict__ sph,
                                                     const uint32_t* __restrict__ child,
                                                     const uint32_t* __restrict__ parent_int,
@@ -1134,7 +1139,7 @@ __global__ void __launch_bounds__(kRefitThreads) k_refit_top(const float4* __res
         const uint32_t item = frontier[i];
         uint32_t p = ((item & kLeafItem) ? parent_leaf[item & ~kLeafItem] : parent_int[item]) & ~kLocalBit;
         for (;;) {
-            if (__hip_atomic_fetch_add(&visit[p], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == 0u) break;
+            if (__hip_atomic_fetch_add(&visit[p], 1u, __ATOMIC_ACQ_REL, SCOPE) == 0u) break;
             const uint32_t cw = child[p];
             const uint32_t g = cw & 0x3FFFFFFFu, flags = cw >> 30;
             float cb[2][6];
@@ -1145,14 +1150,14 @@ __global__ void __launch_bounds__(kRefitThreads) k_refit_top(const float4* __res
                     leaf_box(sph[ch], cb[c]);
                 } else {
                     for (int k = 0; k < 6; k++)
-                        cb[c][k] = __hip_atomic_load(&boxes[ch * 6 + k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    h = max(h, __hip_atomic_load(&height[ch], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+                        cb[c][k] = __hip_atomic_load(&boxes[ch * 6 + k], __ATOMIC_RELAXED, SCOPE);
+                    h = max(h, __hip_atomic_load(&height[ch], __ATOMIC_RELAXED, SCOPE));
                 }
             }
             float nb[6];
             join_boxes(cb, nb);
-            for (int k = 0; k < 6; k++) __hip_atomic_store(&boxes[p * 6 + k], nb[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(&height[p], h + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            for (int k = 0; k < 6; k++) __hip_atomic_store(&boxes[p * 6 + k], nb[k], __ATOMIC_RELAXED, SCOPE);
+            __hip_atomic_store(&height[p], h + 1u, __ATOMIC_RELAXED, SCOPE);
             if (p == 0u) break;
             p = parent_int[p] & ~kLocalBit;
         }
@@ -1884,10 +1889,13 @@ static vzStatus refit_core(vzScene s, hipStream_t st)
     hipLaunchKernelGGL(k_refit_local, dim3(blocks_for(n, kRefitLeaves)), dim3(kRefitThreads), 0, st, s->d_sph,
                        n, s->d_child, s->d_parent_int, s->d_parent_leaf, s->d_boxes, s->d_height,
                        s->d_frontier, s->d_fcount);
-    if (n > kRefitLeaves)  // nodes that cross the workgroups' ranges
-        hipLaunchKernelGGL(k_refit_top, dim3(kTopBlocks), dim3(kRefitThreads), 0, st, s->d_sph, s->d_child,
+    if (n > kRefitLeaves) {  // nodes that cross the workgroups' ranges
+        const bool one = n <= kTopOneLeaves;
+        hipLaunchKernelGGL(one ? k_refit_top<__HIP_MEMORY_SCOPE_WORKGROUP> : k_refit_top<__HIP_MEMORY_SCOPE_AGENT>,
+                           dim3(one ? 1 : kTopBlocks), dim3(kRefitThreads), 0, st, s->d_sph, s->d_child,
                            s->d_parent_int, s->d_parent_leaf, s->d_frontier, s->d_fcount, s->d_visit, s->d_boxes,
                            s->d_height);
+    }
     return collapse_wide(s, st);
 }
 
