@@ -221,15 +221,13 @@ __global__ void __launch_bounds__(path_threads(SRC)) __attribute__((amdgpu_waves
     const uint32_t tid = threadIdx.x, lane = __lane_id();
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(tid >> 6);
     // many requests of many scenes: the lane's own, filled in with its path
-    typename std::conditional<LDSN, SceneView,
-                              typename std::conditional<MANY, LaneScene<COUNT>, SceneArrays>::type>::type sc;
+    typename std::conditional<SRC == kManyMem, LaneScene<COUNT>, SceneArrays>::type sc;
     const SceneView& view = MANY ? G.reqs[0].sc : one.sc;
     if constexpr (SRC == kManyMem) sc = LaneScene<COUNT>{nullptr, nullptr, nullptr};
-    else if constexpr (LDSN) sc = view;
     else sc = scene_arrays<COUNT>(view);
     typename std::conditional<LDSN, PlaneBound, NoBound>::type pb(view);
     if constexpr (LDSN) {
-        stage_scene(sc, sh);
+        stage_scene(view, sh);
         __syncthreads();
     }
     typename std::conditional<LDSN, LdsTraversal<NT>,
@@ -335,7 +333,7 @@ __global__ void __launch_bounds__(path_threads(SRC)) __attribute__((amdgpu_waves
                 // lanes still tracing, or before a queue could overflow (a
                 // visit queues at most 4)
                 const uint64_t pm = __ballot(tr.npend != 0u);
-                if (pm && (__ballot(LDSN ? tr.npend + 4u > kPend : tr.npend == kMemPend) != 0ull ||
+                if (pm && (__ballot(tr.npend == (LDSN ? kLdsPend : kMemPend)) != 0ull ||
                            kFlushDen * (uint32_t)__popcll(pm) >= kFlushNum * (uint32_t)__popcll(busy))) {
                     tr.flush(sc, sh);
                 }
@@ -371,17 +369,11 @@ __global__ void __launch_bounds__(path_threads(SRC)) __attribute__((amdgpu_waves
                 L = mul(thr, sky(tr.d));
             } else if (depth > 0u) {
                 // shade (RayTracer.cu:272-440)
-                float4 s, mat;
-                uint32_t type;
-                if constexpr (LDSN) {
-                    s = sh.spheres[tr.bleaf];
-                    type = ldg(sc.leaf_info + tr.bleaf) >> 30;
-                    mat = ldg(sc.mats + tr.bleaf);
-                } else {
-                    s = ldg(sc.sphere_array() + tr.bleaf);
-                    type = ldg(sc.info_array() + tr.bleaf) >> 30;
-                    mat = ldg(sc.mat_array() + tr.bleaf);
-                }
+                float4 s;
+                if constexpr (LDSN) s = sh.spheres[tr.bleaf];
+                else s = ldg(sc.sphere_array() + tr.bleaf);
+                const uint32_t type = ldg(sc.info_array() + tr.bleaf) >> 30;
+                const float4 mat = ldg(sc.mat_array() + tr.bleaf);
                 const v3 pos = add(tr.o, scl(tr.d, tr.best));
                 v3 n = scl(sub(pos, mk(s.x, s.y, s.z)), recip_rn(s.w));
                 const bool front = dot(tr.d, n) < 0.0f;

@@ -125,11 +125,9 @@ k_trace_hits(SceneView view, const vzRay* __restrict__ rays, uint32_t n, vzHit* 
     __shared__ typename std::conditional<LDSN, LdsScene<NT>, MemScene<NT>>::type sh;
     const uint32_t tid = threadIdx.x, wave = (uint32_t)__builtin_amdgcn_readfirstlane(tid >> 6);
     const typename std::conditional<LDSN, PlaneBound, TraceNoBound>::type pb(view);
-    typename std::conditional<LDSN, SceneView, SceneArrays>::type sc;
-    if constexpr (LDSN) sc = view;
-    else sc = scene_arrays<false>(view);
+    const SceneArrays sc = scene_arrays<false>(view);
     if constexpr (LDSN) {
-        stage_scene(sc, sh);
+        stage_scene(view, sh);
         __syncthreads();
     }
     typename std::conditional<LDSN, LdsTraversal<NT, true>, MemTraversal<NT, true>>::type tr;
@@ -171,7 +169,7 @@ k_trace_hits(SceneView view, const vzRay* __restrict__ rays, uint32_t n, vzHit* 
             }
             busy = __ballot(active && !tdone);
             const uint64_t pm = __ballot(tr.npend != 0u);
-            if (pm && (__ballot(LDSN ? tr.npend + 4u > kPend : tr.npend == kMemPend) != 0ull ||
+            if (pm && (__ballot(tr.npend == (LDSN ? kLdsPend : kMemPend)) != 0ull ||
                        kFlushDen * (uint32_t)__popcll(pm) >= kFlushNum * (uint32_t)__popcll(busy))) {
                 tr.flush(sc, sh);
             }
@@ -179,7 +177,7 @@ k_trace_hits(SceneView view, const vzRay* __restrict__ rays, uint32_t n, vzHit* 
         }
         tr.flush(sc, sh);
         if (active && tdone) {
-            const uint32_t prim = tr.bleaf == 0xFFFFFFFFu ? VZ_MISS : (ldg((LDSN ? view.leaf_info : view.tinfo) + tr.bleaf) & 0x3FFFFFFFu);
+            const uint32_t prim = tr.bleaf == 0xFFFFFFFFu ? VZ_MISS : (ldg(sc.info + tr.bleaf) & 0x3FFFFFFFu);
             reinterpret_cast<uint2*>(hits)[mine] = make_uint2(__float_as_uint(tr.best), prim);
             active = false;
         }

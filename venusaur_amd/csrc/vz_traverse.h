@@ -26,8 +26,6 @@ namespace vz {
 
 constexpr float kRobust = 1.0f + 0x1p-20f;  // >= 1 + 2*gamma_3 (Ize 2013)
 
-constexpr uint32_t kPend = 8;  // queued leaf tests per lane (traversals that do not count)
-
 struct TraceResult {
     float t;
     uint32_t leaf;  // leaf (Morton-order) index, 0xFFFFFFFF on a miss

@@ -15,18 +15,25 @@
 // set-up for camera and scattered rays): a queued test otherwise waits for the
 // L1.  78 KB of LDS per 768 threads keep two workgroups, 24 waves, on a CU.
 //
-// Node, 112 bytes at a byte offset that is also its number:
+// They come from the 48-byte nodes (k_wide_pack, vz_lbvh.hip), whose internal
+// children come first in the slots and whose leaves follow one another, with
+// the leaves in that order.  Node, 112 bytes at a byte offset that is also its
+// number:
 //   0   float lo[4], hi[4] of the slots on x;  32 on y;  64 on z
 //       (an empty slot: lo = +inf, hi = -inf)
-//   96  uint32 per slot: the child node's offset, or 0xFFFF << 16 | leaf (an
-//       empty slot: leaf 0, so that a ray whose terms overflow, which passes
-//       every slot, tests a sphere too many instead of walking astray)
+//   96  uint32 per slot: the child node's offset, or 0xFFFF << 16 for a leaf
+//       or an empty slot.  Slot 3's low 4 bits are the number of internal
+//       children, and if that is below 4 the next 12 the first leaf.
+// An empty slot stands for a leaf further on, which a ray whose terms overflow,
+// and which passes every slot, tests without harm.
 //
-// A stack entry is one word: the entry distance's upper 16 bits (cut, so
-// never beyond the distance) and the LDS address of the slot's child word.
-// Entries compare as distances, so the children hit are put in order by five
-// min/max pairs on such words, leaf and missed slots as words above any
-// distance.
+// A stack entry, and the key by which the children hit are put in order (five
+// min/max pairs), is one word: the entry distance's upper 16 bits (cut, so
+// never beyond the distance) and the child's offset; leaf and missed slots lie
+// above any distance.  A visit's leaves are queued as one word, the first leaf
+// and a mask of four.  With the child's offset behind another LDS load, a
+// queue entry per leaf and a ring of 8 entries whose room each push checked:
+// 1080p book frame at 256 samples 62.3 ms, as it is 59.3.
 #pragma once
 #include "vz_traverse.h"
 
@@ -36,30 +43,27 @@ constexpr uint32_t kLdsNodes = 256;        // a scene of at most this many 4-wid
 constexpr uint32_t kLdsSpheres = 3 * kLdsNodes + 1;  // leaves of so many 4-wide nodes, at most
 constexpr uint32_t kLdsNodeBytes = 112;
 constexpr uint32_t kLdsKeyMask = 0xFFFF0000u;
-constexpr uint32_t kLdsStack = kWideStackS;  // stack words per lane, the oldest beyond them in private memory
+constexpr uint32_t kLdsStack = 10;  // stack words per lane in LDS, later ones in private memory
+constexpr uint32_t kLdsPend = 4;    // queued visits per lane
 
-// LDS of a workgroup of NT threads.
+// LDS of a workgroup of NT threads, [wave][slot][lane].
 template <uint32_t NT>
 struct LdsScene {
     uint4 nodes[kLdsNodes * kLdsNodeBytes / 16];
-    float4 spheres[kLdsSpheres];
-    uint32_t stack[kLdsStack * NT];
-    uint16_t pend[kPend * NT];
+    float4 spheres[kLdsSpheres + 3];
+    uint32_t stack[NT / 64][kLdsStack][64];
+    uint16_t pend[NT / 64][kLdsPend][64];
 };
 
-// Copies the spheres into LDS and decodes the packed nodes (64 bytes,
-// vz_api.h), whole workgroup.
+// Copies the spheres into LDS and decodes the 48-byte nodes, whole workgroup.
 template <uint32_t NT>
 VZ_DEV void stage_scene(const SceneView& sc, LdsScene<NT>& sh)
 {
-    for (uint32_t i = threadIdx.x; i < sc.n; i += NT) sh.spheres[i] = ldg(sc.spheres + i);
+    for (uint32_t i = threadIdx.x; i < sc.n + 3u; i += NT) sh.spheres[i] = ldg(sc.tspheres + i);
     for (uint32_t i = threadIdx.x; i < sc.nw; i += NT) {
-        const uint4 A = ldg(sc.nodes + 4 * i), B = ldg(sc.nodes + 4 * i + 1);
-        const uint4 C = ldg(sc.nodes + 4 * i + 2), D = ldg(sc.nodes + 4 * i + 3);
+        const uint4 A = ldg(sc.tnodes + 3 * i), B = ldg(sc.tnodes + 3 * i + 1), C = ldg(sc.tnodes + 3 * i + 2);
         const float no[3] = {__uint_as_float(A.x), __uint_as_float(A.y), __uint_as_float(A.z)};
-        const uint32_t lo_w[3] = {B.x, B.y, B.z}, hi_w[3] = {B.w, C.x, C.y};
-        const uint32_t ch[4] = {C.z, C.w, D.x, D.y};
-        const uint32_t valid = A.w >> 28, leafm = (A.w >> 24) & 0xFu;
+        const uint32_t lo_w[3] = {B.x, B.y, B.z}, hi_w[3] = {B.w, C.x, C.y}, n_in = A.w >> 24;
         uint4* out = sh.nodes + i * (kLdsNodeBytes / 16);
 #pragma unroll
         for (int k = 0; k < 3; k++) {
@@ -67,20 +71,19 @@ VZ_DEV void stage_scene(const SceneView& sc, LdsScene<NT>& sh)
             uint32_t lo[4], hi[4];
 #pragma unroll
             for (int c = 0; c < 4; c++) {
-                const bool v = ((valid >> c) & 1u) != 0u;
-                lo[c] = __float_as_uint(v ? __builtin_fmaf((float)((lo_w[k] >> (8 * c)) & 0xFFu), s, no[k])
-                                          : __builtin_huge_valf());
-                hi[c] = __float_as_uint(v ? __builtin_fmaf((float)((hi_w[k] >> (8 * c)) & 0xFFu), s, no[k])
-                                          : -__builtin_huge_valf());
+                const uint32_t ql = (lo_w[k] >> (8 * c)) & 0xFFu, qh = (hi_w[k] >> (8 * c)) & 0xFFu;
+                const bool v = ql <= qh;
+                lo[c] = __float_as_uint(v ? __builtin_fmaf((float)ql, s, no[k]) : __builtin_huge_valf());
+                hi[c] = __float_as_uint(v ? __builtin_fmaf((float)qh, s, no[k]) : -__builtin_huge_valf());
             }
             out[2 * k] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
             out[2 * k + 1] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
         }
         uint32_t w[4];
 #pragma unroll
-        for (int c = 0; c < 4; c++)
-            w[c] = ((valid & ~leafm) >> c) & 1u ? ch[c] * kLdsNodeBytes
-                                                : (kLdsKeyMask | (((valid >> c) & 1u) ? ch[c] : 0u));
+        for (uint32_t c = 0; c < 4; c++)
+            w[c] = c < n_in ? (C.z / 3u + c) * kLdsNodeBytes : kLdsKeyMask;
+        w[3] |= n_in < 4u ? n_in | C.w << 4 : 4u;
         out[6] = make_uint4(w[0], w[1], w[2], w[3]);
     }
 }
@@ -94,7 +97,7 @@ struct PlaneBound {
     float p[3];
     VZ_DEV explicit PlaneBound(const SceneView& sc)
     {
-        const uint4 A = ldg(sc.nodes);
+        const uint4 A = ldg(sc.tnodes);
         const float no[3] = {__uint_as_float(A.x), __uint_as_float(A.y), __uint_as_float(A.z)};
         for (int k = 0; k < 3; k++) {
             const float s = scale_of(A.w, k);
@@ -117,7 +120,7 @@ struct LdsTraversal {
     float inv[3], bn[3], bf[3];
     uint32_t off[3];   // 16 where the ray runs towards -k: its near planes are the hi planes
     float tmin, best;
-    uint32_t bleaf, node, sp, bottom, npend;
+    uint32_t bleaf, node, sp, npend;
 
     // Plane distances are fma(p, inv, -o inv), near ones moved down by e and
     // far ones up by 2 e, e = (Pmax + |o|) |inv| 2^-20.  The exact form
@@ -134,7 +137,7 @@ struct LdsTraversal {
         tmin = tmin_;
         best = tmax_;
         bleaf = 0xFFFFFFFFu;
-        node = sp = bottom = npend = 0u;
+        node = sp = npend = 0u;
         const bool ordinary = ray_inverse(d, inv);
         const float oo[3] = {o.x, o.y, o.z};
 #pragma unroll
@@ -153,30 +156,26 @@ struct LdsTraversal {
     }
 
     // Tests the queued leaves; keeps the lexicographic minimum of (t, prim).
-    VZ_DEV void flush(const SceneView& sc, const LdsScene<NT>& sh)
+    VZ_DEV void flush(const SceneArrays& sc, const LdsScene<NT>& sh)
     {
-        while (npend) {
-            npend--;
-            const uint32_t leaf = sh.pend[npend * NT + threadIdx.x];
+        uint32_t m = 0u, leaf0 = 0u;
+        while (m | npend) {
+            if (m == 0u) {
+                npend--;
+                m = sh.pend[threadIdx.x / 64][npend][threadIdx.x % 64];
+                leaf0 = m >> 4;
+                m &= 15u;
+            }
+            const uint32_t leaf = leaf0 + (uint32_t)__builtin_ctz(m);
+            m &= m - 1u;
             float t;
-            if (hit_gated(o, d, inv, tmin, best, sh.spheres[leaf], t))
-                keep_nearer(t, leaf, sc.leaf_info, best, bleaf);
+            if (hit_gated(o, d, inv, tmin, best, sh.spheres[leaf], t)) keep_nearer(t, leaf, sc.info, best, bleaf);
         }
-    }
-
-    VZ_DEV void push(LdsScene<NT>& sh, uint32_t e, LdsOverflow& ov)
-    {
-        if (sp - bottom == kLdsStack) {
-            if (bottom < kWideOverflow) ov.w[bottom] = sh.stack[(bottom % kLdsStack) * NT + threadIdx.x];
-            bottom++;
-        }
-        sh.stack[(sp % kLdsStack) * NT + threadIdx.x] = e;
-        sp++;
     }
 
     // One node visit; returns true when the traversal has finished.  Leaf
-    // slots that are hit are queued (at most 4; the caller flushes before
-    // the queue could overflow, and before it reads the hit).
+    // slots that are hit are queued, an entry a visit (the caller flushes
+    // before the queue could overflow, and before it reads the hit).
     VZ_DEV bool step(LdsScene<NT>& sh, LdsOverflow& ov)
     {
         const char* base = reinterpret_cast<const char*>(sh.nodes);
@@ -204,15 +203,18 @@ struct LdsTraversal {
             const float lo_t = fmaxf(fmaxf(fmaxf(tmin, n3[0]), n3[1]), n3[2]);
             const float hi_t = fminf(fminf(fminf(lim, f3[0]), f3[1]), f3[2]);
             hit[c] = lo_t <= hi_t;
-            const uint32_t e = ((__float_as_uint(ANYT ? fmaxf(lo_t, 0.0f) : lo_t) & kLdsKeyMask) | (node + 96u + 4u * c)) | (w[c] & kLdsKeyMask);
+            const uint32_t e = (__float_as_uint(ANYT ? fmaxf(lo_t, 0.0f) : lo_t) & kLdsKeyMask) | w[c];
             key[c] = hit[c] ? e : 0xFFFFFFFFu;
         }
-#pragma unroll
-        for (int c = 0; c < 4; c++)
-            if (hit[c] && w[c] >= kLdsKeyMask) {
-                sh.pend[npend * NT + threadIdx.x] = (uint16_t)w[c];
-                npend++;
-            }
+        uint32_t leaves = hit[0] ? 1u : 0u;
+        leaves |= hit[1] ? 2u : 0u;
+        leaves |= hit[2] ? 4u : 0u;
+        leaves |= hit[3] ? 8u : 0u;
+        leaves >>= w[3] & 7u;  // internal children come first
+        if (leaves) {
+            sh.pend[threadIdx.x / 64][npend][threadIdx.x % 64] = (uint16_t)((w[3] & 0xFFF0u) | leaves);
+            npend++;
+        }
         // ascending by five compare-exchanges
         auto order = [](uint32_t& a, uint32_t& b) {
             const uint32_t x = min(a, b), y = max(a, b);
@@ -224,31 +226,53 @@ struct LdsTraversal {
         order(key[0], key[2]);
         order(key[1], key[3]);
         order(key[1], key[2]);
-        uint32_t e = key[0];
-        if (e < kLdsKeyMask) {
+        if (key[0] < kLdsKeyMask) {
             if (key[1] < kLdsKeyMask) {
-                if (key[2] < kLdsKeyMask) {
-                    if (key[3] < kLdsKeyMask) push(sh, key[3], ov);
-                    push(sh, key[2], ov);
-                }
-                push(sh, key[1], ov);
-            }
-        } else {
-            // the nearest stacked child that can still hold a closer hit
-            for (;;) {
-                if (sp == 0u) return true;
-                sp--;
-                if (sp < bottom) {
-                    e = ov.w[sp < kWideOverflow ? sp : kWideOverflow - 1u];
-                    bottom = sp;
+                if (sp <= (kLdsStack - 3u) * kRow) {  // room in LDS for three
+                    if (key[2] < kLdsKeyMask) {
+                        if (key[3] < kLdsKeyMask) push(sh, key[3]);
+                        push(sh, key[2]);
+                    }
+                    push(sh, key[1]);
                 } else {
-                    e = sh.stack[(sp % kLdsStack) * NT + threadIdx.x];
+                    for (int c = 3; c >= 1; c--)
+                        if (key[c] < kLdsKeyMask) {
+                            if (sp < kLdsStack * kRow) {
+                                push(sh, key[c]);
+                            } else {
+                                // never more than it holds (kMaxWideDepth)
+                                const uint32_t i = sp / kRow - kLdsStack;
+                                if (i < kWideOverflow) ov.w[i] = key[c];
+                                sp += kRow;
+                            }
+                        }
                 }
-                if (__uint_as_float(e & kLdsKeyMask) <= (ANYT ? fmaxf(lim, 0.0f) : lim)) break;
             }
+            node = key[0] & 0xFFF0u;
+            return false;
         }
-        node = *reinterpret_cast<const uint32_t*>(base + (e & 0xFFFFu));
-        return false;
+        // the nearest stacked child that can still hold a closer hit
+        for (;;) {
+            if (sp == 0u) return true;
+            sp -= kRow;
+            const uint32_t e =
+                sp < kLdsStack * kRow ? *slot(sh, sp) : ov.w[min(sp / kRow - kLdsStack, kWideOverflow - 1u)];
+            node = e & 0xFFF0u;
+            if (__uint_as_float(e & kLdsKeyMask) <= (ANYT ? fmaxf(lim, 0.0f) : lim)) return false;
+        }
+    }
+
+private:
+    static constexpr uint32_t kRow = 256;  // sp counts bytes of a row of the stack, a word a lane
+    static VZ_DEV uint32_t* slot(LdsScene<NT>& sh, uint32_t at)
+    {
+        return reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(&sh.stack[threadIdx.x / 64][0][threadIdx.x % 64]) +
+                                           at);
+    }
+    VZ_DEV void push(LdsScene<NT>& sh, uint32_t e)
+    {
+        *slot(sh, sp) = e;
+        sp += kRow;
     }
 };
 
