@@ -19,8 +19,8 @@ namespace vz {
 // stay well below this for any scene that fits in memory.
 constexpr uint32_t kMaxDepth = 64;
 // Traversal stack of the 4-wide tree: up to 3 entries per wide level above
-// the node being visited, kWideStackS of them per lane in LDS and the oldest
-// kWideOverflow in private memory.  Scenes whose wide depth needs more are
+// the node being visited, kWideStackS of them or more per lane in LDS and
+// kWideOverflow others in private memory.  Scenes whose wide depth needs more are
 // refused at build time.
 constexpr uint32_t kWideStackS = 8;
 constexpr uint32_t kWideOverflow = 96;

@@ -17,12 +17,14 @@
 //                          through LDS so global writes are runs per digit
 //   4. leaf reorder        spheres/materials into Morton (leaf) order
 //   5. Karras linking      one thread per internal node
-//   6. refit + pack        one thread per leaf walks up; the second arrival at
-//                          a node computes its box and writes the 32-byte node
-//   7. 4-wide collapse     level by level, then a structural check
+//   6. refit               one thread per leaf walks up; the second arrival at
+//                          a node computes its box
+//   7. packing, collapse   the 32-byte nodes; the 4-wide tree level by level,
+//                          packed as 64-byte nodes and as the 48-byte ones
+//                          that most traversals read; a structural check
 // A scene of 2 to kSahMaxPrims spheres replaces stages 3 and 5 by a
 // binned-SAH build in one workgroup (k_sah_build) that writes the same node
-// layout, so stages 4, 6 and 7 are shared.
+// layout, and goes through stages 1, 2 and 7 in one workgroup each.
 #include "vz_device.h"
 #include "vz_internal.h"
 

@@ -1,7 +1,7 @@
 // vz_megakernel.hip -- one thread per pixel runs every sample's whole path:
 // __raygen__rg (Core/RayTracer.cu:163-217) with the recursive optixTrace /
 // closest-hit chain (RayTracer.cu:190, 299, 347, 422) unrolled into a loop.
-// Kept beside the wavefront integrator as a second, structurally different
+// Kept beside the path kernels (vz_path.hip) as a second, structurally different
 // GPU path: both must agree with the CPU integrator bit for bit.
 #include "vz_traverse.h"
 

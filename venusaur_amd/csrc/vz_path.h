@@ -45,7 +45,7 @@ struct PathSlot {
     size_t paths_bytes = 0;
     char* pixels = nullptr;    // camera seeds and sums carried between the launches of one request
     size_t pixels_bytes = 0;
-    unsigned long long* stats = nullptr;     // per workgroup, the unit counter, segments per request
+    unsigned long long* stats = nullptr;     // per workgroup, the unit counters, segments per request
     unsigned long long* h_totals = nullptr;  // pinned: kPathStats, then segments per request
     PathReq* reqs = nullptr;   // request table (many requests in one launch)
     PathReq* h_reqs = nullptr; // pinned staging of it

@@ -20,21 +20,22 @@
 // A request with more paths than the buffer holds takes several launches, a
 // chunk of its passes each; its sums and camera seeds carry over.
 //
-// Why.  The queue-driven wavefront this replaces spent a
-// launch per bounce: 304 rounds of three kernels for the 1080p book frame at
-// 256 samples, each as long as its slowest workgroup, its path records
-// written and read back from HBM between them, and no fewer rounds for a
-// small frame.  Tracing whole paths needs one launch, keeps a path in its
-// lane's registers and reads nothing but the scene.  Same box, both sides in
-// turn: 64x36 at 2 samples 817 -> 143 us, 400x225 at 16 samples 2.80 -> 1.12
-// ms, 1200x800 at 16 samples depth 4 3.43 -> 2.04 ms, 1080p at 256 samples
-// 115.2 -> 78.6 ms, a million spheres at 1080p and 64 samples 241 -> 187 ms,
-// 512x512 at 2048 samples in double 355 -> 135 ms, 24 box scenes in a batch
-// 165 -> 121 ms, a burst of 20 requests to a server 336 -> 195 ms; images bit
-// for bit the same.  k_path is bound by VALU issue (traversal and sphere tests with part
-// of the lanes idle); k_path_seeds and k_path_resolve are under 1% each of
-// the 1080p frame (0.27 and 0.60 ms per 128 passes, the latter reading 3.2 GB
-// at 5.3 TB/s).
+// Why.  The queue-driven wavefront this replaces spent a launch per bounce: 304
+// rounds of three kernels for the 1080p book frame at 256 samples, each as
+// long as its slowest workgroup, its path records written and read back from
+// HBM between them, and no fewer rounds for a small frame.  Tracing whole
+// paths needs one launch, keeps a path in its lane's registers and reads
+// nothing but the scene.  Same box, both sides in turn, as first built: 1080p
+// at 256 samples 115.2 -> 78.6 ms, a million spheres at 1080p and 64 samples
+// 241 -> 187 ms, 512x512 at 2048 samples in double 355 -> 135 ms, 400x225 at 16
+// samples 2.80 -> 1.12 ms; with the traversals of vz_traverse_lds.h and
+// vz_traverse_mem.h, queued sphere tests and the counters below 58.4 ms, 143
+// ms, 105 ms and 0.69 ms; images bit for bit the same.  What bounds it is VALU
+// issue at half the lanes with the scene in LDS, the L1 and the latency of
+// node loads as well with it in memory, and the longest path at the end of a
+// small frame.  k_path_seeds and k_path_resolve are under 1% each of the
+// 1080p frame (0.27 and 0.60 ms per 128 passes, the latter reading 3.2 GB at
+// 5.3 TB/s).
 #include <algorithm>
 #include <cstring>
 #include <string>
@@ -211,11 +212,11 @@ struct LaneScene {
 };
 
 // Every wave takes units until none is left: the first by its place (so a
-// small frame spreads over the CUs), the others from its workgroup's counter (a
-// device-wide atomic per unit of up to 512 paths).  Lanes without a path take the next ones of the
-// wave's unit, all lanes with a ray walk the tree until fewer than `refill`
-// of them still do, and the finished ones shade: a path that goes on starts
-// its next segment in place.  A wave never waits for its lanes to finish one
+// small frame spreads over the CUs), the others from its workgroup's counter
+// (a device-wide atomic per unit of up to 512 paths).  Lanes without a path
+// take the next ones of the wave's unit, all lanes with a ray walk the tree
+// until fewer than `refill` of them still do, and the finished ones shade: a
+// path that goes on starts its next segment in place.  A wave never waits for its lanes to finish one
 // request before it starts the next: with kManyMem each lane carries its own
 // scene.
 // COUNT: node visits and sphere tests are counted, with the nodes in memory,

@@ -2,6 +2,10 @@
 // the traversal inside optixTrace (Core/RayTracer.cu:190-202) and the
 // __intersection__hit_sphere program it calls (Core/RayTracer.cu:229-270).
 //
+// This file holds the traversal that counts node visits and sphere tests, and
+// what all share; vz_traverse_lds.h and vz_traverse_mem.h hold the others,
+// which may visit nodes in any order and test spheres late.
+//
 // The tree walked is the 4-wide one collapsed from the binary LBVH: 64-byte
 // nodes holding four quantised child boxes, so a visit is one node fetch
 // (four 16-byte loads that lanes on the same node share) and four box tests
