@@ -2,13 +2,14 @@
 
 Workload (one step): the book final scene (486 spheres, mt19937 seed 5489),
 1920x1080, 256 samples per pixel, max depth 50, FP32, rendered by one
-vzLaunch (LBVH resident, wavefront integrator).  Inputs are resident in HBM
+vzLaunch (BVH resident, persistent path kernels).  Inputs are resident in HBM
 before the timed region; the LBVH build is timed separately.
 
 Prints ONE JSON line.  Besides value/ms_per_step it carries:
-  roofline      the trace kernel (dominant): algorithmic bytes per launch /
+  roofline      the path kernel (dominant): VALU lane operations per launch /
                 its mean launch time from HIP events recorded around every
-                trace launch inside the timed steps, against 8 TB/s HBM
+                launch of it inside the timed steps, against the chip's lane
+                throughput; its algorithmic bytes beside them
   cpu_baseline  the CPU oracle (same integrator, FP32) on a row sample of the
                 same workload, on this host's cores
   checks        segment count vs the oracle on the sample rows, RMSE vs the
@@ -44,7 +45,7 @@ def parse():
     ap.add_argument("--gpus", type=int, default=1)
     ap.add_argument("--steps", type=int, default=3)
     ap.add_argument("--warmup", type=int, default=1)
-    ap.add_argument("--mode", choices=["wavefront", "megakernel"], default="wavefront")
+    ap.add_argument("--mode", choices=["path", "megakernel"], default="path")
     ap.add_argument("--width", type=int, default=1920)
     ap.add_argument("--height", type=int, default=1080)
     ap.add_argument("--spp", type=int, default=256)
@@ -59,7 +60,7 @@ def parse():
     ap.add_argument("--serve-sustainable", type=int, default=0,
                     help="requests in a second serving comparison at 0.8x the plain capacity (0 = skip)")
     ap.add_argument("--batch-eager", action="store_true",
-                    help="batched form without autotuner or hipGraph, each step launch timed (for profiling)")
+                    help="batched form without the autotuner, each launch of the path kernel timed (for profiling)")
     ap.add_argument("--batch-tuning", default="",
                     help="QUEUE,TW,TH,SPLIT[,REFILL] for --batch-eager (default: the context's default tuning), "
                          "e.g. the autotuner's pick from an unprofiled run")
@@ -67,7 +68,7 @@ def parse():
                     help="timed frames of the 1M-sphere traversal-bound scene (0 = skip)")
     ap.add_argument("--summarize", metavar="KERNEL",
                     help="no GPU: summarise rocprofv3 CSVs of profiled bench runs for KERNEL "
-                         "(e.g. 'k_wf_step<false, true, true>') into --out-md / --out-json")
+                         "(e.g. 'k_path_resolve<false>') into --out-md / --out-json")
     ap.add_argument("--trace-csv", help="kernel_stats.csv of the --kernel-trace --stats run")
     ap.add_argument("--fetch-csv", help="counter_collection.csv of the --pmc FETCH_SIZE run")
     ap.add_argument("--write-csv", help="counter_collection.csv of the --pmc WRITE_SIZE run")
@@ -180,7 +181,7 @@ def summarize_sq(a):
                     "lanes_active": round(lanes, 3), "source": os.path.relpath(a.out_md, ROOT)}
         rows.append(f"| `{k}` | {key} | {n} | {v['SQ_INSTS_VALU']:.4g} | {v['SQ_ACTIVE_INST_VALU']:.4g} | "
                     f"{v['SQ_THREAD_CYCLES_VALU']:.4g} | {v['SQ_BUSY_CYCLES']:.4g} | {issue:.2f} | {lanes:.2f} |")
-    md = [f"# rocprofv3 SQ counters of the step kernels", "", "Command (run from the repository root on the MI355X box):",
+    md = [f"# rocprofv3 SQ counters of the path kernels", "", "Command (run from the repository root on the MI355X box):",
           "", "```", *[c.strip() for c in a.commands.split(" ;; ") if c.strip()], "```", "",
           "Means per dispatch.  VALU issue capacity of a dispatch = SQ_BUSY_CYCLES / 32 shader engines x 1024 "
           "SIMDs / 4 cycles per wave64 VALU instruction; lanes active = SQ_THREAD_CYCLES_VALU / "
@@ -210,7 +211,7 @@ def _cpu_model():
 
 
 def _traffic(name, avg_ms):
-    """Measured HBM traffic and L2 figures of a step kernel from its committed
+    """Measured HBM traffic and L2 figures of a path kernel from its committed
     rocprofv3 summary (profiles/*.json), or Nones."""
     tf = os.path.join(ROOT, "profiles", name)
     if not os.path.exists(tf):
@@ -225,30 +226,29 @@ def _traffic(name, avg_ms):
 
 
 def _sq(key):
-    """Per-dispatch SQ counters of a step kernel on a workload (committed
-    rocprofv3 --pmc summary, profiles/step_kernel_sq.json), or None."""
-    tf = os.path.join(ROOT, "profiles", "step_kernel_sq.json")
+    """Per-dispatch SQ counters of a path kernel on a workload (committed
+    rocprofv3 --pmc summary, profiles/path_kernel_sq.json), or None."""
+    tf = os.path.join(ROOT, "profiles", "path_kernel_sq.json")
     if not os.path.exists(tf):
         return None
     return json.load(open(tf)).get(key)
 
 
-NODE_BYTES = 64  # one 4-wide node: four quantised child boxes and the child words
+NODE_BYTES = 48  # one 4-wide node as the kernels that do not count read it
 LDS_WIDE_NODES = 256  # a scene rendered alone with at most this many 4-wide nodes is staged in LDS
 
 
 def record_model_bytes(st, node_bytes=NODE_BYTES):
     """Algorithmic bytes summed over a counting launch under a per-segment
-    model with separate ray, hit and path records: the node bytes fetched (a
-    4-wide node is 64 B; a binary node pair would be 32 B), 16 B per sphere
-    tested, 16 B material per hit, and 144 B of queue traffic per segment
+    model with separate ray, hit and path records: the node bytes fetched,
+    16 B per sphere tested, 16 B material per hit, and 144 B of queue traffic per segment
     (ray record written and read, hit record written and read, path state
     read and written)."""
     return node_bytes * st.node_visits + 16 * st.sphere_tests + 16 * st.hits + 144 * st.segments
 
 
 def valu_roofline(sq, avg_ms):
-    """Useful VALU lane operations per second of a step kernel: the lanes
+    """Useful VALU lane operations per second of a path kernel: the lanes
     active over its VALU instructions per dispatch (SQ_THREAD_CYCLES_VALU, a
     function of the workload) over the live mean dispatch time, against the
     chip's lane throughput."""
@@ -291,9 +291,9 @@ def _cheapest(reqs, k):
 
 def run_batched(ctx, n_scenes, rmse_samples=2, eager=False, eager_tuning=""):
     """Batched form vs sequential plain launches of the same 64-scene mix.
-    eager: skip the autotuner and the hipGraph (default tuning, every step
-    launch timed with HIP events), the form rocprofv3 can profile; adds a
-    counting launch and the step kernel's algorithmic bytes."""
+    eager: skip the autotuner (default tuning, every launch of the path kernel
+    timed with HIP events); adds a counting launch and the path kernel's
+    algorithmic bytes."""
     from venusaur_amd import api, workloads
     from venusaur_amd.hipmem import synchronize
     reqs = workloads.batch_requests(n_scenes)
@@ -318,7 +318,7 @@ def run_batched(ctx, n_scenes, rmse_samples=2, eager=False, eager_tuning=""):
         items = [(scenes[r.scene_key], r.params) for r in reqs]
     else:
         tuning = api.autotune(ctx, items)  # untimed: picks queue capacity and tile shape
-    api.batch_launch(ctx, items, tuning=tuning)  # warm the engine and its graph
+    api.batch_launch(ctx, items, tuning=tuning)  # warm its buffers
     synchronize()
     t0 = time.perf_counter()
     st = api.batch_launch(ctx, items, tuning=tuning)
@@ -332,13 +332,13 @@ def run_batched(ctx, n_scenes, rmse_samples=2, eager=False, eager_tuning=""):
             c.flags = (c.flags & ~api.TIME_STAGES) | api.COUNT_VISITS
             counted.append((scenes[r.scene_key], c))
         cst = api.batch_launch(ctx, counted, tuning=tuning)
-        per_launch = step_bytes(cst) / st.trace_launches
-        step = {"kernel": "k_wf_step (multi-scene)", "launches": st.trace_launches, "avg_launch_ms": round(avg_ms, 4),
+        per_launch = path_bytes(cst) / st.trace_launches
+        step = {"kernel": "k_path (many scenes)", "launches": st.trace_launches, "avg_launch_ms": round(avg_ms, 4),
                 "algorithmic_bytes_per_launch": round(per_launch),
                 "algorithmic_gbs": round(per_launch / (avg_ms * 1e-3) / 1e9, 1),
                 "node_visits_per_segment": round(cst.node_visits / cst.segments, 2),
                 "sphere_tests_per_segment": round(cst.sphere_tests / cst.segments, 2)}
-        step.update(_traffic("step_kernel_traffic_batch64.json", avg_ms))
+        step.update(_traffic("path_kernel_traffic_batch64.json", avg_ms))
     same = all(_sha(r.accum_host()) == w for r, w in zip(reqs, want))
     rmse64 = {f"item{k}_{reqs[k].width}px_{reqs[k].spp}spp_{reqs[k].n_small}sph": _rmse_fp64(reqs[k])
               for k in _cheapest(reqs, rmse_samples)}
@@ -350,22 +350,20 @@ def run_batched(ctx, n_scenes, rmse_samples=2, eager=False, eager_tuning=""):
            "tuning": tuning.as_dict(), "lbvh_build_ms_mean": round(float(np.mean(build_ms)), 3),
            "rmse_vs_fp64_oracle": rmse64}
     if eager:
-        out["mode"] = "eager (no hipGraph, every step launch timed)"
-        out["step_kernel"] = step
+        out["mode"] = "eager (no autotuner, every launch of the path kernel timed)"
+        out["path_kernel"] = step
     for sc in scenes.values():
         sc.close()
     return out
 
 
-def step_bytes(st, node_bytes=NODE_BYTES):
-    """Algorithmic bytes of the step kernel (trace + miss/shade stages) for a
-    counting launch: per segment the 48 B path record read, 64 B per 4-wide
-    BVH node fetched, 16 B per sphere tested; per hit 36 B of sphere, material
-    and type re-read by the shade stage; per surviving path the 48 B record
-    written to the next queue; per ended path its 12 B radiance written to the
-    pass buffer."""
-    return (48 * st.segments + node_bytes * st.node_visits + 16 * st.sphere_tests + 36 * st.hits
-            + 48 * (st.segments - st.paths) + 12 * st.paths)
+def path_bytes(st, node_bytes=NODE_BYTES):
+    """Algorithmic bytes of the path kernel for a counting launch: per 4-wide
+    BVH node visited its bytes, 16 B per sphere tested; per hit 36 B of sphere,
+    material and type; per path 4 B of camera seed and 12 B of radiance.  (The
+    visits are those of the counting kernel, which tests spheres at once; the
+    kernels that queue the tests visit a few nodes more.)"""
+    return node_bytes * st.node_visits + 16 * st.sphere_tests + 36 * st.hits + 16 * st.paths
 
 
 def run_c2(ctx, frames, seed=2024):
@@ -396,24 +394,24 @@ def run_c2(ctx, frames, seed=2024):
     segs = sum(x.segments for x in stats)
     launches = sum(x.trace_launches for x in stats)
     avg_ms = sum(x.trace_ms for x in stats) / launches
-    per_launch = step_bytes(cst) * frames / launches
-    out = {"workload": f"{N} box spheres + ground (seed {seed}), {W}x{H} {SPP}spp depth {DEPTH} plain (wavefront)",
+    per_launch = path_bytes(cst) * frames / launches
+    out = {"workload": f"{N} box spheres + ground (seed {seed}), {W}x{H} {SPP}spp depth {DEPTH} plain (path)",
            "frames": frames, "value": round(segs / wall / 1e6, 2), "unit": "Mray-segments/s",
            "ms_per_frame": round(wall / frames * 1e3, 2), "segments_per_frame": int(stats[0].segments),
            "lbvh_build_ms": round(info.build_ms, 3), "bvh_depth": int(info.depth),
            "wide_nodes": int(info.num_wide_nodes), "wide_depth": int(info.wide_depth),
            "host_generate_s": round(t_gen, 3), "node_visits_per_segment": round(cst.node_visits / cst.segments, 2),
            "sphere_tests_per_segment": round(cst.sphere_tests / cst.segments, 2),
-           "step_kernel": {"launches": launches, "avg_launch_ms": round(avg_ms, 4),
+           "path_kernel": {"launches": launches, "avg_launch_ms": round(avg_ms, 4),
                            "algorithmic_bytes_per_launch": round(per_launch),
                            "algorithmic_gbs": round(per_launch / (avg_ms * 1e-3) / 1e9, 1),
                            "algorithmic_frac_of_hbm": round(per_launch / (avg_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
                            "record_model_frac_of_hbm": round(record_model_bytes(cst) * frames / launches
                                                                / (avg_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4)}}
-    out["step_kernel"].update(_traffic("step_kernel_traffic_c2.json", avg_ms))
+    out["path_kernel"].update(_traffic("path_kernel_traffic_c2.json", avg_ms))
     sq = _sq("box1M_1080p_64spp")
     if sq:
-        out["step_kernel"]["valu"] = valu_roofline(sq, avg_ms)
+        out["path_kernel"]["valu"] = valu_roofline(sq, avg_ms)
     acc.free()
     img.free()
     sc.close()
@@ -465,9 +463,8 @@ def run_served(ctx, n_requests, cap, load=3.0, rmse_samples=3, server_tuning=Non
     t_plain_end = time.perf_counter() - t_start
     want = [_sha(r.accum_host()) for r in reqs]
     # served: a client thread submits at the arrival times
-    # the server runs with the serving defaults (48M-ray queue, 8x8 tiles, queue
-    # split 4): its latency depends on the queue size, which the batch autotuner
-    # does not weigh
+    # the server runs with the serving defaults: its latency depends on how much
+    # work a launch takes, which the batch autotuner does not weigh
     srv = api.Server(ctx, hbm_budget_bytes=64 << 30, max_active=512,
                      tuning=server_tuning if server_tuning is not None else api.Tuning())
     ids = [None] * len(reqs)
@@ -561,7 +558,7 @@ def main():
     pc.flags = flags | api.COUNT_VISITS
     cst = scene.launch(pc)
 
-    # timed region: K full renders; trace launches bracketed by HIP events
+    # timed region: K full renders; launches of the path kernel bracketed by HIP events
     pt = api.LaunchParams.from_buffer_copy(p)
     pt.flags = flags | api.TIME_STAGES
     synchronize()
@@ -574,28 +571,27 @@ def main():
     value = segs / wall / 1e6
     gpu_acc = acc.download(np.float32, (H, W, 4))
 
-    # roofline of the step kernel (trace + miss/shade stages, the dominant
-    # kernel), from the algorithmic bytes of the counting launch; a scene of
-    # at most LDS_WIDE_NODES 4-wide nodes rendered alone is staged in LDS
+    # roofline of the path kernel (the dominant one), with the algorithmic
+    # bytes of the counting launch; a scene of at most LDS_WIDE_NODES 4-wide
+    # nodes rendered alone is staged in LDS
     seg_c, nv_c, ns_c = cst.segments, cst.node_visits, cst.sphere_tests
     lds_staged = scene.info().num_wide_nodes <= LDS_WIDE_NODES
     nb = NODE_BYTES
-    bytes_step = step_bytes(cst, nb)
+    bytes_step = path_bytes(cst, nb)
     trace_ms = sum(s.trace_ms for s in stats)
     launches = sum(s.trace_launches for s in stats)
     roof = None
-    if a.mode == "wavefront" and trace_ms > 0:
+    if a.mode == "path" and trace_ms > 0:
         per_launch_bytes = bytes_step * a.steps / launches
         avg_ms = trace_ms / launches
         achieved = per_launch_bytes / (avg_ms * 1e-3) / 1e9
         full = (W, H, SPP, DEPTH) == (1920, 1080, 256, 50)
         # measured HBM bytes per launch of the same kernel on the same
         # workload: rocprofv3 FETCH_SIZE + WRITE_SIZE, scaled by a copy
-        # kernel of known size (profiles/k_wf_step_book_1080p_256spp.md)
-        meas = _traffic("step_kernel_traffic.json", avg_ms) if full else {"traffic": None, "measured_hbm_gbs": None}
-        # the book scene's nodes are staged in LDS, so its node reads (64 B
-        # per visit) never reach HBM: the HBM-side algorithmic bytes leave
-        # them out
+        # kernel of known size (profiles/k_path_book_1080p_256spp.md)
+        meas = _traffic("path_kernel_traffic.json", avg_ms) if full else {"traffic": None, "measured_hbm_gbs": None}
+        # the book scene's nodes and spheres are staged in LDS, so its node
+        # reads never reach HBM: the HBM-side algorithmic bytes leave them out
         lds_nodes = cst.node_visits if lds_staged else 0
         hbm_alg = (bytes_step - NODE_BYTES * lds_nodes) * a.steps / launches
         svy = record_model_bytes(cst, nb) * a.steps / launches
@@ -616,12 +612,12 @@ def main():
                 if k in meas:
                     hbm[k] = meas[k]
         sq = _sq("book_1080p_256spp") if full else None
-        if sq:  # the step kernel issues VALU at capacity: that is its roof
+        if sq:  # the path kernel is bound by VALU issue: that is its roof
             roof = valu_roofline(sq, avg_ms)
         else:
             roof = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                     "frac": round(achieved / HBM_PEAK_GBS, 4)}
-        roof.update({"traffic": meas.get("traffic"), "kernel": "k_wf_step", "launches": launches,
+        roof.update({"traffic": meas.get("traffic"), "kernel": "k_path", "launches": launches,
                      "avg_launch_ms": round(avg_ms, 4),
                      "trace_share_of_step": round(trace_ms / (sum(s.render_ms for s in stats)), 3),
                      "bytes_per_segment": round(bytes_step / seg_c, 1),
