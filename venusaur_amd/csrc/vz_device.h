@@ -207,61 +207,57 @@ VZ_DEV bool hit_sphere(v3 o, v3 d, float tmin, float tmax, float4 sph, float& to
 }
 
 // ---- miss (RayTracer.cu:442-450) -----------------------------------------
-VZ_DEV v3 sky(v3 d)
+// u: the direction normalised.
+VZ_DEV v3 sky(v3 u)
 {
-    v3 u = normalize(d);
     float t = 0.5f * (u.y + 1.0f);
     return mk(1.0f + t * (0.5f - 1.0f), 1.0f + t * (0.7f - 1.0f), 1.0f + t * (1.0f - 1.0f));
 }
 
 // ---- materials (RayTracer.cu:272-440) --------------------------------------
-// mat = {albedo rgb, fuzz (metal) or ior (dielectric)}.  Returns false when
-// the path is absorbed.  att is the throughput multiplier.
-VZ_DEV bool scatter(uint32_t type, float4 mat, v3 d, v3 n, bool front, uint32_t& seed, v3& nd,
-                    v3& att)
+// In two halves, because a wave holds several materials and misses: what two of
+// them do is done once for the lanes of both.  Lambertian and metal draw a point
+// p in the unit sphere (metal's reflection draws nothing); the Lambertian
+// normalises it, the others d, as does a miss; metal and dielectric reflect.
+VZ_DEV v3 scatter_point(uint32_t type, uint32_t& seed)
 {
-    // Lambertian and metal both draw a point in the unit sphere (metal's
-    // reflection draws nothing) and metal and dielectric both normalise d:
-    // each is done once for the lanes that need it, so a wave holding several
-    // materials runs one rejection loop and one normalisation instead of two
-    v3 p = mk(0.0f, 0.0f, 0.0f);
-    if (type != 2u) p = in_unit_sphere(seed);
+    return type != 2u ? in_unit_sphere(seed) : mk(0.0f, 0.0f, 0.0f);
+}
+// u: p (Lambertian) or d normalised; param: fuzz (metal) or ior (dielectric).
+// Returns false when the path is absorbed.
+VZ_DEV bool scatter(uint32_t type, float param, v3 u, v3 p, v3 n, bool front, uint32_t& seed, v3& nd)
+{
     if (type == 0u) {
-        v3 sd = add(n, normalize(p));
-        if (near_zero(sd)) sd = n;
-        nd = sd;
-        att = mk(mat.x, mat.y, mat.z);
+        nd = add(n, u);
+        if (near_zero(nd)) nd = n;
         return true;
     }
-    const v3 u = normalize(d);
+    nd = reflect(u, n);
     if (type == 1u) {
-        v3 sd = add(reflect(u, n), scl(p, mat.w));
-        if (dot(sd, n) > 0.0f) {
-            nd = sd;
-            att = mk(mat.x, mat.y, mat.z);
-            return true;
-        }
-        return false;
-    } else {
-        float ir = mat.w;
-        float ratio = front ? recip_rn(ir) : ir;
-        float ct = fminf(dot(neg(u), n), 1.0f);
-        float st = sqrtf(1.0f - ct * ct);
-        bool cannot = ratio * st > 1.0f;
-        bool refl = cannot;
-        if (!cannot) {
-            float r0 = (1.0f - ratio) / (1.0f + ratio);
-            r0 = r0 * r0;
-            float x = 1.0f - ct;
-            float x2 = x * x;
-            float x5 = (x2 * x2) * x;
-            float sch = r0 + (1.0f - r0) * x5;
-            refl = sch > rnd(seed);
-        }
-        nd = refl ? reflect(u, n) : refract(u, n, ratio);
-        att = mk(1.0f, 1.0f, 1.0f);
-        return true;
+        nd = add(nd, scl(p, param));
+        return dot(nd, n) > 0.0f;
     }
+    const float ratio = front ? recip_rn(param) : param;
+    const float ct = fminf(dot(neg(u), n), 1.0f);
+    const float st = sqrtf(1.0f - ct * ct);
+    const bool cannot = ratio * st > 1.0f;
+    bool refl = cannot;
+    if (!cannot) {
+        float r0 = (1.0f - ratio) / (1.0f + ratio);
+        r0 = r0 * r0;
+        float x = 1.0f - ct;
+        float x2 = x * x;
+        float x5 = (x2 * x2) * x;
+        float sch = r0 + (1.0f - r0) * x5;
+        refl = sch > rnd(seed);
+    }
+    if (!refl) nd = refract(u, n, ratio);
+    return true;
+}
+// What a scattered ray's throughput is multiplied by.
+VZ_DEV v3 attenuation(uint32_t type, float4 mat)
+{
+    return type == 2u ? mk(1.0f, 1.0f, 1.0f) : mk(mat.x, mat.y, mat.z);
 }
 
 // ---- camera (RayTracer.cu:141-177) ---------------------------------------

@@ -35,7 +35,7 @@ __device__ __forceinline__ v3 trace_path(const SceneView& sc, v3 o, v3 d, uint32
     for (;;) {
         seg++;
         TraceResult r = closest_hit<S, COUNT>(sc, o, d, 0.001f, 1e16f, ln, lt, kMegaBlk, nv, ns);
-        if (r.leaf == 0xFFFFFFFFu) return mul(thr, sky(d));
+        if (r.leaf == 0xFFFFFFFFu) return mul(thr, sky(normalize(d)));
         if (depth <= 0) return mk(0.0f, 0.0f, 0.0f);
         float4 s = sc.spheres[r.leaf];
         uint32_t type = sc.leaf_info[r.leaf] >> 30;
@@ -44,12 +44,11 @@ __device__ __forceinline__ v3 trace_path(const SceneView& sc, v3 o, v3 d, uint32
         v3 n = scl(sub(p, mk(s.x, s.y, s.z)), recip_rn(s.w));
         bool front = dot(d, n) < 0.0f;
         if (!front) n = neg(n);
-        v3 nd, att;
-        if (!scatter(type, mat, d, n, front, seed, nd, att)) return mk(0.0f, 0.0f, 0.0f);
-        thr = mul(thr, att);
+        const v3 in = scatter_point(type, seed), u = normalize(type == 0u ? in : d);
+        if (!scatter(type, mat.w, u, in, n, front, seed, d)) return mk(0.0f, 0.0f, 0.0f);
+        thr = mul(thr, attenuation(type, mat));
         depth -= 1;
         o = p;
-        d = nd;
     }
 }
 

@@ -324,12 +324,16 @@ __global__ void __launch_bounds__(path_threads(SRC)) __attribute__((amdgpu_waves
             continue;
         }
         if (start) {  // new paths and scattered ones alike
-            if constexpr (LDSN) tr.init(pb, tr.o, tr.d, 0.001f, 1e16f);
+            if constexpr (LDSN) tr.begin(tr.o, tr.d, 0.001f, 1e16f);
             else if constexpr (COUNT) tdone = tr.init(sc, tr.o, tr.d, 0.001f, 1e16f, ns);
-            else tdone = tr.init(sc, sh, tr.o, tr.d, 0.001f, 1e16f);
+            else tdone = tr.begin(sc, sh, tr.o, tr.d, 0.001f, 1e16f);
             if (LDSN) tdone = false;
             start = false;
         }
+        // for the lanes still tracing as well: the wave executes this for the
+        // new rays anyway, and need not keep the others' through the shading
+        if constexpr (LDSN) tr.derive(pb);
+        else if constexpr (!COUNT) tr.derive();
         uint64_t busy = __ballot(active && !tdone);
         while (busy) {
             if (active && !tdone) {
@@ -377,29 +381,35 @@ __global__ void __launch_bounds__(path_threads(SRC)) __attribute__((amdgpu_waves
         if (fin) {
             v3 L = mk(0.0f, 0.0f, 0.0f);
             bool ended = true;
-            if (tr.bleaf == 0xFFFFFFFFu) {
-                // miss (RayTracer.cu:442-450)
-                L = mul(thr, sky(tr.d));
-            } else if (depth > 0u) {
-                // shade (RayTracer.cu:272-440)
+            // shade (RayTracer.cu:272-440) or miss (RayTracer.cu:442-450); a
+            // wave with both normalises once
+            const bool miss = tr.bleaf == 0xFFFFFFFFu, shade = !miss && depth > 0u;
+            uint32_t type = 0;
+            float param = 0.0f;
+            bool front = false;
+            v3 n = mk(0.0f, 0.0f, 0.0f), p = n, u = tr.d;
+            if (shade) {
                 float4 s;
                 if constexpr (LDSN) s = sh.spheres[tr.bleaf];
                 else s = ldg(sc.sphere_array() + tr.bleaf);
-                const uint32_t type = ldg(sc.info_array() + tr.bleaf) >> 30;
+                type = ldg(sc.info_array() + tr.bleaf) >> 30;
                 const float4 mat = ldg(sc.mat_array() + tr.bleaf);
-                const v3 pos = add(tr.o, scl(tr.d, tr.best));
-                v3 n = scl(sub(pos, mk(s.x, s.y, s.z)), recip_rn(s.w));
-                const bool front = dot(tr.d, n) < 0.0f;
+                tr.o = add(tr.o, scl(tr.d, tr.best));
+                n = scl(sub(tr.o, mk(s.x, s.y, s.z)), recip_rn(s.w));
+                front = dot(tr.d, n) < 0.0f;
                 if (!front) n = neg(n);
-                v3 att, nd;
-                if (scatter(type, mat, tr.d, n, front, seed, nd, att)) {
-                    thr = mul(thr, att);
-                    depth--;
-                    ended = false;
-                    tr.o = pos;
-                    tr.d = nd;
-                    start = true;
-                }
+                thr = mul(thr, attenuation(type, mat));  // (of no use to a path that ends here)
+                param = mat.w;
+                p = scatter_point(type, seed);
+                if (type == 0u) u = p;
+            }
+            u = normalize(u);
+            if (miss) {
+                L = mul(thr, sky(u));
+            } else if (shade && scatter(type, param, u, p, n, front, seed, tr.d)) {
+                depth--;
+                ended = false;
+                start = true;
             }
             if (ended) {
                 float* q = G.rad + 3 * (size_t)slot;

@@ -146,9 +146,14 @@ k_trace_hits(SceneView view, const vzRay* __restrict__ rays, uint32_t n, vzHit* 
                 mine = base + cur + rk;
                 const float4* rp = reinterpret_cast<const float4*>(rays + mine);
                 const float4 a = ldg(rp), b = ldg(rp + 1);
-                if constexpr (LDSN) tr.init(pb, mk(a.x, a.y, a.z), mk(b.x, b.y, b.z), a.w, b.w);
-                else tdone = tr.init(sc, sh, mk(a.x, a.y, a.z), mk(b.x, b.y, b.z), a.w, b.w);
-                if (LDSN) tdone = false;
+                if constexpr (LDSN) {
+                    tr.begin(mk(a.x, a.y, a.z), mk(b.x, b.y, b.z), a.w, b.w);
+                    tr.derive(pb);
+                    tdone = false;
+                } else {
+                    tdone = tr.begin(sc, sh, mk(a.x, a.y, a.z), mk(b.x, b.y, b.z), a.w, b.w);
+                    tr.derive();
+                }
                 active = true;
             }
             cur += take;

@@ -122,6 +122,18 @@ struct LdsTraversal {
     float tmin, best;
     uint32_t bleaf, node, sp, npend;
 
+    VZ_DEV void begin(v3 o_, v3 d_, float tmin_, float tmax_)
+    {
+        o = o_;
+        d = d_;
+        tmin = tmin_;
+        best = tmax_;
+        bleaf = 0xFFFFFFFFu;
+        node = sp = npend = 0u;
+    }
+
+    // What follows from the ray: after begin(), and wherever it is cheaper than
+    // keeping it (k_path).
     // Plane distances are fma(p, inv, -o inv), near ones moved down by e and
     // far ones up by 2 e, e = (Pmax + |o|) |inv| 2^-20.  The exact form
     // fl(fl(p - o) inv) and the unmoved fma differ by less than 5.2 u (Pmax +
@@ -130,14 +142,8 @@ struct LdsTraversal {
     // (16 u more): the test passes whenever the sphere gate's does.  An
     // overflow of a term leaves an infinity or a NaN that min and max drop:
     // the slot passes.
-    VZ_DEV void init(const PlaneBound& pb, v3 o_, v3 d_, float tmin_, float tmax_)
+    VZ_DEV void derive(const PlaneBound& pb)
     {
-        o = o_;
-        d = d_;
-        tmin = tmin_;
-        best = tmax_;
-        bleaf = 0xFFFFFFFFu;
-        node = sp = npend = 0u;
         const bool ordinary = ray_inverse(d, inv);
         const float oo[3] = {o.x, o.y, o.z};
 #pragma unroll

@@ -59,7 +59,7 @@ struct MemTraversal {
 
     // Returns true when there is nothing to walk: a single sphere, queued.
     template <class Scene>
-    VZ_DEV bool init(const Scene& sc, MemScene<NT>& sh, v3 o_, v3 d_, float tmin_, float tmax_)
+    VZ_DEV bool begin(const Scene& sc, MemScene<NT>& sh, v3 o_, v3 d_, float tmin_, float tmax_)
     {
         o = o_;
         d = d_;
@@ -67,11 +67,14 @@ struct MemTraversal {
         best = tmax_;
         bleaf = kMiss;
         node = sp = npend = 0u;
-        ray_inverse(d, inv);
         if (sc.node_array() != nullptr) return false;
         queue(sh, 0u, 1u);
         return true;
     }
+
+    // What follows from the ray: after begin(), and wherever it is cheaper than
+    // keeping it (k_path).
+    VZ_DEV void derive() { ray_inverse(d, inv); }
 
     // Tests the queued leaves; keeps the lexicographic minimum of (t, prim).
     template <class Scene>
