@@ -261,8 +261,16 @@ struct LdsTraversal {
         for (;;) {
             if (sp == 0u) return true;
             sp -= kRow;
-            const uint32_t e =
-                sp < kLdsStack * kRow ? *slot(sh, sp) : ov.w[min(sp / kRow - kLdsStack, kWideOverflow - 1u)];
+            uint32_t e;
+            if (sp < kLdsStack * kRow) {
+                e = *slot(sh, sp);
+                // kept apart from the other load: the two become one flat load
+                // otherwise, and every pop waits for the memory pipe (1080p
+                // book frame 55.6 ms against 56.2)
+                asm volatile("" : "+v"(e));
+            } else {
+                e = ov.w[min(sp / kRow - kLdsStack, kWideOverflow - 1u)];
+            }
             node = e & 0xFFF0u;
             if (__uint_as_float(e & kLdsKeyMask) <= (ANYT ? fmaxf(lim, 0.0f) : lim)) return false;
         }
