@@ -29,8 +29,8 @@
 // at 256 samples 115.2 -> 78.6 ms, a million spheres at 1080p and 64 samples
 // 241 -> 187 ms, 512x512 at 2048 samples in double 355 -> 135 ms, 400x225 at 16
 // samples 2.80 -> 1.12 ms; with the traversals of vz_traverse_lds.h and
-// vz_traverse_mem.h, queued sphere tests and the counters below 58.4 ms, 143
-// ms, 105 ms and 0.69 ms; images bit for bit the same.  What bounds it is VALU
+// vz_traverse_mem.h, queued sphere tests, shared shading and the counters below
+// 55.6 ms, 134 ms, 102 ms and 0.66 ms; images bit for bit the same.  What bounds it is VALU
 // issue at half the lanes with the scene in LDS, the L1 and the latency of
 // node loads as well with it in memory, and the longest path at the end of a
 // small frame.  k_path_seeds and k_path_resolve are under 1% each of the
