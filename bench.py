@@ -125,7 +125,7 @@ def summarize(a):
     ffac, wfac = f["copy"][0] / true_kib, w["copy"][0] / true_kib
     kf, kw = statistics.mean(f["kern"]), statistics.mean(w["kern"])
     fetch_b, write_b = kf * 1024 / ffac, kw * 1024 / wfac
-    md = [f"# rocprofv3 summary: {kern}", "", "Commands (run from the repository root on the MI355X box):", "",
+    md = [f"# rocprofv3 summary: {kern}", "", "Commands (run from the repository root on an MI355X):", "",
           "```", *[c.strip() for c in a.commands.split(" ;; ") if c.strip()], "```", "",
           "## Kernel time (kernel trace, --stats)", "", *table, "",
           "## HBM traffic of the dominant kernel (PMC)", "",
@@ -181,7 +181,7 @@ def summarize_sq(a):
                     "lanes_active": round(lanes, 3), "source": os.path.relpath(a.out_md, ROOT)}
         rows.append(f"| `{k}` | {key} | {n} | {v['SQ_INSTS_VALU']:.4g} | {v['SQ_ACTIVE_INST_VALU']:.4g} | "
                     f"{v['SQ_THREAD_CYCLES_VALU']:.4g} | {v['SQ_BUSY_CYCLES']:.4g} | {issue:.2f} | {lanes:.2f} |")
-    md = [f"# rocprofv3 SQ counters of the path kernels", "", "Command (run from the repository root on the MI355X box):",
+    md = [f"# rocprofv3 SQ counters of the path kernels", "", "Command (run from the repository root on an MI355X):",
           "", "```", *[c.strip() for c in a.commands.split(" ;; ") if c.strip()], "```", "",
           "Means per dispatch.  VALU issue capacity of a dispatch = SQ_BUSY_CYCLES / 32 shader engines x 1024 "
           "SIMDs / 4 cycles per wave64 VALU instruction; lanes active = SQ_THREAD_CYCLES_VALU / "
