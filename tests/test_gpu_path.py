@@ -192,3 +192,23 @@ def test_uneven_tree(ctx, n):
         out.append(h.download(api.HIT_DT))
     assert out[0].tobytes() == out[1].tobytes() == O.trace_brute(s, rays).tobytes()
     sc.close()
+
+
+# launches of few paths, whose tiles' passes are split among waves: from one
+# path a wave to whole tiles, plain and in a batch
+@pytest.mark.parametrize("kind", ["book", "mem"])
+@pytest.mark.parametrize("w,h,spp", [(2, 2, 1), (8, 8, 1), (64, 36, 2), (57, 31, 5), (100, 60, 4), (128, 128, 12),
+                                     (160, 160, 13)])
+def test_launches_of_few_paths(ctx, book, kind, w, h, spp):
+    say(f"case: few paths {kind} {w}x{h} spp={spp}")
+    (s, m), look = _scene(kind, book)
+    cam = look(w, h)
+    sc = api.Scene(ctx, s, m)
+    want, _, ost = O.render(s, m, oracle_params(w, h, spp, 12, cam), bvh=O.BVH(s))
+    tgt = GpuTarget(w, h)
+    st = sc.launch(tgt.bind(gpu_params(w, h, spp, 12, cam)))
+    assert np.array_equal(tgt.accum_host(), want) and st.segments == ost.segments
+    two = [GpuTarget(w, h), GpuTarget(w, h)]
+    st = api.batch_launch(ctx, [(sc, t.bind(gpu_params(w, h, spp, 12, cam))) for t in two])
+    assert all(np.array_equal(t.accum_host(), want) for t in two) and st.segments == 2 * ost.segments
+    sc.close()

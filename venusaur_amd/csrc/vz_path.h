@@ -31,6 +31,7 @@ struct PathReq {               // one request of a launch, read by scalar loads
     uint32_t tiles_x, npad;    // npad: pixels of all tiles
     uint32_t s0, ns;           // the launch's passes [s0, s0 + ns)
     uint32_t spu, groups;      // passes per unit, units per tile
+    uint32_t parts;            // log2 of the units that share a pass of a tile (spu 1)
     uint32_t unit0, pix0, slot0;  // its first unit, padded pixel and path in the launch
     uint32_t* camseed;         // npad: camera seed of the next launch's first pass (ns < spp)
     void* sums;                // 3 * npad float or double, carried between launches (ns < spp)
