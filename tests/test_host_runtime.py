@@ -1,0 +1,76 @@
+"""What libvz.so does on the host, without a GPU: run in a process of its own
+over tests/host_hip, a stand-in for the HIP runtime whose device memory is
+host memory and whose kernels do nothing."""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+PRELUDE = """
+import ctypes as C, sys
+hip = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+sys.path.insert(0, sys.argv[2])
+for f in ("host_hip_used", "host_hip_peak", "host_hip_log"):
+    getattr(hip, f).restype = C.c_size_t
+hip.host_hip_limit.argtypes = [C.c_size_t]
+FREED = C.CFUNCTYPE(None)
+hip.host_hip_on_free.argtypes = [FREED, C.c_size_t]
+import time
+import numpy as np
+from venusaur_amd import api
+MB = 1 << 20
+
+def calls():
+    buf = C.create_string_buffer(hip.host_hip_log(None, 0) + 1)
+    hip.host_hip_log(buf, len(buf))
+    return buf.value.decode().split("\\n")[:-1]
+
+def params(w, h, spp, flags=0):
+    p = api.launch_params(w, h, spp, 8, [13, 2, 3], [0, 0, 0], 20.0, 0.1, 10.0, flags=flags)
+    p.accum = 256  # no kernel runs: never read
+    return p
+
+ctx = api.Context(0)
+scene = api.Scene(ctx, *api.box_scene(500, 1))
+"""
+
+
+@pytest.fixture(scope="module")
+def stand_in(tmp_path_factory):
+    cxx = shutil.which("g++")
+    if cxx is None:
+        pytest.skip("no g++")
+    out = str(tmp_path_factory.mktemp("host_hip") / "libhost_hip.so")
+    subprocess.run([cxx, "-std=c++17", "-O1", "-Wall", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__",
+                    "-I/opt/rocm/include", os.path.join(HERE, "host_hip", "host_hip.cpp"), "-o", out], check=True)
+    return out
+
+
+def run(stand_in, code):
+    r = subprocess.run([sys.executable, "-c", PRELUDE + code, stand_in, ROOT], capture_output=True, text=True,
+                       timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_context_cannot_go_while_a_scene_gives_back_its_memory(stand_in):
+    """A scene's block returns to its context's pool: until that is done the
+    context counts the scene as alive.  4e6 spheres are above what the pool
+    keeps, so their block is freed inside vzSceneDestroy; there, vzDestroy
+    (another thread's, say) has to refuse."""
+    run(stand_in, """
+scene.close()
+big = api.Scene(ctx, *api.box_scene(4_000_000, 1))
+seen = []
+cb = FREED(lambda: seen.append(api.lib().vzDestroy(ctx.h)))
+hip.host_hip_on_free(cb, 1 << 30)
+assert api.lib().vzSceneDestroy(big.h) == 0
+assert seen == [1], seen
+hip.host_hip_on_free(FREED(), 0)
+assert api.lib().vzDestroy(ctx.h) == 0
+ctx.h = big.h = None
+""")

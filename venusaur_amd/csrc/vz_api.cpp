@@ -246,9 +246,10 @@ vzStatus vzSceneDestroy(vzScene scene)
                                                      " queued or running server request(s)");
     (void)hipSetDevice(scene->ctx->device);
     (void)hipDeviceSynchronize();
-    scene->ctx->live_scenes--;
-    lbvh_free(scene);
+    vzContext ctx = scene->ctx;
+    lbvh_free(scene);  // gives memory back to the context, which has to be there
     delete scene;
+    ctx->live_scenes--;
     return VZ_SUCCESS;
 }
 
