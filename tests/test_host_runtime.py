@@ -74,3 +74,32 @@ hip.host_hip_on_free(FREED(), 0)
 assert api.lib().vzDestroy(ctx.h) == 0
 ctx.h = big.h = None
 """)
+
+
+def test_little_memory_makes_more_chunks(stand_in):
+    """2048x2048 at 131 samples in double takes 44 passes at a time (2.95 GB)
+    and 117 MB of sums.  With room for the first alone the launch goes on in
+    smaller chunks, for which the larger buffer is given back."""
+    run(stand_in, """
+p = params(2048, 2048, 131, api.ACCUM_FP64)
+base = hip.host_hip_used()
+hip.host_hip_limit(base + 2900 * MB)
+for _ in range(2):
+    st = scene.launch(p)
+    assert st.iterations == 6, st.iterations   # 22 passes each
+    assert hip.host_hip_used() <= base + 2900 * MB
+other = api.Context(0)
+s2 = api.Scene(other, *api.box_scene(500, 1))
+hip.host_hip_limit(hip.host_hip_used() + 250 * MB)
+st = s2.launch(p)
+assert st.iterations == 66, st.iterations      # two passes (134 MB) at a time
+third = api.Context(0)
+hip.host_hip_limit(1 << 60)
+s3 = api.Scene(third, *api.box_scene(500, 1))
+hip.host_hip_limit(hip.host_hip_used() + 100 * MB)
+try:
+    s3.launch(p)
+    raise SystemExit("not refused")
+except api.VzError as e:
+    assert e.status == 2
+""")

@@ -523,13 +523,19 @@ __global__ void __launch_bounds__(kBlk) k_path_resolve(PathGroup G, PathReq one)
 
 inline uint64_t align256(uint64_t v) { return (v + 255) & ~255ull; }
 
+// Gives back a buffer that nothing in flight uses.
+void drop(char** p, size_t* have)
+{
+    if (*p) (void)hipFree(*p);
+    *p = nullptr;
+    *have = 0;
+}
+
 // Grows a buffer that nothing in flight uses.
 bool grow(vzContext ctx, char** p, size_t* have, size_t need)
 {
     if (*have >= need) return true;
-    if (*p) (void)hipFree(*p);
-    *p = nullptr;
-    *have = 0;
+    drop(p, have);
     if (hipMalloc((void**)p, need) != hipSuccess) {
         (void)hipGetLastError();
         ctx->scene_blocks.trim();
@@ -771,6 +777,10 @@ vzStatus path_enqueue_one(PathWork* w, PathSlot& s, const PathItem& item, const 
         if (rs == VZ_SUCCESS && grow(s.ctx, &s.pixels, &s.pixels_bytes, pix)) break;
         if (chunk == 1u) return rs != VZ_SUCCESS ? rs : set_error(VZ_ERROR_OUT_OF_MEMORY, "launch buffers do not fit");
         chunk = split((chunk + 1) / 2);
+        // neither buffer is kept larger than the smaller chunk needs: the one
+        // that fitted would go on taking the room of the one that did not
+        drop(&s.paths, &s.paths_bytes);
+        drop(&s.pixels, &s.pixels_bytes);
     }
     const bool lds = fits_lds(item.scene) && !opt.count;
     const uint32_t resident = lds ? w->grid_lds : w->grid_mem;
