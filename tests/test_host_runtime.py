@@ -103,3 +103,27 @@ try:
 except api.VzError as e:
     assert e.status == 2
 """)
+
+
+def test_render_time_holds_no_allocation(stand_in):
+    """render_ms runs between two events: the buffers of a launch, of a
+    batch's groups and of its large items are there before the first."""
+    run(stand_in, """
+def check(what):
+    log = calls()
+    first = log.index("record")
+    assert any("k_path" in c for c in log[first:]), what
+    late = [c for c in log[first:] if c.startswith(("malloc", "free", "refuse"))]
+    assert late == [], (what, late)
+
+calls()
+scene.launch(params(64, 36, 2))
+check("a first launch")
+scene.launch(params(2048, 2048, 131, api.ACCUM_FP64))
+check("a launch of several chunks")
+t = api.Tuning()
+t.queue_capacity = 1 << 20                     # 256 MB: 16M paths
+big = [params(1024, 1024, 40), params(2048, 1024, 12, api.ACCUM_FP64), params(4096, 4096, 2)]
+api.batch_launch(ctx, [(scene, params(512, 512, 4)), (scene, big[0]), (scene, big[1]), (scene, big[2])], tuning=t)
+check("a batch with large items")
+""")

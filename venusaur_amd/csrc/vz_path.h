@@ -97,9 +97,15 @@ uint64_t path_count(const vzLaunchParams& p, const PathOptions& opt);
 // Makes room in the slot for launches of up to `paths` paths; nothing on its
 // stream may still run.
 vzStatus slot_reserve(PathSlot& s, uint64_t paths);
-// Enqueues one request, in as many launches as its passes need within
-// `budget` bytes.  add: its totals add to those of the slot's launch before.
-vzStatus path_enqueue_one(PathWork* w, PathSlot& s, const PathItem& item, const PathOptions& opt, uint64_t budget,
+// Makes room for a request's launches, of *passes passes each: as many as fit
+// *budget bytes, fewer where the memory is not there (*budget is then what
+// they take), with room for at least `least` paths.  Nothing on the slot's
+// stream may still run.
+vzStatus path_reserve_one(PathSlot& s, const PathItem& item, const PathOptions& opt, uint64_t* budget, uint64_t least,
+                          uint32_t* passes);
+// Enqueues one request in launches of `passes` passes.  add: its totals add to
+// those of the slot's launch before.
+vzStatus path_enqueue_one(PathWork* w, PathSlot& s, const PathItem& item, const PathOptions& opt, uint32_t passes,
                           bool add, hipStream_t st, uint32_t* launches);
 // Enqueues n requests as one launch (their paths fit the slot).
 vzStatus path_enqueue_many(PathWork* w, PathSlot& s, const PathItem* const* items, uint32_t n, const PathOptions& opt,

@@ -523,6 +523,14 @@ __global__ void __launch_bounds__(kBlk) k_path_resolve(PathGroup G, PathReq one)
 
 inline uint64_t align256(uint64_t v) { return (v + 255) & ~255ull; }
 
+// What a request's launches carry from one to the next: the sums of every
+// padded pixel, then the camera seeds.
+uint64_t sum_bytes(const vzLaunchParams& p, uint64_t npad)
+{
+    return align256(((p.flags & VZ_ACCUM_FP64) ? 24ull : 12ull) * npad);
+}
+uint64_t carry_bytes(const vzLaunchParams& p, uint64_t npad) { return sum_bytes(p, npad) + 4ull * npad; }
+
 // Gives back a buffer that nothing in flight uses.
 void drop(char** p, size_t* have)
 {
@@ -755,46 +763,57 @@ vzStatus slot_reserve(PathSlot& s, uint64_t paths)
     return VZ_SUCCESS;
 }
 
-vzStatus path_enqueue_one(PathWork* w, PathSlot& s, const PathItem& item, const PathOptions& opt, uint64_t budget,
-                          bool add, hipStream_t st, uint32_t* launches)
+vzStatus path_reserve_one(PathSlot& s, const PathItem& item, const PathOptions& opt, uint64_t* budget, uint64_t least,
+                          uint32_t* passes)
 {
     const uint64_t ntiles = tile_count(item.params, tile_lw(item.params, opt));
     if (ntiles * kTile > 0xFFFFFF00ull) return set_error(VZ_ERROR_CAPACITY, "image too large");
-    PathReq A;
-    fill_request(A, item, opt);
+    const uint64_t npad = ntiles * kTile, spp = item.params.samples_per_pixel;
     // the passes in as few equal chunks as the budget allows; less memory
     // than that makes more chunks
     auto split = [&](uint64_t most) {
-        const uint64_t chunks = (A.spp + most - 1) / most;
-        return (uint32_t)((A.spp + chunks - 1) / chunks);
+        const uint64_t chunks = (spp + most - 1) / most;
+        return (spp + chunks - 1) / chunks;
     };
-    budget = std::min(budget, kMaxSlotBudget);
-    uint32_t chunk = split(std::max<uint64_t>(1, std::min<uint64_t>(A.spp, budget / (kPathBytes * A.npad))));
-    const uint64_t sum_bytes = align256((A.fp64 ? 24ull : 12ull) * A.npad);
+    *budget = std::min(*budget, kMaxSlotBudget);
+    uint64_t chunk = split(std::max<uint64_t>(1, std::min<uint64_t>(spp, *budget / (kPathBytes * npad))));
     for (;;) {
-        const uint64_t pix = chunk < A.spp ? sum_bytes + 4ull * A.npad : 0ull;
-        const vzStatus rs = slot_reserve(s, (uint64_t)A.npad * chunk);
+        const uint64_t pix = chunk < spp ? carry_bytes(item.params, npad) : 0ull;
+        const vzStatus rs = slot_reserve(s, std::max(npad * chunk, least));
         if (rs == VZ_SUCCESS && grow(s.ctx, &s.pixels, &s.pixels_bytes, pix)) break;
         if (chunk == 1u) return rs != VZ_SUCCESS ? rs : set_error(VZ_ERROR_OUT_OF_MEMORY, "launch buffers do not fit");
         chunk = split((chunk + 1) / 2);
+        *budget = chunk * npad * kPathBytes;
         // neither buffer is kept larger than the smaller chunk needs: the one
         // that fitted would go on taking the room of the one that did not
         drop(&s.paths, &s.paths_bytes);
         drop(&s.pixels, &s.pixels_bytes);
     }
+    *passes = (uint32_t)chunk;
+    return VZ_SUCCESS;
+}
+
+vzStatus path_enqueue_one(PathWork* w, PathSlot& s, const PathItem& item, const PathOptions& opt, uint32_t passes,
+                          bool add, hipStream_t st, uint32_t* launches)
+{
+    PathReq A;
+    fill_request(A, item, opt);
+    const uint64_t ntiles = A.npad / kTile;
+    if ((uint64_t)A.npad * passes * kPathBytes + 256 > s.paths_bytes)
+        return set_error(VZ_ERROR_INTERNAL, "launch larger than its slot");
     const bool lds = fits_lds(item.scene) && !opt.count;
     const uint32_t resident = lds ? w->grid_lds : w->grid_mem;
     const uint32_t waves = resident * (lds ? kLdsBlk : kMemBlk) / 64;
     PathGroup G;
     fill_group(G, s, add);
     G.seeds = (uint32_t*)s.paths;
-    G.rad = (float*)(s.paths + align256(4ull * A.npad * chunk));
+    G.rad = (float*)(s.paths + align256(4ull * A.npad * passes));
     G.pixels = A.npad;
     G.refill = refill_of(opt, lds ? kRefillLds : kRefillGlobal);
     A.sums = s.pixels;
-    A.camseed = (uint32_t*)(s.pixels + sum_bytes);
-    for (A.s0 = 0; A.s0 < A.spp; A.s0 += chunk) {
-        A.ns = std::min(chunk, A.spp - A.s0);
+    A.camseed = (uint32_t*)(s.pixels + sum_bytes(item.params, A.npad));
+    for (A.s0 = 0; A.s0 < A.spp; A.s0 += passes) {
+        A.ns = std::min(passes, A.spp - A.s0);
         A.spu = unit_passes(ntiles * A.ns, waves);
         A.parts = unit_parts(ntiles * A.ns, waves);
         A.groups = ((A.ns + A.spu - 1) / A.spu) << A.parts;
@@ -888,9 +907,12 @@ vzStatus path_launch(vzContext ctx, const PathItem& item, hipStream_t st, RunRes
     if (item.params.flags & VZ_TIME_STAGES) opt.events = &ev;
     *res = RunResult();
     res->paths = (unsigned long long)item.params.width * item.params.height * item.params.samples_per_pixel;
+    uint64_t budget = kPlainBudget;
+    uint32_t passes = 0;
+    VZ_TRY(path_reserve_one(w->plain, item, opt, &budget, 0, &passes));
     auto enqueue = [&]() -> vzStatus {
         VZ_HIP_TRY(hipEventRecord(w->t0.e, st));
-        VZ_TRY(path_enqueue_one(w, w->plain, item, opt, kPlainBudget, false, st, &res->iterations));
+        VZ_TRY(path_enqueue_one(w, w->plain, item, opt, passes, false, st, &res->iterations));
         VZ_HIP_TRY(hipEventRecord(w->t1.e, st));
         return VZ_SUCCESS;
     };
@@ -929,7 +951,6 @@ vzStatus path_batch(vzContext ctx, const std::vector<PathItem>& items, const vzT
     if (slot.paths_bytes > budget + 256) slot.free();  // a smaller tuning gives memory back
     VZ_TRY(slot.init(ctx, true));
     slot.used = 0;
-    // small items first, so that the slot has its size before anything runs
     std::vector<std::vector<const PathItem*>> groups(1);
     std::vector<const PathItem*> large;
     uint64_t open = 0, need = 0;
@@ -947,7 +968,15 @@ vzStatus path_batch(vzContext ctx, const std::vector<PathItem>& items, const vzT
         open += n;
         need = std::max(need, open);
     }
+    // the buffers before anything runs; an item that has to make do with less
+    // leaves no more to the others
     if (need) VZ_TRY(slot_reserve(slot, need));
+    std::vector<uint32_t> passes(large.size());
+    for (uint64_t most = budget, before = 0; most != before;) {
+        before = most;
+        for (size_t i = 0; i < large.size(); i++)
+            VZ_TRY(path_reserve_one(slot, *large[i], opt, &most, need, &passes[i]));
+    }
     auto enqueue = [&]() -> vzStatus {
         VZ_HIP_TRY(hipEventRecord(w->t0.e, st));
         for (const auto& g : groups) {
@@ -955,10 +984,8 @@ vzStatus path_batch(vzContext ctx, const std::vector<PathItem>& items, const vzT
             VZ_TRY(path_enqueue_many(w, slot, g.data(), (uint32_t)g.size(), opt, res->iterations != 0, st));
             res->iterations++;
         }
-        for (const PathItem* it : large) {
-            VZ_HIP_TRY(hipStreamSynchronize(st));  // its buffers may have to grow
-            VZ_TRY(path_enqueue_one(w, slot, *it, opt, budget, res->iterations != 0, st, &res->iterations));
-        }
+        for (size_t i = 0; i < large.size(); i++)
+            VZ_TRY(path_enqueue_one(w, slot, *large[i], opt, passes[i], res->iterations != 0, st, &res->iterations));
         VZ_HIP_TRY(hipEventRecord(w->t1.e, st));
         return VZ_SUCCESS;
     };

@@ -158,7 +158,12 @@ vzStatus vzServer_st::start(Flight& f, const std::vector<Pending>& group)
     for (const PathItem& it : items) paths += path_count(it.params, opt);
     f.slot.used = 0;
     f.large = group.size() == 1 && paths * kPathBytes > slot_budget;
-    if (f.large) return path_enqueue_one(work, f.slot, items[0], opt, slot_budget, false, f.stream, nullptr);
+    if (f.large) {
+        uint64_t budget = slot_budget;
+        uint32_t passes = 0;
+        VZ_TRY(path_reserve_one(f.slot, items[0], opt, &budget, 0, &passes));
+        return path_enqueue_one(work, f.slot, items[0], opt, passes, false, f.stream, nullptr);
+    }
     VZ_TRY(slot_reserve(f.slot, paths));
     return path_enqueue_many(work, f.slot, ptr.data(), (uint32_t)ptr.size(), opt, false, f.stream);
 }
