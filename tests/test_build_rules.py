@@ -1,4 +1,5 @@
-"""The library's Makefile rebuilds what includes a changed header."""
+"""The library's Makefile and sources: a changed header rebuilds what includes
+it; indices that outgrow 32 bits are formed in 64."""
 import os
 import re
 import shutil
@@ -36,3 +37,14 @@ def test_a_changed_header_rebuilds_every_object_that_includes_it(tmp_path, heade
     users = [f for f in sources if header in _includes(f)]
     assert users
     assert [f for f in users if f"-c {f}" not in told] == []
+
+
+def test_node_box_indices_are_64_bit():
+    """Six floats a node: from 715,827,883 nodes on (a scene may have 2^30
+    spheres) node * 6 no longer fits 32 bits.  Every box is found through
+    node_box, which multiplies in 64."""
+    with open(os.path.join(CSRC, "vz_lbvh.hip")) as f:
+        text = f.read()
+    helper = re.search(r"node_box\(.*?\)\s*\{(.*?)\}", text, re.S).group(1)
+    assert "(size_t)node * 6" in helper
+    assert re.findall(r"boxes\s*(?:\[|\+)[^;\n]*\*\s*6", text.replace(helper, "")) == []

@@ -980,6 +980,14 @@ __device__ __forceinline__ void leaf_box(const float4 sp, float* b)
     b[3] = sp.x + r; b[4] = sp.y + r; b[5] = sp.z + r;
 }
 
+// A node's box (lo, hi), six floats: in 64 bits, since node * 6 outgrows 32
+// below the 2^30 spheres a scene may have.
+template <class F>
+__device__ __forceinline__ F* node_box(F* boxes, uint32_t node)
+{
+    return boxes + (size_t)node * 6;
+}
+
 // Union of the two child boxes.
 __device__ __forceinline__ void join_boxes(const float (&cb)[2][6], float (&nb)[6])
 {
@@ -1001,7 +1009,7 @@ __device__ __forceinline__ void pack_node(uint32_t p, const float4* __restrict__
     for (uint32_t c = 0; c < 2; c++) {
         if ((flags >> c) & 1u) leaf_box(sph[g + c], cb[c]);
         else
-            for (int k = 0; k < 6; k++) cb[c][k] = boxes[(size_t)(g + c) * 6 + k];
+            for (int k = 0; k < 6; k++) cb[c][k] = node_box(boxes, g + c)[k];
     }
     join_boxes(cb, nb);
     uint32_t meta = 0, q[3];
@@ -1105,7 +1113,7 @@ __global__ void __launch_bounds__(kRefitThreads) k_refit_local(const float4* __r
             nh = h + 1u;
             for (int k = 0; k < 6; k++) {
                 __hip_atomic_store(&s_box[k][slot], nb[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                boxes[(size_t)p * 6 + k] = nb[k];  // every node's exact box: packing and the 4-wide collapse read them
+                node_box(boxes, p)[k] = nb[k];  // every node's exact box: packing and the 4-wide collapse read them
             }
             __hip_atomic_store(&s_h[slot], nh, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             done = p;
@@ -1117,7 +1125,7 @@ __global__ void __launch_bounds__(kRefitThreads) k_refit_local(const float4* __r
             if (done != 0u) continue;
         }
         if (!(done & kLeafItem)) {  // a finished local node: publish its box and height
-            for (int k = 0; k < 6; k++) boxes[done * 6 + k] = nb[k];
+            for (int k = 0; k < 6; k++) node_box(boxes, done)[k] = nb[k];
             height[done] = nh;
         }
         if (done != 0u) frontier[atomicAdd(fcount, 1u)] = done;
@@ -1152,13 +1160,13 @@ __global__ void __launch_bounds__(kRefitThreads) k_refit_top(const float4* __res
                     leaf_box(sph[ch], cb[c]);
                 } else {
                     for (int k = 0; k < 6; k++)
-                        cb[c][k] = __hip_atomic_load(&boxes[ch * 6 + k], __ATOMIC_RELAXED, SCOPE);
+                        cb[c][k] = __hip_atomic_load(node_box(boxes, ch) + k, __ATOMIC_RELAXED, SCOPE);
                     h = max(h, __hip_atomic_load(&height[ch], __ATOMIC_RELAXED, SCOPE));
                 }
             }
             float nb[6];
             join_boxes(cb, nb);
-            for (int k = 0; k < 6; k++) __hip_atomic_store(&boxes[p * 6 + k], nb[k], __ATOMIC_RELAXED, SCOPE);
+            for (int k = 0; k < 6; k++) __hip_atomic_store(node_box(boxes, p) + k, nb[k], __ATOMIC_RELAXED, SCOPE);
             __hip_atomic_store(&height[p], h + 1u, __ATOMIC_RELAXED, SCOPE);
             if (p == 0u) break;
             p = parent_int[p] & ~kLocalBit;
@@ -1215,7 +1223,7 @@ __device__ __forceinline__ uint32_t wide_children(uint32_t r, const uint32_t* __
     ks[2] = ks[3] = 0u;
     bool internal[4] = {!(ks[0] & kLeafRef), !(ks[1] & kLeafRef), false, false};
     for (int k = 0; k < 2; k++)
-        if (internal[k]) area[k] = box_area(boxes + (size_t)ks[k] * 6);
+        if (internal[k]) area[k] = box_area(node_box(boxes, ks[k]));
     uint32_t n_k = 2;
 #pragma unroll
     for (int round = 0; round < 2; round++) {
@@ -1232,8 +1240,8 @@ __device__ __forceinline__ uint32_t wide_children(uint32_t r, const uint32_t* __
         const uint32_t ow = child[opened];
         const uint32_t c0 = child_ref(ow, 0), c1 = child_ref(ow, 1);
         const bool i0 = !(c0 & kLeafRef), i1 = !(c1 & kLeafRef);
-        const float a0 = i0 ? box_area(boxes + (size_t)c0 * 6) : -1.0f;
-        const float a1 = i1 ? box_area(boxes + (size_t)c1 * 6) : -1.0f;
+        const float a0 = i0 ? box_area(node_box(boxes, c0)) : -1.0f;
+        const float a1 = i1 ? box_area(node_box(boxes, c1)) : -1.0f;
         // c0 takes the opened slot, c1 the next; the slots after move up
 #pragma unroll
         for (int k = 3; k >= 0; k--) {
@@ -1487,7 +1495,7 @@ __device__ __forceinline__ void wide_pack(uint32_t r, const float4* sph, const u
     const uint32_t fl = wflag[r];
     if (!(fl & kWideRoot)) return;
     const uint32_t cnt = fl & 7u;
-    const float* nb = boxes + (size_t)r * 6;
+    const float* nb = node_box(boxes, r);
     uint32_t meta = 0, qlo[3] = {0u, 0u, 0u}, qhi[3] = {0u, 0u, 0u}, ch[4] = {0u, 0u, 0u, 0u};
     uint32_t tlo[3] = {0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu}, thi[3] = {0u, 0u, 0u};
     float sc[3];
@@ -1517,7 +1525,7 @@ __device__ __forceinline__ void wide_pack(uint32_t r, const float4* sph, const u
             T.tinfo[at] = T.info[leaf];
             T.tmat[at] = T.mat[leaf];
         } else {
-            for (int k = 0; k < 6; k++) cb[k] = boxes[(size_t)ref[c] * 6 + k];
+            for (int k = 0; k < 6; k++) cb[k] = node_box(boxes, ref[c])[k];
             ch[c] = widx[ref[c]];
             t = slot_in++;
         }
