@@ -116,6 +116,12 @@ vzStatus vzCreate(int device, vzContext* out);
 /* Fails with VZ_ERROR_INVALID_VALUE while scenes or servers of the context
  * are alive: destroy them first. */
 vzStatus vzDestroy(vzContext ctx);
+/* Gives back the device memory the context keeps for later calls: up to 1 GiB
+ * of blocks of destroyed scenes, and the buffers of its largest plain launch
+ * (up to 4 GiB) and batch (by its tuning).  Waits for a launch of the context
+ * that another thread runs.  For callers whose own allocations need the room;
+ * the next calls allocate again. */
+vzStatus vzContextTrim(vzContext ctx);
 /* Device properties used by the autotuner/admission: CU count, HBM bytes. */
 vzStatus vzDeviceInfo(vzContext ctx, uint32_t* num_cus, uint64_t* hbm_bytes, char* name,
                       size_t name_len);

@@ -127,3 +127,44 @@ big = [params(1024, 1024, 40), params(2048, 1024, 12, api.ACCUM_FP64), params(40
 api.batch_launch(ctx, [(scene, params(512, 512, 4)), (scene, big[0]), (scene, big[1]), (scene, big[2])], tuning=t)
 check("a batch with large items")
 """)
+
+
+def test_kept_memory_is_given_back(stand_in):
+    """What a context keeps between calls (blocks of destroyed scenes, launch
+    buffers) makes room when one of its allocations fails, whichever it is,
+    and goes back when the caller asks."""
+    run(stand_in, """
+L = api.lib()
+base = hip.host_hip_used()
+
+def keep(n=1_000_000):
+    api.Scene(ctx, *api.box_scene(n, 1)).close()   # about 350 MB
+    assert hip.host_hip_used() > base + 300 * MB
+
+rays = api.RAY_DT
+def no_room(f):
+    keep()
+    hip.host_hip_limit(hip.host_hip_used())
+    out = f()
+    hip.host_hip_limit(1 << 60)
+    assert hip.host_hip_used() < base + 3500 * MB
+    return out
+
+buf = C.c_void_p(4096)
+st = api.Stats()
+no_room(lambda: api.check(L.vzTraceClosest(scene.h, buf, 1000, buf, None, C.byref(st))))
+no_room(lambda: scene.launch(params(64, 36, 2, api.MEGAKERNEL)))
+no_room(lambda: scene.launch(params(64, 36, 2)))
+scene.launch(params(1920, 1080, 64))              # 2.1 GB of launch buffers, kept
+hip.host_hip_limit(hip.host_hip_used() + 400 * MB)
+big = api.Scene(ctx, *api.box_scene(4_000_000, 1))  # 1.4 GB
+big.close()
+hip.host_hip_limit(1 << 60)
+scene.launch(params(1920, 1080, 64))
+t = api.Tuning()
+api.batch_launch(ctx, [(scene, params(512, 512, 16))] * 2, tuning=t)
+keep()
+ctx.trim()
+assert hip.host_hip_used() <= base, (hip.host_hip_used(), base)
+scene.launch(params(64, 36, 2))                   # and goes on
+""")

@@ -103,6 +103,7 @@ def _declare(L):
     sig = {
         "vzCreate": (st, [C.c_int, P(vp)]),
         "vzDestroy": (st, [vp]),
+        "vzContextTrim": (st, [vp]),
         "vzDeviceInfo": (st, [vp, P(u32), P(u64), C.c_char_p, C.c_size_t]),
         "vzSceneCreate": (st, [vp, vp, vp, u32, vp, P(vp)]),
         "vzSceneCreateDevice": (st, [vp, vp, vp, u32, vp, P(vp)]),
@@ -287,6 +288,10 @@ class Context:
         self.h = C.c_void_p()
         self._children = weakref.WeakSet()  # scenes and servers, closed before the context
         check(lib().vzCreate(device, C.byref(self.h)))
+
+    def trim(self):
+        """Gives back the device memory kept for later calls."""
+        check(lib().vzContextTrim(self.h))
 
     def close(self):
         if self.h:

@@ -84,6 +84,25 @@ static void adopt_cached_tuning(vzContext ctx)
     }
 }
 
+// Gives back all device memory that the context keeps for later calls.
+static void trim_context(vzContext ctx)
+{
+    std::lock_guard<std::mutex> lk(ctx->mu);
+    path_trim(ctx->path);
+    ctx->scene_blocks.trim();
+}
+
+// A scene's memory, the launch buffers making room for it if they have to.
+static vzStatus scene_alloc(vzScene s)
+{
+    vzStatus rs = lbvh_alloc(s);
+    if (rs == VZ_ERROR_OUT_OF_MEMORY) {
+        trim_context(s->ctx);
+        rs = lbvh_alloc(s);
+    }
+    return rs;
+}
+
 struct DevCounters {   // per-call counters for the non-engine kernels
     unsigned long long* d = nullptr;
     ~DevCounters()
@@ -157,6 +176,13 @@ vzStatus vzDestroy(vzContext ctx)
     return VZ_SUCCESS;
 }
 
+vzStatus vzContextTrim(vzContext ctx)
+{
+    if (!ctx) return set_error(VZ_ERROR_INVALID_VALUE, "ctx is NULL");
+    trim_context(ctx);
+    return VZ_SUCCESS;
+}
+
 vzStatus vzDeviceInfo(vzContext ctx, uint32_t* num_cus, uint64_t* hbm_bytes, char* name, size_t name_len)
 {
     if (!ctx) return set_error(VZ_ERROR_INVALID_VALUE, "ctx is NULL");
@@ -184,7 +210,7 @@ vzStatus vzSceneCreate(vzContext ctx, const vzSphere* spheres, const vzMaterial*
     s->ctx = ctx;
     s->n = n;
     s->uid = g_next_scene_uid.fetch_add(1);
-    vzStatus rs = lbvh_alloc(s);
+    vzStatus rs = scene_alloc(s);
     hipStream_t st = as_stream(stream);
     if (rs == VZ_SUCCESS && (hipMemcpyAsync(s->d_sph_in, spheres, sizeof(vzSphere) * n, hipMemcpyHostToDevice, st) != hipSuccess ||
                              hipMemcpyAsync(s->d_mat_in, materials, sizeof(vzMaterial) * n, hipMemcpyHostToDevice, st) != hipSuccess))
@@ -212,7 +238,7 @@ vzStatus vzSceneCreateDevice(vzContext ctx, const vzSphere* spheres, const vzMat
     s->ctx = ctx;
     s->n = n;
     s->uid = g_next_scene_uid.fetch_add(1);
-    vzStatus rs = lbvh_alloc(s);
+    vzStatus rs = scene_alloc(s);
     hipStream_t st = as_stream(stream);
     if (rs == VZ_SUCCESS &&
         (hipMemcpyAsync(s->d_sph_in, spheres, sizeof(vzSphere) * n, hipMemcpyDeviceToDevice, st) != hipSuccess ||
@@ -274,7 +300,11 @@ vzStatus vzSceneUpdateSpheresDevice(vzScene scene, const vzSphere* spheres, vzSt
     hipStream_t st = as_stream(stream);
     // check a copy first, so a rejected update leaves the scene unchanged
     vzSphere* tmp = nullptr;
-    VZ_HIP_TRY(hipMallocAsync((void**)&tmp, sizeof(vzSphere) * scene->n, st));
+    if (hipMallocAsync((void**)&tmp, sizeof(vzSphere) * scene->n, st) != hipSuccess) {
+        (void)hipGetLastError();
+        scene->ctx->scene_blocks.trim();
+        VZ_HIP_TRY(hipMallocAsync((void**)&tmp, sizeof(vzSphere) * scene->n, st));
+    }
     vzStatus rs = VZ_SUCCESS;
     if (hipMemcpyAsync(tmp, spheres, sizeof(vzSphere) * scene->n, hipMemcpyDeviceToDevice, st) != hipSuccess)
         rs = set_error(VZ_ERROR_HIP, "sphere copy failed");
@@ -352,7 +382,8 @@ vzStatus vzTraceClosest(vzScene scene, const vzRay* rays, uint32_t n, vzHit* hit
     // per-workgroup partial counters, then the 4 summed counters
     const size_t nparts = (size_t)trace_blocks(n) * kTraceParts;
     DevCounters c;
-    VZ_HIP_TRY(hipMalloc(&c.d, (nparts + 8) * sizeof(unsigned long long)));
+    if (!device_alloc(scene->ctx, (void**)&c.d, (nparts + 8) * sizeof(unsigned long long)))
+        return set_error(VZ_ERROR_HIP, "hipMalloc of the trace counters failed");
     Event e0, e1;
     VZ_EVENT_TRY(e0);
     VZ_EVENT_TRY(e1);
@@ -420,7 +451,8 @@ vzStatus vzLaunch(vzScene scene, const vzLaunchParams* params, vzStream stream, 
     std::lock_guard<std::mutex> lk(ctx->mu);
     if (params->flags & VZ_MEGAKERNEL) {
         DevCounters c;
-        VZ_HIP_TRY(hipMalloc(&c.d, 8 * sizeof(unsigned long long)));
+        if (!device_alloc(ctx, (void**)&c.d, 8 * sizeof(unsigned long long)))
+            return set_error(VZ_ERROR_HIP, "hipMalloc of the counters failed");
         VZ_HIP_TRY(hipMemsetAsync(c.d, 0, 8 * sizeof(unsigned long long), st));
         Event e0, e1;
         VZ_EVENT_TRY(e0);

@@ -106,12 +106,14 @@ namespace vz {
 // Blocks of destroyed scenes, kept for the next ones: mapping and unmapping
 // the 300 MB of a million-sphere scene takes longer than building it.  At
 // most kKeepBytes are kept, given back when an allocation of the context
-// fails and with the context.  A scene is destroyed after the device has
-// gone idle, so a kept block is free for any stream.
+// fails (device_alloc), by vzContextTrim and with the context.  A scene is
+// destroyed after the device has gone idle, so a kept block is free for any
+// stream.
 class SceneBlocks {
 public:
     static constexpr size_t kKeepBytes = 1ull << 30;
-    // A block of at least `bytes`; *got is its size.  NULL when out of memory.
+    // A kept block of at least `bytes`, its size in *got; NULL, and `bytes`,
+    // if there is none.
     void* take(size_t bytes, size_t* got);
     void give(void* p, size_t bytes);
     void trim();
@@ -226,6 +228,9 @@ vzStatus lbvh_refit(vzScene s, hipStream_t st);   // same topology, new d_sph_in
 vzStatus lbvh_check_input(vzScene s, const vzMaterial* mat, hipStream_t st, uint32_t* bad_sphere,
                           uint32_t* bad_material);
 void lbvh_free(vzScene s);
+// hipMalloc, and once more without the context's kept blocks if there is no
+// room.  Records no error message.
+bool device_alloc(vzContext ctx, void** p, size_t bytes);
 
 // vz_trace.hip
 // Workgroups of a trace of n rays (each writes kTraceParts partial counters).
@@ -244,7 +249,9 @@ vzStatus trace_scratch_address(unsigned long long** out);
 // vz_api.cpp: the process-wide autotune cache, keyed by device name and CU count
 void tuning_cache_store(vzContext ctx, const vzTuning& t);
 
-// vz_path.hip: gives back what a context kept for its launches
+// vz_path.hip: gives back what a context kept for its launches (the latter
+// with it, the former until the next launch; no launch may run)
+void path_trim(PathWork* w);
 void path_free(PathWork* w);
 
 // vz_megakernel.hip

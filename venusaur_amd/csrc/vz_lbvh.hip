@@ -1619,17 +1619,8 @@ void* SceneBlocks::take(size_t bytes, size_t* got)
             return p;
         }
     }
-    void* p = nullptr;
-    if (hipMalloc(&p, bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        trim();
-        if (hipMalloc(&p, bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            return nullptr;
-        }
-    }
     *got = bytes;
-    return p;
+    return nullptr;
 }
 
 void SceneBlocks::give(void* p, size_t bytes)
@@ -1651,6 +1642,17 @@ void SceneBlocks::trim()
     for (const Block& b : kept_) (void)hipFree(b.p);
     kept_.clear();
     kept_bytes_ = 0;
+}
+
+bool device_alloc(vzContext ctx, void** p, size_t bytes)
+{
+    if (hipMalloc(p, bytes) == hipSuccess) return true;
+    (void)hipGetLastError();
+    ctx->scene_blocks.trim();
+    if (hipMalloc(p, bytes) == hipSuccess) return true;
+    (void)hipGetLastError();
+    *p = nullptr;
+    return false;
 }
 
 vzStatus lbvh_alloc(vzScene s)
@@ -1701,7 +1703,8 @@ vzStatus lbvh_alloc(vzScene s)
     part(&s->d_wfront[1], sizeof(uint32_t) * ni);
     part(&s->d_wcnt, sizeof(uint32_t) * kWideWords);
     s->arena = s->ctx->scene_blocks.take(at, &s->arena_bytes);
-    if (!s->arena) return set_error(VZ_ERROR_OUT_OF_MEMORY, "hipMalloc of scene buffers failed");
+    if (!s->arena && !device_alloc(s->ctx, &s->arena, at))
+        return set_error(VZ_ERROR_OUT_OF_MEMORY, "hipMalloc of scene buffers failed");
     for (const Part& q : parts) *q.p = (char*)s->arena + q.at;
     s->device_bytes = bytes;
     return VZ_SUCCESS;

@@ -78,11 +78,7 @@ struct PathWork {              // what a context keeps between launches
     PathSlot plain, batch;
     Event t0, t1;
     uint32_t grid_lds = 0, grid_mem = 0;  // resident k_path workgroups by variant
-    ~PathWork()
-    {
-        plain.free();
-        batch.free();
-    }
+    ~PathWork() { path_trim(this); }
 };
 
 vzStatus path_work(vzContext ctx, PathWork** out);

@@ -544,15 +544,7 @@ bool grow(vzContext ctx, char** p, size_t* have, size_t need)
 {
     if (*have >= need) return true;
     drop(p, have);
-    if (hipMalloc((void**)p, need) != hipSuccess) {
-        (void)hipGetLastError();
-        ctx->scene_blocks.trim();
-        if (hipMalloc((void**)p, need) != hipSuccess) {
-            (void)hipGetLastError();
-            *p = nullptr;
-            return false;
-        }
-    }
+    if (!device_alloc(ctx, (void**)p, need)) return false;
     *have = need;
     return true;
 }
@@ -705,12 +697,12 @@ size_t request_bytes(const vzLaunchParams& p)
 vzStatus PathSlot::init(vzContext c, bool table)
 {
     ctx = c;
-    bool ok = stats || hipMalloc((void**)&stats, (kMaxPathBlocks * kPathStats + kCounterWords + kMaxRequests) *
-                                                     sizeof(unsigned long long)) == hipSuccess;
+    bool ok = stats || device_alloc(ctx, (void**)&stats, (kMaxPathBlocks * kPathStats + kCounterWords + kMaxRequests) *
+                                                             sizeof(unsigned long long));
     ok = ok && (h_totals || hipHostMalloc((void**)&h_totals, (kPathStats + kMaxRequests) *
                                                                  sizeof(unsigned long long)) == hipSuccess);
     if (table) {
-        ok = ok && (reqs || hipMalloc((void**)&reqs, kMaxRequests * sizeof(PathReq)) == hipSuccess);
+        ok = ok && (reqs || device_alloc(ctx, (void**)&reqs, kMaxRequests * sizeof(PathReq)));
         ok = ok && (h_reqs || hipHostMalloc((void**)&h_reqs, kMaxRequests * sizeof(PathReq)) == hipSuccess);
     }
     if (!ok) {
@@ -746,6 +738,13 @@ vzStatus path_work(vzContext ctx, PathWork** out)
     }
     *out = ctx->path;
     return VZ_SUCCESS;
+}
+
+void path_trim(PathWork* w)
+{
+    if (!w) return;
+    w->plain.free();
+    w->batch.free();
 }
 
 void path_free(PathWork* w) { delete w; }
