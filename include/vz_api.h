@@ -220,7 +220,11 @@ vzStatus vzAutotune(vzContext ctx, const vzBatchItem* items, uint32_t n, vzStrea
                     vzTuning* out);
 vzStatus vzDefaultTuning(vzContext ctx, vzTuning* out);
 
-/* ---- serving form --------------------------------------------------- */
+/* ---- serving form ---------------------------------------------------
+ * Requests are admitted in arrival order and rendered in turn, several in one
+ * launch and two launches at a time.  One of more paths than a launch takes is
+ * rendered a slice of its samples at a time, after each of which the others
+ * have their turn; requests of one launch finish together. */
 typedef struct vzServeConfig {
     uint64_t hbm_budget_bytes;   /* admission budget: requests are admitted while the sum of their
                                     vzRequestFootprint fits (the server's own buffers are sized by
@@ -250,7 +254,7 @@ vzStatus vzServerPoll(vzServer srv, uint64_t request_id, vzRequestResult* out);
 /* Block until every submitted request finished. */
 vzStatus vzServerDrain(vzServer srv);
 /* Finishes every submitted request, then stops the loop and frees the
- * server's engine and stream. */
+ * server's buffers and streams. */
 vzStatus vzServerDestroy(vzServer srv);
 /* Bytes of device memory a request of these params needs (admission). */
 uint64_t vzRequestFootprint(const vzLaunchParams* params);

@@ -1,0 +1,55 @@
+"""Served requests of more paths than a launch takes, rendered a slice of
+their passes at a time in turn with others: bit for bit what a plain launch
+gives."""
+import numpy as np
+import pytest
+
+from util import GpuTarget, book_lookat, box_lookat, gpu_params, sha
+from venusaur_amd import api
+
+pytestmark = pytest.mark.gpu
+
+
+# the smallest queue gives launches of 8M paths: three slices of a float image
+# and of a double one, slices whose last shares its launch with small
+# requests, an image of one pass above a launch, and progressive frames
+@pytest.mark.parametrize("kind", ["book", "mem"])
+def test_sliced_requests_equal_plain_launches(ctx, book, kind):
+    print(f"case: served slices {kind}", flush=True)
+    (s, m), look = (book, book_lookat) if kind == "book" else (api.box_scene(3000, 9), box_lookat)
+    other = api.Scene(ctx, *api.box_scene(700, 3))
+    sc = api.Scene(ctx, s, m)
+    jobs = []
+    for w, h, spp, fp64, scene in [(1021, 763, 24, False, sc), (128, 130, 1100, True, sc), (64, 36, 2, False, sc),
+                                   (4099, 2301, 2, False, sc), (640, 360, 37, False, other), (33, 17, 1, False, other),
+                                   (256, 256, 300, False, sc)]:
+        t = GpuTarget(w, h, fp64=fp64)
+        p = t.bind(gpu_params(w, h, spp, 6, look(w, h), flags=api.ACCUM_FP64 if fp64 else 0))
+        jobs.append((scene, p, t))
+    frames = (1, 2)
+    want, segs = [], []
+    for f in frames:
+        for scene, p, t in jobs:
+            p.subframe_index = f
+            segs.append(scene.launch(p).segments)
+            want.append((sha(t.accum_host()), sha(t.image_host())))
+    for _, _, t in jobs:
+        t.accum.zero()
+        t.image.zero()
+    srv = api.Server(ctx, 4 << 30, tuning=api.Tuning(queue_capacity=1))
+    k = 0
+    for f in frames:
+        ids = []
+        for scene, p, t in jobs:
+            p.subframe_index = f
+            ids.append(srv.submit(scene, p))
+        srv.drain()
+        for i, (_, p, t) in zip(ids, jobs):
+            r = srv.poll(i)
+            what = (f, p.width, p.height, p.samples_per_pixel)
+            assert r.status == 0 and r.segments == segs[k], what
+            assert (sha(t.accum_host()), sha(t.image_host())) == want[k], what
+            k += 1
+    srv.close()
+    sc.close()
+    other.close()

@@ -168,3 +168,50 @@ ctx.trim()
 assert hip.host_hip_used() <= base, (hip.host_hip_used(), base)
 scene.launch(params(64, 36, 2))                   # and goes on
 """)
+
+
+SERVE = """
+class Steps:
+    # the flights of a server, finished one at a time
+    def __init__(self):
+        hip.host_hip_hold(1)
+
+    def settle(self, flights):
+        for _ in range(200):
+            if hip.host_hip_held() == flights:
+                return
+            time.sleep(0.01)
+        raise AssertionError(f"{hip.host_hip_held()} flights, not {flights}")
+
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *exc):
+        hip.host_hip_hold(0)
+        while hip.host_hip_release():
+            pass
+"""
+
+
+def test_small_request_does_not_wait_for_large_ones(stand_in):
+    """Two requests of 2.1e9 paths each are running when a thumbnail comes: it
+    is rendered within a few launches, long before either is done."""
+    run(stand_in, SERVE + """
+srv = api.Server(ctx, 8 << 30)
+with Steps() as steps:
+    large = [srv.submit(scene, params(2048, 2048, 512)) for _ in range(2)]
+    steps.settle(2)
+    thumb = srv.submit(scene, params(64, 36, 2))
+    time.sleep(0.1)
+    for turn in range(1, 5):
+        assert hip.host_hip_release()
+        time.sleep(0.1)
+        if srv.poll(thumb) is not None:
+            break
+    assert srv.poll(thumb) is not None and turn <= 3, turn
+    assert [srv.poll(i) for i in large] == [None, None]
+srv.drain()
+assert all(srv.poll(i).status == 0 for i in large)
+assert hip.host_hip_launches("k_path_resolve") > 2 * 40    # in slices
+srv.close()
+""")

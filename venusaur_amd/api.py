@@ -441,7 +441,8 @@ def autotune(ctx, scenes_params, stream=None):
 
 
 class Server:
-    """Serving loop: continuous batching over resident scenes."""
+    """Serving loop: requests over resident scenes, admitted in arrival order
+    and rendered in turn, a large one a slice of its samples at a time."""
 
     def __init__(self, ctx, hbm_budget_bytes, max_active=256, tuning=None):
         cfg = ServeConfig()

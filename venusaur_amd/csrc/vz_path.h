@@ -21,8 +21,9 @@ constexpr uint64_t kPathBytes = 16;
 constexpr uint64_t kRayBytes = 96;
 // A plain launch: 4 GiB hold 129 passes of a 1080p frame.
 constexpr uint64_t kPlainBudget = 4ull << 30;
-// The most a slot is used for, so that a path's index fits 32 bits.
+// The most a slot is used for, beyond one pass of a large image.
 constexpr uint64_t kMaxSlotBudget = 16ull << 30;
+constexpr uint64_t kMaxLaunchPaths = 0xFFFFFF00ull;  // a path's index has 32 bits
 
 struct PathReq {               // one request of a launch, read by scalar loads
     Cam cam;
@@ -61,6 +62,15 @@ struct PathItem {
     vzLaunchParams params;
 };
 
+// Passes [s0, s0 + ns) of a request: one launch's share of it.  carry holds
+// its sums and camera seeds from slice to slice (carry_bytes), and may be null
+// for a slice of all passes.
+struct PathSlice {
+    const PathItem* item;
+    uint32_t s0, ns;
+    char* carry;
+};
+
 struct PathOptions {
     uint32_t refill = 0;       // 0: the kernel variant's default
     uint32_t tile_w = 8, tile_h = 8;
@@ -88,8 +98,13 @@ Cam make_cam(const vzLaunchParams& p);
 // (at most max_depth + 2), its per-pixel sums and camera seeds.
 size_t request_bytes(const vzLaunchParams& p);
 
-// Paths of a request with its tiles' padding.
+// Pixels of a request with its tiles' padding, and its paths.
+uint64_t padded_pixels(const vzLaunchParams& p, const PathOptions& opt);
 uint64_t path_count(const vzLaunchParams& p, const PathOptions& opt);
+// Device memory that a request of several launches carries between them.
+uint64_t carry_bytes(const vzLaunchParams& p, uint64_t npad);
+// Bytes of a slot for launches of up to `paths` paths.
+inline uint64_t slot_bytes(uint64_t paths) { return paths * kPathBytes + 256; }
 // Makes room in the slot for launches of up to `paths` paths; nothing on its
 // stream may still run.
 vzStatus slot_reserve(PathSlot& s, uint64_t paths);
@@ -103,9 +118,11 @@ vzStatus path_reserve_one(PathSlot& s, const PathItem& item, const PathOptions& 
 // those of the slot's launch before.
 vzStatus path_enqueue_one(PathWork* w, PathSlot& s, const PathItem& item, const PathOptions& opt, uint32_t passes,
                           bool add, hipStream_t st, uint32_t* launches);
-// Enqueues n requests as one launch (their paths fit the slot).
-vzStatus path_enqueue_many(PathWork* w, PathSlot& s, const PathItem* const* items, uint32_t n, const PathOptions& opt,
+// Enqueues n slices of different requests as one launch (their paths fit the slot).
+vzStatus path_enqueue_many(PathWork* w, PathSlot& s, const PathSlice* slices, uint32_t n, const PathOptions& opt,
                            bool add, hipStream_t st);
+// Segments of slice i of the slot's last launch, of n slices, once it is done.
+unsigned long long slice_segments(const PathSlot& s, uint32_t n, uint32_t i);
 
 // Renders one frame and waits for it.
 vzStatus path_launch(vzContext ctx, const PathItem& item, hipStream_t st, RunResult* res);

@@ -529,8 +529,6 @@ uint64_t sum_bytes(const vzLaunchParams& p, uint64_t npad)
 {
     return align256(((p.flags & VZ_ACCUM_FP64) ? 24ull : 12ull) * npad);
 }
-uint64_t carry_bytes(const vzLaunchParams& p, uint64_t npad) { return sum_bytes(p, npad) + 4ull * npad; }
-
 // Gives back a buffer that nothing in flight uses.
 void drop(char** p, size_t* have)
 {
@@ -662,6 +660,8 @@ uint32_t refill_of(const PathOptions& opt, uint32_t dflt)
 
 }  // namespace
 
+uint64_t carry_bytes(const vzLaunchParams& p, uint64_t npad) { return sum_bytes(p, npad) + 4ull * npad; }
+
 Cam make_cam(const vzLaunchParams& p)
 {
     auto nrm = [](v3 v) {
@@ -749,14 +749,16 @@ void path_trim(PathWork* w)
 
 void path_free(PathWork* w) { delete w; }
 
+uint64_t padded_pixels(const vzLaunchParams& p, const PathOptions& opt) { return tile_count(p, tile_lw(p, opt)) * kTile; }
+
 uint64_t path_count(const vzLaunchParams& p, const PathOptions& opt)
 {
-    return tile_count(p, tile_lw(p, opt)) * kTile * p.samples_per_pixel;
+    return padded_pixels(p, opt) * p.samples_per_pixel;
 }
 
 vzStatus slot_reserve(PathSlot& s, uint64_t paths)
 {
-    const uint64_t need = paths * kPathBytes + 256;
+    const uint64_t need = slot_bytes(paths);
     if (!grow(s.ctx, &s.paths, &s.paths_bytes, need))
         return set_error(VZ_ERROR_OUT_OF_MEMORY, "launch buffers (" + std::to_string(need) + " bytes) do not fit");
     return VZ_SUCCESS;
@@ -766,7 +768,7 @@ vzStatus path_reserve_one(PathSlot& s, const PathItem& item, const PathOptions& 
                           uint32_t* passes)
 {
     const uint64_t ntiles = tile_count(item.params, tile_lw(item.params, opt));
-    if (ntiles * kTile > 0xFFFFFF00ull) return set_error(VZ_ERROR_CAPACITY, "image too large");
+    if (ntiles * kTile > kMaxLaunchPaths) return set_error(VZ_ERROR_CAPACITY, "image too large");
     const uint64_t npad = ntiles * kTile, spp = item.params.samples_per_pixel;
     // the passes in as few equal chunks as the budget allows; less memory
     // than that makes more chunks
@@ -798,7 +800,7 @@ vzStatus path_enqueue_one(PathWork* w, PathSlot& s, const PathItem& item, const 
     PathReq A;
     fill_request(A, item, opt);
     const uint64_t ntiles = A.npad / kTile;
-    if ((uint64_t)A.npad * passes * kPathBytes + 256 > s.paths_bytes)
+    if (slot_bytes((uint64_t)A.npad * passes) > s.paths_bytes)
         return set_error(VZ_ERROR_INTERNAL, "launch larger than its slot");
     const bool lds = fits_lds(item.scene) && !opt.count;
     const uint32_t resident = lds ? w->grid_lds : w->grid_mem;
@@ -826,21 +828,30 @@ vzStatus path_enqueue_one(PathWork* w, PathSlot& s, const PathItem& item, const 
     return VZ_SUCCESS;
 }
 
-vzStatus path_enqueue_many(PathWork* w, PathSlot& s, const PathItem* const* items, uint32_t n, const PathOptions& opt,
+vzStatus path_enqueue_many(PathWork* w, PathSlot& s, const PathSlice* slices, uint32_t n, const PathOptions& opt,
                            bool add, hipStream_t st)
 {
     if (s.used + n > kMaxRequests) return set_error(VZ_ERROR_INTERNAL, "request table overrun");
     PathReq* const h = s.h_reqs + s.used;
     PathReq* const d = s.reqs + s.used;
-    bool lds = fits_lds(items[0]->scene) && !opt.count;
+    bool lds = fits_lds(slices[0].item->scene) && !opt.count;
     uint64_t tile_passes = 0, paths = 0;
     for (uint32_t i = 0; i < n; i++) {
-        fill_request(h[i], *items[i], opt);
-        lds = lds && items[i]->scene == items[0]->scene;
-        tile_passes += (uint64_t)h[i].npad / kTile * h[i].spp;
-        paths += (uint64_t)h[i].npad * h[i].spp;
+        const PathSlice& sl = slices[i];
+        fill_request(h[i], *sl.item, opt);
+        h[i].s0 = sl.s0;
+        h[i].ns = sl.ns;
+        if (sl.carry) {
+            h[i].sums = sl.carry;
+            h[i].camseed = (uint32_t*)(sl.carry + sum_bytes(sl.item->params, h[i].npad));
+        } else if (sl.ns != h[i].spp) {
+            return set_error(VZ_ERROR_INTERNAL, "a slice of a request without its sums");
+        }
+        lds = lds && sl.item->scene == slices[0].item->scene;
+        tile_passes += (uint64_t)h[i].npad / kTile * sl.ns;
+        paths += (uint64_t)h[i].npad * sl.ns;
     }
-    if (paths * kPathBytes + 256 > s.paths_bytes || paths * kPathBytes > kMaxSlotBudget)
+    if (slot_bytes(paths) > s.paths_bytes || paths > kMaxLaunchPaths)
         return set_error(VZ_ERROR_INTERNAL, "launch larger than its slot");
     const uint32_t resident = lds ? w->grid_lds : w->grid_mem;
     const uint32_t waves = resident * (lds ? kLdsBlk : kMemBlk) / 64;
@@ -850,8 +861,7 @@ vzStatus path_enqueue_many(PathWork* w, PathSlot& s, const PathItem* const* item
     uint32_t slot0 = 0;
     for (uint32_t i = 0; i < n; i++) {
         PathReq& A = h[i];
-        A.ns = A.spp;
-        A.spu = std::min(spu, A.spp);
+        A.spu = std::min(spu, A.ns);
         A.parts = parts;
         A.groups = ((A.ns + A.spu - 1) / A.spu) << parts;
         A.unit0 = G.units;
@@ -859,18 +869,24 @@ vzStatus path_enqueue_many(PathWork* w, PathSlot& s, const PathItem* const* item
         A.slot0 = slot0;
         G.units += A.npad / kTile * A.groups;
         G.pixels += A.npad;
-        slot0 += A.npad * A.spp;
+        slot0 += A.npad * A.ns;
     }
-    G.reqs = d;
-    G.n = n;
     G.seeds = (uint32_t*)s.paths;
     G.rad = (float*)(s.paths + align256(4ull * paths));
     G.refill = refill_of(opt, lds ? kRefillLds : kRefillGlobal);
     G.grid = std::min(resident, G.units);
     G.log_counters = log_counters(G.grid);
+    if (n == 1) return launch_group<false>(G, h[0], lds, opt, st);  // by value: no table
+    G.reqs = d;
+    G.n = n;
     VZ_HIP_TRY(hipMemcpyAsync(d, h, n * sizeof(PathReq), hipMemcpyHostToDevice, st));
     s.used += n;
     return launch_group<true>(G, PathReq{}, lds, opt, st);
+}
+
+unsigned long long slice_segments(const PathSlot& s, uint32_t n, uint32_t i)
+{
+    return n == 1 ? s.h_totals[0] : s.h_totals[kPathStats + i];
 }
 
 // Waits for the launches of a slot, whose buffers are then free for the next
@@ -950,7 +966,7 @@ vzStatus path_batch(vzContext ctx, const std::vector<PathItem>& items, const vzT
     if (slot.paths_bytes > budget + 256) slot.free();  // a smaller tuning gives memory back
     VZ_TRY(slot.init(ctx, true));
     slot.used = 0;
-    std::vector<std::vector<const PathItem*>> groups(1);
+    std::vector<std::vector<PathSlice>> groups(1);
     std::vector<const PathItem*> large;
     uint64_t open = 0, need = 0;
     for (const PathItem& it : items) {
@@ -963,7 +979,7 @@ vzStatus path_batch(vzContext ctx, const std::vector<PathItem>& items, const vzT
             groups.emplace_back();
             open = 0;
         }
-        groups.back().push_back(&it);
+        groups.back().push_back(PathSlice{&it, 0u, it.params.samples_per_pixel, nullptr});
         open += n;
         need = std::max(need, open);
     }

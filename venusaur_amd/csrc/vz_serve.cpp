@@ -1,16 +1,18 @@
 // vz_serve.cpp -- the serving form and the autotuner.
 //
 // Serving: a host thread owns a few streams, each with the buffers of its
-// launches (a slot).  Requests are queued FIFO by vzServerSubmit; whenever a
-// slot is idle the requests at the head of the queue that fit it and the HBM
-// budget are rendered as one launch on its stream, at once and beside the
+// launches (a slot).  Requests are queued FIFO by vzServerSubmit and admitted
+// while they fit the HBM budget.  Whenever a slot is idle the admitted requests
+// next in turn are rendered as one launch on its stream, at once and beside the
 // launches of the other slots, which the GPU works through in the order they
 // came: new work overlaps with requests already on the GPU (continuous
-// batching) and takes over the CUs that finishing launches leave.  BVHs stay
-// resident (vzScene objects owned by the caller) and the slots' buffers are
-// kept, so admission and release never synchronise the device.  The nearest
-// reference analogue is the interactive loop that keeps the GAS and
-// accumulator resident across frames (Core/Core.cpp:358-430,
+// batching) and takes over the CUs that finishing launches leave.  A request of
+// more paths than a launch takes is rendered a slice of its passes at a time
+// and goes to the end of the queue between them, so that no request waits for
+// another to finish.  BVHs stay resident (vzScene objects owned by the caller)
+// and the slots' buffers are kept, so admission and release never synchronise
+// the device.  The nearest reference analogue is the interactive loop that
+// keeps the GAS and accumulator resident across frames (Core/Core.cpp:358-430,
 // Core/Renderer.h:37-54).
 //
 // Autotuner: times the caller's batch over candidate buffer sizes, camera
@@ -21,6 +23,7 @@
 #include <condition_variable>
 #include <cstring>
 #include <deque>
+#include <memory>
 #include <thread>
 #include <unordered_map>
 
@@ -31,39 +34,49 @@ using namespace vz;
 
 namespace {
 
-struct Pending {
+struct Request {
     uint64_t id;
-    const vzScene_st* scene;
-    vzLaunchParams params;
-    size_t bytes;
-    double submit_ms;
+    PathItem item;
+    size_t bytes;               // counted against the budget
+    uint64_t npad;              // its pixels, padded
+    double submit_ms, admit_ms = 0.0;
+    uint32_t done = 0;          // passes rendered or in flight
+    char* carry = nullptr;      // what its slices hand on
+    unsigned long long segments = 0;
+
+    uint32_t left() const { return item.params.samples_per_pixel - done; }
+};
+using RequestPtr = std::unique_ptr<Request>;
+
+struct Share {                  // of a request, in a launch
+    RequestPtr r;
+    uint32_t s0, ns;
 };
 
-struct Active {
-    uint64_t id;
-    const vzScene_st* scene;
-    size_t bytes;
-    double submit_ms, admit_ms;
-};
-
-// Requests rendered by one launch, or one request of several launches.
+// One launch.
 struct Flight {
     PathSlot slot;
     hipStream_t stream = nullptr;
     Event done{hipEventDisableTiming};
-    std::vector<Active> active;  // empty: idle
-    bool large = false;
+    std::vector<Share> shares;  // empty: idle
 };
 
 // Launches side by side: the second takes over the CUs that the first one's
 // last paths leave.  A burst of 20 requests (1k to 200k spheres, 256 to 1024
-// pixels square, 4 to 64 samples, one of 1088) took 195 ms with 2, 209 with
-// 1, 202 with 3 and 203 with 4.
+// pixels square, 4 to 64 samples, one of 1088) takes 147.9 ms with 2 and 150.3
+// with 3 at 16M paths a launch, 143.6 and 145.4 at 32M.
 constexpr uint32_t kServeStreams = 2;
-// Paths of a launch of several requests at most.  A launch's requests finish
-// together: the burst's p50 latency is 92 ms at 8M paths, 101 at 32M and 116
-// at 64M, its throughput the same within 1%.
-constexpr uint64_t kServeGroupPaths = 16u << 20;
+// Paths of a launch at most while other requests wait; one that has the server
+// to itself takes as many as the slot may hold, since its slices follow one
+// another and each leaves the GPU idle at its end (1080p at 512 samples: 473 ms
+// in launches of 128M, 493 of 64M).  A launch's requests finish together and the
+// next in turn start after it: with 16M, 32M, 48M, 64M and 128M the same burst
+// takes 147.9, 143.6, 140.8, 139.5 and 139.4 ms, 600 such requests at 0.8 of
+// the capacity have a p50 of 102, 174, 234, 292 and 489 ms, and 256x256 at 4
+// samples behind two frames of 1080p at 512 samples 11, 25, 24, 10 to 39 and 38
+// to 165 ms.  (Requests up to 150M paths whole, in order of arrival: 141.2 ms,
+// 923 ms and 730 ms.)
+constexpr uint64_t kServePaths = 48u << 20;
 
 }  // namespace
 
@@ -72,12 +85,13 @@ struct vzServer_st {
     vzServeConfig cfg{};
     PathWork* work = nullptr;
     PathOptions opt;
-    uint64_t slot_budget = 0;
+    uint64_t launch_paths = kServePaths, alone_paths = kServePaths;
     std::vector<Flight> flights;
     std::thread worker;
     std::mutex mu;
     std::condition_variable cv_work, cv_done;
-    std::deque<Pending> pending;
+    std::deque<RequestPtr> pending;    // in arrival order
+    std::deque<RequestPtr> ready;      // admitted, in turn (the worker's)
     std::unordered_map<uint64_t, vzRequestResult> results;
     size_t n_active = 0;
     uint64_t next_id = 1;
@@ -92,102 +106,163 @@ struct vzServer_st {
         return std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     }
     void loop();
-    std::vector<Pending> admit();
-    vzStatus start(Flight& f, const std::vector<Pending>& group);
+    void admit();
+    uint64_t pick(Flight& f, uint64_t most);
+    vzStatus start(Flight& f);
+    void put_back(Flight& f);
     void harvest(Flight& f);
-    // A request no longer needs its scene (finished, rejected or dropped).
-    static void release_scene(const vzScene_st* sc)
+    bool others_busy(const Flight& f) const
     {
-        const_cast<vzScene_st*>(sc)->server_refs.fetch_sub(1);
+        for (const Flight& o : flights)
+            if (&o != &f && !o.shares.empty()) return true;
+        return false;
     }
-    // A request that will never run (mu held).
-    void reject(const Pending& p, vzStatus status)
+    // A request no longer needs its scene (finished, rejected or dropped).
+    static void release_scene(const Request& r)
     {
-        release_scene(p.scene);
-        vzRequestResult r{};
-        r.request_id = p.id;
-        r.submit_ms = p.submit_ms;
-        r.admit_ms = r.finish_ms = now_ms();
-        r.status = status;
-        results[p.id] = r;
+        const_cast<vzScene_st*>(r.item.scene)->server_refs.fetch_sub(1);
+    }
+    // A request is over (mu held).
+    void finish(const Request& r, vzStatus status)
+    {
+        release_scene(r);
+        vzRequestResult out{};
+        out.request_id = r.id;
+        out.submit_ms = r.submit_ms;
+        out.finish_ms = now_ms();
+        out.admit_ms = r.admit_ms > 0.0 ? r.admit_ms : out.finish_ms;
+        out.segments = r.segments;
+        out.status = status;
+        results[r.id] = out;
     }
     ~vzServer_st()
     {
+        // after a fatal error requests may remain; they will never run
+        for (const RequestPtr& r : pending) release_scene(*r);
+        for (const RequestPtr& r : ready) drop(*r);
+        for (Flight& f : flights)
+            for (const Share& s : f.shares) drop(*s.r);
         for (Flight& f : flights) {
             f.slot.free();
             if (f.stream) (void)hipStreamDestroy(f.stream);
         }
     }
+    void drop(const Request& r)
+    {
+        release_scene(r);
+        if (r.carry) (void)hipFreeAsync(r.carry, flights.front().stream);
+    }
 };
 
-// The next launch's requests, in arrival order, while they fit the budget,
-// the table and the slot (mu held).
-std::vector<Pending> vzServer_st::admit()
+// Queued requests, in arrival order, while they fit the budget.
+void vzServer_st::admit()
 {
-    std::vector<Pending> group;
-    uint64_t paths = 0;
-    const uint64_t most = std::min<uint64_t>(slot_budget / kPathBytes, kServeGroupPaths);
+    std::lock_guard<std::mutex> lk(mu);
     while (!pending.empty() && n_active < cfg.max_active) {
-        const Pending& p = pending.front();
-        if (p.bytes > cfg.hbm_budget_bytes) {  // can never fit
-            reject(p, VZ_ERROR_CAPACITY);
+        Request& p = *pending.front();
+        if (p.bytes > cfg.hbm_budget_bytes || p.npad > kMaxLaunchPaths) {  // can never fit
+            finish(p, VZ_ERROR_CAPACITY);
             pending.pop_front();
+            cv_done.notify_all();
             continue;
         }
         if (used_bytes + p.bytes > cfg.hbm_budget_bytes) break;  // wait for memory
-        const uint64_t n = path_count(p.params, opt);
-        if (!group.empty() && paths + n > most) break;
-        paths += n;
+        p.admit_ms = now_ms();
         used_bytes += p.bytes;
         n_active++;
-        group.push_back(p);
+        ready.push_back(std::move(pending.front()));
         pending.pop_front();
-        if (paths > most) break;  // a large request renders by itself
     }
-    return group;
 }
 
-vzStatus vzServer_st::start(Flight& f, const std::vector<Pending>& group)
+// The requests next in turn, as many as a launch of `most` paths takes; returns
+// their paths.  A request it does not take whole has a launch to itself, of
+// one of as few equal slices as there can be.
+uint64_t vzServer_st::pick(Flight& f, uint64_t most)
 {
-    std::vector<PathItem> items;
-    std::vector<const PathItem*> ptr;
-    items.reserve(group.size());
-    for (const Pending& p : group) items.push_back(PathItem{p.scene, p.params});
-    for (const PathItem& it : items) ptr.push_back(&it);
     uint64_t paths = 0;
-    for (const PathItem& it : items) paths += path_count(it.params, opt);
-    f.slot.used = 0;
-    f.large = group.size() == 1 && paths * kPathBytes > slot_budget;
-    if (f.large) {
-        uint64_t budget = slot_budget;
-        uint32_t passes = 0;
-        VZ_TRY(path_reserve_one(f.slot, items[0], opt, &budget, 0, &passes));
-        return path_enqueue_one(work, f.slot, items[0], opt, passes, false, f.stream, nullptr);
+    while (!ready.empty() && f.shares.size() < kMaxRequests) {
+        Request& r = *ready.front();
+        const uint64_t left = r.left();
+        uint64_t take = (most - std::min(most, paths)) / r.npad;
+        if (take < left) {
+            if (!f.shares.empty()) break;
+            const uint64_t slices = (left + std::max<uint64_t>(take, 1) - 1) / std::max<uint64_t>(take, 1);
+            take = (left + slices - 1) / slices;
+        } else {
+            take = left;
+        }
+        paths += r.npad * take;
+        f.shares.push_back(Share{std::move(ready.front()), r.done, (uint32_t)take});
+        ready.pop_front();
+        if (take < left) break;
     }
-    VZ_TRY(slot_reserve(f.slot, paths));
-    return path_enqueue_many(work, f.slot, ptr.data(), (uint32_t)ptr.size(), opt, false, f.stream);
+    return paths;
 }
 
-// Results of a flight whose launches have finished.
+void vzServer_st::put_back(Flight& f)
+{
+    while (!f.shares.empty()) {
+        ready.push_front(std::move(f.shares.back().r));
+        f.shares.pop_back();
+    }
+}
+
+// Renders the requests next in turn on an idle flight.  VZ_ERROR_OUT_OF_MEMORY:
+// they are back in the queue.
+vzStatus vzServer_st::start(Flight& f)
+{
+    bool alone;
+    {
+        std::lock_guard<std::mutex> lk(mu);
+        alone = ready.size() == 1 && pending.empty() && !others_busy(f);
+    }
+    const uint64_t paths = pick(f, alone ? std::max(alone_paths, launch_paths) : launch_paths);
+    Share& first = f.shares.front();
+    vzStatus rs = slot_reserve(f.slot, paths);
+    if (rs == VZ_SUCCESS && !first.r->carry && first.ns < first.r->item.params.samples_per_pixel) {
+        if (hipMallocAsync((void**)&first.r->carry, carry_bytes(first.r->item.params, first.r->npad), f.stream) !=
+            hipSuccess) {
+            (void)hipGetLastError();
+            first.r->carry = nullptr;
+            ctx->scene_blocks.trim();
+            rs = set_error(VZ_ERROR_OUT_OF_MEMORY, "no memory for the sums of a request");
+        }
+    }
+    if (rs == VZ_SUCCESS) {
+        std::vector<PathSlice> slices;
+        for (const Share& s : f.shares) slices.push_back(PathSlice{&s.r->item, s.s0, s.ns, s.r->carry});
+        f.slot.used = 0;
+        rs = path_enqueue_many(work, f.slot, slices.data(), (uint32_t)slices.size(), opt, false, f.stream);
+    }
+    if (rs == VZ_ERROR_OUT_OF_MEMORY) {
+        put_back(f);
+        return rs;
+    }
+    if (rs == VZ_SUCCESS && hipEventRecord(f.done.e, f.stream) != hipSuccess)
+        rs = set_error(VZ_ERROR_HIP, "hipEventRecord failed");
+    for (Share& s : f.shares) s.r->done += s.ns;
+    return rs;
+}
+
+// A flight's launch has finished.
 void vzServer_st::harvest(Flight& f)
 {
     std::lock_guard<std::mutex> lk(mu);
-    const double t = now_ms();
-    for (size_t i = 0; i < f.active.size(); i++) {
-        const Active& a = f.active[i];
-        release_scene(a.scene);
-        vzRequestResult r{};
-        r.request_id = a.id;
-        r.submit_ms = a.submit_ms;
-        r.admit_ms = a.admit_ms;
-        r.finish_ms = t;
-        r.segments = f.large ? f.slot.h_totals[0] : f.slot.h_totals[kPathStats + i];
-        r.status = VZ_SUCCESS;
-        results[a.id] = r;
-        used_bytes -= a.bytes;
+    const uint32_t n = (uint32_t)f.shares.size();
+    for (uint32_t i = 0; i < n; i++) {
+        RequestPtr r = std::move(f.shares[i].r);
+        r->segments += slice_segments(f.slot, n, i);
+        if (r->left()) {
+            ready.push_back(std::move(r));
+            continue;
+        }
+        if (r->carry) (void)hipFreeAsync(r->carry, f.stream);
+        used_bytes -= r->bytes;
         n_active--;
+        finish(*r, VZ_SUCCESS);
     }
-    f.active.clear();
+    f.shares.clear();
     cv_done.notify_all();
 }
 
@@ -203,9 +278,11 @@ void vzServer_st::loop()
     };
     for (;;) {
         bool progress = false, busy = false;
-        // 1. finished launches
+        // 1. finished launches; requests that came meanwhile go before those
+        // whose turn ends
+        admit();
         for (Flight& f : flights) {
-            if (f.active.empty()) continue;
+            if (f.shares.empty()) continue;
             const hipError_t e = hipEventQuery(f.done.e);
             if (e == hipSuccess) {
                 harvest(f);
@@ -218,46 +295,33 @@ void vzServer_st::loop()
                 goto out;
             }
         }
-        // 2. queued requests onto idle slots
+        if (progress) admit();
+        // 2. the next launches onto idle slots
         for (Flight& f : flights) {
-            if (!f.active.empty()) continue;
-            std::vector<Pending> group;
-            {
-                std::lock_guard<std::mutex> lk(mu);
-                if (pending.empty()) break;
-                group = admit();
-                const double t = now_ms();
-                for (const Pending& p : group)
-                    f.active.push_back(Active{p.id, p.scene, p.bytes, p.submit_ms, t});
-                if (group.empty()) {
-                    cv_done.notify_all();  // rejected ones, if any
-                    break;
-                }
-            }
-            const vzStatus s = start(f, group);
-            if (s == VZ_ERROR_CAPACITY || s == VZ_ERROR_OUT_OF_MEMORY) {
-                // nothing of the group was enqueued beyond what the stream
-                // finishes: wait for it, and for memory if others run
-                (void)hipStreamSynchronize(f.stream);
-                std::lock_guard<std::mutex> lk(mu);
-                f.active.clear();
-                for (auto p = group.rbegin(); p != group.rend(); ++p) {
-                    used_bytes -= p->bytes;
+            if (!f.shares.empty() || ready.empty()) continue;
+            const vzStatus s = start(f);
+            if (s == VZ_ERROR_OUT_OF_MEMORY) {
+                if (others_busy(f)) break;  // until one of them has finished
+                // even an idle device does not hold the launch: fewer paths at
+                // a time, down to one pass of one request
+                if (launch_paths > ready.front()->npad || alone_paths > launch_paths) {
+                    launch_paths = std::max<uint64_t>(std::min(launch_paths, alone_paths) / 2, 1);
+                    alone_paths = launch_paths;
+                } else {
+                    std::lock_guard<std::mutex> lk(mu);
+                    Request& r = *ready.front();
+                    if (r.carry) (void)hipFreeAsync(r.carry, f.stream);
+                    used_bytes -= r.bytes;
                     n_active--;
-                    if (busy || group.size() > 1) pending.push_front(*p);
-                    else reject(*p, s);
+                    finish(r, s);
+                    ready.pop_front();
+                    cv_done.notify_all();
                 }
-                if (!busy && group.size() > 1) {
-                    // even an idle device does not hold the group: fewer at a time
-                    slot_budget = std::max<uint64_t>(slot_budget / 2, kPathBytes);
-                    progress = true;
-                }
-                cv_done.notify_all();
+                progress = true;
                 break;
             }
-            if (s != VZ_SUCCESS || hipEventRecord(f.done.e, f.stream) != hipSuccess) {
-                if (s == VZ_SUCCESS) set_error(VZ_ERROR_HIP, "hipEventRecord failed");
-                fail(VZ_ERROR_HIP);
+            if (s != VZ_SUCCESS) {
+                fail(s);
                 goto out;
             }
             progress = busy = true;
@@ -267,12 +331,10 @@ void vzServer_st::loop()
         std::unique_lock<std::mutex> lk(mu);
         if (busy) {
             cv_work.wait_for(lk, std::chrono::microseconds(20));
-        } else {
-            if (pending.empty()) {
-                cv_done.notify_all();
-                if (stop) break;
-                cv_work.wait(lk, [&] { return stop || !pending.empty(); });
-            }
+        } else if (pending.empty()) {
+            cv_done.notify_all();
+            if (stop) break;
+            cv_work.wait(lk, [&] { return stop || !pending.empty(); });
         }
     }
 out:
@@ -299,7 +361,9 @@ vzStatus vzServerCreate(vzContext ctx, const vzServeConfig* cfg, vzServer* out)
     s->opt.tile_h = t.tile_h ? t.tile_h : 8u;
     s->opt.refill = std::min<uint32_t>(t.refill_lanes, 65u);  // 0: the kernel variant's default
     const uint32_t n = std::min<uint32_t>(kServeStreams, s->cfg.max_active);
-    s->slot_budget = tuning_budget(t) / kServeStreams;
+    const uint64_t slot_paths = std::max<uint64_t>(tuning_budget(t) / kServeStreams / kPathBytes, 1);
+    s->launch_paths = std::min(kServePaths, slot_paths);
+    s->alone_paths = slot_paths;
     vzStatus rs;
     {
         std::lock_guard<std::mutex> lk(ctx->mu);
@@ -311,7 +375,7 @@ vzStatus vzServerCreate(vzContext ctx, const vzServeConfig* cfg, vzServer* out)
         if (rs == VZ_SUCCESS && hipStreamCreateWithFlags(&f.stream, hipStreamNonBlocking) != hipSuccess)
             rs = set_error(VZ_ERROR_HIP, "hipStreamCreateWithFlags failed");
         if (rs == VZ_SUCCESS) rs = f.slot.init(ctx, true);
-        if (rs == VZ_SUCCESS) rs = slot_reserve(f.slot, s->slot_budget / kPathBytes);
+        if (rs == VZ_SUCCESS) rs = slot_reserve(f.slot, s->launch_paths);
     }
     if (rs != VZ_SUCCESS) {
         delete s;
@@ -332,15 +396,15 @@ vzStatus vzServerSubmit(vzServer srv, vzScene scene, const vzLaunchParams* param
     if (params->flags & VZ_MEGAKERNEL) return set_error(VZ_ERROR_INVALID_VALUE, "VZ_MEGAKERNEL is not a serving mode");
     std::lock_guard<std::mutex> lk(srv->mu);
     if (srv->fatal != VZ_SUCCESS) return set_error(srv->fatal, "server stopped: " + srv->fatal_msg);
-    Pending p;
-    p.id = srv->next_id++;
-    p.scene = scene;
+    RequestPtr p(new Request());
+    p->id = srv->next_id++;
+    p->item = PathItem{scene, *params};
     scene->server_refs.fetch_add(1);  // vzSceneDestroy refuses until the request is done
-    p.params = *params;
-    p.bytes = request_bytes(*params);
-    p.submit_ms = srv->now_ms();
-    srv->pending.push_back(p);
-    *request_id = p.id;
+    p->bytes = request_bytes(*params);
+    p->npad = padded_pixels(*params, srv->opt);
+    p->submit_ms = srv->now_ms();
+    *request_id = p->id;
+    srv->pending.push_back(std::move(p));
     srv->cv_work.notify_one();
     return VZ_SUCCESS;
 }
@@ -379,12 +443,9 @@ vzStatus vzServerDestroy(vzServer srv)
         srv->cv_work.notify_all();
     }
     if (srv->worker.joinable()) srv->worker.join();
-    // after a fatal error requests may remain; they will never run
-    for (const Pending& p : srv->pending) vzServer_st::release_scene(p.scene);
-    for (const Flight& f : srv->flights)
-        for (const Active& a : f.active) vzServer_st::release_scene(a.scene);
-    srv->ctx->live_servers--;
+    vzContext ctx = srv->ctx;
     delete srv;
+    ctx->live_servers--;
     return VZ_SUCCESS;
 }
 
