@@ -226,10 +226,12 @@ vzStatus vzDefaultTuning(vzContext ctx, vzTuning* out);
  * rendered a slice of its samples at a time, after each of which the others
  * have their turn; requests of one launch finish together. */
 typedef struct vzServeConfig {
-    uint64_t hbm_budget_bytes;   /* admission budget: requests are admitted while the sum of their
-                                    vzRequestFootprint fits (the server's own buffers are sized by
-                                    the tuning's queue_capacity).  Scenes are the caller's and already resident;
-                                    they are not counted (vzAccelInfo.device_bytes gives theirs) */
+    uint64_t hbm_budget_bytes;   /* what the server allocates for its requests stays within it, beside
+                                    about 1 MB of tables (0: half the GPU's memory).  Requests are
+                                    admitted while the sum of their footprints (vzRequestFootprint)
+                                    fits, and refused if their own does not.  Scenes are the caller's
+                                    and already resident; they are not counted
+                                    (vzAccelInfo.device_bytes gives theirs) */
     uint32_t max_active;         /* max requests admitted at a time (<= 1024) */
     vzTuning tuning;             /* 0 fields take the serving defaults: 48M x 96 bytes, 8x8 tiles */
 } vzServeConfig;
@@ -256,7 +258,10 @@ vzStatus vzServerDrain(vzServer srv);
 /* Finishes every submitted request, then stops the loop and frees the
  * server's buffers and streams. */
 vzStatus vzServerDestroy(vzServer srv);
-/* Bytes of device memory a request of these params needs (admission). */
+/* Bytes of device memory a server of the default tuning takes for a request of
+ * these params: 16 for each path of one slice of its samples (768 MiB at most,
+ * or one sample), and its sums and camera seeds, 16 or 28 a pixel, if there are
+ * several slices.  Pixels count with their tiles' padding. */
 uint64_t vzRequestFootprint(const vzLaunchParams* params);
 
 /* ---- wire format (input of the serving form) ------------------------

@@ -53,3 +53,26 @@ def test_sliced_requests_equal_plain_launches(ctx, book, kind):
     srv.close()
     sc.close()
     other.close()
+
+
+# budgets of one footprint and of a little more: slots that shrink and grow
+# between a request of several slices and small ones
+@pytest.mark.parametrize("factor", [1.0, 1.4, 2.5])
+def test_tight_budget_same_results(ctx, book, factor):
+    print(f"case: served within a budget of {factor} footprints", flush=True)
+    sc = api.Scene(ctx, *book)
+    jobs, want = [], []
+    for w, h, spp in [(640, 480, 40), (61, 33, 4), (512, 512, 20), (640, 480, 40), (900, 301, 33)]:
+        t = GpuTarget(w, h)
+        p = t.bind(gpu_params(w, h, spp, 5, book_lookat(w, h)))
+        sc.launch(p)
+        want.append(sha(t.accum_host()))
+        t.accum.zero()
+        jobs.append((p, t))
+    srv = api.Server(ctx, int(factor * max(api.footprint(p) for p, _ in jobs)), tuning=api.Tuning(queue_capacity=1))
+    ids = [srv.submit(sc, p) for p, _ in jobs]
+    srv.drain()
+    assert [srv.poll(i).status for i in ids] == [0] * len(ids)
+    assert [sha(t.accum_host()) for _, t in jobs] == want
+    srv.close()
+    sc.close()

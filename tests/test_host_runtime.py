@@ -215,3 +215,35 @@ assert all(srv.poll(i).status == 0 for i in large)
 assert hip.host_hip_launches("k_path_resolve") > 2 * 40    # in slices
 srv.close()
 """)
+
+
+def test_server_memory_stays_within_its_budget(stand_in):
+    """What a server allocates for its requests is within hbm_budget_bytes
+    (beside 2 MB of tables), for budgets from one small request's footprint to
+    the default buffers', and each of them is rendered; a request whose own
+    footprint is above the budget is refused."""
+    run(stand_in, """
+TABLES = 2 * MB
+small = params(96, 64, 4)
+fp = lambda p: api.footprint(p)
+assert fp(small) == 96 * 64 * 4 * 16 + 256                      # seeds and radiances of its paths
+sliced = params(2048, 2048, 100, api.ACCUM_FP64)                # 9 slices of at most 12 passes
+px = 2048 * 2048
+assert fp(sliced) == px * 12 * 16 + 256 + px * 28
+big = [params(2048, 2048, 7), params(1024, 1024, 64), sliced, params(512, 512, 16), params(1920, 1080, 300)]
+mixes = [(fp(small), [small] * 5), (fp(small) * 3 // 2, [small] * 5),
+         (max(map(fp, big)), big * 2 + [small] * 20), (1 << 30, big * 3), (2 << 30, big * 4), (64 << 30, big * 2)]
+for budget, reqs in mixes:
+    for tuning in (None, api.Tuning(queue_capacity=1)):
+        base = hip.host_hip_used()
+        hip.host_hip_reset_peak()
+        srv = api.Server(ctx, budget, tuning=tuning)
+        over = srv.submit(scene, params(8192, 8192, 256)) if budget < 4 << 30 else None
+        ids = [srv.submit(scene, p) for p in reqs]
+        srv.drain()
+        assert [srv.poll(i).status for i in ids] == [0] * len(ids), budget
+        assert over is None or srv.poll(over).status == 5
+        assert hip.host_hip_peak() - base <= budget + TABLES, (budget, tuning, hip.host_hip_peak() - base)
+        srv.close()
+        assert hip.host_hip_used() <= base
+""")

@@ -25,6 +25,18 @@ constexpr uint64_t kPlainBudget = 4ull << 30;
 constexpr uint64_t kMaxSlotBudget = 16ull << 30;
 constexpr uint64_t kMaxLaunchPaths = 0xFFFFFF00ull;  // a path's index has 32 bits
 
+// Paths of a server's launch at most while other requests wait; one that has the server
+// to itself takes as many as the slot may hold, since its slices follow one
+// another and each leaves the GPU idle at its end (1080p at 512 samples: 473 ms
+// in launches of 128M, 493 of 64M).  A launch's requests finish together and the
+// next in turn start after it: with 16M, 32M, 48M, 64M and 128M the same burst
+// takes 147.9, 143.6, 140.8, 139.5 and 139.4 ms, 600 such requests at 0.8 of
+// the capacity have a p50 of 102, 174, 234, 292 and 489 ms, and 256x256 at 4
+// samples behind two frames of 1080p at 512 samples 11, 25, 24, 10 to 39 and 38
+// to 165 ms.  (Requests up to 150M paths whole, in order of arrival: 141.2 ms,
+// 923 ms and 730 ms.)
+constexpr uint64_t kServePaths = 48u << 20;
+
 struct PathReq {               // one request of a launch, read by scalar loads
     Cam cam;
     uint32_t subframe, max_depth, spp, fp64;
@@ -94,10 +106,6 @@ struct PathWork {              // what a context keeps between launches
 vzStatus path_work(vzContext ctx, PathWork** out);
 
 Cam make_cam(const vzLaunchParams& p);
-// The device memory a served request is admitted by: a ring of its passes
-// (at most max_depth + 2), its per-pixel sums and camera seeds.
-size_t request_bytes(const vzLaunchParams& p);
-
 // Pixels of a request with its tiles' padding, and its paths.
 uint64_t padded_pixels(const vzLaunchParams& p, const PathOptions& opt);
 uint64_t path_count(const vzLaunchParams& p, const PathOptions& opt);
@@ -105,9 +113,17 @@ uint64_t path_count(const vzLaunchParams& p, const PathOptions& opt);
 uint64_t carry_bytes(const vzLaunchParams& p, uint64_t npad);
 // Bytes of a slot for launches of up to `paths` paths.
 inline uint64_t slot_bytes(uint64_t paths) { return paths * kPathBytes + 256; }
+// Passes of the next slice of `passes` that are left, where a launch takes at
+// most `most` paths: of as few equal slices as there can be.
+uint64_t slice_passes(uint64_t passes, uint64_t npad, uint64_t most);
+// The device memory a served request is admitted by: the paths of one of its
+// slices, and what they carry if there are several.
+size_t request_bytes(const vzLaunchParams& p, const PathOptions& opt, uint64_t most);
 // Makes room in the slot for launches of up to `paths` paths; nothing on its
 // stream may still run.
 vzStatus slot_reserve(PathSlot& s, uint64_t paths);
+// Gives the buffer back (likewise).
+void slot_drop(PathSlot& s);
 // Makes room for a request's launches, of *passes passes each: as many as fit
 // *budget bytes, fewer where the memory is not there (*budget is then what
 // they take), with room for at least `least` paths.  Nothing on the slot's

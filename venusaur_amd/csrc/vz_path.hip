@@ -685,13 +685,17 @@ Cam make_cam(const vzLaunchParams& p)
     return c;
 }
 
-size_t request_bytes(const vzLaunchParams& p)
+uint64_t slice_passes(uint64_t passes, uint64_t npad, uint64_t most)
 {
-    const size_t npix = (size_t)p.width * p.height;
-    const size_t K = std::min<uint32_t>(std::min<uint32_t>(p.max_depth + 2u, p.samples_per_pixel), 255u);
-    const bool fp64 = (p.flags & VZ_ACCUM_FP64) != 0;
-    return align256(K * 3 * npix * 4) + align256(3 * npix * (fp64 ? 8 : 4)) + align256(npix * 4) + align256(K * 4) +
-           align256(K * 8) + 1024;
+    const uint64_t take = std::max<uint64_t>(most / npad, 1);
+    const uint64_t slices = (passes + take - 1) / take;
+    return (passes + slices - 1) / slices;
+}
+
+size_t request_bytes(const vzLaunchParams& p, const PathOptions& opt, uint64_t most)
+{
+    const uint64_t npad = padded_pixels(p, opt), passes = slice_passes(p.samples_per_pixel, npad, most);
+    return slot_bytes(npad * passes) + (passes < p.samples_per_pixel ? carry_bytes(p, npad) : 0);
 }
 
 vzStatus PathSlot::init(vzContext c, bool table)
@@ -755,6 +759,8 @@ uint64_t path_count(const vzLaunchParams& p, const PathOptions& opt)
 {
     return padded_pixels(p, opt) * p.samples_per_pixel;
 }
+
+void slot_drop(PathSlot& s) { drop(&s.paths, &s.paths_bytes); }
 
 vzStatus slot_reserve(PathSlot& s, uint64_t paths)
 {

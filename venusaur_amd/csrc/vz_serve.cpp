@@ -42,6 +42,7 @@ struct Request {
     double submit_ms, admit_ms = 0.0;
     uint32_t done = 0;          // passes rendered or in flight
     char* carry = nullptr;      // what its slices hand on
+    size_t carry_size = 0;
     unsigned long long segments = 0;
 
     uint32_t left() const { return item.params.samples_per_pixel - done; }
@@ -66,17 +67,6 @@ struct Flight {
 // pixels square, 4 to 64 samples, one of 1088) takes 147.9 ms with 2 and 150.3
 // with 3 at 16M paths a launch, 143.6 and 145.4 at 32M.
 constexpr uint32_t kServeStreams = 2;
-// Paths of a launch at most while other requests wait; one that has the server
-// to itself takes as many as the slot may hold, since its slices follow one
-// another and each leaves the GPU idle at its end (1080p at 512 samples: 473 ms
-// in launches of 128M, 493 of 64M).  A launch's requests finish together and the
-// next in turn start after it: with 16M, 32M, 48M, 64M and 128M the same burst
-// takes 147.9, 143.6, 140.8, 139.5 and 139.4 ms, 600 such requests at 0.8 of
-// the capacity have a p50 of 102, 174, 234, 292 and 489 ms, and 256x256 at 4
-// samples behind two frames of 1080p at 512 samples 11, 25, 24, 10 to 39 and 38
-// to 165 ms.  (Requests up to 150M paths whole, in order of arrival: 141.2 ms,
-// 923 ms and 730 ms.)
-constexpr uint64_t kServePaths = 48u << 20;
 
 }  // namespace
 
@@ -85,7 +75,8 @@ struct vzServer_st {
     vzServeConfig cfg{};
     PathWork* work = nullptr;
     PathOptions opt;
-    uint64_t launch_paths = kServePaths, alone_paths = kServePaths;
+    uint64_t request_paths = kServePaths;  // of a slice, by the tuning
+    uint64_t launch_paths = kServePaths, alone_paths = kServePaths;  // lower where memory is short (the worker's)
     std::vector<Flight> flights;
     std::thread worker;
     std::mutex mu;
@@ -95,7 +86,8 @@ struct vzServer_st {
     std::unordered_map<uint64_t, vzRequestResult> results;
     size_t n_active = 0;
     uint64_t next_id = 1;
-    size_t used_bytes = 0;
+    size_t used_bytes = 0;             // footprints of the admitted
+    size_t carried = 0;                // allocated for slices (the worker's)
     bool stop = false;
     vzStatus fatal = VZ_SUCCESS;
     std::string fatal_msg;
@@ -108,6 +100,14 @@ struct vzServer_st {
     void loop();
     void admit();
     uint64_t pick(Flight& f, uint64_t most);
+    bool make_room(Flight& f, size_t slot, size_t carry);
+    void free_carry(Request& r, hipStream_t st)
+    {
+        if (!r.carry) return;
+        (void)hipFreeAsync(r.carry, st);
+        carried -= r.carry_size;
+        r.carry = nullptr;
+    }
     vzStatus start(Flight& f);
     void put_back(Flight& f);
     void harvest(Flight& f);
@@ -147,10 +147,10 @@ struct vzServer_st {
             if (f.stream) (void)hipStreamDestroy(f.stream);
         }
     }
-    void drop(const Request& r)
+    void drop(Request& r)
     {
         release_scene(r);
-        if (r.carry) (void)hipFreeAsync(r.carry, flights.front().stream);
+        free_carry(r, flights.front().stream);
     }
 };
 
@@ -184,13 +184,10 @@ uint64_t vzServer_st::pick(Flight& f, uint64_t most)
     while (!ready.empty() && f.shares.size() < kMaxRequests) {
         Request& r = *ready.front();
         const uint64_t left = r.left();
-        uint64_t take = (most - std::min(most, paths)) / r.npad;
-        if (take < left) {
+        uint64_t take = left;
+        if (paths + r.npad * left > most) {
             if (!f.shares.empty()) break;
-            const uint64_t slices = (left + std::max<uint64_t>(take, 1) - 1) / std::max<uint64_t>(take, 1);
-            take = (left + slices - 1) / slices;
-        } else {
-            take = left;
+            take = slice_passes(left, r.npad, most);
         }
         paths += r.npad * take;
         f.shares.push_back(Share{std::move(ready.front()), r.done, (uint32_t)take});
@@ -208,6 +205,25 @@ void vzServer_st::put_back(Flight& f)
     }
 }
 
+// Whether the budget has room for a flight's slot of `slot` bytes and `carry`
+// more for slices.  Slots keep the size of their largest launch; where that
+// leaves no room, those of idle flights go.
+bool vzServer_st::make_room(Flight& f, size_t slot, size_t carry)
+{
+    for (;;) {
+        size_t total = carried + carry + std::max(slot, f.slot.paths_bytes);
+        Flight* idle = f.slot.paths_bytes > slot ? &f : nullptr;
+        for (Flight& o : flights) {
+            if (&o == &f) continue;
+            total += o.slot.paths_bytes;
+            if (o.shares.empty() && o.slot.paths_bytes) idle = &o;
+        }
+        if (total <= cfg.hbm_budget_bytes) return true;
+        if (!idle) return false;
+        slot_drop(idle->slot);
+    }
+}
+
 // Renders the requests next in turn on an idle flight.  VZ_ERROR_OUT_OF_MEMORY:
 // they are back in the queue.
 vzStatus vzServer_st::start(Flight& f)
@@ -217,14 +233,27 @@ vzStatus vzServer_st::start(Flight& f)
         std::lock_guard<std::mutex> lk(mu);
         alone = ready.size() == 1 && pending.empty() && !others_busy(f);
     }
-    const uint64_t paths = pick(f, alone ? std::max(alone_paths, launch_paths) : launch_paths);
-    Share& first = f.shares.front();
-    vzStatus rs = slot_reserve(f.slot, paths);
-    if (rs == VZ_SUCCESS && !first.r->carry && first.ns < first.r->item.params.samples_per_pixel) {
-        if (hipMallocAsync((void**)&first.r->carry, carry_bytes(first.r->item.params, first.r->npad), f.stream) !=
-            hipSuccess) {
+    uint64_t paths = 0;
+    size_t carry = 0;
+    vzStatus rs = VZ_SUCCESS;
+    for (;;) {
+        paths = pick(f, alone ? std::max(alone_paths, launch_paths) : launch_paths);
+        const Share& s = f.shares.front();
+        carry = !s.r->carry && s.ns < s.r->item.params.samples_per_pixel ? carry_bytes(s.r->item.params, s.r->npad) : 0;
+        if (make_room(f, slot_bytes(paths), carry)) break;
+        put_back(f);
+        if (!alone) return set_error(VZ_ERROR_OUT_OF_MEMORY, "the budget has no room for a launch");
+        alone = false;
+    }
+    Request& first = *f.shares.front().r;
+    rs = slot_reserve(f.slot, paths);
+    if (rs == VZ_SUCCESS && carry) {
+        if (hipMallocAsync((void**)&first.carry, carry, f.stream) == hipSuccess) {
+            first.carry_size = carry;
+            carried += carry;
+        } else {
             (void)hipGetLastError();
-            first.r->carry = nullptr;
+            first.carry = nullptr;
             ctx->scene_blocks.trim();
             rs = set_error(VZ_ERROR_OUT_OF_MEMORY, "no memory for the sums of a request");
         }
@@ -257,7 +286,7 @@ void vzServer_st::harvest(Flight& f)
             ready.push_back(std::move(r));
             continue;
         }
-        if (r->carry) (void)hipFreeAsync(r->carry, f.stream);
+        free_carry(*r, f.stream);
         used_bytes -= r->bytes;
         n_active--;
         finish(*r, VZ_SUCCESS);
@@ -310,7 +339,7 @@ void vzServer_st::loop()
                 } else {
                     std::lock_guard<std::mutex> lk(mu);
                     Request& r = *ready.front();
-                    if (r.carry) (void)hipFreeAsync(r.carry, f.stream);
+                    free_carry(r, f.stream);
                     used_bytes -= r.bytes;
                     n_active--;
                     finish(r, s);
@@ -362,8 +391,11 @@ vzStatus vzServerCreate(vzContext ctx, const vzServeConfig* cfg, vzServer* out)
     s->opt.refill = std::min<uint32_t>(t.refill_lanes, 65u);  // 0: the kernel variant's default
     const uint32_t n = std::min<uint32_t>(kServeStreams, s->cfg.max_active);
     const uint64_t slot_paths = std::max<uint64_t>(tuning_budget(t) / kServeStreams / kPathBytes, 1);
-    s->launch_paths = std::min(kServePaths, slot_paths);
+    s->request_paths = s->launch_paths = std::min(kServePaths, slot_paths);
     s->alone_paths = slot_paths;
+    // what a flight starts with; larger ones as launches need them
+    const uint64_t share = s->cfg.hbm_budget_bytes / kServeStreams;
+    const uint64_t first = std::min(s->launch_paths, share > slot_bytes(0) ? (share - slot_bytes(0)) / kPathBytes : 0);
     vzStatus rs;
     {
         std::lock_guard<std::mutex> lk(ctx->mu);
@@ -375,7 +407,7 @@ vzStatus vzServerCreate(vzContext ctx, const vzServeConfig* cfg, vzServer* out)
         if (rs == VZ_SUCCESS && hipStreamCreateWithFlags(&f.stream, hipStreamNonBlocking) != hipSuccess)
             rs = set_error(VZ_ERROR_HIP, "hipStreamCreateWithFlags failed");
         if (rs == VZ_SUCCESS) rs = f.slot.init(ctx, true);
-        if (rs == VZ_SUCCESS) rs = slot_reserve(f.slot, s->launch_paths);
+        if (rs == VZ_SUCCESS) rs = slot_reserve(f.slot, first);
     }
     if (rs != VZ_SUCCESS) {
         delete s;
@@ -400,7 +432,7 @@ vzStatus vzServerSubmit(vzServer srv, vzScene scene, const vzLaunchParams* param
     p->id = srv->next_id++;
     p->item = PathItem{scene, *params};
     scene->server_refs.fetch_add(1);  // vzSceneDestroy refuses until the request is done
-    p->bytes = request_bytes(*params);
+    p->bytes = request_bytes(*params, srv->opt, srv->request_paths);
     p->npad = padded_pixels(*params, srv->opt);
     p->submit_ms = srv->now_ms();
     *request_id = p->id;
