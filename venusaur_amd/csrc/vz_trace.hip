@@ -49,8 +49,9 @@ __global__ void __launch_bounds__(kTraceBlk) k_trace(SceneView sc, const vzRay* 
     if (i < n) {
         const float4* rp = reinterpret_cast<const float4*>(rays + i);
         float4 a = rp[0], b = rp[1];
+        Overflow ov;
         TraceResult r = closest_hit<S, COUNT>(sc, mk(a.x, a.y, a.z), mk(b.x, b.y, b.z), a.w, b.w,
-                                              s_node + threadIdx.x, s_t + threadIdx.x, kTraceBlk, nv, ns);
+                                              s_node + threadIdx.x, s_t + threadIdx.x, kTraceBlk, ov, nv, ns);
         uint32_t prim = r.leaf == 0xFFFFFFFFu ? VZ_MISS : (sc.leaf_info[r.leaf] & 0x3FFFFFFFu);
         reinterpret_cast<uint2*>(hits)[i] = make_uint2(__float_as_uint(r.t), prim);
         seg = 1;
@@ -108,6 +109,11 @@ __global__ void __launch_bounds__(kTraceBlk) k_trace_reduce(const unsigned long 
 // 355 -> 207 us, 131072 in 200k spheres 457 -> 317 us.  Packets of 64 keep
 // neighbouring rays together: 81 us with packets of 16, 73 us with an equal
 // share of consecutive rays per wave.
+//
+// Rays whose closest hit depends on the order of the tests (ordered) are left
+// to the end of their wave and walked as before, so that hits with and without
+// stats agree for every ray.  Sorting them out costs a million ordinary rays 1
+// us of 81.
 constexpr uint32_t kTraceLdsBlk = 768;
 constexpr uint32_t kTraceMemBlk = kMemThreads;
 constexpr uint32_t kTraceRefill = 32;
@@ -126,18 +132,27 @@ k_trace_hits(SceneView view, const vzRay* __restrict__ rays, uint32_t n, vzHit* 
     const uint32_t tid = threadIdx.x, wave = (uint32_t)__builtin_amdgcn_readfirstlane(tid >> 6);
     const typename std::conditional<LDSN, PlaneBound, TraceNoBound>::type pb(view);
     const SceneArrays sc = scene_arrays<false>(view);
+    float bound = 0.0f;
+    if (LDSN || view.nw != 0u) {
+        const v3 m = plane_bounds(view);
+        bound = fmaxf(fmaxf(m.x, m.y), m.z);
+    }
     if constexpr (LDSN) {
         stage_scene(view, sh);
         __syncthreads();
     }
     typename std::conditional<LDSN, LdsTraversal<NT, true>, MemTraversal<NT, true>>::type tr;
-    typename std::conditional<LDSN, LdsOverflow, MemOverflow>::type ov;
+    union {  // one after the other
+        typename std::conditional<LDSN, LdsOverflow, MemOverflow>::type ov;
+        Overflow odd_ov;
+    };
     tr.npend = 0;
     uint32_t mine = 0;
     bool active = false, tdone = false;
     // the wave's next ray, the end of its packet and the packets' stride
-    const uint32_t stride = gridDim.x * NT;
-    uint32_t base = (wave * gridDim.x + blockIdx.x) * 64u, cur = 0;
+    const uint32_t stride = gridDim.x * NT, first = (wave * gridDim.x + blockIdx.x) * 64u;
+    uint32_t base = first, cur = 0;
+    bool odd = false;
     for (;;) {
         for (uint64_t m; base < n && (m = __ballot(!active)) != 0ull;) {
             const uint32_t left = min(64u, n - base) - cur, take = min((uint32_t)__popcll(m), left);
@@ -146,15 +161,19 @@ k_trace_hits(SceneView view, const vzRay* __restrict__ rays, uint32_t n, vzHit* 
                 mine = base + cur + rk;
                 const float4* rp = reinterpret_cast<const float4*>(rays + mine);
                 const float4 a = ldg(rp), b = ldg(rp + 1);
-                if constexpr (LDSN) {
-                    tr.begin(mk(a.x, a.y, a.z), mk(b.x, b.y, b.z), a.w, b.w);
-                    tr.derive(pb);
-                    tdone = false;
+                if (ordered(mk(a.x, a.y, a.z), mk(b.x, b.y, b.z), b.w, bound)) {
+                    if constexpr (LDSN) {
+                        tr.begin(mk(a.x, a.y, a.z), mk(b.x, b.y, b.z), a.w, b.w);
+                        tr.derive(pb);
+                        tdone = false;
+                    } else {
+                        tdone = tr.begin(sc, sh, mk(a.x, a.y, a.z), mk(b.x, b.y, b.z), a.w, b.w);
+                        tr.derive();
+                    }
+                    active = true;
                 } else {
-                    tdone = tr.begin(sc, sh, mk(a.x, a.y, a.z), mk(b.x, b.y, b.z), a.w, b.w);
-                    tr.derive();
+                    odd = true;
                 }
-                active = true;
             }
             cur += take;
             if (take == left) {
@@ -186,6 +205,25 @@ k_trace_hits(SceneView view, const vzRay* __restrict__ rays, uint32_t n, vzHit* 
             reinterpret_cast<uint2*>(hits)[mine] = make_uint2(__float_as_uint(tr.best), prim);
             active = false;
         }
+    }
+    // the wave's rays whose hit depends on the order of the tests, in that
+    // order, on its stacks of before
+    if (__builtin_expect(__ballot(odd) == 0ull, 1)) return;
+    uint32_t* stack;
+    if constexpr (LDSN) stack = &sh.stack[wave][0][__lane_id()];
+    else stack = &sh.node[wave][0][__lane_id()];
+    for (base = first; base < n; base = n - base > stride ? base + stride : n) {
+        mine = base + __lane_id();
+        if (mine >= n) continue;
+        const float4* rp = reinterpret_cast<const float4*>(rays + mine);
+        const float4 a = ldg(rp), b = ldg(rp + 1);
+        const v3 o = mk(a.x, a.y, a.z), d = mk(b.x, b.y, b.z);
+        if (ordered(o, d, b.w, bound)) continue;
+        uint32_t nv = 0, ns = 0;
+        const TraceResult r =
+            closest_hit<4, false>(view, o, d, a.w, b.w, stack, reinterpret_cast<float*>(stack + 4 * 64), 64, odd_ov, nv, ns);
+        const uint32_t prim = r.leaf == 0xFFFFFFFFu ? VZ_MISS : (ldg(view.leaf_info + r.leaf) & 0x3FFFFFFFu);
+        reinterpret_cast<uint2*>(hits)[mine] = make_uint2(__float_as_uint(r.t), prim);
     }
 }
 

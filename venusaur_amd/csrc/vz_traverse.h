@@ -80,6 +80,32 @@ VZ_DEV void keep_nearer(float t, uint32_t leaf, const uint32_t* info, float& bes
     }
 }
 
+// Whether every root of the ray in a scene is a number: with |d| below D and all
+// distances below M, disc's terms stay below 18 (D M)^2, and an infinite root
+// is compared like any other.  Only then does the closest hit not depend on the
+// order of the tests (a root, or a tmax, that is not a number is neither nearer
+// nor farther than others, and culls what comes after it); other rays keep the
+// order of Traversal.  bound: the largest of plane_bounds, 0 for a single
+// sphere, where there is no order.
+VZ_DEV bool ordered(v3 o, v3 d, float tmax, float bound)
+{
+    const float D = fabsf(d.x) + fabsf(d.y) + fabsf(d.z), M = fabsf(o.x) + fabsf(o.y) + fabsf(o.z) + bound;
+    // and each below 2^62, in one test; false for a NaN in any
+    return __builtin_fmaf(D, M, 0.25f * (D + M)) < 0x1p60f && tmax == tmax;
+}
+// At least the largest |coordinate| of a scene's boxes on each axis: every lo
+// plane is at or above the root box's lo corner, every hi plane at most one
+// step of its node's grid above an exact box, and no node's grid is coarser
+// than the root's.
+VZ_DEV v3 plane_bounds(const SceneView& sc)
+{
+    const uint4 A = ldg(sc.tnodes);
+    const float no[3] = {__uint_as_float(A.x), __uint_as_float(A.y), __uint_as_float(A.z)};
+    float m[3];
+    for (int k = 0; k < 3; k++) m[k] = fmaxf(fabsf(no[k]), fabsf(__builtin_fmaf(257.0f, scale_of(A.w, k), no[k])));
+    return mk(m[0], m[1], m[2]);
+}
+
 // The arrays of a scene in memory that a traversal reads, with its nodes null
 // for a single sphere: the 64-byte nodes and the leaves in their order for
 // the traversal that counts, the 48-byte ones and theirs for the others.
@@ -106,8 +132,9 @@ VZ_DEV SceneArrays scene_arrays(const SceneView& sc)
 // only splits an aggregate into registers when nothing in it is indexed
 // dynamically.
 struct Overflow {
-    uint32_t node[kWideOverflow];
-    float t[kWideOverflow];
+    static constexpr uint32_t kSize = kWideOverflow + kWideStackS - 4u;  // beside 4 LDS slots, the fewest
+    uint32_t node[kSize];
+    float t[kSize];
 };
 
 // Resumable traversal of one ray: init() sets it up, every step() visits
@@ -282,7 +309,7 @@ struct Traversal {
         if (m > 1u) {
             // room in the LDS ring for m - 1 entries: the oldest go to the overflow
             while (sp + (m - 1u) - bottom > (uint32_t)S) {
-                if (bottom >= kWideOverflow) return true;
+                if (bottom >= Overflow::kSize) return true;
                 ov.node[bottom] = lds_node[(bottom & (S - 1)) * stride];
                 ov.t[bottom] = lds_t[(bottom & (S - 1)) * stride];
                 bottom++;
@@ -306,11 +333,10 @@ struct Traversal {
 // Whole-ray traversal: init, then step until done.
 template <int S, bool COUNT>
 VZ_DEV TraceResult closest_hit(const SceneView& view, v3 o, v3 d, float tmin, float tmax, uint32_t* lds_node,
-                               float* lds_t, uint32_t stride, uint32_t& nv, uint32_t& ns)
+                               float* lds_t, uint32_t stride, Overflow& ov, uint32_t& nv, uint32_t& ns)
 {
     const SceneArrays sc = scene_arrays<true>(view);
     Traversal<S, COUNT> tr;
-    Overflow ov;
     if (!tr.init(sc, o, d, tmin, tmax, ns))
         while (!tr.step(sc, lds_node, lds_t, stride, ov, nv, ns)) {
         }

@@ -89,20 +89,15 @@ VZ_DEV void stage_scene(const SceneView& sc, LdsScene<NT>& sh)
 }
 
 // 2^-20 of the largest |plane| of a scene on each axis, at least 2^-70 (|1/d|
-// of an ordinary ray is above 2^-41, so that its bound stays a normal number):
-// every lo plane is at or above
-// the root box's lo corner, every hi plane at most one step of its node's
-// grid above an exact box, and no node's grid is coarser than the root's.
+// of an ordinary ray is above 2^-41, so that its bound stays a normal number).
 struct PlaneBound {
     float p[3];
     VZ_DEV explicit PlaneBound(const SceneView& sc)
     {
-        const uint4 A = ldg(sc.tnodes);
-        const float no[3] = {__uint_as_float(A.x), __uint_as_float(A.y), __uint_as_float(A.z)};
-        for (int k = 0; k < 3; k++) {
-            const float s = scale_of(A.w, k);
-            p[k] = fmaxf(0x1p-20f * fmaxf(fabsf(no[k]), fabsf(__builtin_fmaf(257.0f, s, no[k]))), 0x1p-70f);
-        }
+        const v3 m = plane_bounds(sc);
+        p[0] = fmaxf(0x1p-20f * m.x, 0x1p-70f);
+        p[1] = fmaxf(0x1p-20f * m.y, 0x1p-70f);
+        p[2] = fmaxf(0x1p-20f * m.z, 0x1p-70f);
     }
 };
 
