@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 import oracle as O
+from util import GpuTarget, book_lookat, gpu_params
 from venusaur_amd import api
 from venusaur_amd.hipmem import DeviceBuffer
 
@@ -38,7 +39,8 @@ def _rays(s, rng):
 
 def _grow(r, names, by):
     for f in names:
-        r[f] = (r[f].astype(np.float64) * by).astype(np.float32)
+        with np.errstate(over="ignore"):
+            r[f] = (r[f].astype(np.float64) * by).astype(np.float32)
     r["tmin"], r["tmax"] = 0.0, 3e38
 
 
@@ -74,3 +76,60 @@ def test_hits_keep_their_order(ctx, book, kind):
             same_t = (g["t"].view(np.uint32) == want["t"].view(np.uint32)) | (np.isnan(g["t"]) & np.isnan(want["t"]))
             assert same_t.all() and (g["prim"] == want["prim"]).all(), (what, v)
     sc.close()
+
+
+def _odd_launch(what, p, m):
+    if what == "far view":
+        p.w[:] = [x * 1e19 for x in p.w]
+    elif what == "far eye":
+        p.origin[:] = [x * 1e18 for x in p.origin]
+    elif what == "no frame":
+        p.u[:] = [0.0, 0.0, 0.0]
+    elif what == "fuzz":
+        m["type"][5::7], m["fuzz"][5::7] = api.METAL, np.float32(3e38)
+    elif what == "index":
+        m["type"][5::7], m["ir"][5::7] = api.DIELECTRIC, np.float32(np.nan)
+    elif what == "index 0":
+        m["type"][5::7], m["ir"][5::7] = api.DIELECTRIC, np.float32(0.0)
+
+
+# plain, in a batch with an ordinary item, and served, against the megakernel,
+# which walks every ray in the one order
+@pytest.mark.parametrize("kind", ["book", "mem", "far"])
+@pytest.mark.parametrize("what", ["far view", "far eye", "no frame", "fuzz", "index", "index 0", "none"])
+def test_launches_keep_their_order(ctx, book, kind, what):
+    print(f"case: odd launch {kind} {what}", flush=True)
+    s, m = (a.copy() for a in _scene(kind, book))
+    p = gpu_params(96, 54, 4, 8, book_lookat(96, 54))
+    _odd_launch(what, p, m)
+    sc = api.Scene(ctx, s, m)
+    ordinary = api.Scene(ctx, *book)
+    q = gpu_params(96, 54, 4, 8, book_lookat(96, 54))
+    out = []
+    for form in ("mega", "plain", "batch", "serve"):
+        t, u = GpuTarget(96, 54), GpuTarget(96, 54)
+        p.flags = api.MEGAKERNEL if form == "mega" else 0
+        t.bind(p)
+        u.bind(q)
+        if form in ("mega", "plain"):
+            st = sc.launch(p)
+            segs = st.segments
+            ordinary.launch(q)
+            assert form == "mega" or (st.node_visits, st.sphere_tests) == (0, 0)
+        elif form == "batch":
+            st = api.batch_launch(ctx, [(sc, p), (ordinary, q)])
+            assert (st.node_visits, st.sphere_tests) == (0, 0)
+            segs = None
+        else:
+            srv = api.Server(ctx, 1 << 30)
+            ids = [srv.submit(sc, p), srv.submit(ordinary, q)]
+            srv.drain()
+            segs = srv.poll(ids[0]).segments
+            srv.close()
+        out.append((form, segs, t.accum_host(), u.accum_host()))
+    for form, segs, a, b in out[1:]:
+        assert np.array_equal(a, out[0][2], equal_nan=True), form
+        assert np.array_equal(b, out[0][3], equal_nan=True), form
+        assert segs in (None, out[0][1]), form
+    sc.close()
+    ordinary.close()

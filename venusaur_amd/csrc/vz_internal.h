@@ -70,6 +70,8 @@ struct SceneView {           // what kernels need to traverse one scene
     const float4* tmats;
 };
 
+constexpr float kOrderedBound = 0x1p26f;
+
 struct PathWork;
 
 // A HIP event owned by the enclosing scope, so early error returns do not
@@ -197,6 +199,11 @@ struct vzScene_st {
     uint32_t nw = 0;                  // wide nodes
     uint32_t wdepth = 0;              // wide levels from the root to the deepest leaf
     uint32_t builder = 0;             // VZ_BUILD_LBVH or VZ_BUILD_SAH
+    // Every root of a path's rays is a number, given an ordinary camera: the
+    // boxes lie within kOrderedBound and no material makes a direction longer
+    // than 2^22 (fuzz, or index of refraction either way, below 2^20).  Other
+    // scenes keep the one order of tests that their closest hits depend on.
+    bool ordered = true;
     uint32_t depth = 0;
     uint64_t device_bytes = 0;
     double build_ms = 0.0;

@@ -25,6 +25,8 @@
 // A scene of 2 to kSahMaxPrims spheres replaces stages 3 and 5 by a
 // binned-SAH build in one workgroup (k_sah_build) that writes the same node
 // layout, and goes through stages 1, 2 and 7 in one workgroup each.
+#include <cstring>
+
 #include "vz_device.h"
 #include "vz_internal.h"
 
@@ -37,6 +39,7 @@ constexpr int kTile = kBlk * kItems;  // keys per radix tile
 constexpr uint32_t kLocalBit = 0x80000000u;  // parent link flag (see k_karras)
 constexpr uint32_t kLargeKey = 0x40000000u;  // sort-key bit of a large sphere (see k_morton)
 constexpr uint32_t kRefitLeaves = 2048;       // leaves per k_refit_local workgroup
+constexpr uint32_t kOddWord = 16;             // of the counter block: materials out of the ordinary
 
 __device__ __forceinline__ uint32_t lane_id() { return __lane_id(); }
 __device__ __forceinline__ uint32_t mbcnt(uint64_t m)
@@ -155,10 +158,12 @@ __device__ __forceinline__ uint32_t morton_key(const float4 c, const float* grid
 __global__ void __launch_bounds__(kBlk) k_morton(const float4* __restrict__ sph, uint32_t n,
                                                  const float* __restrict__ grid_a,
                                                  const float* __restrict__ grid_b,
-                                                 uint32_t* __restrict__ keys, uint32_t* __restrict__ vals)
+                                                 uint32_t* __restrict__ keys, uint32_t* __restrict__ vals,
+                                                 uint32_t* __restrict__ odd)
 {
     uint32_t i = blockIdx.x * kBlk + threadIdx.x;
     if (i >= n) return;
+    if (i == 0u) *odd = 0u;
     keys[i] = morton_key(sph[i], grid_a, grid_b);
     vals[i] = i;
 }
@@ -305,11 +310,13 @@ __global__ void __launch_bounds__(kBlk) k_radix_scatter(const uint32_t* __restri
 }
 
 // ---- 4. leaf reorder -----------------------------------------------------------
+// *odd: some material may send rays on in directions far longer than the
+// normal, or of no length (see vzScene_st::ordered).
 __global__ void __launch_bounds__(kBlk) k_reorder(const float4* __restrict__ sph_in,
                                                   const vzMaterial* __restrict__ mat_in,
                                                   const uint32_t* __restrict__ perm, uint32_t n,
                                                   float4* __restrict__ sph, uint32_t* __restrict__ info,
-                                                  float4* __restrict__ mat)
+                                                  float4* __restrict__ mat, uint32_t* __restrict__ odd)
 {
     uint32_t i = blockIdx.x * kBlk + threadIdx.x;
     if (i >= n) return;
@@ -320,6 +327,7 @@ __global__ void __launch_bounds__(kBlk) k_reorder(const float4* __restrict__ sph
     info[i] = p | (type << 30);
     float param = type == 1u ? m.fuzz : (type == 2u ? m.ir : 0.0f);
     mat[i] = make_float4(m.albedo[0], m.albedo[1], m.albedo[2], param);
+    if (!(fabsf(param) < 0x1p20f) || (type == 2u && !(fabsf(param) > 0x1p-20f))) *odd = 1u;
 }
 
 // refit reads spheres in leaf order but geometry updates arrive in prim order
@@ -515,11 +523,13 @@ __device__ __forceinline__ void wave_order()
 constexpr uint32_t kSmallThreads = 1024;
 static_assert(kSahMaxPrims <= kSmallThreads, "a thread per sphere");
 __global__ void __launch_bounds__(kSmallThreads) k_small_keys(const float4* __restrict__ sph, uint32_t n,
-                                                              uint32_t* __restrict__ keys, uint32_t* __restrict__ vals)
+                                                              uint32_t* __restrict__ keys, uint32_t* __restrict__ vals,
+                                                              uint32_t* __restrict__ odd)
 {
     __shared__ float part[6][kSmallThreads / 64];
     __shared__ float grid[2][10];
     const uint32_t t = threadIdx.x, w = t / 64;
+    if (t == 0u) *odd = 0u;
     const float4 c = t < n ? sph[t] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     for (uint32_t g = 0; g < 2u; g++) {  // grid A: every centroid; grid B: those of the small spheres
         const bool in = t < n && (g == 0u || !(2.0f * fabsf(c.w) > grid[0][9]));
@@ -1194,7 +1204,9 @@ constexpr uint32_t kLeafCount = kMaxDepth + 2;   // leaves given a place so far
 constexpr uint32_t kWideError = kMaxDepth + 3;   // the structural check's result
 constexpr uint32_t kTreeHeight = kMaxDepth + 4;  // of the binary tree
 constexpr uint32_t kFirstLevel = kMaxDepth + 5;  // first level that k_wide_few left
-constexpr uint32_t kWideWords = kMaxDepth + 6;
+constexpr uint32_t kOddMaterials = kMaxDepth + 6;  // as k_reorder found them
+constexpr uint32_t kBound = kMaxDepth + 7;       // largest |coordinate| of the root box (float)
+constexpr uint32_t kWideWords = kMaxDepth + 8;
 constexpr uint32_t kScanItems = 4;            // root flags per thread in the index scan
 constexpr uint32_t kScanTile = kBlk * kScanItems;
 
@@ -1350,10 +1362,10 @@ __device__ __forceinline__ void few_levels(const LevelArrays& A, uint32_t* cnt, 
 // Clears the level words and sets up level 0: the root, unless the tree is
 // deeper than the host will take.
 __device__ __forceinline__ uint32_t first_level(const LevelArrays& A, uint32_t* cnt, const uint32_t* height,
-                                                FewShared& sh)
+                                                const uint32_t* odd, FewShared& sh)
 {
     const uint32_t t = threadIdx.x, h = height[0], count = h + 1u <= kMaxDepth ? 1u : 0u;
-    if (t < kWideWords) cnt[t] = t == 0u ? count : (t == kTreeHeight ? h : 0u);
+    if (t < kWideWords) cnt[t] = t == 0u ? count : (t == kTreeHeight ? h : (t == kOddMaterials ? *odd : 0u));
     if (t == 0u) {
         A.wflag[0] = kWideRoot;
         A.front[0][0] = 0u;
@@ -1372,12 +1384,12 @@ __device__ __forceinline__ uint32_t first_level(const LevelArrays& A, uint32_t* 
 // take some 4 us each, no longer than a launch.
 constexpr uint32_t kFewRoots = 2048;
 __global__ void __launch_bounds__(kFewThreads) k_wide_few(LevelArrays A, uint32_t* cnt, const uint32_t* height,
-                                                          uint32_t resume, uint32_t mids)
+                                                          const uint32_t* odd, uint32_t resume, uint32_t mids)
 {
     __shared__ FewShared sh;
     uint32_t level = 0, count, before = 0;
     if (!resume) {
-        count = first_level(A, cnt, height, sh);
+        count = first_level(A, cnt, height, odd, sh);
         few_levels(A, cnt, level, count, 0u, kFewRoots, sh);
         if (threadIdx.x == 0u) {
             cnt[kFirstLevel] = level;
@@ -1487,6 +1499,7 @@ struct TravOut {
     float4* sph;            // traversal order, 3 spare at the end
     uint32_t* tinfo;
     float4* tmat;
+    uint32_t* bound;        // see kBound
 };
 
 __device__ __forceinline__ void wide_pack(uint32_t r, const float4* sph, const uint32_t* wkids, const uint32_t* wflag,
@@ -1547,12 +1560,17 @@ __device__ __forceinline__ void wide_pack(uint32_t r, const float4* sph, const u
     v[0] = make_uint4(__float_as_uint(nb[0]), __float_as_uint(nb[1]), __float_as_uint(nb[2]), scales | n_in << 24);
     v[1] = make_uint4(tlo[0], tlo[1], tlo[2], thi[0]);
     v[2] = make_uint4(thi[1], thi[2], 3u * T.tchild[r], leaf0);
-    if (r == 0u)  // the spare leaves are one of the scene's once more
+    if (r == 0u) {
+        float m = 0.0f;
+        for (int k = 0; k < 6; k++) m = fmaxf(m, fabsf(nb[k]));
+        *T.bound = __float_as_uint(m);
+        // the spare leaves are one of the scene's once more
         for (uint32_t k = 0; k < 3; k++) {
             T.sph[T.n + k] = sph[0];
             T.tinfo[T.n + k] = T.info[0];
             T.tmat[T.n + k] = T.mat[0];
         }
+    }
 }
 __global__ void __launch_bounds__(kBlk) k_wide_pack(const float4* __restrict__ sph, const uint32_t* __restrict__ wkids,
                                                     const uint32_t* __restrict__ wflag,
@@ -1795,7 +1813,8 @@ __global__ void __launch_bounds__(kBlk) k_wide_verify(const uint32_t* __restrict
 // once between them: loading and tracing the book scene 440 -> 324 us with
 // k_small_keys.
 __global__ void __launch_bounds__(kSmallThreads) k_wide_small(LevelArrays A, const float4* sph, uint32_t n,
-                                                              uint4* nodes, const uint32_t* height, uint32_t* cnt,
+                                                              uint4* nodes, const uint32_t* height,
+                                                              const uint32_t* odd, uint32_t* cnt,
                                                               uint32_t* widx, uint4* wnodes, TravOut T)
 {
     __shared__ FewShared sh;
@@ -1804,7 +1823,7 @@ __global__ void __launch_bounds__(kSmallThreads) k_wide_small(LevelArrays A, con
     wref[t] = tref[t] = lref[t] = 0u;
     if (t > 0u && t < ni) A.wflag[t] = 0u;
     if (t < ni) pack_node(t, sph, A.child, A.boxes, nodes);
-    uint32_t level = 0, count = first_level(A, cnt, height, sh);
+    uint32_t level = 0, count = first_level(A, cnt, height, odd, sh);
     if (count == 0u) return;
     few_levels(A, cnt, level, count, 0u, 0xFFFFFFFFu, sh);
     const uint32_t fl = t < ni ? A.wflag[t] : 0u;
@@ -1838,10 +1857,11 @@ static vzStatus collapse_wide(vzScene s, hipStream_t st)
     const LevelArrays A{s->d_child, s->d_boxes, {s->d_wfront[0], s->d_wfront[1]}, s->d_wkids, s->d_wflag,
                         s->d_visit, s->d_keys[1], s->d_vals[1]};
     const TravOut T{A.tidx, A.tchild, A.tleaf, s->d_leaf_info, s->d_mat, n, s->d_tnodes, s->d_tsph, s->d_tinfo,
-                    s->d_tmat};
+                    s->d_tmat, cnt + kBound};
+    const uint32_t* odd = s->d_fcount + kOddWord;
     if (n <= kSahMaxPrims) {
         hipLaunchKernelGGL(k_wide_small, dim3(1), dim3(kSmallThreads), 0, st, A, s->d_sph, n, s->d_nodes, s->d_height,
-                           cnt, s->d_widx, s->d_wnodes, T);
+                           odd, cnt, s->d_widx, s->d_wnodes, T);
     } else {
         const dim3 all(blocks_for(n, kBlk));
         hipLaunchKernelGGL(k_pack_nodes, all, dim3(kBlk), 0, st, s->d_sph, s->d_child, s->d_boxes, ni, s->d_nodes);
@@ -1852,10 +1872,10 @@ static vzStatus collapse_wide(vzScene s, hipStream_t st)
         if (ni > kFewRoots)
             for (uint32_t v = ni; v > 4u; v /= 4u) mids++;
         const uint32_t grid = std::min<uint32_t>(1024u, blocks_for(ni, kBlk));
-        hipLaunchKernelGGL(k_wide_few, dim3(1), dim3(kFewThreads), 0, st, A, cnt, s->d_height, 0u, 0u);
+        hipLaunchKernelGGL(k_wide_few, dim3(1), dim3(kFewThreads), 0, st, A, cnt, s->d_height, odd, 0u, 0u);
         for (uint32_t m = 0; m < mids; m++)
             hipLaunchKernelGGL(k_wide_level, dim3(grid), dim3(kBlk), 0, st, A, cnt, m);
-        if (mids) hipLaunchKernelGGL(k_wide_few, dim3(1), dim3(kFewThreads), 0, st, A, cnt, s->d_height, 1u, mids);
+        if (mids) hipLaunchKernelGGL(k_wide_few, dim3(1), dim3(kFewThreads), 0, st, A, cnt, s->d_height, odd, 1u, mids);
         uint32_t* tsum = s->d_widx + ni;
         const uint32_t ntile = blocks_for(ni, kScanTile);
         hipLaunchKernelGGL(k_wscan_tiles, dim3(ntile), dim3(kBlk), 0, st, s->d_wflag, ni, tsum);
@@ -1882,6 +1902,9 @@ static vzStatus collapse_wide(vzScene s, hipStream_t st)
                                                 " exceeds the traversal stack (" +
                                                 std::to_string(kMaxDepth) + ")");
     s->nw = h[kWideCount];
+    float bound;
+    std::memcpy(&bound, &h[kBound], sizeof(bound));
+    s->ordered = h[kOddMaterials] == 0u && bound < kOrderedBound;
     s->wdepth = 1;  // the leaf level below the deepest roots'
     for (uint32_t L = 0; L <= kMaxDepth; L++)
         if (h[L]) s->wdepth = L + 2;
@@ -1925,14 +1948,14 @@ vzStatus lbvh_build(vzScene s, hipStream_t st)
     float* grid_b = fin + 16;
     if (n <= kSahMaxPrims) {
         hipLaunchKernelGGL(k_small_keys, dim3(1), dim3(kSmallThreads), 0, st, s->d_sph_in, n, s->d_keys[0],
-                           s->d_vals[0]);
+                           s->d_vals[0], s->d_fcount + kOddWord);
     } else {
         hipLaunchKernelGGL(k_bounds_partial, dim3(nb), dim3(kBlk), 0, st, s->d_sph_in, n, nullptr, partial);
         hipLaunchKernelGGL(k_bounds_final, dim3(1), dim3(kBlk), 0, st, partial, nb, 0u, fin);
         hipLaunchKernelGGL(k_bounds_partial, dim3(nb), dim3(kBlk), 0, st, s->d_sph_in, n, fin, partial);
         hipLaunchKernelGGL(k_bounds_final, dim3(1), dim3(kBlk), 0, st, partial, nb, 1u, grid_b);
         hipLaunchKernelGGL(k_morton, dim3(blocks_for(n, kBlk)), dim3(kBlk), 0, st, s->d_sph_in, n, fin, grid_b,
-                           s->d_keys[0], s->d_vals[0]);
+                           s->d_keys[0], s->d_vals[0], s->d_fcount + kOddWord);
     }
     s->builder = (n >= 2 && n <= kSahMaxPrims) ? VZ_BUILD_SAH : VZ_BUILD_LBVH;
     // keys and leaf order end in buffers 0 either way
@@ -1971,7 +1994,7 @@ vzStatus lbvh_build(vzScene s, hipStream_t st)
         }
     }
     hipLaunchKernelGGL(k_reorder, dim3(blocks_for(n, kBlk)), dim3(kBlk), 0, st, s->d_sph_in,
-                       s->d_mat_in, s->d_leaf_prim, n, s->d_sph, s->d_leaf_info, s->d_mat);
+                       s->d_mat_in, s->d_leaf_prim, n, s->d_sph, s->d_leaf_info, s->d_mat, s->d_fcount + kOddWord);
     VZ_HIP_TRY(hipGetLastError());
     vzStatus rs = refit_core(s, st);
     VZ_HIP_TRY(hipEventRecord(e1.e, st));

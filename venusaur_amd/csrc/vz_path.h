@@ -86,7 +86,7 @@ struct PathSlice {
 struct PathOptions {
     uint32_t refill = 0;       // 0: the kernel variant's default
     uint32_t tile_w = 8, tile_h = 8;
-    bool count = false;        // count node visits and sphere tests
+    bool count = false;        // count node visits and sphere tests; test spheres in the one order
     std::vector<Event>* events = nullptr;  // appended to: a pair around every k_path launch
 };
 
@@ -106,6 +106,8 @@ struct PathWork {              // what a context keeps between launches
 vzStatus path_work(vzContext ctx, PathWork** out);
 
 Cam make_cam(const vzLaunchParams& p);
+// Whether a request may go through the traversals that do not count.
+bool ordered_paths(const PathItem& item);
 // Pixels of a request with its tiles' padding, and its paths.
 uint64_t padded_pixels(const vzLaunchParams& p, const PathOptions& opt);
 uint64_t path_count(const vzLaunchParams& p, const PathOptions& opt);

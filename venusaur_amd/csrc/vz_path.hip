@@ -662,6 +662,20 @@ uint32_t refill_of(const PathOptions& opt, uint32_t dflt)
 
 uint64_t carry_bytes(const vzLaunchParams& p, uint64_t npad) { return sum_bytes(p, npad) + 4ull * npad; }
 
+// Whether the closest hits of a request's paths are free of the order of the
+// tests (vz_traverse.h, ordered): directions stay below 2^24 and distances
+// below 2^28, so the product keeps far below 2^60.  Other requests go through
+// the traversal that counts, which keeps the order.
+bool ordered_paths(const PathItem& item)
+{
+    if (item.scene->n < 2) return true;
+    const Cam c = make_cam(item.params);
+    auto sum = [](v3 v) { return fabsf(v.x) + fabsf(v.y) + fabsf(v.z); };
+    const float lens = 4.0f * fabsf(c.lr) * (sum(c.un) + sum(c.vn));  // NaN without a frame
+    return item.scene->ordered && 2.0f * (sum(c.U) + sum(c.V) + sum(c.W)) + lens < 0x1p24f &&
+           sum(c.O) + lens < kOrderedBound;
+}
+
 Cam make_cam(const vzLaunchParams& p)
 {
     auto nrm = [](v3 v) {
@@ -897,15 +911,18 @@ unsigned long long slice_segments(const PathSlot& s, uint32_t n, uint32_t i)
 
 // Waits for the launches of a slot, whose buffers are then free for the next
 // ones on any stream, and reads their counters and times.
-static vzStatus finish(PathWork* w, PathSlot& s, vzStatus rs, const std::vector<Event>& ev, hipStream_t st, RunResult* res)
+static vzStatus finish(PathWork* w, PathSlot& s, vzStatus rs, bool visits, const std::vector<Event>& ev, hipStream_t st,
+                       RunResult* res)
 {
     if (hipStreamSynchronize(st) != hipSuccess && rs == VZ_SUCCESS)
         rs = set_error(VZ_ERROR_HIP, "hipStreamSynchronize failed");
     VZ_TRY(rs);
     res->segments = s.h_totals[0];
     res->hits = s.h_totals[1];
-    res->node_visits = s.h_totals[2];
-    res->sphere_tests = s.h_totals[3];
+    if (visits) {  // (others may have been counted on the way)
+        res->node_visits = s.h_totals[2];
+        res->sphere_tests = s.h_totals[3];
+    }
     float ms = 0.0f;
     VZ_HIP_TRY(hipEventElapsedTime(&ms, w->t0.e, w->t1.e));
     res->render_ms = ms;
@@ -924,7 +941,8 @@ vzStatus path_launch(vzContext ctx, const PathItem& item, hipStream_t st, RunRes
     VZ_TRY(w->plain.init(ctx, false));
     std::vector<Event> ev;
     PathOptions opt;
-    opt.count = (item.params.flags & VZ_COUNT_VISITS) != 0;
+    const bool asked = (item.params.flags & VZ_COUNT_VISITS) != 0;
+    opt.count = asked || !ordered_paths(item);
     if (item.params.flags & VZ_TIME_STAGES) opt.events = &ev;
     *res = RunResult();
     res->paths = (unsigned long long)item.params.width * item.params.height * item.params.samples_per_pixel;
@@ -937,7 +955,7 @@ vzStatus path_launch(vzContext ctx, const PathItem& item, hipStream_t st, RunRes
         VZ_HIP_TRY(hipEventRecord(w->t1.e, st));
         return VZ_SUCCESS;
     };
-    return finish(w, w->plain, enqueue(), ev, st, res);
+    return finish(w, w->plain, enqueue(), asked, ev, st, res);
 }
 
 uint64_t tuning_budget(const vzTuning& t)
@@ -963,8 +981,10 @@ vzStatus path_batch(vzContext ctx, const std::vector<PathItem>& items, const vzT
     opt.refill = t.refill_lanes;
     opt.tile_w = t.tile_w;
     opt.tile_h = t.tile_h;
+    bool asked = false;
     for (const PathItem& it : items) {
-        opt.count |= (it.params.flags & VZ_COUNT_VISITS) != 0;
+        asked |= (it.params.flags & VZ_COUNT_VISITS) != 0;
+        opt.count |= asked || !ordered_paths(it);
         if (it.params.flags & VZ_TIME_STAGES) opt.events = &ev;
         res->paths += (unsigned long long)it.params.width * it.params.height * it.params.samples_per_pixel;
     }
@@ -1010,7 +1030,7 @@ vzStatus path_batch(vzContext ctx, const std::vector<PathItem>& items, const vzT
         VZ_HIP_TRY(hipEventRecord(w->t1.e, st));
         return VZ_SUCCESS;
     };
-    VZ_TRY(finish(w, slot, enqueue(), ev, st, res));
+    VZ_TRY(finish(w, slot, enqueue(), asked, ev, st, res));
     return VZ_SUCCESS;
 }
 

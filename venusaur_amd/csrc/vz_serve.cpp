@@ -261,8 +261,10 @@ vzStatus vzServer_st::start(Flight& f)
     if (rs == VZ_SUCCESS) {
         std::vector<PathSlice> slices;
         for (const Share& s : f.shares) slices.push_back(PathSlice{&s.r->item, s.s0, s.ns, s.r->carry});
+        PathOptions o = opt;
+        for (const Share& s : f.shares) o.count |= !ordered_paths(s.r->item);
         f.slot.used = 0;
-        rs = path_enqueue_many(work, f.slot, slices.data(), (uint32_t)slices.size(), opt, false, f.stream);
+        rs = path_enqueue_many(work, f.slot, slices.data(), (uint32_t)slices.size(), o, false, f.stream);
     }
     if (rs == VZ_ERROR_OUT_OF_MEMORY) {
         put_back(f);
