@@ -76,3 +76,31 @@ def test_tight_budget_same_results(ctx, book, factor):
     assert [sha(t.accum_host()) for _, t in jobs] == want
     srv.close()
     sc.close()
+
+
+# the smallest memory a tuning gives a batch is 16M paths: groups of several
+# items and of one, an item that fills it exactly, items above it (in double and
+# float, several chunks each), counted and not
+@pytest.mark.parametrize("count", [False, True])
+def test_batch_groups_and_large_items(ctx, book, count):
+    print(f"case: batch groups and large items, visits counted: {count}", flush=True)
+    scenes = [api.Scene(ctx, *book), api.Scene(ctx, *api.box_scene(3000, 9))]
+    jobs, want, segs = [], [], 0
+    for i, (w, h, spp, fp64) in enumerate([(512, 512, 40, False), (64, 36, 2, False), (512, 512, 24, False),
+                                           (512, 512, 64, False), (640, 480, 70, True), (33, 17, 3, False),
+                                           (1024, 768, 33, False), (256, 256, 8, False)]):
+        t = GpuTarget(w, h, fp64=fp64)
+        flags = (api.ACCUM_FP64 if fp64 else 0) | (api.COUNT_VISITS if count else 0)
+        p = t.bind(gpu_params(w, h, spp, 4, (book_lookat, box_lookat)[i % 2](w, h), flags=flags))
+        segs += scenes[i % 2].launch(p).segments
+        want.append(sha(t.accum_host()))
+        t.accum.zero()
+        jobs.append((scenes[i % 2], p, t))
+    st = api.batch_launch(ctx, [(sc, p) for sc, p, _ in jobs], tuning=api.Tuning(queue_capacity=1))
+    assert st.segments == segs and (st.node_visits > 0) == count
+    # the first two, the third (5120 paths too many for it), the one of exactly
+    # 16M, the last two; and the images of 21.5M and 26M paths in two chunks each
+    assert st.iterations == 4 + 2 + 2, st.iterations
+    assert [sha(t.accum_host()) for _, _, t in jobs] == want
+    for sc in scenes:
+        sc.close()
