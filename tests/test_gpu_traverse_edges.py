@@ -85,3 +85,23 @@ def test_planes_and_interval_ends(ctx, n, lds, away):
         r["tmin"] = end[hit]
         assert _hits(sc, r).tobytes() == O.trace_brute(s, r).tobytes()
     sc.close()
+
+
+# either side of the size from which many workgroups refit the nodes across
+# workgroups' ranges, and of the one it was before
+@pytest.mark.parametrize("n", [393216, 393217, 655360, 655361])
+def test_refit_lines(ctx, n):
+    print(f"case: refit of {n} spheres", flush=True)
+    s, m = api.box_scene(n - 1, 7)
+    sc = api.Scene(ctx, s, m)
+    s["cx"][1:] += np.random.default_rng(n).uniform(-0.2, 0.2, n - 1).astype(np.float32)
+    sc.update_spheres(s)
+    rays = np.zeros(400, api.RAY_DT)
+    rng = np.random.default_rng([n, 1])
+    pick = s[rng.integers(0, n, len(rays))]
+    for f, c in (("ox", "cx"), ("oy", "cy"), ("oz", "cz")):
+        rays[f] = rng.uniform(-100, 100, len(rays))
+        rays["d" + f[1]] = pick[c] - rays[f]
+    rays["tmin"], rays["tmax"] = 0.001, 1e16
+    assert _hits(sc, rays).tobytes() == O.trace_brute(s, rays).tobytes()
+    sc.close()

@@ -1061,8 +1061,9 @@ __global__ void __launch_bounds__(kBlk) k_pack_nodes(const float4* __restrict__ 
 //                  at agent scope, where each step writes back what its L2
 //                  holds dirty (little: the kernel boundary wrote the local
 //                  results back) and so takes some 4 us, but many run at a
-//                  time.  200k spheres: 37 us by one workgroup, 76 by many; a
-//                  million: 190 and 122; the lines cross near 490k.  With
+//                  time.  Whole refits by one workgroup and by many, us: 200k
+//                  spheres 255 and 298, 393k 344 and 381, 550k 422 and 435,
+//                  700k 489 and 498 (504 and 501), a million 673 and 607.  With
 //                  every node at agent scope in one kernel the build of a
 //                  million spheres took 10 ms.
 constexpr uint32_t kLeafItem = 0x80000000u;  // frontier entry is a leaf index
@@ -1143,7 +1144,7 @@ __global__ void __launch_bounds__(kRefitThreads) k_refit_local(const float4* __r
 }
 
 constexpr uint32_t kTopBlocks = 64;
-constexpr uint32_t kTopOneLeaves = 192 * kRefitLeaves;
+constexpr uint32_t kTopOneLeaves = 320 * kRefitLeaves;
 
 template <int SCOPE>  // of the climbs' counters, boxes and heights
 __global__ void __launch_bounds__(kRefitThreads) k_refit_top(const float4* __restrict__ sph,
