@@ -16,7 +16,6 @@
 namespace vz {
 
 static thread_local std::string g_last_error;
-static std::atomic<uint64_t> g_next_scene_uid{1};
 
 vzStatus set_error(vzStatus s, const std::string& msg)
 {
@@ -209,7 +208,6 @@ vzStatus vzSceneCreate(vzContext ctx, const vzSphere* spheres, const vzMaterial*
     vzScene s = new vzScene_st();
     s->ctx = ctx;
     s->n = n;
-    s->uid = g_next_scene_uid.fetch_add(1);
     vzStatus rs = scene_alloc(s);
     hipStream_t st = as_stream(stream);
     if (rs == VZ_SUCCESS && (hipMemcpyAsync(s->d_sph_in, spheres, sizeof(vzSphere) * n, hipMemcpyHostToDevice, st) != hipSuccess ||
@@ -237,7 +235,6 @@ vzStatus vzSceneCreateDevice(vzContext ctx, const vzSphere* spheres, const vzMat
     vzScene s = new vzScene_st();
     s->ctx = ctx;
     s->n = n;
-    s->uid = g_next_scene_uid.fetch_add(1);
     vzStatus rs = scene_alloc(s);
     hipStream_t st = as_stream(stream);
     if (rs == VZ_SUCCESS &&

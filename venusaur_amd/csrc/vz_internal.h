@@ -149,10 +149,6 @@ struct vzContext_st {
 struct vzScene_st {
     vzContext ctx = nullptr;
     uint32_t n = 0;
-    // Unique over the process lifetime: tables that cache a scene's device
-    // view key it by this id, never by the object's address (a destroyed
-    // scene's address can be reused by the next one created).
-    uint64_t uid = 0;
     // Server requests (queued or running) that name this scene; while any
     // remain, vzSceneDestroy refuses.
     std::atomic<uint32_t> server_refs{0};

@@ -437,11 +437,8 @@ static_assert(kSahWaves * kSahBinWords >= (int)kSahMaxPrims, "the bins hold a tr
 // queue from kSahShare spheres up (at most kSahMaxPrims / kSahShare of them),
 // and is finished first otherwise.  Ranges of up to kSahFew spheres are built
 // to the end by sah_few.
-#ifndef SSH
-#define SSH 8
-#endif
 constexpr uint32_t kSahFew = 21;  // times 3 axes in a wave
-constexpr uint32_t kSahShare = SSH;
+constexpr uint32_t kSahShare = 8;
 constexpr uint32_t kSahTasks = 192;
 static_assert(kSahMaxPrims / kSahShare + 1 + kSahSoloWaves <= kSahTasks, "a ticket per task and waiting wave");
 static_assert(kSahShare <= kSahFew, "what a wave finishes first is built by sah_few");
