@@ -102,7 +102,7 @@ static vzStatus scene_alloc(vzScene s)
     return rs;
 }
 
-struct DevCounters {   // per-call counters for the non-engine kernels
+struct DevCounters {   // a call's counters on the device
     unsigned long long* d = nullptr;
     ~DevCounters()
     {

@@ -30,7 +30,7 @@
 // 241 -> 187 ms, 512x512 at 2048 samples in double 355 -> 135 ms, 400x225 at 16
 // samples 2.80 -> 1.12 ms; with the traversals of vz_traverse_lds.h and
 // vz_traverse_mem.h, queued sphere tests, shared shading and the counters below
-// 55.6 ms, 134 ms, 102 ms and 0.66 ms; images bit for bit the same.  What bounds it is VALU
+// 53.8 ms, 134 ms, 106 ms and 0.66 ms; images bit for bit the same.  What bounds it is VALU
 // issue at half the lanes with the scene in LDS, the L1 and the latency of
 // node loads as well with it in memory, and the longest path at the end of a
 // small frame.  k_path_seeds and k_path_resolve are under 1% each of the
@@ -58,32 +58,32 @@ constexpr int kStackS = kWideStackS;  // LDS stack slots per lane
 constexpr int kBlk = 256;
 constexpr uint32_t kMaxPathBlocks = 8192;
 // A wave leaves the traversal to shade and take new paths once fewer than
-// this many of its lanes still trace.  Nodes in LDS, 1080p book frame: 66.2
-// ms at 1, 61.7 at 5, 61.3 at 9, 61.4 at 13, 62.1 at 17, 64.6 at 25.  Many
-// scenes in memory, 24-scene batch: 141 ms at 9, 128 at 17, 121 at 25, 117 at
-// 33, 115 at 41, 119 at 49 (64-byte nodes, 24 waves); 93.3 at 33, 93.4 at 41,
-// 93.5 at 49 now, where a million spheres take 143.9, 142.9 and 146.6.
+// this many of its lanes still trace.  Nodes in LDS, 1080p book frame: 54.1
+// ms at 5, 53.8 at 9, 54.6 at 17 (66.2, 61.3 and 64.6 at 1, 9 and 25 as first
+// built).  Nodes in memory: a million spheres 136.4 ms at 33, 134.0 at 41,
+// 134.3 at 49, a 24-scene batch 90.5, 90.5 and 90.3 (141, 128 and 115 at 9, 17
+// and 41 as first built).
 constexpr uint32_t kRefillLds = 9;
 constexpr uint32_t kRefillGlobal = 41;
 // Queued sphere tests run once two thirds of the tracing lanes hold some:
-// 1080p book frame 61.1 ms against 61.3 at a half, 61.7 at a third and 65.8
-// when tested at once; a million spheres 142.9 against 144.2 at a half and
-// 143.2 when all of them do.
+// 1080p book frame 53.8 ms, 53.9 at a half and 53.6 when all of them do, a
+// million spheres 134.0, 135.6 and 133.4 (tested at once as first built 65.8
+// against 61.1 for the book frame).
 constexpr uint32_t kFlushNum = 2, kFlushDen = 3;
 constexpr uint32_t kTile = 64;        // pixels of a camera tile: one wave of camera rays
 // A unit is what a wave claims at a time: up to kUnitPasses passes of one
 // tile, fewer while the units would not go round the waves kUnitRounds times.
-// 1200x800 at 16 samples depth 4: 1680 us at 4 rounds, 1523 at 8, 1462 at 16,
-// 1508 at 32; a million spheres 145.1, 144.3, 144.1, 144.3 ms, with up to 4
-// passes 143.3, with up to 16 147.6 (1080p book frame 59.5 and 59.7 ms against
-// 59.1 with 8).
+// 1200x800 at 16 samples depth 4: 1377 us at 8 rounds, 1354 at 16, 1398 at 32;
+// a million spheres 133.9, 134.0 and 133.9 ms.  With up to 4, 8 and 16 passes a
+// million spheres 132.9, 134.0 and 136.5 ms, the 1080p book frame 54.0, 53.8 and
+// 54.2.
 constexpr uint32_t kUnitPasses = 8;
 constexpr uint32_t kUnitRounds = 16;
 // Units beyond the first ones are dealt out to up to 2^kLogCounters counters
 // (128 bytes apart), each of which serves every so-many-th workgroup alone.  One
 // counter for all waves served a unit every 12 ns and no more: 400x225 at 16
-// samples 775 us, 680 with 8 counters, 676 with 16, 672 with 32; 1200x800 at 16
-// samples depth 4 1535, 1515, 1515, 1514.
+// samples 775 us with one and 680 with 8 as first built; 656 with 8, 657 with
+// 16 and 652 with 32 now.
 constexpr uint32_t kLogCounters = 4;
 constexpr uint32_t kCounterStride = 32;
 constexpr uint32_t kCounterWords = (kCounterStride << kLogCounters) / 2;  // in 8 bytes
@@ -350,7 +350,7 @@ __global__ void __launch_bounds__(path_threads(SRC)) __attribute__((amdgpu_waves
             if constexpr (!COUNT) {
                 // flush once enough lanes hold queued tests, relative to the
                 // lanes still tracing, or before a queue could overflow (a
-                // visit queues at most 4)
+                // visit queues one entry)
                 const uint64_t pm = __ballot(tr.npend != 0u);
                 if (pm && (__ballot(tr.npend == (LDSN ? kLdsPend : kMemPend)) != 0ull ||
                            kFlushDen * (uint32_t)__popcll(pm) >= kFlushNum * (uint32_t)__popcll(busy))) {
@@ -558,7 +558,8 @@ bool fits_lds(const vzScene_st* s) { return s->n >= 2 && s->nw <= kLdsNodes && s
 
 // Tile shape of a request: the options' where it is 64 pixels of powers of
 // two, 8x8 otherwise; images less than 8 pixels high or wide get tiles of
-// their shape, so that padding never multiplies the pixels by more than 4.
+// their shape (2x2 takes a tile of 64 all the same; from a tile's pixels on
+// padding less than quadruples them).
 uint32_t tile_lw(const vzLaunchParams& p, const PathOptions& opt)
 {
     if (p.height < 8u) return 5u;
@@ -967,8 +968,8 @@ uint64_t tuning_budget(const vzTuning& t)
 // launch; an item too large for the slot renders by itself, a chunk of passes
 // at a time.  One stream: with the groups side by side on 2, 4 and 8 streams,
 // so that a group takes over the CUs another's last paths leave, a 24-scene
-// batch took 139-143 ms instead of 121 (groups that share the GPU also share
-// its caches).
+// batch took 139-143 ms when one stream took 121 (groups that share the GPU
+// also share its caches).
 vzStatus path_batch(vzContext ctx, const std::vector<PathItem>& items, const vzTuning& t, hipStream_t st, RunResult* res)
 {
     *res = RunResult();

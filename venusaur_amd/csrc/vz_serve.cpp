@@ -64,8 +64,8 @@ struct Flight {
 
 // Launches side by side: the second takes over the CUs that the first one's
 // last paths leave.  A burst of 20 requests (1k to 200k spheres, 256 to 1024
-// pixels square, 4 to 64 samples, one of 1088) takes 147.9 ms with 2 and 150.3
-// with 3 at 16M paths a launch, 143.6 and 145.4 at 32M.
+// pixels square, 4 to 64 samples, one of 1088) takes 153.6 ms with 1, 141.1 with
+// 2 and 144.2 with 3.
 constexpr uint32_t kServeStreams = 2;
 
 }  // namespace

@@ -19,7 +19,7 @@
 // and a mask of four.  12 entries and 3 visits are 87 bytes a lane, 28 waves
 // on a CU, and hardly an entry goes to private memory: the same frame 162 ms
 // with 8 entries of 8 bytes and 24 waves, 193 with 4, 148 with 14 of 6 bytes
-// and 24 waves, 143 as it is, 146 with 10 and 32 waves (64 registers).
+// and 24 waves, 143 with 12 and 28, 146 with 10 and 32 waves (64 registers).
 #pragma once
 #include "vz_traverse.h"
 
