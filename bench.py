@@ -34,10 +34,12 @@ import numpy as np  # noqa: E402
 
 METRIC = "Mray-segments/s @1080p; batched/served vs plain, p50/p99 latency, RMSE≤1e-3"
 HBM_PEAK_GBS = 8000.0
-# VALU lane throughput of MI355X for unpacked FP32/INT32 operations: 256 CUs x
-# 4 SIMDs x 16 lanes x 2.4 GHz (a wave64 instruction issues over 4 cycles);
-# the published 157.3 TFLOP/s FP32 is this x 2 (FMA) x 2 (packed pairs)
-VALU_PEAK_TLANE = 256 * 4 * 16 * 2.4e9 / 1e12
+# VALU lane throughput of MI355X: 256 CUs x 4 SIMDs x 32 lanes x 2.4 GHz.  Its
+# fastest wave64 instructions (multiply-adds, adds, moves) issue every 2 cycles,
+# measured 0.45 a cycle and SIMD; conversions, compares, min and max every 4.
+# The published 157.3 TFLOP/s FP32 is this x 2 (a multiply-add).
+VALU_CYCLES = 2
+VALU_PEAK_TLANE = 256 * 4 * (64 / VALU_CYCLES) * 2.4e9 / 1e12
 
 
 def parse():
@@ -156,9 +158,10 @@ def summarize(a):
 def summarize_sq(a):
     """Per-dispatch means of SQ counters for the kernels of --sq-map, with
     the VALU issue fraction (instructions over the issue capacity of the
-    busy cycles: 1024 SIMDs, one wave64 VALU instruction per 4 cycles, the
-    busy-cycle counter summed over 32 shader engines) and the fraction of
-    lanes active per VALU instruction."""
+    busy cycles: 1024 SIMDs, one of the fastest wave64 VALU instructions per 2
+    cycles, the busy-cycle counter summed over 32 shader engines; slower
+    instructions take twice as much of it) and the fraction of lanes active
+    per VALU instruction."""
     import csv
     import statistics
     want = dict(x.split("=", 1) for x in a.sq_map.split(";") if x.strip())
@@ -173,7 +176,7 @@ def summarize_sq(a):
     for k, key in want.items():
         v = {c: statistics.mean(x) for c, x in vals[k].items()}
         n = len(vals[k]["SQ_INSTS_VALU"])
-        issue = v["SQ_INSTS_VALU"] / (v["SQ_BUSY_CYCLES"] / 32 * 1024 / 4)
+        issue = v["SQ_INSTS_VALU"] / (v["SQ_BUSY_CYCLES"] / 32 * 1024 / VALU_CYCLES)
         lanes = v["SQ_THREAD_CYCLES_VALU"] / (64 * v["SQ_ACTIVE_INST_VALU"])
         out[key] = {"kernel": k, "dispatches": n, "insts_valu": v["SQ_INSTS_VALU"],
                     "active_inst_valu": v["SQ_ACTIVE_INST_VALU"], "thread_cycles_valu": v["SQ_THREAD_CYCLES_VALU"],
@@ -184,8 +187,8 @@ def summarize_sq(a):
     md = [f"# rocprofv3 SQ counters of the path kernels", "", "Command (run from the repository root on an MI355X):",
           "", "```", *[c.strip() for c in a.commands.split(" ;; ") if c.strip()], "```", "",
           "Means per dispatch.  VALU issue capacity of a dispatch = SQ_BUSY_CYCLES / 32 shader engines x 1024 "
-          "SIMDs / 4 cycles per wave64 VALU instruction; lanes active = SQ_THREAD_CYCLES_VALU / "
-          "(64 x SQ_ACTIVE_INST_VALU).", "", *rows]
+          "SIMDs / 2 cycles of the fastest wave64 VALU instructions (others take 4); lanes active = "
+          "SQ_THREAD_CYCLES_VALU / (64 x SQ_ACTIVE_INST_VALU).", "", *rows]
     open(a.out_md, "w").write("\n".join(md) + "\n")
     json.dump(out, open(a.out_json, "w"), indent=1)
 
