@@ -184,7 +184,7 @@ vzStatus vzTraceClosestNoAlloc(vzScene scene, const vzRay* rays, uint32_t n, vzH
                                vzStream stream, vzStats* stats);
 /* One frame: the OptiX launch of Renderer::Draw (Renderer.h:75) plus the
  * accumulation of __raygen__rg (RayTracer.cu:163-217).  Synchronises the
- * stream when stats != NULL, otherwise returns after enqueueing. */
+ * stream. */
 vzStatus vzLaunch(vzScene scene, const vzLaunchParams* params, vzStream stream, vzStats* stats);
 
 /* ---- batched form --------------------------------------------------- */

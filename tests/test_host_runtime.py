@@ -18,6 +18,7 @@ sys.path.insert(0, sys.argv[2])
 for f in ("host_hip_used", "host_hip_peak", "host_hip_log"):
     getattr(hip, f).restype = C.c_size_t
 hip.host_hip_limit.argtypes = [C.c_size_t]
+hip.host_hip_launches.argtypes = [C.c_char_p]
 FREED = C.CFUNCTYPE(None)
 hip.host_hip_on_free.argtypes = [FREED, C.c_size_t]
 import time
@@ -212,7 +213,7 @@ with Steps() as steps:
     assert [srv.poll(i) for i in large] == [None, None]
 srv.drain()
 assert all(srv.poll(i).status == 0 for i in large)
-assert hip.host_hip_launches("k_path_resolve") > 2 * 40    # in slices
+assert hip.host_hip_launches(b"k_path_resolve") > 2 * 40    # in slices
 srv.close()
 """)
 
@@ -246,4 +247,28 @@ for budget, reqs in mixes:
         assert hip.host_hip_peak() - base <= budget + TABLES, (budget, tuning, hip.host_hip_peak() - base)
         srv.close()
         assert hip.host_hip_used() <= base
+""")
+
+
+def test_server_short_of_memory_takes_smaller_launches(stand_in):
+    """A request alone on a server would take 150M paths a launch (2.4 GB).
+    Where that is not there it goes on with the usual 48M, and with less where
+    those are not; the next requests are rendered too."""
+    run(stand_in, """
+p = params(2048, 2048, 100)                       # 67 MB a pass, 67 MB carried
+for room, launches in ((200 * MB, 9), (0, 9), (-1400 * MB, 100)):
+    srv = api.Server(ctx, 8 << 30)                # two slots of 805 MB
+    hip.host_hip_limit(hip.host_hip_used() + room)
+    before = hip.host_hip_launches(b"k_path_resolve")
+    i = srv.submit(scene, p)
+    srv.drain()
+    assert srv.poll(i).status == 0, room
+    done = hip.host_hip_launches(b"k_path_resolve") - before
+    print(room, done)
+    j = [srv.submit(scene, params(64, 36, 2)) for _ in range(5)]
+    srv.drain()
+    assert [srv.poll(k).status for k in j] == [0] * 5
+    hip.host_hip_limit(1 << 60)
+    srv.close()
+    assert done == launches, (room, done)
 """)

@@ -334,10 +334,12 @@ void vzServer_st::loop()
             if (s == VZ_ERROR_OUT_OF_MEMORY) {
                 if (others_busy(f)) break;  // until one of them has finished
                 // even an idle device does not hold the launch: fewer paths at
-                // a time, down to one pass of one request
-                if (launch_paths > ready.front()->npad || alone_paths > launch_paths) {
-                    launch_paths = std::max<uint64_t>(std::min(launch_paths, alone_paths) / 2, 1);
+                // a time, down to one pass of one request, in slots of their size
+                for (Flight& o : flights) slot_drop(o.slot);
+                if (alone_paths > launch_paths) {
                     alone_paths = launch_paths;
+                } else if (launch_paths > ready.front()->npad) {
+                    alone_paths = launch_paths = launch_paths / 2;
                 } else {
                     std::lock_guard<std::mutex> lk(mu);
                     Request& r = *ready.front();
