@@ -105,3 +105,47 @@ def test_refit_lines(ctx, n):
     rays["tmin"], rays["tmax"] = 0.001, 1e16
     assert _hits(sc, rays).tobytes() == O.trace_brute(s, rays).tobytes()
     sc.close()
+
+
+# without stats the call only enqueues: captured once, replayed on other rays,
+# scenes in LDS and in memory, odd rays (a NaN limit) among them
+@pytest.mark.parametrize("kind", ["lds", "mem"])
+def test_captured_trace(ctx, book, kind):
+    print(f"case: captured hits {kind}", flush=True)
+    torch = pytest.importorskip("torch")
+    s, m = book if kind == "lds" else api.box_scene(5000, 9)
+    sc = api.Scene(ctx, s, m)
+    n = 30001
+
+    def make(seed):
+        rng = np.random.default_rng(seed)
+        r = np.zeros(n, api.RAY_DT)
+        pick = s[rng.integers(0, len(s), n)]
+        for f, c in (("ox", "cx"), ("oy", "cy"), ("oz", "cz")):
+            r[f] = rng.uniform(-30, 30, n)
+            r["d" + f[1]] = pick[c] - r[f]
+        r["tmin"], r["tmax"] = 0.001, 1e16
+        r["tmax"][::97] = np.nan
+        return r
+
+    dev = lambda a: torch.from_numpy(a.view(np.uint8).reshape(-1).copy()).cuda()  # noqa: E731
+    rays, hits = dev(make(0)), torch.zeros(n * 2, dtype=torch.int32, device="cuda")
+    api.check(api.lib().vzTraceClosestNoAlloc(sc.h, rays.data_ptr(), n, hits.data_ptr(), None, None))
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        st = torch.cuda.current_stream().cuda_stream
+        api.check(api.lib().vzTraceClosestNoAlloc(sc.h, rays.data_ptr(), n, hits.data_ptr(), st, None))
+    for seed in range(1, 5):
+        r = make(seed)
+        rays.copy_(dev(r))
+        hits.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        got = hits.cpu().numpy().view(np.uint8).view(api.HIT_DT)
+        want = O.BVH(s).trace(r)[0]
+        same_t = (got["t"].view(np.uint32) == want["t"].view(np.uint32)) | (np.isnan(got["t"]) & np.isnan(want["t"]))
+        assert same_t.all() and (got["prim"] == want["prim"]).all(), seed
+        sc2 = api.Scene(ctx, s[:100].copy(), m[:100].copy())  # eager work of the program between replays
+        sc2.close()
+    sc.close()
