@@ -259,7 +259,7 @@ vzStatus vzServerDrain(vzServer srv);
  * server's buffers and streams. */
 vzStatus vzServerDestroy(vzServer srv);
 /* Bytes of device memory a server of the default tuning takes for a request of
- * these params: 16 for each path of one slice of its samples (768 MiB at most,
+ * these params: 16 for each path of one slice of its samples (1152 MiB at most,
  * or one sample), and its sums and camera seeds, 16 or 28 a pixel, if there are
  * several slices.  Pixels count with their tiles' padding. */
 uint64_t vzRequestFootprint(const vzLaunchParams* params);

@@ -213,7 +213,7 @@ with Steps() as steps:
     assert [srv.poll(i) for i in large] == [None, None]
 srv.drain()
 assert all(srv.poll(i).status == 0 for i in large)
-assert hip.host_hip_launches(b"k_path_resolve") > 2 * 40    # in slices
+assert hip.host_hip_launches(b"k_path_resolve") > 2 * 25    # in slices
 srv.close()
 """)
 
@@ -228,12 +228,12 @@ TABLES = 2 * MB
 small = params(96, 64, 4)
 fp = lambda p: api.footprint(p)
 assert fp(small) == 96 * 64 * 4 * 16 + 256                      # seeds and radiances of its paths
-sliced = params(2048, 2048, 100, api.ACCUM_FP64)                # 9 slices of at most 12 passes
+sliced = params(2048, 2048, 100, api.ACCUM_FP64)                # 6 slices of at most 17 passes
 px = 2048 * 2048
-assert fp(sliced) == px * 12 * 16 + 256 + px * 28
+assert fp(sliced) == px * 17 * 16 + 256 + px * 28
 big = [params(2048, 2048, 7), params(1024, 1024, 64), sliced, params(512, 512, 16), params(1920, 1080, 300)]
 mixes = [(fp(small), [small] * 5), (fp(small) * 3 // 2, [small] * 5),
-         (max(map(fp, big)), big * 2 + [small] * 20), (1 << 30, big * 3), (2 << 30, big * 4), (64 << 30, big * 2)]
+         (max(map(fp, big)), big * 2 + [small] * 20), (3 << 29, big * 3), (2 << 30, big * 4), (64 << 30, big * 2)]
 for budget, reqs in mixes:
     for tuning in (None, api.Tuning(queue_capacity=1)):
         base = hip.host_hip_used()
@@ -251,20 +251,20 @@ for budget, reqs in mixes:
 
 
 def test_server_short_of_memory_takes_smaller_launches(stand_in):
-    """A request alone on a server would take 150M paths a launch (2.4 GB).
-    Where that is not there it goes on with the usual 48M, and with less where
-    those are not; the next requests are rendered too."""
+    """A request alone on a server takes up to 150M paths a launch (2.3 GB),
+    for which the two slots of 1.2 GB go.  Where that is not there it goes on
+    with the usual 72M, and with less where those are not; the next requests are
+    rendered too, also after one that not a single pass of fitted."""
     run(stand_in, """
 p = params(2048, 2048, 100)                       # 67 MB a pass, 67 MB carried
-for room, launches in ((200 * MB, 9), (0, 9), (-1400 * MB, 100)):
-    srv = api.Server(ctx, 8 << 30)                # two slots of 805 MB
+for room, launches in ((0, 3), (-600 * MB, 6), (-1400 * MB, 12), (-2150 * MB, 100), (-2200 * MB, 0)):
+    srv = api.Server(ctx, 8 << 30)
     hip.host_hip_limit(hip.host_hip_used() + room)
     before = hip.host_hip_launches(b"k_path_resolve")
     i = srv.submit(scene, p)
     srv.drain()
-    assert srv.poll(i).status == 0, room
+    assert srv.poll(i).status == (0 if launches else 2), room
     done = hip.host_hip_launches(b"k_path_resolve") - before
-    print(room, done)
     j = [srv.submit(scene, params(64, 36, 2)) for _ in range(5)]
     srv.drain()
     assert [srv.poll(k).status for k in j] == [0] * 5

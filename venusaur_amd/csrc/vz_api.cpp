@@ -550,7 +550,7 @@ vzStatus vzBatchLaunch(vzContext ctx, const vzBatchItem* items, uint32_t n, cons
 uint64_t vzRequestFootprint(const vzLaunchParams* params)
 {
     if (!params) return 0;
-    return (uint64_t)request_bytes(*params, PathOptions(), kServePaths);
+    return (uint64_t)request_bytes(*params, PathOptions(), kServeSlicePaths);
 }
 
 // ---- host helpers -------------------------------------------------------------

@@ -25,17 +25,18 @@ constexpr uint64_t kPlainBudget = 4ull << 30;
 constexpr uint64_t kMaxSlotBudget = 16ull << 30;
 constexpr uint64_t kMaxLaunchPaths = 0xFFFFFF00ull;  // a path's index has 32 bits
 
-// Paths of a server's launch at most while other requests wait; a request that
-// has the server to itself takes as many as the slot may hold, since its slices
-// follow one another and each leaves the GPU idle at its end (1080p at 512
-// samples: 474 ms in launches of 150M, 493 of 64M).  A launch's requests finish
-// together and the next in turn start after it: with 16M, 32M, 48M, 64M and 128M
-// a burst of 20 requests (vz_serve.cpp) takes 147.9, 143.6, 140.8, 139.5 and
-// 139.4 ms, 600 such requests at 0.8 of the capacity have a p50 of 102, 174, 234,
-// 292 and 489 ms, and 256x256 at 4 samples behind two frames of 1080p at 512
-// samples takes 11, 25, 24, 10 to 39 and 38 to 165 ms.  (Requests up to 150M
-// paths whole, in order of arrival: 141.2, 923 and 730 ms.)
+// Paths of a server's launch of several requests, and of a slice of one request,
+// at most.  A launch's requests finish together and the next in turn start after
+// it; each launch's end leaves part of the GPU idle.  Launches and slices of up
+// to 16M, 32M, 48M, 64M and 128M: a burst of 20 requests (vz_serve.cpp) takes
+// 147.9, 143.6, 140.8, 139.5 and 139.4 ms, 600 such requests at 0.8 of the
+// capacity have a p50 of 102, 174, 234, 292 and 489 ms, and 256x256 at 4 samples
+// behind two 1080p frames at 512 samples takes 11, 25, 24, 10 to 39 and 38 to 165
+// ms.  With 48M and 72M 139.6, 287 and 12 to 79, and bursts of 2 to 5 requests,
+// one of 71M paths, take 2 to 4% less than with 48M for both.  (Requests up to
+// 150M paths whole, in order of arrival: 141.2, 923 and 724 ms.)
 constexpr uint64_t kServePaths = 48u << 20;
+constexpr uint64_t kServeSlicePaths = kServePaths + kServePaths / 2;
 
 struct PathReq {               // one request of a launch, read by scalar loads
     Cam cam;

@@ -75,8 +75,14 @@ struct vzServer_st {
     vzServeConfig cfg{};
     PathWork* work = nullptr;
     PathOptions opt;
-    uint64_t request_paths = kServePaths;  // of a slice, by the tuning
-    uint64_t launch_paths = kServePaths, alone_paths = kServePaths;  // lower where memory is short (the worker's)
+    uint64_t footprint_slice = kServeSlicePaths;  // by the tuning
+    // paths of a launch of several requests, of a slice, and of a slice of a
+    // request that has the server to itself: its slices follow one another, so
+    // it takes as many as the tuning's memory holds (1080p at 512 samples: 474
+    // ms in launches of 150M, 493 of 64M).  Lower where memory is short (the
+    // worker's)
+    uint64_t launch_paths = kServePaths, slice_paths = kServeSlicePaths, alone_paths = kServeSlicePaths;
+    bool trimmed = false;              // idle slots have made room for the next launch (the worker's)
     std::vector<Flight> flights;
     std::thread worker;
     std::mutex mu;
@@ -99,7 +105,7 @@ struct vzServer_st {
     }
     void loop();
     void admit();
-    uint64_t pick(Flight& f, uint64_t most);
+    uint64_t pick(Flight& f, uint64_t most, uint64_t slice);
     bool make_room(Flight& f, size_t slot, size_t carry);
     void free_carry(Request& r, hipStream_t st)
     {
@@ -176,9 +182,9 @@ void vzServer_st::admit()
 }
 
 // The requests next in turn, as many as a launch of `most` paths takes; returns
-// their paths.  A request it does not take whole has a launch to itself, of
-// one of as few equal slices as there can be.
-uint64_t vzServer_st::pick(Flight& f, uint64_t most)
+// their paths.  A request of more has a launch to itself, whole or, above `slice`
+// paths, one of as few equal slices as there can be.
+uint64_t vzServer_st::pick(Flight& f, uint64_t most, uint64_t slice)
 {
     uint64_t paths = 0;
     while (!ready.empty() && f.shares.size() < kMaxRequests) {
@@ -187,7 +193,7 @@ uint64_t vzServer_st::pick(Flight& f, uint64_t most)
         uint64_t take = left;
         if (paths + r.npad * left > most) {
             if (!f.shares.empty()) break;
-            take = slice_passes(left, r.npad, most);
+            take = slice_passes(left, r.npad, slice);
         }
         paths += r.npad * take;
         f.shares.push_back(Share{std::move(ready.front()), r.done, (uint32_t)take});
@@ -237,7 +243,7 @@ vzStatus vzServer_st::start(Flight& f)
     size_t carry = 0;
     vzStatus rs = VZ_SUCCESS;
     for (;;) {
-        paths = pick(f, alone ? std::max(alone_paths, launch_paths) : launch_paths);
+        paths = alone ? pick(f, alone_paths, alone_paths) : pick(f, launch_paths, slice_paths);
         const Share& s = f.shares.front();
         carry = !s.r->carry && s.ns < s.r->item.params.samples_per_pixel ? carry_bytes(s.r->item.params, s.r->npad) : 0;
         if (make_room(f, slot_bytes(paths), carry)) break;
@@ -333,13 +339,17 @@ void vzServer_st::loop()
             const vzStatus s = start(f);
             if (s == VZ_ERROR_OUT_OF_MEMORY) {
                 if (others_busy(f)) break;  // until one of them has finished
-                // even an idle device does not hold the launch: fewer paths at
-                // a time, down to one pass of one request, in slots of their size
+                // even an idle device does not hold the launch beside the slots:
+                // without them, then fewer paths at a time, down to one pass of
+                // one request
                 for (Flight& o : flights) slot_drop(o.slot);
-                if (alone_paths > launch_paths) {
-                    alone_paths = launch_paths;
-                } else if (launch_paths > ready.front()->npad) {
-                    alone_paths = launch_paths = launch_paths / 2;
+                if (!trimmed) {
+                    trimmed = true;
+                } else if (alone_paths > slice_paths) {
+                    alone_paths = slice_paths;
+                } else if (slice_paths > ready.front()->npad) {
+                    launch_paths = std::max<uint64_t>(launch_paths / 2, 1);
+                    alone_paths = slice_paths = slice_paths / 2;
                 } else {
                     std::lock_guard<std::mutex> lk(mu);
                     Request& r = *ready.front();
@@ -357,6 +367,7 @@ void vzServer_st::loop()
                 fail(s);
                 goto out;
             }
+            trimmed = false;
             progress = busy = true;
         }
         if (progress) continue;
@@ -395,11 +406,12 @@ vzStatus vzServerCreate(vzContext ctx, const vzServeConfig* cfg, vzServer* out)
     s->opt.refill = std::min<uint32_t>(t.refill_lanes, 65u);  // 0: the kernel variant's default
     const uint32_t n = std::min<uint32_t>(kServeStreams, s->cfg.max_active);
     const uint64_t slot_paths = std::max<uint64_t>(tuning_budget(t) / kServeStreams / kPathBytes, 1);
-    s->request_paths = s->launch_paths = std::min(kServePaths, slot_paths);
+    s->launch_paths = std::min(kServePaths, slot_paths);
+    s->footprint_slice = s->slice_paths = std::min(kServeSlicePaths, slot_paths);
     s->alone_paths = slot_paths;
     // what a flight starts with; larger ones as launches need them
     const uint64_t share = s->cfg.hbm_budget_bytes / kServeStreams;
-    const uint64_t first = std::min(s->launch_paths, share > slot_bytes(0) ? (share - slot_bytes(0)) / kPathBytes : 0);
+    const uint64_t first = std::min(s->slice_paths, share > slot_bytes(0) ? (share - slot_bytes(0)) / kPathBytes : 0);
     vzStatus rs;
     {
         std::lock_guard<std::mutex> lk(ctx->mu);
@@ -436,7 +448,7 @@ vzStatus vzServerSubmit(vzServer srv, vzScene scene, const vzLaunchParams* param
     p->id = srv->next_id++;
     p->item = PathItem{scene, *params};
     scene->server_refs.fetch_add(1);  // vzSceneDestroy refuses until the request is done
-    p->bytes = request_bytes(*params, srv->opt, srv->request_paths);
+    p->bytes = request_bytes(*params, srv->opt, srv->footprint_slice);
     p->npad = padded_pixels(*params, srv->opt);
     p->submit_ms = srv->now_ms();
     *request_id = p->id;
